@@ -671,6 +671,41 @@ def test_attention_does_not_depend_on_the_batch(K):
     assert torch.equal(out_a.cpu()[0], out_b.cpu()[0])
 
 
+SAMPLE_ROWS = {   # name -> (row of logits, settings (temperature, top_k, top_p))
+    "ties beyond the list": (lambda V, g: (torch.randn(V, generator=g) * 2).round(), [(1.0, 0, 0.7), (0.7, 3000, 1.0), (1.3, 50, 0.5)]),
+    "all equal": (lambda V, g: torch.full((V,), 1.5), [(1.0, 0, 0.5), (1.0, 7, 0.9)]),
+    "mostly masked": (lambda V, g: torch.where(torch.rand(V, generator=g) < 0.9, -math.inf, torch.randn(V, generator=g)), [(1.0, 0, 0.9), (0.8, 40, 0.9)]),
+    "masked to the lowest number": (lambda V, g: torch.where(torch.rand(V, generator=g) < 0.999, -3.4028234663852886e38, torch.randn(V, generator=g)),
+                                    [(1.0, 0, 0.9), (1.0, 5000, 1.0)]),
+    "k in the last bin": (lambda V, g: torch.randn(V, generator=g) * 4, [(0.05, 60, 1.0), (0.05, 2500, 1.0), (0.02, 0, 0.999)]),
+    "k beyond the list": (lambda V, g: torch.randn(V, generator=g), [(1.0, 2048, 1.0), (1.0, 2049, 0.95), (1.0, 6000, 0.9), (5.0, 0, 0.99)]),
+}
+
+
+@pytest.mark.parametrize("V", [1, 3, 255, 2049, 16385, 122753, 300001])
+@pytest.mark.parametrize("name", list(SAMPLE_ROWS))
+def test_sampling_where_thresholds_are_hard(K, name, V):
+    """Every way to a threshold (list, radix, last bin) and to a token (list, tiles), rows that begin at any alignment, against the
+    plain distribution.  A token's interval is met within 1e-5: the plain masses are float64, the kernel's exponentials float32
+    (a few 2^-24 each, and 2^-43 a mass); ties and masked entries are exact."""
+    make, settings = SAMPLE_ROWS[name]
+    g = torch.Generator().manual_seed(V)
+    row = make(V, g)
+    row[0] = max(float(row[0]), 0.5)     # (one entry at least is not masked)
+    us = [0.0, 1e-4, 0.13, 0.5, 0.77, 0.99, 1.0 - 2.0 ** -24]
+    n = len(us)
+    for temp, k, p in settings:
+        mk = lambda v, dt: torch.tensor(v, dtype=dt, device=DEV)
+        rows = row.expand(n, V).contiguous().to(DEV)
+        got = K.sample(rows, mk([temp] * n, torch.float32), mk([k] * n, torch.int32), mk([p] * n, torch.float32), mk(us, torch.float32)).tolist()
+        dist = P.plain_sample_distribution(row, temp, k, p)
+        cdf = torch.cumsum(dist, 0)
+        for u, tok in zip(us, got):
+            assert 0 <= tok < V and dist[tok] > 0, f"token {tok} is outside the kept set (T={temp}, k={k}, p={p})"
+            lo, hi = float(cdf[tok] - dist[tok]), float(cdf[tok])
+            assert lo - 1e-5 <= u <= hi + 1e-5, f"u={u} not in token {tok}'s interval [{lo}, {hi}] (T={temp}, k={k}, p={p})"
+
+
 def test_argmax_and_sampling(K):
     V = 73448
     logits = _rand((5, V), 20, scale=3.0)

@@ -306,3 +306,12 @@ def test_sampling_distribution_and_inverse_cdf():
     assert P.plain_sample(l, 1.0, 0, 0.5, 0.49) == 3
     assert P.plain_sample(l, 1.0, 0, 0.5, 0.51) == 5
     assert P.plain_sample(l, 1.0, 0, 0.5, 0.999999) == 5
+
+
+def test_uniform_numbers_of_many_rows_are_those_of_each():
+    from infinilm_amd.sampling.sampler import uniform_for, uniforms_for
+
+    rows = [(s, k, i) for s in (0, 7, -1, 1 << 63, (1 << 70) + 3) for k in (0, -5, 1 << 64, 123456789) for i in (0, 1, 1 << 31)]
+    for n in (1, 23, 24, len(rows)):
+        got = uniforms_for(*zip(*rows[:n]))
+        assert got.tolist() == [uniform_for(*r) for r in rows[:n]]     # (24 bits: a float32 holds them)
