@@ -1,55 +1,64 @@
-// C[M,N] = alpha * (X[M,K] W[N,K]^T + bias) in true 32-bit for few rows of X (M <= 64): the
-// projections of a decode step on the 32-bit path, bound by reading W once.
+// C[M,N] = alpha * (X[M,K] W[N,K]^T + bias) in 32-bit for few rows of X (M <= 64): the projections of a decode step
+// on the 32-bit path, bound by reading W once.
 //
-// v_mfma_f32_16x16x4_f32 (IEEE float products and sums, no reduced-precision mode) with W rows on the
-// A side and tokens on the B side.  A lane loads 16 bytes (4 consecutive k) of its W row and of its
-// token's X row and feeds them to four matrix instructions, one per element: instruction j
-// reduces over the k values {4 q + j}.  The waves of a workgroup split K into contiguous slices;
-// their partial tiles are summed through LDS in wave order.  The order of an output's sum depends on
-// K alone (the eight slices, the 16-wide steps inside them, the four instructions of a step), not on
-// M, on the batch or on the place of the row in it: rows of any two calls of this kernel agree bit
-// for bit.  It is not the ascending-k order of the many-rows kernel (gemm_basic.hip), from which a
-// result differs by rounding.
+// The products run on the bfloat16 matrix cores in three pieces a float (f32_split.h), W rows on the A side and tokens on
+// the B side.  The eight waves of a workgroup take the eight slices of K and keep DEPTH steps of loads in flight; a load
+// instruction takes eight rows' whole 128-byte lines (32 k).  Lanes that gather a fragment from 16 rows, as this kernel had
+// it, are taken in at 31 GB/s a compute unit whatever the source, X as slowly as W.  A wave cuts what has arrived into pieces and
+// turns it into fragments through LDS of its own: no barrier until the partial tiles meet, in wave order.
+// Eight rows, before and after: 6912 x 2304 19.8 -> 14.3 us (4.5 TB/s), 2304 x 5760 23.3 -> 17.7, 122753 x 2304 266 -> 195,
+// 32768 x 4096 111 -> 91 (5.9 TB/s); 64 rows 58 -> 28, 69 -> 43, 852 -> 412 and 346 -> 174.
 // K must be a multiple of 4 and rows 16-byte aligned.
-#include "common.h"
+#include "f32_split.h"
 
-typedef __attribute__((ext_vector_type(4))) float f32x4;
+#define FS_WAVES F3_SLICES
 
-#define FS_UNROLL 4   // 16-wide k-steps whose loads are in flight together, twice over
-
-__device__ __forceinline__ f32x4 fs_mfma(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-#define FS_WAVES 8   // the same for every shape: it fixes the order of the sums
-
-// MG: groups of 16 rows of X; RT: tiles of 16 W rows a workgroup
-template <int MG, int RT>
-__global__ void __launch_bounds__(FS_WAVES * 64)
+// XG: groups of 8 rows of X; RT: tiles of 16 W rows a workgroup; DEPTH: steps of 32 k in flight
+template <int XG, int RT, int DEPTH>
+__global__ void __launch_bounds__(FS_WAVES * 64, XG <= 2 ? 4 : 2)
 gemm_f32_skinny_kernel(float* __restrict__ C, const float* __restrict__ X, const float* __restrict__ W,
                        const float* __restrict__ bias, int M, int N, int K, int lda, int ldw, int ldc, float alpha) {
-    __shared__ float part[FS_WAVES][RT][MG][64][4];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r = lane & 15, q = lane >> 4;
+    constexpr int MG = (XG + 1) / 2;
+    struct Frags {
+        uint4 at[RT + MG][3][64];   // [tile of W, then group of X][piece][slot]
+    };
+    union Lds {
+        Frags frag[FS_WAVES];
+        float part[FS_WAVES][RT][MG][64][4];
+    };
+    __shared__ Lds lds;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int r = lane & 15, q = lane >> 4;       // place in a fragment
+    const int lrow = lane >> 3, lk4 = lane & 7;   // place in a load: row, 16-byte piece of its line
     const int n0 = blockIdx.x * (16 * RT);
-    const int steps_total = (K + 15) >> 4;
-    const int per = (steps_total + FS_WAVES - 1) / FS_WAVES;
+    const int steps_total = (K + F3_STEP - 1) / F3_STEP;
+    const int per = (steps_total + F3_SLICES - 1) / F3_SLICES;
     const int s0 = wave * per;
     const int s1 = (s0 + per < steps_total) ? s0 + per : steps_total;
     const int k4_last = (K >> 2) - 1;   // last valid group of 4 elements of a row
 
-    const float4* wp[RT];
+    const float4* wp[2 * RT];
 #pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        const int row = (n0 + t * 16 + r < N) ? n0 + t * 16 + r : N - 1;
-        wp[t] = reinterpret_cast<const float4*>(W + (size_t)row * ldw);
+    for (int i = 0; i < 2 * RT; ++i) {
+        const int row = n0 + 8 * i + lrow;
+        wp[i] = reinterpret_cast<const float4*>(W + (size_t)(row < N ? row : N - 1) * ldw);
     }
-    const float4* xp[MG];
-    bool xok[MG];
+    const float4* xp[XG];
+    bool xok[XG];
 #pragma unroll
-    for (int g = 0; g < MG; ++g) {
-        xok[g] = g * 16 + r < M;
-        xp[g] = reinterpret_cast<const float4*>(X + (size_t)(xok[g] ? g * 16 + r : 0) * lda);
+    for (int i = 0; i < XG; ++i) {
+        const int row = 8 * i + lrow;
+        xok[i] = row < M;
+        xp[i] = reinterpret_cast<const float4*>(X + (size_t)(xok[i] ? row : M - 1) * lda);
+    }
+    Frags& mine = lds.frag[wave];
+    const int get = f3_slot(r, q);
+    int put[2];   // in 8 bytes: rows 0 .. 7 and 8 .. 15 of a group
+#pragma unroll
+    for (int h = 0; h < 2; ++h) put[h] = f3_slot(lrow + 8 * h, lk4 & 3) * 2 + (lk4 >> 2);
+    if (XG & 1) {   // the last group's rows 8 .. 15 hold nothing
+#pragma unroll
+        for (int p = 0; p < 3; ++p) reinterpret_cast<uint2*>(&mine.at[RT + MG - 1][p][0])[put[1]] = make_uint2(0u, 0u);
     }
     f32x4 acc[RT][MG];
 #pragma unroll
@@ -57,50 +66,69 @@ gemm_f32_skinny_kernel(float* __restrict__ C, const float* __restrict__ X, const
 #pragma unroll
         for (int g = 0; g < MG; ++g) acc[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Unconditional 16-byte loads from clamped addresses; what lies beyond K, beyond the wave's slice or
-    // beyond M is replaced by zeros on the X side.  The chunk after the one being multiplied is on its way.
+    // Unconditional 16-byte loads from clamped addresses, the steps after the slice's end those of its last one again; what
+    // lies beyond K, beyond the slice or beyond M is replaced by zeros on the X side.
+    float4 a[DEPTH][2 * RT], b[DEPTH][XG];
+    auto load = [&](int i, int s) {
+        const int k4 = 8 * (s < s1 ? s : s1 - 1) + lk4, k4c = k4 < k4_last ? k4 : k4_last;
+#pragma unroll
+        for (int t = 0; t < 2 * RT; ++t) a[i][t] = wp[t][k4c];
+#pragma unroll
+        for (int g = 0; g < XG; ++g) b[i][g] = xp[g][k4c];
+    };
+    auto cut = [&](int at, int h, const float4& v) {
+        const F3Pair c = f3_split2(v.x, v.y), d = f3_split2(v.z, v.w);
+        uint2* to = reinterpret_cast<uint2*>(&mine.at[at][0][0]) + put[h];
+        to[0] = make_uint2(c.h, d.h);
+        to[128] = make_uint2(c.m, d.m);
+        to[256] = make_uint2(c.l, d.l);
+    };
+    auto frag = [&](int at) { return F3Frag{mine.at[at][0][get], mine.at[at][1][get], mine.at[at][2][get]}; };
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 a[2][FS_UNROLL][RT];
-    float4 b[2][FS_UNROLL][MG];
-#define FS_LOAD(BUF_, S_)                                                          \
-    _Pragma("unroll") for (int u = 0; u < FS_UNROLL; ++u) {                        \
-        const int k4 = ((S_) + u) * 4 + q;                                         \
-        const int k4c = k4 < k4_last ? k4 : k4_last;                               \
-        _Pragma("unroll") for (int t = 0; t < RT; ++t) a[BUF_][u][t] = wp[t][k4c]; \
-        _Pragma("unroll") for (int g = 0; g < MG; ++g) b[BUF_][u][g] = xp[g][k4c]; \
+    if (s0 < s1) {
+#pragma unroll
+        for (int i = 0; i < DEPTH; ++i) {   // (in the loop's order: the waits count loads, and take the worse of two orders)
+            load(i, s0 + i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        auto step = [&](int i, int s, bool more) {
+            const bool live = 8 * s + lk4 <= k4_last;
+#pragma unroll
+            for (int t = 0; t < 2 * RT; ++t) cut(t >> 1, t & 1, a[i][t]);
+#pragma unroll
+            for (int g = 0; g < XG; ++g) cut(RT + (g >> 1), g & 1, live && xok[g] ? b[i][g] : zero);
+            if (more) load(i, s + DEPTH);
+            // the wave's own writes before its reads: LDS serves a wave in order, the compiler keeps the order here
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            F3Frag w[RT];
+#pragma unroll
+            for (int t = 0; t < RT; ++t) w[t] = frag(t);
+#pragma unroll
+            for (int g = 0; g < MG; ++g) {
+                const F3Frag x = frag(RT + g);
+                f3_step(w, x, acc, 0, g);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int s = s0;
+        for (; s + DEPTH < s1; s += DEPTH) {
+#pragma unroll
+            for (int i = 0; i < DEPTH; ++i) step(i, s + i, true);
+        }
+#pragma unroll
+        for (int i = 0; i < DEPTH; ++i)
+            if (s + i < s1) step(i, s + i, false);
     }
-#define FS_MUL(BUF_, S_)                                                           \
-    _Pragma("unroll") for (int u = 0; u < FS_UNROLL; ++u) {                        \
-        const int k4 = ((S_) + u) * 4 + q;                                         \
-        const bool ok = ((S_) + u < s1) && (k4 <= k4_last);                        \
-        _Pragma("unroll") for (int g = 0; g < MG; ++g) {                           \
-            const float4 xv = (ok && xok[g]) ? b[BUF_][u][g] : zero;               \
-            _Pragma("unroll") for (int t = 0; t < RT; ++t) {                       \
-                const float4 wv = a[BUF_][u][t];                                   \
-                acc[t][g] = fs_mfma(wv.x, xv.x, acc[t][g]);                        \
-                acc[t][g] = fs_mfma(wv.y, xv.y, acc[t][g]);                        \
-                acc[t][g] = fs_mfma(wv.z, xv.z, acc[t][g]);                        \
-                acc[t][g] = fs_mfma(wv.w, xv.w, acc[t][g]);                        \
-            }                                                                      \
-        }                                                                          \
-    }
-    if (s0 < s1) FS_LOAD(0, s0)
-    for (int s = s0; s < s1; s += 2 * FS_UNROLL) {
-        if (s + FS_UNROLL < s1) FS_LOAD(1, s + FS_UNROLL)
-        __builtin_amdgcn_sched_barrier(0);
-        FS_MUL(0, s)
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + 2 * FS_UNROLL < s1) FS_LOAD(0, s + 2 * FS_UNROLL)
-        __builtin_amdgcn_sched_barrier(0);
-        if (s + FS_UNROLL < s1) FS_MUL(1, s + FS_UNROLL)
-        __builtin_amdgcn_sched_barrier(0);
-    }
-#undef FS_LOAD
-#undef FS_MUL
+    __syncthreads();   // (the partial tiles lie where the fragments lay)
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int g = 0; g < MG; ++g) *reinterpret_cast<f32x4*>(&part[wave][t][g][lane][0]) = acc[t][g];
+        for (int g = 0; g < MG; ++g) *reinterpret_cast<f32x4*>(&lds.part[wave][t][g][lane][0]) = acc[t][g];
     __syncthreads();
     // acc[t][g][e] of lane (r, q) is output row n0 + t*16 + q*4 + e for token g*16 + r
     for (int idx = threadIdx.x; idx < RT * MG * 64 * 4; idx += FS_WAVES * 64) {
@@ -108,7 +136,7 @@ gemm_f32_skinny_kernel(float* __restrict__ C, const float* __restrict__ X, const
         const int t = tg / MG, g = tg % MG;
         float v = 0.f;
 #pragma unroll
-        for (int w = 0; w < FS_WAVES; ++w) v += part[w][t][g][l][e];
+        for (int w = 0; w < FS_WAVES; ++w) v += lds.part[w][t][g][l][e];
         const int n = n0 + t * 16 + (l >> 4) * 4 + e;
         const int m = g * 16 + (l & 15);
         if (n < N && m < M) {
@@ -124,17 +152,28 @@ extern "C" int ilm_gemm_f32_skinny(void* C, const void* X, const void* W, const 
     ILM_REQUIRE(K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && lda >= K && ldw >= K && ldc >= N,
                 "gemm_f32_skinny: K=%d lda=%d ldw=%d ldc=%d", K, lda, ldw, ldc);
     ILM_REQUIRE(((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0, "gemm_f32_skinny: operands must be 16-byte aligned");
-    const int mg = (M + 15) / 16;
-#define FS_CASE(MG_, RT_)                                                                                       \
-    gemm_f32_skinny_kernel<MG_, RT_><<<(N + 16 * RT_ - 1) / (16 * RT_), FS_WAVES * 64, 0, stream>>>(            \
+#define FS_CASE(XG_, RT_, DEPTH_)                                                                               \
+    gemm_f32_skinny_kernel<XG_, RT_, DEPTH_><<<(N + 16 * RT_ - 1) / (16 * RT_), FS_WAVES * 64, 0, stream>>>(    \
         (float*)C, (const float*)X, (const float*)W, (const float*)bias, M, N, K, lda, ldw, ldc, alpha)
-    // two tiles a workgroup where W is tall enough to still fill the chip: an X fragment read once serves both
-    const bool tall = N >= 16384;
-    switch (mg) {
-        case 1: if (tall) FS_CASE(1, 2); else FS_CASE(1, 1); break;
-        case 2: if (tall) FS_CASE(2, 2); else FS_CASE(2, 1); break;
-        case 3: FS_CASE(3, 1); break;
-        default: FS_CASE(4, 1); break;
+    // Two tiles a workgroup, for which X is read and cut once, where one a workgroup would be more than one a compute unit
+    // (M 8, K 2304: 14.3 us against 16.7 at N 6912, 11.6 against 9.6 at N 2304; K 4096: 18.5 against 15.9 at N 4096).  Not where
+    // X is eight rows and K long: the deeper pipeline of one tile counts more (N 32768, K 4096: 100.6 against 91.2 us).
+    const bool tall = N > 16 * ilm_num_cus() && (M > 8 || N < 16384 || K < 4096);
+    if (M <= 8) {
+        if (tall) FS_CASE(1, 2, 3);
+        else FS_CASE(1, 1, 6);
+    } else if (M <= 16) {
+        if (tall) FS_CASE(2, 2, 2);
+        else FS_CASE(2, 1, 4);
+    } else if (M <= 32) {
+        if (tall) FS_CASE(4, 2, 3);
+        else FS_CASE(4, 1, 4);
+    } else if (M <= 48) {
+        if (tall) FS_CASE(6, 2, 2);
+        else FS_CASE(6, 1, 2);
+    } else {
+        if (tall) FS_CASE(8, 2, 2);
+        else FS_CASE(8, 1, 2);
     }
 #undef FS_CASE
     ILM_LAUNCH_CHECK("gemm_f32_skinny");

@@ -399,18 +399,18 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, 
         with _timed("library_gemm"):
             torch.matmul(a, w.t(), out=out)
         return out
-    if (a.dtype == F32 and out_dtype == F32 and not FORCE_BASIC and M <= F32_FEW_ROWS and K % 4 == 0 and a.stride(0) % 4 == 0
-            and w.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
-        # the 32-bit path's few rows (decoded tokens): W streamed once on the float matrix instruction
+    pieces = (a.dtype == F32 and out_dtype == F32 and not FORCE_BASIC and K % 4 == 0 and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0
+              and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and max(a.stride(0), w.stride(0)) < 1 << 24)
+    if pieces and M <= F32_FEW_ROWS:
+        # the 32-bit path's few rows (decoded tokens): W streamed once, products in three pieces a float
         _run("ilm_gemm_f32_skinny", out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K, a.stride(0),
              w.stride(0), out.stride(0), float(alpha), _stream())
         return out
-    if (a.dtype == F32 and out_dtype == F32 and not FORCE_BASIC and F32_FEW_ROWS > 0 and K % 4 == 0 and a.stride(0) % 4 == 0
-            and w.stride(0) % 4 == 0 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
-        # the 32-bit path's many rows (portions of prompts): tiles on the float matrix instruction, every
+    if pieces and F32_FEW_ROWS > 0:
+        # the 32-bit path's many rows (portions of prompts): tiles on the same products, every
         # output summed in the few-rows kernel's order, so a row's bits do not depend on the rows around it
         _run("ilm_gemm_f32_tile", out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K, a.stride(0),
-             w.stride(0), out.stride(0), float(alpha), _stream())
+             w.stride(0), out.stride(0), float(alpha), 0, _stream())
         return out
     _run("ilm_gemm_basic", out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K, a.stride(0), w.stride(0),
          out.stride(0), float(alpha), _dt(a), _DT[out_dtype], _stream())

@@ -222,6 +222,32 @@ def test_gemm_float32_is_true_float32(K, M, N, K_):
     assert torch.equal(more[:M].cpu(), out.cpu())
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 15, 4), (8, 4097, 36), (9, 33, 1028), (17, 16385, 68), (40, 260, 260), (64, 257, 4096), (65, 63, 8),
+                                    (127, 129, 2052), (129, 257, 1024), (192, 4100, 516), (333, 640, 8192)])
+def test_gemm_float32_in_pieces(K, M, N, K_):
+    """The products in three bfloat16 pieces a float, at the edges of their tiles, rows and slices: every tile gives the same bits, and
+    the error against float64 stays below that of sums of floats rounded every four k, 2.1e-7 sqrt(K / 1024) of the norm
+    (measured with the float matrix instruction at K 1024, 4096 and 16,384), here with operands over six decades and
+    with the largest numbers of the type."""
+    from infinilm_amd.csrc import lib
+    g = torch.Generator().manual_seed(M * 7 + N)
+    a, w = torch.randn((M, K_), generator=g), torch.randn((N, K_), generator=g)
+    a *= torch.exp(1.5 * torch.randn((M, K_), generator=g))
+    a[0] *= 1e30
+    a[M // 2, K_ - 1] = 3.4028234663852886e38
+    w[:, K_ - 1] *= 1e-30
+    ad, wd = a.to(DEV), w.to(DEV)
+    out = K.gemm(ad, wd)
+    want = ad.to(F64) @ wd.to(F64).T
+    rel = ((out.to(F64) - want).norm(dim=1) / want.norm(dim=1)).max()
+    assert float(rel) < 2.1e-7 * math.sqrt(max(K_, 1024) / 1024)
+    for tile in (1, 2, 3):
+        c = torch.full_like(out, float("nan"))
+        assert lib.load().ilm_gemm_f32_tile(c.data_ptr(), ad.data_ptr(), wd.data_ptr(), None, M, N, K_, K_, K_, N, 1.0, tile,
+                                            torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(c, out), f"tile {tile}"
+
+
 @pytest.mark.parametrize("M,N,K_,out_dtype", [
     (1, 16, 32, torch.bfloat16), (1, 4608, 4096, torch.bfloat16), (8, 331, 80, torch.float32), (17, 96, 200, torch.bfloat16),
     (33, 200, 96, torch.bfloat16), (64, 73448, 128, torch.float32), (48, 100, 2048, torch.bfloat16),
