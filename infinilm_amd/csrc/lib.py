@@ -50,7 +50,7 @@ _SIGNATURES = {
     "ilm_attn_mfma_static": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P],
     "ilm_attn_tile": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _F, _I, _P],
     "ilm_argmax": [_P, _P, _I, _I, _I, _P],
-    "ilm_sample": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+    "ilm_sample": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
     "ilm_unary": [_P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "ilm_lin_prep": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "ilm_decay_scan": [_P, _I, _P, _P, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _I, _P],
@@ -142,6 +142,8 @@ def load(verbose: bool = True) -> ctypes.CDLL:
     lib.ilm_mlstm_chunk_ws.argtypes = [c_int, c_int, c_int]
     lib.ilm_delta_chunk_ws.restype = c_int
     lib.ilm_delta_chunk_ws.argtypes = [c_int, c_int]
+    lib.ilm_sample_ws.restype = c_long
+    lib.ilm_sample_ws.argtypes = [c_int, c_int]
     lib.ilm_attn_static_init.restype = c_int
     lib.ilm_attn_static_init.argtypes = []
     lib.ilm_attn_static_scratch_floats.restype = c_long

@@ -823,8 +823,10 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
     if top_k.numel() != n:
         raise KernelError("top_k must have one entry a row")
     out = torch.empty((n,), dtype=torch.int32, device=logits.device)
+    per_row = _lib().ilm_sample_ws(n, V)
+    ws = torch.empty((n * per_row,), dtype=torch.uint8, device=logits.device) if per_row else None
     _run("ilm_sample", out.data_ptr(), logits.data_ptr(), temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(),
-         uniform.data_ptr(), n, V, logits.stride(0), _stream())
+         uniform.data_ptr(), _ptr(ws), n, V, logits.stride(0), _stream())
     return out
 
 

@@ -34,20 +34,31 @@ def uniform_for(seed: int, request_key: int, index: int) -> float:
     return (x >> 40) / float(1 << 24)
 
 
+def _words(values: Sequence[int]) -> np.ndarray:
+    try:
+        return np.array(values, dtype=np.uint64)
+    except (OverflowError, ValueError, TypeError):     # negative, or of more than 64 bits
+        return np.array([v & _MASK for v in values], dtype=np.uint64)
+
+
 def uniforms_for(seeds: Sequence[int], request_keys: Sequence[int], indices: Sequence[int]) -> np.ndarray:
-    """`uniform_for` of every row.  From 24 rows on all at once, in whole numbers of 64 bits that wrap: 42 us for 64 rows
-    against 89 one by one (1.4 us a row; the arrays' own cost is that of 20 rows)."""
+    """`uniform_for` of every row.  From 24 rows on all at once, in whole numbers of 64 bits that wrap: 23 us for 64 rows
+    against 89 one by one (1.4 us a row)."""
     if len(seeds) < 24:
         return np.array([uniform_for(*row) for row in zip(seeds, request_keys, indices)], dtype=np.float32)
 
     def mix(x):
         x = x + np.uint64(0x9E3779B97F4A7C15)
-        x = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
-        x = (x ^ (x >> np.uint64(27))) * np.uint64(0x94D2049BB133111B)
-        return x ^ (x >> np.uint64(31))
+        x ^= x >> np.uint64(30)
+        x *= np.uint64(0xBF58476D1CE4E5B9)
+        x ^= x >> np.uint64(27)
+        x *= np.uint64(0x94D2049BB133111B)
+        x ^= x >> np.uint64(31)
+        return x
 
-    seeds, keys, indices = (np.array([v & _MASK for v in vs], dtype=np.uint64) for vs in (seeds, request_keys, indices))
-    x = mix(mix(mix(seeds) ^ keys) ^ indices)
+    one = len(set(seeds)) == 1      # the engine's own seed, as a rule
+    seeds = np.uint64(_mix(seeds[0] & _MASK)) if one else mix(_words(seeds))
+    x = mix(mix(seeds ^ _words(request_keys)) ^ _words(indices))
     return (x >> np.uint64(40)).astype(np.float32) / np.float32(1 << 24)
 
 

@@ -714,6 +714,7 @@ def test_sampling_where_thresholds_are_hard(K, name, V):
     """Every way to a threshold (list, radix, last bin) and to a token (list, tiles), rows that begin at any alignment, against the
     plain distribution.  A token's interval is met within 1e-5: the plain masses are float64, the kernel's exponentials float32
     (a few 2^-24 each, and 2^-43 a mass); ties and masked entries are exact."""
+    from infinilm_amd.csrc import lib
     make, settings = SAMPLE_ROWS[name]
     g = torch.Generator().manual_seed(V)
     row = make(V, g)
@@ -723,7 +724,12 @@ def test_sampling_where_thresholds_are_hard(K, name, V):
     for temp, k, p in settings:
         mk = lambda v, dt: torch.tensor(v, dtype=dt, device=DEV)
         rows = row.expand(n, V).contiguous().to(DEV)
-        got = K.sample(rows, mk([temp] * n, torch.float32), mk([k] * n, torch.int32), mk([p] * n, torch.float32), mk(us, torch.float32)).tolist()
+        rest = mk([temp] * n, torch.float32), mk([k] * n, torch.int32), mk([p] * n, torch.float32), mk(us, torch.float32)
+        got = K.sample(rows, *rest).tolist()
+        alone = torch.full((n,), -1, dtype=torch.int32, device=DEV)     # the same rows by one workgroup each, as many rows are
+        assert lib.load().ilm_sample(alone.data_ptr(), rows.data_ptr(), *(t.data_ptr() for t in rest), None, n, V, V,
+                                     torch.cuda.current_stream().cuda_stream) == 0
+        assert alone.tolist() == got
         dist = P.plain_sample_distribution(row, temp, k, p)
         cdf = torch.cumsum(dist, 0)
         for u, tok in zip(us, got):

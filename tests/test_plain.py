@@ -315,3 +315,5 @@ def test_uniform_numbers_of_many_rows_are_those_of_each():
     for n in (1, 23, 24, len(rows)):
         got = uniforms_for(*zip(*rows[:n]))
         assert got.tolist() == [uniform_for(*r) for r in rows[:n]]     # (24 bits: a float32 holds them)
+    same = [(-3, k, k + 1) for k in range(30)]                         # (one seed for all)
+    assert uniforms_for(*zip(*same)).tolist() == [uniform_for(*r) for r in same]
