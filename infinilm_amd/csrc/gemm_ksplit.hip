@@ -34,7 +34,7 @@ gemm_ksplit_kernel(TC* __restrict__ C, const bf16* __restrict__ X, const bf16* _
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, q = lane >> 4;
     const int kslice = blockIdx.y;
-    static_assert(GF_WAVES * GF_KSTEPS * 32 == GF_KSPAN, "a workgroup covers GF_KSPAN of K");
+    static_assert(GF_WAVES * GF_KSTEPS * 32 <= GF_KSPAN, "a workgroup covers at most GF_KSPAN of K");
     const int k_lo = kslice * kspan;              // this workgroup's K range starts here
     const int k_hi = (k_lo + kspan < K) ? k_lo + kspan : K;
     const int s0 = wave * ks;
@@ -153,7 +153,10 @@ extern "C" int ilm_gemm_ksplit(void* C, int out_dtype, int ldc, long c_part_stri
                 "gemm_ksplit: X and W rows must be 16-byte aligned, X rows %d long", act ? 2 * K : K);
     const int ntiles = (N + 15) / 16;
     const int kspan = ((K + kb - 1) / kb + 31) / 32 * 32;   // K spread evenly over the parts
-    int gx = ilm_num_cus() / kb;
+    // up to 16 rows over a short part (a small matrix cut into many): 8 waves x 4 k-steps, two workgroups a unit.  With 16 waves x 8
+    // every wave would take two of its eight steps and load the first again for the others.
+    const bool narrow = M <= 16 && !act && kspan <= 8 * 4 * 32 && out_dtype == ILM_DTYPE_F32;
+    int gx = (narrow ? 2 : 1) * ilm_num_cus() / kb;
     if (gx < 1) gx = 1;
     if (gx > ntiles) gx = ntiles;
     dim3 grid(gx, kb);
@@ -164,7 +167,9 @@ extern "C" int ilm_gemm_ksplit(void* C, int out_dtype, int ldc, long c_part_stri
 #define KS_LAUNCH(ACT, TC)                                   \
     if (M <= 16) KS_LAUNCH_(16, 8, 1, ACT, TC);              \
     else KS_LAUNCH_(8, 16, 2, ACT, TC)
-    if (out_dtype == ILM_DTYPE_BF16) {
+    if (narrow) {
+        KS_LAUNCH_(8, 4, 1, false, float);
+    } else if (out_dtype == ILM_DTYPE_BF16) {
         if (act) { KS_LAUNCH(true, bf16); } else { KS_LAUNCH(false, bf16); }
     } else if (out_dtype == ILM_DTYPE_F32) {
         if (act) { KS_LAUNCH(true, float); } else { KS_LAUNCH(false, float); }

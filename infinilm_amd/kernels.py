@@ -283,6 +283,7 @@ def gather_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
 
 _LIBRARY_F32_OUT = [True]   # cleared when torch.mm refuses out_dtype
 KSPLIT_SPAN = 4096  # K range of one part of the K-split few-rows product (ilm_gemm_ksplit_max_k(1))
+KSPLIT_FEW_SPAN = 1024   # ... and with up to 16 rows of up to KSPLIT_SPAN
 # Rows up to which the products keep X in registers (16 or 32; 32 only for K up to 4096 a workgroup)
 FEW_ROWS = int(os.environ.get("INFINILM_AMD_FEW_ROWS", "32"))
 
@@ -352,8 +353,12 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, 
             _run("ilm_gemm_rows64", parts.data_ptr(), N, M * N, kb, w.data_ptr(), w.stride(0), M, N, K, a.data_ptr(),
                  a.stride(0), 0, _stream())
         return parts
-    if fast and aligned and plain and allow_parts and out is None and M <= max(16, FEW_ROWS) and K > KSPLIT_SPAN and USE_KSPLIT:
-        kb = -(-K // KSPLIT_SPAN)
+    # Up to 16 rows and 4,096 k: parts of 1,024 k, which give a small matrix as many workgroups as the chip takes and every wave
+    # a short chain of loads (8 rows: 1024 x 4096 4.6 us against 8.6 with all of K in one workgroup, 1024 x 2048 3.9 / 5.4,
+    # 2048 x 2048 4.5 / 5.9, 2304 x 2304 5.8 / 7.4, 4096 x 4096 8.3 / 10.2).
+    span = KSPLIT_FEW_SPAN if M <= 16 and K <= KSPLIT_SPAN else KSPLIT_SPAN
+    if fast and aligned and plain and allow_parts and out is None and M <= max(16, FEW_ROWS) and K > span and USE_KSPLIT:
+        kb = -(-K // span)
         parts = torch.empty((kb, M, N), dtype=F32, device=a.device)
         _run("ilm_gemm_ksplit", parts.data_ptr(), _DT[F32], N, M * N, kb, w.data_ptr(), w.stride(0), None, 1.0,
              M, N, K, a.data_ptr(), a.stride(0), 0, _stream())

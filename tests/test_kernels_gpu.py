@@ -222,6 +222,18 @@ def test_gemm_float32_is_true_float32(K, M, N, K_):
     assert torch.equal(more[:M].cpu(), out.cpu())
 
 
+@pytest.mark.parametrize("M,N,K_", [(1, 1024, 1032), (16, 1000, 2048), (3, 2305, 2056), (16, 40, 3080), (9, 5000, 4096), (2, 300, 4096)])
+def test_gemm_few_rows_in_short_parts(K, M, N, K_):
+    """Up to 16 rows on their way into a residual sum, K in parts of 1,024: parts that do not fill up, more tiles than
+    workgroups.  bfloat16 operands are exact in float64, the parts' sum is float: 2^-24 a sum of K products."""
+    a, w = _rand((M, K_), 50, torch.bfloat16), _rand((N, K_), 51, torch.bfloat16)
+    parts = K.gemm(a.to(DEV), w.to(DEV), allow_parts=True)
+    assert parts.dtype == torch.float32 and parts.shape == (-(-K_ // K.KSPLIT_FEW_SPAN), M, N)
+    _close(parts.sum(0), P.plain_linear(a.to(F64), w.to(F64)), 2e-6 * math.sqrt(K_))
+    one = K.gemm(a[M - 1:].to(DEV), w.to(DEV), allow_parts=True)
+    assert torch.equal(one[:, 0], parts[:, M - 1])      # a row's bits do not depend on the rows around it
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 15, 4), (8, 4097, 36), (9, 33, 1028), (17, 16385, 68), (40, 260, 260), (64, 257, 4096), (65, 63, 8),
                                     (127, 129, 2052), (129, 257, 1024), (192, 4100, 516), (333, 640, 8192)])
 def test_gemm_float32_in_pieces(K, M, N, K_):
