@@ -61,7 +61,10 @@ __device__ __forceinline__ float att_cap(float raw, float capq, float icapq) {
 }
 
 // WF: the softmax weights enter the second product as two bfloat16 terms each (the rounded weight and the rest)
-template <int D16, bool WF>
+// PAIR: two chunks of ATT_STEP keys, both walked by one workgroup, which keeps the first one's result in registers and merges the two
+// as the merge kernel does, bit for bit.  That kernel costs more than a second step: one token, 16 heads of 64: 3.7 us instead
+// of 6.5 over 60 keys and 5.9 instead of 7.2 over 200; eight tokens, 32 heads of 128: 4.8 / 7.2 and 8.3 / 8.3.
+template <int D16, bool WF, bool PAIR>
 __global__ void __launch_bounds__(ATT_WAVES * 64, 2)
 attn_mfma_kernel(bf16* __restrict__ out, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
                  const bf16* __restrict__ q, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
@@ -87,7 +90,7 @@ attn_mfma_kernel(bf16* __restrict__ out, float* __restrict__ ws_acc, float* __re
 
     // the chunk's valid keys [c_begin, c_end); empty: nothing to do for the whole workgroup (the
     // merge reads only the chunks between the first and the last key the token sees)
-    int c_begin = split * span, c_end = c_begin + span;
+    int c_begin = split * span, c_end = c_begin + (PAIR ? 2 * ATT_STEP : span);
     if (c_begin < lo) c_begin = lo;
     if (c_end > p + 1) c_end = p + 1;
     if (c_begin >= c_end) return;
@@ -202,6 +205,80 @@ attn_mfma_kernel(bf16* __restrict__ out, float* __restrict__ ws_acc, float* __re
     }
     uint4 kfa[2][KS], vfa[D16], kfb[2][KS], vfb[D16];
     ATT_LOAD(kfa, vfa, first_step)
+    if constexpr (PAIR) {
+        // acc[db][e] is dim db*16 + qg*4 + e of head column r; o[i] the four waves' sum of db = wave + 4 i
+        constexpr int DBW = (D16 + ATT_WAVES - 1) / ATT_WAVES;
+        float M = NEG_BIG, L = 0.f;
+        f32x4 o[DBW];
+        auto merge_waves = [&]() {
+#pragma unroll
+            for (int db = 0; db < D16; ++db) *reinterpret_cast<f32x4*>(&sm_acc[wave][db][lane][0]) = acc[db];
+            if (qg == 0) {
+                sm_ml[wave][r][0] = m;
+                sm_ml[wave][r][1] = lsum;
+            }
+            __syncthreads();
+            M = NEG_BIG;
+#pragma unroll
+            for (int w = 0; w < ATT_WAVES; ++w) M = fmaxf(M, sm_ml[w][r][0]);
+            float wgt[ATT_WAVES];
+            L = 0.f;
+#pragma unroll
+            for (int w = 0; w < ATT_WAVES; ++w) {
+                wgt[w] = __builtin_amdgcn_exp2f(sm_ml[w][r][0] - M);
+                L += sm_ml[w][r][1] * wgt[w];
+            }
+#pragma unroll
+            for (int i = 0; i < DBW; ++i) {
+                const int db = wave + i * ATT_WAVES;
+                o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (db >= D16) continue;
+#pragma unroll
+                for (int w = 0; w < ATT_WAVES; ++w) {
+                    const f32x4 a = *reinterpret_cast<const f32x4*>(&sm_acc[w][db][lane][0]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[i][e] += a[e] * wgt[w];
+                }
+            }
+        };
+        if (first_step < last_step) ATT_LOAD(kfb, vfb, last_step)
+        __builtin_amdgcn_sched_barrier(0);
+        ATT_COMPUTE(kfa, vfa, first_step)
+        merge_waves();
+        if (first_step < last_step) {
+            const float M0 = M, L0 = L;
+            f32x4 o0[DBW];
+#pragma unroll
+            for (int i = 0; i < DBW; ++i) o0[i] = o[i];
+#pragma unroll
+            for (int db = 0; db < D16; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+            m = NEG_BIG;
+            lsum = 0.f;
+            __syncthreads();   // (the first chunk's sums have been read)
+            ATT_COMPUTE(kfb, vfb, last_step)
+            merge_waves();
+            const float M1 = M;
+            M = fmaxf(M0, M1);
+            const float w0 = __builtin_amdgcn_exp2f(M0 - M), w1 = __builtin_amdgcn_exp2f(M1 - M);
+            L = __fadd_rn(__fmul_rn(L0, w0), __fmul_rn(L, w1));
+#pragma unroll
+            for (int i = 0; i < DBW; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[i][e] = fmaf(o[i][e], w1, __fmul_rn(o0[i][e], w0));
+        }
+        if (!head_ok) return;
+#pragma unroll
+        for (int i = 0; i < DBW; ++i) {
+            const int db = wave + i * ATT_WAVES;
+            if (db >= D16) continue;
+            const float inv = 1.0f / L;
+            uint2 wv;
+            wv.x = pack_bf16x2(o[i][0] * inv, o[i][1] * inv);
+            wv.y = pack_bf16x2(o[i][2] * inv, o[i][3] * inv);
+            *reinterpret_cast<uint2*>(out + (size_t)t * out_stride + (size_t)head * D + db * 16 + qg * 4) = wv;
+        }
+        return;
+    }
     for (int st = first_step; st <= last_step; st += 2) {
         if (st + 1 <= last_step) ATT_LOAD(kfb, vfb, st + 1)
         __builtin_amdgcn_sched_barrier(0);
@@ -1035,10 +1112,12 @@ static int attn_mfma_launch(void* out, void* ws_acc, void* ws_ml, const void* q,
     ILM_REQUIRE(page % 16 == 0 && page > 0, "attn_mfma: page size %d is not a multiple of 16", page);
     ILM_REQUIRE(q_stride % 8 == 0 && out_stride % 4 == 0 && ((uintptr_t)q & 15) == 0 && ((uintptr_t)out & 7) == 0,
                 "attn_mfma: q and out rows must be 16-byte / 8-byte aligned");
-    ILM_REQUIRE(nsplit >= 1 && (nsplit == 1 || (ws_acc != nullptr && ws_ml != nullptr)), "attn_mfma: workspace missing");
+    const bool pair = nsplit == 2 && span == ATT_STEP;   // (no workspace, no merge)
+    ILM_REQUIRE(nsplit >= 1 && (nsplit == 1 || pair || (ws_acc != nullptr && ws_ml != nullptr)), "attn_mfma: workspace missing");
     ILM_REQUIRE(span > 0 && span % ATT_STEP == 0, "attn_mfma: chunk of %d keys is no multiple of %d", span, ATT_STEP);
     const int G = nh / nkv, HG = (G + 15) / 16;
     ILM_REQUIRE(nkv * HG <= 65535 && nsplit <= ATT_MERGE_MAX_CHUNKS, "attn_mfma: at most %d chunks, got %d", ATT_MERGE_MAX_CHUNKS, nsplit);
+    if (pair) nsplit = 1;
     dim3 grid(T_, nkv * HG, nsplit);
     const float sl2 = scale * 1.4426950408889634f;
     const float capq = softcap > 0.f ? softcap / scale : 0.f;
@@ -1047,8 +1126,10 @@ static int attn_mfma_launch(void* out, void* ws_acc, void* ws_ml, const void* q,
                 max_blocks, q_stride, out_stride, sl2, capq, reach, nsplit, span
 #define AM_CASE(D16)                                                                                           \
     case D16:                                                                                                  \
-        if (float_weights) attn_mfma_kernel<D16, true><<<grid, ATT_WAVES * 64, 0, stream>>>(AM_ARGS);          \
-        else attn_mfma_kernel<D16, false><<<grid, ATT_WAVES * 64, 0, stream>>>(AM_ARGS);                       \
+        if (float_weights && pair) attn_mfma_kernel<D16, true, true><<<grid, ATT_WAVES * 64, 0, stream>>>(AM_ARGS); \
+        else if (float_weights) attn_mfma_kernel<D16, true, false><<<grid, ATT_WAVES * 64, 0, stream>>>(AM_ARGS); \
+        else if (pair) attn_mfma_kernel<D16, false, true><<<grid, ATT_WAVES * 64, 0, stream>>>(AM_ARGS);       \
+        else attn_mfma_kernel<D16, false, false><<<grid, ATT_WAVES * 64, 0, stream>>>(AM_ARGS);                \
         break
     switch (d / 16) {
         AM_CASE(1); AM_CASE(2); AM_CASE(3); AM_CASE(4); AM_CASE(5); AM_CASE(6); AM_CASE(7); AM_CASE(8);

@@ -769,7 +769,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         # (the tokens counted as the recorded steps round them, so that an eager step and a replayed one cut alike)
         span, nsplit = attention_chunks(int(max_total_len), page, bound_rows(n_single) * nkv * (-(-(nh // nkv) // 16)), q.device)
         ws_acc = ws_ml = None
-        if nsplit > 1:
+        if nsplit > 1 and (span, nsplit) != (ATT_STEP, 2):   # (two chunks of one step meet inside a workgroup)
             # partial results of the rows served here (not of every token of the step)
             ws_acc = torch.empty((n_single * nh * nsplit * d,), dtype=F32, device=q.device)
             ws_ml = torch.empty((n_single * nh * nsplit * 2,), dtype=F32, device=q.device)

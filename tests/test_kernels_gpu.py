@@ -691,6 +691,24 @@ def test_attention_bfloat16_many_single_tokens(K, nh, nkv, d, page, n):
     _close(out, want, 1.2e-2)
 
 
+@pytest.mark.parametrize("nh,nkv,d,page", [(16, 2, 64, 64), (32, 2, 128, 64), (3, 1, 48, 16), (20, 1, 112, 32), (4, 4, 16, 128)])
+def test_attention_bfloat16_two_chunks_in_one_workgroup(K, monkeypatch, nh, nkv, d, page):
+    """Up to 256 keys in chunks of 128: one workgroup merges the two chunks as the merge kernel does, bit for bit (that kernel
+    serves when a third, empty chunk is asked for); contexts at the chunks' edges, a window that leaves the first out."""
+    attention = K.paged_attention
+    lens = [1, 31, 127, 128, 129, 160, 255, 256]
+    for window, softcap, fw in ((0, 0.0, False), (100, 0.0, False), (0, 20.0, True)):
+        got = []
+        for chunks in (2, 3):
+            monkeypatch.setattr(K, "attention_chunks", lambda *a: (K.ATT_STEP, chunks))
+            monkeypatch.setattr(K, "paged_attention", lambda *a, **k: attention(*a, softcap=softcap, float_weights=fw, **k))
+            out, want = _attention_case(K, torch.bfloat16, nh, nkv, d, page, lens=lens, qlens=[1] * len(lens), seed=60 + d, window=window)
+            got.append(out.cpu())
+        if not softcap:
+            _close(got[0], want, 1.2e-2)
+        assert torch.equal(got[0], got[1])
+
+
 def test_attention_bfloat16_with_a_block_table_beyond_lds(K):
     """33,000 keys in pages of 16: more block-table entries than the tile kernel keeps in LDS, and
     the most chunks the single-token kernel cuts a context into."""
