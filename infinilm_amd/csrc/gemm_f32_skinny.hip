@@ -9,15 +9,33 @@
 // Eight rows, before and after: 6912 x 2304 19.8 -> 14.3 us (4.5 TB/s), 2304 x 5760 23.3 -> 17.7, 122753 x 2304 266 -> 195,
 // 32768 x 4096 111 -> 91 (5.9 TB/s); 64 rows 58 -> 28, 69 -> 43, 852 -> 412 and 346 -> 174.
 // K must be a multiple of 4 and rows 16-byte aligned.
+//
+// Two more forms have the kernel that would follow in their epilogue, for which a workgroup takes two tiles whose outputs belong
+// together and the thread that reduces one output reduces its partner: gate and up rows of a feed-forward (SwiGLU), and the
+// halves of 16 rotation pairs of a query or key head, with the write into the paged cache.  Bit for bit what the
+// two kernels give, without a launch of 4.8 and 5.6 us each, which is what such small kernels take.
 #include "f32_split.h"
 
 #define FS_WAVES F3_SLICES
+#define FS_PLAIN 0
+#define FS_GLU 1
+#define FS_ROPE 2
 
-// XG: groups of 8 rows of X; RT: tiles of 16 W rows a workgroup; DEPTH: steps of 32 k in flight
-template <int XG, int RT, int DEPTH>
+struct FsRope {   // what FS_ROPE's epilogue needs (as gemm_qkv_rope.hip)
+    const int* pos;
+    const float *cosT, *sinT;
+    float *kc, *vc;
+    const int* slots;
+    int nh, nkv, d, page;
+};
+
+// XG: groups of 8 rows of X; RT: tiles of 16 W rows a workgroup; DEPTH: steps of 32 k in flight.  FORM: FS_GLU: N outputs from 2 N
+// rows of W; FS_ROPE: C is the queries' rows
+template <int XG, int RT, int DEPTH, int FORM>
 __global__ void __launch_bounds__(FS_WAVES * 64, XG <= 2 ? 4 : 2)
 gemm_f32_skinny_kernel(float* __restrict__ C, const float* __restrict__ X, const float* __restrict__ W,
-                       const float* __restrict__ bias, int M, int N, int K, int lda, int ldw, int ldc, float alpha) {
+                       const float* __restrict__ bias, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int act, FsRope rope) {
+    static_assert(FORM == FS_PLAIN || RT == 2, "outputs in pairs");
     constexpr int MG = (XG + 1) / 2;
     struct Frags {
         uint4 at[RT + MG][3][64];   // [tile of W, then group of X][piece][slot]
@@ -30,7 +48,9 @@ gemm_f32_skinny_kernel(float* __restrict__ C, const float* __restrict__ X, const
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 15, q = lane >> 4;       // place in a fragment
     const int lrow = lane >> 3, lk4 = lane & 7;   // place in a load: row, 16-byte piece of its line
-    const int n0 = blockIdx.x * (16 * RT);
+    const int n0 = FORM == FS_ROPE ? (int)(blockIdx.x / (rope.d / 32)) * rope.d + (int)(blockIdx.x % (rope.d / 32)) * 16
+                                   : blockIdx.x * (FORM == FS_GLU ? 16 : 16 * RT);
+    const int second = FORM == FS_ROPE ? rope.d / 2 : N;   // the partner's row after an output's (FS_GLU, FS_ROPE)
     const int steps_total = (K + F3_STEP - 1) / F3_STEP;
     const int per = (steps_total + F3_SLICES - 1) / F3_SLICES;
     const int s0 = wave * per;
@@ -40,8 +60,11 @@ gemm_f32_skinny_kernel(float* __restrict__ C, const float* __restrict__ X, const
     const float4* wp[2 * RT];
 #pragma unroll
     for (int i = 0; i < 2 * RT; ++i) {
-        const int row = n0 + 8 * i + lrow;
-        wp[i] = reinterpret_cast<const float4*>(W + (size_t)(row < N ? row : N - 1) * ldw);
+        const int in = FORM == FS_PLAIN ? 8 * i : 8 * (i & 1);
+        int row = n0 + in + lrow;
+        if (FORM != FS_ROPE) row = row < N ? row : N - 1;
+        if (FORM != FS_PLAIN && i >= 2) row += second;
+        wp[i] = reinterpret_cast<const float4*>(W + (size_t)row * ldw);
     }
     const float4* xp[XG];
     bool xok[XG];
@@ -131,6 +154,48 @@ gemm_f32_skinny_kernel(float* __restrict__ C, const float* __restrict__ X, const
         for (int g = 0; g < MG; ++g) *reinterpret_cast<f32x4*>(&lds.part[wave][t][g][lane][0]) = acc[t][g];
     __syncthreads();
     // acc[t][g][e] of lane (r, q) is output row n0 + t*16 + q*4 + e for token g*16 + r
+    if (FORM != FS_PLAIN) {
+        for (int idx = threadIdx.x; idx < MG * 64 * 4; idx += FS_WAVES * 64) {
+            const int e = idx & 3, l = (idx >> 2) & 63, g = idx >> 8;
+            const int n = n0 + (l >> 4) * 4 + e, m = g * 16 + (l & 15);
+            float a = 0.f, b = 0.f;
+#pragma unroll
+            for (int w = 0; w < FS_WAVES; ++w) {
+                a += lds.part[w][0][g][l][e];
+                b += lds.part[w][RT - 1][g][l][e];
+            }
+            if (m >= M || (FORM == FS_GLU && n >= N)) continue;
+            if (bias != nullptr) {
+                a += bias[n];
+                b += bias[n + second];
+            }
+            if (FORM == FS_GLU) {
+                C[(size_t)m * ldc + n] = glu_act(a, act) * b;
+                continue;
+            }
+            const int d = rope.d, half = d / 2, hs = n / d, i = n % d, slot = rope.slots != nullptr ? rope.slots[m] : -1;
+            if (hs >= rope.nh + rope.nkv) {   // values are cached transposed, [pages, nkv, d, page]
+                if (slot < 0) continue;
+                float* to = rope.vc + ((size_t)(slot / rope.page) * rope.nkv + (hs - rope.nh - rope.nkv)) * d * rope.page + (slot % rope.page);
+                to[(size_t)i * rope.page] = a;
+                to[(size_t)(i + half) * rope.page] = b;
+                continue;
+            }
+            const size_t at = (size_t)rope.pos[m] * half + i;
+            const float cs = rope.cosT[at], sn = rope.sinT[at];
+            const float ra = a * cs - b * sn, rb = b * cs + a * sn;
+            float* to;
+            if (hs < rope.nh) {
+                to = C + (size_t)m * ldc + n;
+            } else {
+                if (slot < 0) continue;
+                to = rope.kc + (((size_t)(slot / rope.page) * rope.nkv + (hs - rope.nh)) * rope.page + (slot % rope.page)) * d + i;
+            }
+            to[0] = ra;
+            to[half] = rb;
+        }
+        return;
+    }
     for (int idx = threadIdx.x; idx < RT * MG * 64 * 4; idx += FS_WAVES * 64) {
         const int e = idx & 3, l = (idx >> 2) & 63, tg = idx >> 8;
         const int t = tg / MG, g = tg % MG;
@@ -146,36 +211,73 @@ gemm_f32_skinny_kernel(float* __restrict__ C, const float* __restrict__ X, const
     }
 }
 
+#define FS_RUN(XG_, RT_, DEPTH_, FORM_, BLOCKS_)                                                                 \
+    gemm_f32_skinny_kernel<XG_, RT_, DEPTH_, FORM_><<<BLOCKS_, FS_WAVES * 64, 0, stream>>>(                      \
+        (float*)C, (const float*)X, (const float*)W, (const float*)bias, M, N, K, lda, ldw, ldc, alpha, act, rope)
+#define FS_PAIRS(FORM_, BLOCKS_)                                                                                 \
+    {                                                                                                            \
+        if (M <= 8) FS_RUN(1, 2, 3, FORM_, BLOCKS_);                                                             \
+        else if (M <= 16) FS_RUN(2, 2, 2, FORM_, BLOCKS_);                                                       \
+        else if (M <= 32) FS_RUN(4, 2, 3, FORM_, BLOCKS_);                                                       \
+        else if (M <= 48) FS_RUN(6, 2, 2, FORM_, BLOCKS_);                                                       \
+        else FS_RUN(8, 2, 2, FORM_, BLOCKS_);                                                                    \
+    }
+
+static int fs_check(const char* name, const void* X, const void* W, int M, int N, int K, int lda, int ldw) {
+    ILM_REQUIRE(M > 0 && M <= 64 && N > 0 && K > 0, "%s: needs 1 <= M <= 64, got M=%d N=%d K=%d", name, M, N, K);
+    ILM_REQUIRE(K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && lda >= K && ldw >= K, "%s: K=%d lda=%d ldw=%d", name, K, lda, ldw);
+    ILM_REQUIRE(((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0, "%s: operands must be 16-byte aligned", name);
+    return 0;
+}
+
 extern "C" int ilm_gemm_f32_skinny(void* C, const void* X, const void* W, const void* bias, int M, int N, int K,
                                    int lda, int ldw, int ldc, float alpha, hipStream_t stream) {
-    ILM_REQUIRE(M > 0 && M <= 64 && N > 0 && K > 0, "gemm_f32_skinny: needs 1 <= M <= 64, got M=%d N=%d K=%d", M, N, K);
-    ILM_REQUIRE(K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && lda >= K && ldw >= K && ldc >= N,
-                "gemm_f32_skinny: K=%d lda=%d ldw=%d ldc=%d", K, lda, ldw, ldc);
-    ILM_REQUIRE(((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0, "gemm_f32_skinny: operands must be 16-byte aligned");
-#define FS_CASE(XG_, RT_, DEPTH_)                                                                               \
-    gemm_f32_skinny_kernel<XG_, RT_, DEPTH_><<<(N + 16 * RT_ - 1) / (16 * RT_), FS_WAVES * 64, 0, stream>>>(    \
-        (float*)C, (const float*)X, (const float*)W, (const float*)bias, M, N, K, lda, ldw, ldc, alpha)
+    if (fs_check("gemm_f32_skinny", X, W, M, N, K, lda, ldw) != 0) return -1;
+    ILM_REQUIRE(ldc >= N, "gemm_f32_skinny: N=%d ldc=%d", N, ldc);
+    const int act = 0;
+    const FsRope rope = {};
     // Two tiles a workgroup, for which X is read and cut once, where one a workgroup would be more than one a compute unit
     // (M 8, K 2304: 14.3 us against 16.7 at N 6912, 11.6 against 9.6 at N 2304; K 4096: 18.5 against 15.9 at N 4096).  Not where
     // X is eight rows and K long: the deeper pipeline of one tile counts more (N 32768, K 4096: 100.6 against 91.2 us).
     const bool tall = N > 16 * ilm_num_cus() && (M > 8 || N < 16384 || K < 4096);
-    if (M <= 8) {
-        if (tall) FS_CASE(1, 2, 3);
-        else FS_CASE(1, 1, 6);
-    } else if (M <= 16) {
-        if (tall) FS_CASE(2, 2, 2);
-        else FS_CASE(2, 1, 4);
-    } else if (M <= 32) {
-        if (tall) FS_CASE(4, 2, 3);
-        else FS_CASE(4, 1, 4);
-    } else if (M <= 48) {
-        if (tall) FS_CASE(6, 2, 2);
-        else FS_CASE(6, 1, 2);
-    } else {
-        if (tall) FS_CASE(8, 2, 2);
-        else FS_CASE(8, 1, 2);
-    }
-#undef FS_CASE
+    const int blocks = (N + 15) / 16;
+    if (tall) FS_PAIRS(FS_PLAIN, (N + 31) / 32)
+    else if (M <= 8) FS_RUN(1, 1, 6, FS_PLAIN, blocks);
+    else if (M <= 16) FS_RUN(2, 1, 4, FS_PLAIN, blocks);
+    else if (M <= 32) FS_RUN(4, 1, 4, FS_PLAIN, blocks);
+    else if (M <= 48) FS_RUN(6, 1, 2, FS_PLAIN, blocks);
+    else FS_RUN(8, 1, 2, FS_PLAIN, blocks);
     ILM_LAUNCH_CHECK("gemm_f32_skinny");
+    return 0;
+}
+
+// C[M, ldc] = act(X Wg^T + bg) * (X Wu^T + bu), W = [Wg; Wu] of I rows each, bias [2 I] or null
+extern "C" int ilm_gemm_f32_glu(void* C, const void* X, const void* W, const void* bias, int M, int I, int K,
+                                int lda, int ldw, int ldc, int act, hipStream_t stream) {
+    if (fs_check("gemm_f32_glu", X, W, M, I, K, lda, ldw) != 0) return -1;
+    ILM_REQUIRE(ldc >= I, "gemm_f32_glu: I=%d ldc=%d", I, ldc);
+    const float alpha = 1.f;
+    const int N = I;
+    const FsRope rope = {};
+    FS_PAIRS(FS_GLU, (I + 15) / 16)
+    ILM_LAUNCH_CHECK("gemm_f32_glu");
+    return 0;
+}
+
+// C [M, ldc] receives the rotated query heads; k (rotated) and v go to the cache slots (slots may be null: nothing
+// is cached).  W [(nh + 2 nkv) d, ldw] holds the q, k, v rows in this order, bias as many numbers or null; all of a head is rotated.
+extern "C" int ilm_gemm_f32_rope(void* C, int ldc, const void* X, int lda, const void* W, int ldw, const void* bias, int M, int K,
+                                 const void* pos, const void* cosT, const void* sinT, void* kc, void* vc, const void* slots,
+                                 int nh, int nkv, int d, int page, hipStream_t stream) {
+    ILM_REQUIRE(nh > 0 && nkv >= 0 && d > 0 && d % 32 == 0, "gemm_f32_rope: %d + 2 * %d heads of %d", nh, nkv, d);
+    const int N = (nh + 2 * nkv) * d;
+    if (fs_check("gemm_f32_rope", X, W, M, N, K, lda, ldw) != 0) return -1;
+    ILM_REQUIRE(ldc >= nh * d, "gemm_f32_rope: rows of %d for %d heads of %d", ldc, nh, d);
+    ILM_REQUIRE(slots == nullptr || (page > 0 && kc != nullptr && vc != nullptr), "gemm_f32_rope: cache missing");
+    const float alpha = 1.f;
+    const int act = 0;
+    const FsRope rope = {(const int*)pos, (const float*)cosT, (const float*)sinT, (float*)kc, (float*)vc, (const int*)slots, nh, nkv, d, page};
+    FS_PAIRS(FS_ROPE, N / 32)
+    ILM_LAUNCH_CHECK("gemm_f32_rope");
     return 0;
 }

@@ -228,11 +228,25 @@ def qkv_rope_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]
             and K % 8 == 0 and K <= 8192 and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0
             and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
         return None
+    return _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)
+
+
+def qkv_rope_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], positions: torch.Tensor,
+                 cos: torch.Tensor, sin: torch.Tensor, k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor],
+                 slots: Optional[torch.Tensor], nh: int, nkv: int, d: int, rd: int) -> Optional[torch.Tensor]:
+    """The same in float32, up to 64 rows: bit for bit the projection and `rope_kvwrite` one after the other."""
+    if not (USE_QKV_ROPE and rd == d and d % 32 == 0 and _f32_few_rows(x, w)):
+        return None
+    return _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)
+
+
+def _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d):
+    M, K = x.shape
     _dev(x, w, bias, positions, cos, sin, k_cache, v_cache, slots)
     _i32(positions, "positions")
     if w.shape != ((nh + 2 * nkv) * d, K) or positions.numel() != M:
         raise KernelError(f"fused projection {tuple(w.shape)} does not fit {nh}+2*{nkv} heads of {d} over {K}")
-    if bias is not None and (bias.shape != (w.shape[0],) or bias.dtype != BF16 or not bias.is_contiguous()):
+    if bias is not None and (bias.shape != (w.shape[0],) or bias.dtype != x.dtype or not bias.is_contiguous()):
         raise KernelError("bias does not fit the fused projection")
     if cos.dtype != F32 or sin.dtype != F32 or cos.shape != sin.shape or cos.shape[1] != d // 2 \
             or not cos.is_contiguous() or not sin.is_contiguous():
@@ -240,12 +254,12 @@ def qkv_rope_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]
     page = 0
     if slots is not None:
         _i32(slots, "slots")
-        if k_cache is None or v_cache is None or k_cache.dtype != BF16 or v_cache.dtype != BF16:
+        if k_cache is None or v_cache is None or k_cache.dtype != x.dtype or v_cache.dtype != x.dtype:
             raise KernelError("cache tensors missing or of another dtype than the activations")
         page = _check_cache(k_cache, v_cache, nkv, d)
-    q = torch.empty((M, nh * d), dtype=BF16, device=x.device)
-    _run("ilm_gemm_qkv_rope", q.data_ptr(), q.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), _ptr(bias),
-         M, K, positions.data_ptr(), cos.data_ptr(), sin.data_ptr(), _ptr(k_cache) if slots is not None else None,
+    q = torch.empty((M, nh * d), dtype=x.dtype, device=x.device)
+    _run("ilm_gemm_qkv_rope" if x.dtype == BF16 else "ilm_gemm_f32_rope", q.data_ptr(), q.stride(0), x.data_ptr(), x.stride(0),
+         w.data_ptr(), w.stride(0), _ptr(bias), M, K, positions.data_ptr(), cos.data_ptr(), sin.data_ptr(), _ptr(k_cache) if slots is not None else None,
          _ptr(v_cache) if slots is not None else None, _ptr(slots), nh, nkv, d, page, _stream())
     return q
 
@@ -294,6 +308,14 @@ def _few_rows(M: int, K: int) -> bool:
     beside the W fragments in flight."""
     groups = max(1, min(FEW_ROWS // 16, 8192 // max(K, 4096)))
     return M <= 16 * groups
+
+
+def _f32_few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the 32-bit products of few rows take these operands (`gemm` goes to the same kernels then)."""
+    K = x.shape[1]
+    return (x.dtype == F32 and w.dtype == F32 and not FORCE_BASIC and x.shape[0] <= F32_FEW_ROWS and K % 4 == 0 and x.stride(1) == 1
+            and w.stride(1) == 1 and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and max(x.stride(0), w.stride(0)) < 1 << 24)
 
 
 def _frag_of(frag_w):
@@ -615,6 +637,20 @@ def gateup_swiglu_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Te
     out = torch.empty((M, I), dtype=BF16, device=x.device)
     _run("ilm_gemm_gateup_swiglu", out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
          _ptr(bias), M, I, K, _ptr(row_ss), 0 if row_ss is None else row_ss.shape[0], float(eps), glu_code(act), _stream())
+    return out
+
+
+def gateup_glu_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], act: str = "silu") -> Optional[torch.Tensor]:
+    """The same in float32, up to 64 rows: bit for bit the projection and the activation kernel one after the other."""
+    if not (USE_GATEUP_SWIGLU and _f32_few_rows(x, w) and w.shape[0] % 2 == 0 and w.shape[1] == x.shape[1]):
+        return None
+    _dev(x, w, bias)
+    M, I = x.shape[0], w.shape[0] // 2
+    if bias is not None and (bias.shape != (2 * I,) or bias.dtype != F32 or not bias.is_contiguous()):
+        raise KernelError("bias does not fit the fused gate/up projection")
+    out = torch.empty((M, I), dtype=F32, device=x.device)
+    _run("ilm_gemm_f32_glu", out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias), M, I, x.shape[1], x.stride(0), w.stride(0),
+         out.stride(0), glu_code(act), _stream())
     return out
 
 

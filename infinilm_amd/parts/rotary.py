@@ -151,8 +151,8 @@ class RotaryEmbedding(PositionEncoding):
         if isinstance(x, kernels.FragRows):   # rows in fragment order, as `takes_frag` offered
             return kernels.gemm_frag_rope(x, proj.frag_weight("qkv", nh=nh, nkv=nkv, d=d), proj.bias, batch.positions,
                                           self.cos, self.sin, view.k, view.v, view.slots, nh, nkv, d)
-        return kernels.qkv_rope_gemm(x, proj.weight, proj.bias, batch.positions, self.cos, self.sin, view.k, view.v,
-                                     view.slots, nh, nkv, d, self.rotary_dim)
+        fused = kernels.qkv_rope_f32 if x.dtype == torch.float32 else kernels.qkv_rope_gemm
+        return fused(x, proj.weight, proj.bias, batch.positions, self.cos, self.sin, view.k, view.v, view.slots, nh, nkv, d, self.rotary_dim)
 
     def encode_and_store(self, qkv, batch, view, nh, nkv, d):
         kernels.rope_kvwrite(qkv, batch.positions, self.cos, self.sin, view.k, view.v, view.slots, nh, nkv, d,

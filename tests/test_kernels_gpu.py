@@ -222,6 +222,39 @@ def test_gemm_float32_is_true_float32(K, M, N, K_):
     assert torch.equal(more[:M].cpu(), out.cpu())
 
 
+@pytest.mark.parametrize("M,I,K_,bias,act", [(1, 15, 36, False, "silu"), (8, 4100, 260, True, "gelu_tanh"), (16, 33, 1028, False, "silu"),
+                                             (33, 100, 64, True, "silu"), (64, 5760, 96, False, "gelu_tanh")])
+def test_gemm_float32_with_the_activation_in_its_epilogue(K, M, I, K_, bias, act):
+    """Bit for bit the projection and the activation kernel one after the other, at the edges of tiles and row groups."""
+    x, w = _rand((M, K_), 70).to(DEV), _rand((2 * I, K_), 71, scale=0.1).to(DEV)
+    b = _rand((2 * I,), 72).to(DEV) if bias else None
+    got = K.gateup_glu_f32(x, w, b, act=act)
+    assert torch.equal(got, K.swiglu(K.gemm(x, w, b), act))
+
+
+@pytest.mark.parametrize("M,nh,nkv,d,page,K_,bias", [(1, 4, 2, 32, 4, 64, False), (9, 3, 3, 64, 64, 132, True), (17, 6, 1, 128, 16, 1028, False),
+                                                     (40, 2, 2, 96, 8, 36, True), (64, 36, 36, 64, 64, 96, False)])
+def test_gemm_float32_with_the_rotation_in_its_epilogue(K, M, nh, nkv, d, page, K_, bias):
+    """Bit for bit the projection and the kernel that rotates and writes the cache; a row without a slot writes nothing."""
+    x, w = _rand((M, K_), 73).to(DEV), _rand(((nh + 2 * nkv) * d, K_), 74, scale=0.1).to(DEV)
+    b = _rand(((nh + 2 * nkv) * d,), 75).to(DEV) if bias else None
+    g = torch.Generator().manual_seed(M)
+    pos = torch.randint(0, 500, (M,), generator=g, dtype=torch.int32).to(DEV)
+    ang = torch.rand((500, d // 2), generator=g) * 6.28
+    cos, sin = torch.cos(ang).to(DEV), torch.sin(ang).to(DEV)
+    pages = -(-M // page) + 1
+    slots = torch.randperm(pages * page, generator=g)[:M].to(torch.int32)
+    slots[M // 2] = -1
+    slots = slots.to(DEV)
+    caches = [[torch.zeros((pages, nkv, page, d), device=DEV), torch.zeros((pages, nkv, d, page), device=DEV)] for _ in range(2)]
+    got = K.qkv_rope_f32(x, w, b, pos, cos, sin, *caches[0], slots, nh, nkv, d, d)
+    rows = K.gemm(x, w, b)
+    K.rope_kvwrite(rows, pos, cos, sin, *caches[1], slots, nh, nkv, d, d)
+    assert torch.equal(got, rows[:, :nh * d])
+    assert torch.equal(caches[0][0], caches[1][0]) and torch.equal(caches[0][1], caches[1][1])
+    assert K.qkv_rope_f32(x, w, b, pos, cos, sin, None, None, None, nh, nkv, d, d).equal(got)
+
+
 @pytest.mark.parametrize("M,N,K_", [(1, 1024, 1032), (16, 1000, 2048), (3, 2305, 2056), (16, 40, 3080), (9, 5000, 4096), (2, 300, 4096)])
 def test_gemm_few_rows_in_short_parts(K, M, N, K_):
     """Up to 16 rows on their way into a residual sum, K in parts of 1,024: parts that do not fill up, more tiles than
