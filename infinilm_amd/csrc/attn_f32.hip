@@ -41,7 +41,8 @@ __device__ __forceinline__ void fa_fold_scales(float& M, float& L, float m, floa
 
 // DT: head size / 16.  !SPLIT: gridDim.z == 1 and the wave walks all chunks; SPLIT: blockIdx.z is the
 // chunk and the partial result goes to ws[((t * nh + h) * gridDim.z + chunk) * (d + FA_WS_PAD)].
-template <int DT, bool SPLIT>
+// P16: pages hold whole tiles of 16 keys.
+template <int DT, bool SPLIT, bool P16>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DT <= 8 ? 2 : 1)))
 attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __restrict__ qp, const float* __restrict__ kc,
                 const float* __restrict__ vc, const int* __restrict__ block_tables, const int* __restrict__ seg,
@@ -49,7 +50,12 @@ attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __
                 int out_stride, float scale, int reach, float softcap) {
     constexpr int d = DT * 16;
     // tiles of keys (and of values) in flight: two, or one where the running result of the wave that walks all
-    // chunks leaves no registers for the second (another wave of the SIMD then covers the wait)
+    // chunks leaves no registers for the second (another wave of the SIMD then covers the wait).  A wave with one chunk is a
+    // chain of memory latencies, and each removed from it counts: with pages looked up once a tile and loads behind no
+    // branch, a decode step of 8 tokens over 1,250 keys of 36 heads of 64 takes 42.8 us (46.4 with a lookup a lane before each
+    // tile's loads), one token 16.2 (19.6), 64 tokens over 1,000 keys 223 (264, 5.3 TB/s now), 8 tokens over 4,000 keys of
+    // 2 heads of 128 31.3 (36.6).  Four tiles in flight with the values started before the softmax spilled at four waves a
+    // SIMD and was slower.
     constexpr int NB = (!SPLIT && DT > 6) ? 1 : 2;
     const int t = blockIdx.x, lane = threadIdx.x, r = lane & 15, q = lane >> 4;
     const int G = nh / nkv;
@@ -86,22 +92,35 @@ attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __
         // ---- scores of the chunk's tiles; the next tile's keys are on their way while one is multiplied
         f32x4 S[FA_TILES];
         float4 kf[NB][DT];
+        // where a tile's keys lie: the page and the place in it.  Pages of whole tiles are looked up once a tile by the scalar unit; else
+        // every lane looks up its own key's, a load that the tile's own loads then wait for
+        auto place = [&](int kt, int key, int& at) {
+            if (P16) {
+                const int base = c * FA_CHUNK + 16 * (kt < t_first ? t_first : (kt > t_last ? t_last : kt));
+                const int pg = bt[base / page];
+                at = base % page + (key - base);
+                return pg;
+            }
+            at = key % page;
+            return bt[key / page];
+        };
 #define FA_LOAD_K(BUF_, KT_)                                                                                  \
         {                                                                                                     \
-            int key = c * FA_CHUNK + (KT_) * 16 + r;                                                          \
+            int key = c * FA_CHUNK + (KT_) * 16 + r, at;                                                      \
             key = key < k_lo ? k_lo : (key > k_hi ? k_hi : key);   /* rows the token does not see: a row it sees */ \
-            const int pg = bt[key / page];                                                                    \
-            const float4* krow = reinterpret_cast<const float4*>(kc + (((size_t)pg * nkv + kvh) * page + (key % page)) * d); \
+            const int pg = place(KT_, key, at);                                                               \
+            const float4* krow = reinterpret_cast<const float4*>(kc + (((size_t)pg * nkv + kvh) * page + at) * d); \
             _Pragma("unroll") for (int j = 0; j < DT; ++j) kf[BUF_][j] = krow[4 * j + q];                      \
         }
+        // (the loads are unconditional, those of tiles beyond the last one of its rows again: behind a branch they are waited for at once)
         if (NB == 2) FA_LOAD_K(0, 0)
 #pragma unroll
         for (int kt = 0; kt < FA_TILES; ++kt) {
             S[kt] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+            if (NB == 2 && kt + 1 < FA_TILES) FA_LOAD_K((kt + 1) & (NB - 1), kt + 1)
+            __builtin_amdgcn_sched_barrier(0);
             if (kt > t_last) continue;
             if (NB == 1) FA_LOAD_K(0, kt)
-            else if (kt + 1 < FA_TILES && kt < t_last) FA_LOAD_K((kt + 1) & (NB - 1), kt + 1)
-            __builtin_amdgcn_sched_barrier(0);
             f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int j = 0; j < DT; ++j) {
@@ -146,21 +165,21 @@ attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __
         float4 vf[NB][DT];
 #define FA_LOAD_V(BUF_, KT_)                                                                                   \
         {                                                                                                      \
-            int gk = c * FA_CHUNK + (KT_) * 16 + 4 * q;   /* the lane's four keys; groups wholly outside: a group inside */ \
+            int gk = c * FA_CHUNK + (KT_) * 16 + 4 * q, at;   /* the lane's four keys; groups wholly outside: a group inside */ \
             if (gk > k_hi) gk = k_hi & ~3;                                                                     \
             if (gk + 3 < k_lo) gk = k_lo & ~3;                                                                 \
-            const int pg = bt[gk / page];                                                                      \
-            const float* vbase = vc + ((size_t)pg * nkv + kvh) * d * page + (gk % page);                       \
+            const int pg = place(KT_, gk, at);                                                                 \
+            const float* vbase = vc + ((size_t)pg * nkv + kvh) * d * page + at;                                \
             _Pragma("unroll") for (int i = 0; i < DT; ++i)                                                     \
                 vf[BUF_][i] = *reinterpret_cast<const float4*>(vbase + (size_t)(16 * i + r) * page);           \
         }
         if (NB == 2) FA_LOAD_V(0, 0)
 #pragma unroll
         for (int kt = 0; kt < FA_TILES; ++kt) {
+            if (NB == 2 && kt + 1 < FA_TILES) FA_LOAD_V((kt + 1) & (NB - 1), kt + 1)
+            __builtin_amdgcn_sched_barrier(0);
             if (kt > t_last) continue;
             if (NB == 1) FA_LOAD_V(0, kt)
-            else if (kt + 1 < FA_TILES && kt < t_last) FA_LOAD_V((kt + 1) & (NB - 1), kt + 1)
-            __builtin_amdgcn_sched_barrier(0);
             // values of keys the token does not see may be anything (pages are not cleared): they count as zeros
             const int key0 = c * FA_CHUNK + kt * 16 + 4 * q;
             const bool edge = (kt <= t_first || kt == t_last);
@@ -276,12 +295,15 @@ extern "C" int ilm_attn_f32(void* out, void* ws, int nchunks, const void* q, con
     const int G = nh / nkv, nsub = (G + 15) / 16;
     ILM_REQUIRE((long long)nkv * nsub <= 65535 && nh <= 65535, "attn_f32: too many heads");
     dim3 grid(T_, nkv * nsub, ws != nullptr ? nchunks : 1);
+    const bool p16 = page % 16 == 0;
 #define FA_ARGS (float*)out, (float*)ws, (const float*)q, (const float*)kc, (const float*)vc, (const int*)block_tables, \
                 (const int*)seg, (const int*)pos, nh, nkv, nsub, page, max_blocks, q_stride, out_stride, scale, reach, softcap
 #define FA_CASE(DT_)                                                                        \
     case DT_:                                                                               \
-        if (ws != nullptr) attn_f32_kernel<DT_, true><<<grid, 64, 0, stream>>>(FA_ARGS);    \
-        else attn_f32_kernel<DT_, false><<<grid, 64, 0, stream>>>(FA_ARGS);                 \
+        if (ws != nullptr && p16) attn_f32_kernel<DT_, true, true><<<grid, 64, 0, stream>>>(FA_ARGS);  \
+        else if (ws != nullptr) attn_f32_kernel<DT_, true, false><<<grid, 64, 0, stream>>>(FA_ARGS);    \
+        else if (p16) attn_f32_kernel<DT_, false, true><<<grid, 64, 0, stream>>>(FA_ARGS);              \
+        else attn_f32_kernel<DT_, false, false><<<grid, 64, 0, stream>>>(FA_ARGS);                      \
         break;
     switch (d / 16) {
         FA_CASE(1) FA_CASE(2) FA_CASE(3) FA_CASE(4) FA_CASE(5) FA_CASE(6) FA_CASE(7) FA_CASE(8)

@@ -631,6 +631,22 @@ def test_attention_float32_matrix_cores_one_wave_a_chunk_gives_the_same_bits(K, 
     assert torch.equal(alone.cpu()[0], among.cpu()[39])
 
 
+@pytest.mark.parametrize("nh,nkv,d", [(6, 2, 48), (3, 3, 64), (16, 1, 128), (2, 1, 256)])
+@pytest.mark.parametrize("window", [0, 100, 21])
+def test_attention_float32_pages_of_whole_tiles(K, monkeypatch, nh, nkv, d, window):
+    """Pages that hold whole tiles of 16 keys are looked up once a tile, others once a lane: the same keys give the
+    same bits either way, at the edges of tiles, chunks and windows and in both launch shapes."""
+    case = dict(lens=[1, 16, 17, 128, 129, 300], qlens=[1, 1, 2, 1, 1, 3], window=window, seed=11)
+    outs = []
+    for split in (True, False):
+        monkeypatch.setattr(K, "F32_ATTN_SPLIT", split)
+        for page in (12, 16, 48):
+            out, want = _attention_case(K, torch.float32, nh, nkv, d, page, **case)
+            outs.append(out.cpu())
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    _close(outs[0], want, 3e-6)
+
+
 def test_attention_float32_refuses_a_bound_below_a_position_loudly(K):
     """A caller's bound on the lengths that is too small for a token must not lose a chunk silently: the
     fold marks the token's row with NaNs."""
