@@ -8,7 +8,7 @@ ends.  One JSON line is printed: `value` is decoded tokens a second at the defau
 `prefill` is one 2,048-token prompt in one step (the median of seven passes timed with events);
 `roofline` prices the decode step against HBM bandwidth (every weight it uses read once, plus the
 cache of the live requests); `points` holds decode at batch 1, 32 and 64 and `points_frac` the same
-pricing of each; `fp32` the batch-8 step and the prefill on the true 32-bit path.  Peaks are MI355X's
+pricing of each; `fp32` the batch-8 step and the prefill on the true 32-bit path (its projections run as bfloat16 pieces, so a prefill can pass the float matrix peak it is priced against).  Peaks are MI355X's
 published ones (HBM 8 TB/s; dense MFMA bf16 2.5 PFLOP/s, fp32 157.3 TFLOP/s).  Weights are random (N(0, 0.02), norms 1 + N(0, 0.02)) and the
 cache of the context is filled with random keys and values instead of being computed: the timed
 steps do all of their work.
