@@ -8,7 +8,7 @@ time, the kernels raise.
 from __future__ import annotations
 
 import ctypes
-from ctypes import c_float, c_int, c_long, c_void_p
+from ctypes import c_float, c_int, c_long, c_uint64, c_void_p
 from typing import Optional
 
 _lib: Optional[ctypes.CDLL] = None
@@ -53,6 +53,7 @@ _SIGNATURES = {
     "ilm_attn_tile": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _F, _I, _P],
     "ilm_argmax": [_P, _P, _I, _I, _I, _P],
     "ilm_sample": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+    "ilm_uniforms": [_P, _P, c_uint64, _P, _P, _I],
     "ilm_unary": [_P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "ilm_lin_prep": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "ilm_decay_scan": [_P, _I, _P, _P, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _I, _P],
@@ -146,6 +147,8 @@ def load(verbose: bool = True) -> ctypes.CDLL:
     lib.ilm_delta_chunk_ws.argtypes = [c_int, c_int]
     lib.ilm_sample_ws.restype = c_long
     lib.ilm_sample_ws.argtypes = [c_int, c_int]
+    lib.ilm_sample_few_k.restype = c_int
+    lib.ilm_sample_few_k.argtypes = []
     lib.ilm_attn_static_init.restype = c_int
     lib.ilm_attn_static_init.argtypes = []
     lib.ilm_attn_static_scratch_floats.restype = c_long

@@ -17,11 +17,13 @@
 // changes with the code around it, at 1 to 30 us a call of the sampler.)
 //
 // What bounds it is arithmetic, some 40 instructions an element and pass for its mass and bin: one compute unit a row takes
-// 110 us for 122,753 elements.  So few long rows are cut into chunks over the chip, four short kernels
+// 103 us for 122,753 elements.  So few long rows are cut into chunks over the chip, four short kernels
 // one after the other (maximum; histogram; list and masses of 256-element tiles; the token), the rows' results meeting in
-// a workspace, and only rows whose threshold falls where lists overflow are done again by one workgroup.
-// A call with its host's work, against 32 + 32 rounds of bitwise search over a row in registers (or in memory beyond
-// 98,304): 64 rows x 73,448 with top-k 50 and top-p 0.9 55 us against 187, 5 rows x 122,753 with top-p 0.95 49 against 802.
+// a workspace, and only rows whose threshold falls where lists overflow are done again by one workgroup.  A row with a small top-k
+// needs neither masses nor bins for all of its elements (top_k_of_few).
+// A call with its host's work, against histograms for every row (and 32 + 32 rounds of bitwise search before them): 64 rows x 73,448 with
+// top-k 50 and top-p 0.9 33 us against 55 (187), 5 rows x 122,753 with top-p 0.95 37 against 49 (802), of which the kernels take 20 against 35
+// and 30 (4.8, 6.4, 8.0 and 10.6) against 43 (4.9, 6.6, 14.1 and 17.5).
 //
 // Masses are summed as whole numbers (e * 2^43): every sum is exact in its terms whatever the order, so the
 // result depends on no order of atomics, and finer than sums of floats.
@@ -397,6 +399,58 @@ __device__ __forceinline__ uint32_t rank_list(SampleLds& S, int n, uint32_t leas
     return block_max_u32(best, (uint32_t*)S.red);
 }
 
+// rank_list of one bin's elements, which lie even over a short range of keys: a long list falls into 2,048 steps of that range, one or two
+// elements a step, and the step that holds the threshold is ranked by every wave for itself (one histogram instead of radix's three:
+// 5 rows of 122,753, top-p 0.95, about 390 listed: the kernel that ends in it
+// 14.3 -> 10.6 us)
+#define STEP_MAX 64
+__device__ __forceinline__ uint32_t rank_bin(SampleLds& S, int n, uint32_t least, u64 base, double need) {
+    if (n <= RANK_MAX) return rank_list<false>(S, n, least, base, need);
+    u64 ends = 0;     // the largest key, and the largest complement of one
+    for (int i = threadIdx.x; i < n; i += SB) {
+        const uint32_t key = S.list.key[i];
+        const u64 one = (u64)key << 32 | (uint32_t)~key;
+        ends = i == (int)threadIdx.x ? one : ((ends >> 32) > key ? ends >> 32 : key) << 32 | ((uint32_t)ends > (uint32_t)~key ? (uint32_t)ends : (uint32_t)~key);
+    }
+    ends = block_reduce<SB>(ends, S.red, [](u64 a, u64 b) {
+        const u64 h = (a >> 32) > (b >> 32) ? a >> 32 : b >> 32;
+        return h << 32 | ((uint32_t)a > (uint32_t)b ? (uint32_t)a : (uint32_t)b);
+    });
+    const uint32_t hi = (uint32_t)(ends >> 32), range = hi - ~(uint32_t)ends;
+    const int bits = range == 0 ? 0 : 32 - __builtin_clz(range), shift = bits > 11 ? bits - 11 : 0;
+    clear_hist(S);
+    for (int i = threadIdx.x; i < n; i += SB)
+        if (S.list.key[i] >= least) atomicAdd(&S.hist[(hi - S.list.key[i]) >> shift], S.list.mass[i]);
+    const Found f = find_in<SB>(S.hist, base, need, S.red, &S.found);
+    if (f.at < 0) return 0;
+    if (threadIdx.x == 0) S.listed = 0;
+    __syncthreads();
+    u64* mass = S.hist;                                              // of the step's elements, and behind them their keys
+    uint32_t* key = reinterpret_cast<uint32_t*>(S.hist + STEP_MAX);
+    for (int i = threadIdx.x; i < n; i += SB)
+        if (S.list.key[i] >= least && (int)((hi - S.list.key[i]) >> shift) == f.at) {
+            const int to = atomicAdd(&S.listed, 1);
+            if (to < STEP_MAX) {
+                mass[to] = S.list.mass[i];
+                key[to] = S.list.key[i];
+            }
+        }
+    __syncthreads();
+    const int m = S.listed;
+    if (m > STEP_MAX) return radix_list<false>(S, n, least, base, need);
+    const int lane = threadIdx.x & 63;
+    const uint32_t mine = lane < m ? key[lane] : 0u;
+    u64 sum = f.before;
+    for (int j = 0; j < m; ++j) sum += key[j] >= mine ? mass[j] : 0ull;
+    uint32_t best = lane < m && (double)sum >= need ? mine : 0u;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const uint32_t v = __shfl_xor(best, o, 64);
+        best = v > best ? v : best;
+    }
+    return best;
+}
+
 // tau of a top-p over what the list holds from `tau` on
 __device__ __forceinline__ uint32_t top_p_of_list(SampleLds& S, int listed, uint32_t tau, float pp) {
     u64 total = 0;
@@ -594,7 +648,7 @@ __device__ __noinline__ void sample_row(SampleLds& S, const float* row, int V, f
                 // (a bin of ties has one key, as a rule, which the first of radix_bin's passes finds)
                 const int n = TIES ? LIST_CAP + 1
                                    : collect(row, V, S, mass, [&](float l) { return okey(l) >= tau && bin_of(l, mx, per) == bin; });
-                tp = n <= LIST_CAP ? rank_list<false>(S, n, tau, base, need) : radix_bin<false>(row, V, S, mass, bin, per, tau, base, need);
+                tp = n <= LIST_CAP ? rank_bin(S, n, tau, base, need) : radix_bin<false>(row, V, S, mass, bin, per, tau, base, need);
             }
         }
         if (!(pp > 0.f)) tp = okey(mx);
@@ -628,6 +682,178 @@ __device__ __noinline__ void sample_row(SampleLds& S, const float* row, int V, f
     if (w == 0) token_of_tiles(S, row, V, mass, tau, uniform, last, amax, out);
 }
 
+// ---- a top-k of few ----------------------------------------------------------------------------------------
+// Four threads' elements are a group, whose maxima are distinct elements: the k-th largest of 256 maxima is a bound that at least k
+// elements reach, and few more do (of independent numbers 56 for k = 50, 532 for 224).  So the row is read once for the maxima, at one
+// instruction an element instead of some 40 for bins, the bound is found by one wave bit by bit in registers, and only threads with an element
+// that reaches it read theirs again.  64 rows of 73,448, top-k 50, top-p 0.9: 35 us ->
+// 20, top-k 200 45 -> 36, 5 rows of 122,753, top-k 50 46 -> 24.
+#define FEW_K 224
+#define FEW_GROUPS (SB / 4)
+#define FEW_FROM (4 * SB)   // vocabulary from which every thread has elements
+#define FEW_TIES 64     // groups beyond k at the bound from which a row is left to the histograms (rows of ties)
+
+// Threshold and token of a list of up to 64 E elements that holds all of the top-k: by the first wave, E elements a lane, each weighed
+// against all (rank_list, top_p_of_list and token_of_list in one wave, without their barriers: some 12 us for a list of 60)
+template <int E>
+__device__ __forceinline__ void token_of_few(const SampleLds& S, int n, int k, float pp, float uniform, int* out) {
+    const int lane = threadIdx.x & 63;
+    uint32_t key[E];
+    int index[E];
+    u64 mass[E];
+    int count[E];
+    u64 above[E];    // mass of the elements with keys from this one's on
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int i = e * 64 + lane;
+        key[e] = i < n ? S.list.key[i] : 0u;
+        index[e] = i < n ? S.list.index[i] : -1;
+        mass[e] = i < n ? S.list.mass[i] : 0ull;
+        count[e] = 0;
+        above[e] = 0;
+    }
+#pragma unroll 4
+    for (int j = 0; j < n; ++j) {
+        const uint32_t kj = S.list.key[j];
+        const u64 mj = S.list.mass[j];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            count[e] += kj >= key[e] ? 1 : 0;
+            above[e] += kj >= key[e] ? mj : 0ull;
+        }
+    }
+    auto largest = [&](auto of) {    // (of: a key, or 0)
+        uint32_t best = 0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const uint32_t v = of(e);
+            best = v > best ? v : best;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint32_t v = __shfl_xor(best, o, 64);
+            best = v > best ? v : best;
+        }
+        return best;
+    };
+    auto kept = [&](uint32_t tau) {    // mass of the elements from tau on
+        u64 sum = 0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) sum += key[e] >= tau ? mass[e] : 0ull;
+        return wave_sum_u64(sum);
+    };
+    uint32_t tau = largest([&](int e) { return count[e] >= k ? key[e] : 0u; });
+    u64 total = kept(tau);
+    if (pp < 1.0f) {
+        const double need = (double)pp * (double)total;
+        const uint32_t tp = !(pp > 0.f) ? largest([&](int e) { return key[e]; })
+                            : total > 0 ? largest([&](int e) { return key[e] >= tau && (double)above[e] >= need ? key[e] : 0u; })
+                                        : 0u;
+        if (tp > tau) {
+            tau = tp;
+            total = kept(tau);
+        }
+    }
+    const double target = (double)uniform * (double)total;
+    u64 run[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) run[e] = 0;
+#pragma unroll 4
+    for (int j = 0; j < n; ++j) {
+        const int ij = S.list.index[j];
+        const u64 mj = S.list.key[j] >= tau ? S.list.mass[j] : 0ull;
+#pragma unroll
+        for (int e = 0; e < E; ++e) run[e] += ij <= index[e] ? mj : 0ull;
+    }
+    uint32_t pick = 0;    // the first index that passes the target (as its complement), else the last kept one
+    pick = largest([&](int e) { return key[e] >= tau && mass[e] > 0 && target < (double)run[e] ? ~(uint32_t)index[e] : 0u; });
+    if (pick != 0) pick = ~pick;
+    else pick = largest([&](int e) { return index[e] >= 0 && key[e] >= tau ? (uint32_t)index[e] + 1u : 0u; }) - 1u;
+    if (lane == 0) *out = (int)pick;
+}
+
+// The row's top-k of 2 to FEW_K; false: the list does not hold it (ties, masked rows, NaN)
+__device__ __forceinline__ bool top_k_of_few(SampleLds& S, const float* row, int V, float temp, int k, float pp, float uniform, int cut, int* out) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    uint32_t* group = reinterpret_cast<uint32_t*>(S.hist);      // [FEW_GROUPS]; behind them the waves' results
+    uint32_t* bound = group + FEW_GROUPS;
+    float most = -INFINITY;
+    over_row<SB>(row, V, [&](int, float l) { most = fmaxf(most, l); });     // (a NaN is dropped)
+    float m = fmaxf(most, __shfl_xor(most, 1, 64));
+    m = fmaxf(m, __shfl_xor(m, 2, 64));
+    if ((lane & 3) == 0) group[threadIdx.x >> 2] = okey(m);
+    if (threadIdx.x == 0) S.listed = 0;
+    __syncthreads();
+    if (w == 0) {
+        uint32_t own[FEW_GROUPS / 64], top = 0;
+#pragma unroll
+        for (int i = 0; i < FEW_GROUPS / 64; ++i) {
+            own[i] = group[i * 64 + lane];
+            top = own[i] > top ? own[i] : top;
+        }
+        auto reach = [&](uint32_t at) {
+            int n = 0;
+#pragma unroll
+            for (int i = 0; i < FEW_GROUPS / 64; ++i) n += __popcll(__builtin_amdgcn_ballot_w64(own[i] >= at));
+            return n;
+        };
+        uint32_t at = 0;
+#pragma unroll 1
+        for (int bit = 31; bit >= 0; --bit) {
+            const uint32_t c = at | (1u << bit);
+            if (reach(c) >= k) at = c;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const uint32_t v = __shfl_xor(top, o, 64);
+            top = v > top ? v : top;
+        }
+        if (lane == 0) {
+            bound[0] = at;
+            bound[1] = top;
+            bound[2] = (uint32_t)reach(at);
+        }
+    }
+    __syncthreads();
+    const uint32_t at = bound[0];
+    const float mx = key_to_float(bound[1]);
+    if ((int)bound[2] > k + FEW_TIES) return false;
+    const Mass mass = {mx, 1.0f / temp, cut};
+    if (okey(most) >= at)
+        over_row<SB>(row, V, [&](int i, float l) {
+            if (okey(l) >= at && l == l) {
+                const int to = atomicAdd(&S.listed, 1);
+                if (to < LIST_CAP) {
+                    S.list.key[to] = okey(l);
+                    S.list.index[to] = i;
+                    S.list.mass[to] = mass(l);
+                }
+            }
+        });
+    __syncthreads();
+    const int n = S.listed;
+    if (n < k || n > LIST_CAP) return false;
+    if (n > 128) {
+        uint32_t tau = rank_list<true>(S, n, 0, 0, (double)k);
+        if (pp < 1.0f) {
+            const uint32_t tp = pp > 0.f ? top_p_of_list(S, n, tau, pp) : okey(mx);
+            tau = tp > tau ? tp : tau;
+        }
+        if (n <= RANK_MAX) {
+            token_of_list(S, n, tau, uniform, 0, out);
+        } else {
+            const int g = tile_groups(V);
+            clear_tiles(S, (V + 256 * g - 1) / (256 * g));
+            list_to_tiles(S, n, tau, g);
+            if (w == 0) token_of_tiles(S, row, V, mass, tau, uniform, S.pick - 1, 0, out);
+        }
+    } else if (w == 0) {
+        if (n <= 64) token_of_few<1>(S, n, k, pp, uniform, out);
+        else token_of_few<2>(S, n, k, pp, uniform, out);
+    }
+    return true;
+}
+
 __global__ void __launch_bounds__(SB)
 sample_kernel(int* __restrict__ out, const float* __restrict__ logits, const float* __restrict__ temperature,
               const int* __restrict__ top_k, const float* __restrict__ top_p,
@@ -636,6 +862,7 @@ sample_kernel(int* __restrict__ out, const float* __restrict__ logits, const flo
     const int r = blockIdx.x, k = top_k[r];
     const float* row = logits + (size_t)r * stride;
     const float temp = temperature[r];
+    if (k > 1 && k <= FEW_K && k < V && V >= FEW_FROM && temp != 0.0f && top_k_of_few(S, row, V, temp, k, top_p[r], uniform[r], cut, out + r)) return;
     const RowMax m = block_argmax<SB>(row, V, sample_of(row[(size_t)threadIdx.x * V / SB]), S.meet);
     const float mx = m.value;
     const int amax = m.index == 0x7fffffff ? 0 : m.index;
@@ -653,6 +880,9 @@ sample_kernel(int* __restrict__ out, const float* __restrict__ logits, const flo
 struct RowWork {
     u64 hist[NBINS];
     u64 rest;                   // mass of the last bin
+    double need;                // the threshold's, as the list's kernel found it: what it has to reach,
+    Found found;                // ... its bin,
+    int whole;                  // ... and whether the row is left to one workgroup
     int listed, last;           // elements listed; the last element of the bins ahead of the threshold's, + 1
     RowMax max[MAX_CHUNKS];     // of each chunk
     uint32_t key[LIST_CAP];
@@ -755,26 +985,50 @@ sample_hist_kernel(char* __restrict__ ws, size_t ws_row, const float* __restrict
 }
 
 // Where the row's first threshold lies, from its histogram: found.at < 0 and no top-k or top-p: everything is kept; `whole`: the row
-// is left to one workgroup (a threshold in the last bin, a top-k beyond the list, no mass, p not above 0)
+// is left to one workgroup (a threshold in the last bin, a top-k beyond the list, no mass, p not above 0).  `mine`: a thread's bins; their
+// scan gives the row's mass, by which a top-p's threshold is known, and then its bin.
 template <int NT>
-__device__ __forceinline__ Found row_threshold(const RowWork* W, u64* red, Found* shared, bool count, int k, float pp, bool* whole, double* need) {
+__device__ __forceinline__ Found row_threshold(const u64 (&mine)[NBINS / NT], u64 rest, u64* red, Found* shared, bool count, int k, float pp, bool* whole,
+                                               double* need) {
+    constexpr int PER = NBINS / NT;
     Found f = {-1, 0, 0};
     *whole = false;
     *need = 0;
     if (!count && !(pp < 1.0f)) return f;
-    if (count) {
-        *need = (double)k;
-    } else {
-        u64 total = 0;
-        for (int i = threadIdx.x; i < NBINS; i += NT) total += W->hist[i];
-        total = block_sum_u64<NT>(total, red) + W->rest;
-        *need = (double)pp * (double)total;
-        if (!(pp > 0.f) || total == 0) {
-            *whole = true;
-            return f;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    u64 sum = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) sum += mine[i];
+    u64 incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const u64 n = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += n;
+    }
+    if (lane == 63) red[w] = incl;
+    if (threadIdx.x == 0) *shared = f;
+    __syncthreads();
+    u64 run = incl - sum, total = rest;
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) {
+        const u64 v = red[i];
+        if (i < w) run += v;
+        total += v;
+    }
+    *need = count ? (double)k : (double)pp * (double)total;
+    if (!count && (!(pp > 0.f) || total == 0)) {
+        *whole = true;
+        return f;
+    }
+    if (!((double)run >= *need)) {   // (not reached before this thread's entries)
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            if (!((double)run >= *need) && (double)(run + mine[i]) >= *need) *shared = {(int)threadIdx.x * PER + i, run, mine[i]};
+            run += mine[i];
         }
     }
-    f = find_in<NT>(W->hist, 0, *need, red, shared);
+    __syncthreads();
+    f = *shared;
     *whole = f.at < 0 || (count && f.before + f.in > LIST_CAP);
     return f;
 }
@@ -784,52 +1038,103 @@ sample_list_kernel(char* __restrict__ ws, size_t ws_row, const float* __restrict
                    const int* __restrict__ top_k, const float* __restrict__ top_p, int V, int stride, int cut) {
     __shared__ u64 red[CHUNK_THREADS / 64];
     __shared__ Found shared;
+    __shared__ uint32_t keys[LIST_CAP];   // the chunk's listed elements: a place in the row's list costs a round trip through memory, so a chunk asks
+    __shared__ int indices[LIST_CAP];     // once for all of its own
+    __shared__ int own, from, last;
     const int r = blockIdx.y, k = top_k[r];
     RowWork* W = reinterpret_cast<RowWork*>(ws + (size_t)r * ws_row);
     const float* row = logits + (size_t)r * stride;
     const float temp = temperature[r], pp = top_p[r];
     const bool count = k > 0 && k < V;
     if (temp == 0.0f || k == 1) return;
-    bool whole;
-    double need;
-    const Found f = row_threshold<CHUNK_THREADS>(W, red, &shared, count, k, pp, &whole, &need);
-    if (whole) return;
+    if (threadIdx.x == 0) own = 0, last = 0;
+    // what the kernel reads is on its way at once: the bins, the chunks' maxima, and a wave's first two tiles
+    u64 mine[NBINS / CHUNK_THREADS];
+#pragma unroll
+    for (int i = 0; i < NBINS / CHUNK_THREADS; ++i) mine[i] = W->hist[threadIdx.x * (NBINS / CHUNK_THREADS) + i];
+    const u64 rest = W->rest;
+    const Chunk c = chunk_of(V);
+    const int m = tile_groups(V), t0 = c.first + (int)(threadIdx.x >> 6), lane4 = 4 * (int)(threadIdx.x & 63);
+    float ahead[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = (t0 + u * (CHUNK_THREADS / 64)) * 256 + lane4 + e;
+            ahead[u][e] = row[i < V ? i : V - 1];
+        }
     float mx, low;
     bool ties;
     row_max(W, gridDim.x, &mx, &ties, &low);
+    bool whole;
+    double need;
+    const Found f = row_threshold<CHUNK_THREADS>(mine, rest, red, &shared, count, k, pp, &whole, &need);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        W->need = need;
+        W->found = f;
+        W->whole = whole ? 1 : 0;
+    }
+    if (whole) return;
     const Mass mass = {mx, 1.0f / temp, cut};
     const float per = bins_per(mx, low, mass.inv_t);
+    __syncthreads();   // (`own`)
     auto list = [&](int i, float l) {
-        const int at = atomicAdd(&W->listed, 1);
+        const int at = atomicAdd(&own, 1);
         if (at < LIST_CAP) {
-            W->key[at] = okey(l);
-            W->index[at] = i;
+            keys[at] = okey(l);
+            indices[at] = i;
         }
     };
-    const Chunk c = chunk_of(V);
     if (count) {   // everything down to the threshold's bin
         over_row<CHUNK_THREADS>(row + c.begin, c.size, [&](int i, float l) {
             if (bin_of(l, mx, per) <= f.at) list(c.begin + i, l);
         });
-        return;
+    } else {
+        const int above = f.at >= 0 ? f.at : NBINS;   // the bins ahead of the threshold's are kept whole
+        int my_last = -1;
+        auto tile = [&](int t, auto over) {
+            u64 sum = 0;
+            over([&](int i, float l) {
+                const int b = bin_of(l, mx, per);
+                if (b < above) {
+                    sum += mass(l);
+                    my_last = i;
+                } else if (b == above) {
+                    list(i, l);
+                }
+            });
+            sum = wave_sum_u64(sum);
+            if ((threadIdx.x & 63) == 0) W->tile[t] = sum;
+        };
+        int t = t0;
+        if (m == 1) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u, t += CHUNK_THREADS / 64)
+                if (t < c.first + c.count)
+                    tile(t, [&](auto f) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (t * 256 + lane4 + e < V) f(t * 256 + lane4 + e, ahead[u][e]);
+                    });
+        }
+        for (; t < c.first + c.count; t += CHUNK_THREADS / 64) tile(t, [&](auto f) { over_tile(row, V, t, m, f); });
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const int v = __shfl_xor(my_last, o, 64);
+            my_last = v > my_last ? v : my_last;
+        }
+        if ((threadIdx.x & 63) == 0) atomicMax(&last, my_last + 1);
     }
-    const int m = tile_groups(V), above = f.at >= 0 ? f.at : NBINS;   // the bins ahead of the threshold's are kept whole
-    int my_last = -1;
-    for (int t = c.first + (int)(threadIdx.x >> 6); t < c.first + c.count; t += CHUNK_THREADS / 64) {
-        u64 sum = 0;
-        over_tile(row, V, t, m, [&](int i, float l) {
-            const int b = bin_of(l, mx, per);
-            if (b < above) {
-                sum += mass(l);
-                my_last = i;
-            } else if (b == above) {
-                list(i, l);
-            }
-        });
-        sum = wave_sum_u64(sum);
-        if ((threadIdx.x & 63) == 0) W->tile[t] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0 && last != 0) atomicMax(&W->last, last);   // (an atomic a chunk: one of every thread held the row's address for half the kernel)
+    const int n = own;
+    if (n == 0) return;
+    if (threadIdx.x == 0) from = atomicAdd(&W->listed, n);
+    __syncthreads();
+    for (int i = threadIdx.x; i < n && i < LIST_CAP && from + i < LIST_CAP; i += CHUNK_THREADS) {
+        W->key[from + i] = keys[i];
+        W->index[from + i] = indices[i];
     }
-    if (my_last >= 0) atomicMax(&W->last, my_last + 1);
 }
 
 __global__ void __launch_bounds__(SB)
@@ -849,12 +1154,11 @@ sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row,
         if (threadIdx.x == 0) out[r] = amax;
         return;
     }
-    bool whole;
-    double need;
-    const Found f = row_threshold<SB>(W, S.red, &S.found, count, k, pp, &whole, &need);
+    const Found f = W->found;
+    const double need = W->need;
     const int listed = W->listed;
     const Mass mass = {mx, 1.0f / temp, cut};
-    if (whole || listed > LIST_CAP) {
+    if (W->whole != 0 || listed > LIST_CAP) {
         uint32_t tau = 0;
         int known = 0;
         const float per = bins_per(mx, low, mass.inv_t);
@@ -873,8 +1177,12 @@ sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row,
         S.list.index[i] = W->index[i];
         S.list.mass[i] = mass(key_to_float(key));
     }
-    __syncthreads();
     const int m = tile_groups(V), tiles = (V + 256 * m - 1) / (256 * m);
+    if (!count) {
+        for (int t = threadIdx.x; t < tiles; t += SB) S.tile[t] = W->tile[t];
+        if (threadIdx.x == 0) S.pick = W->last;
+    }
+    __syncthreads();
     uint32_t tau = 0;
     if (count) {
         tau = rank_list<true>(S, listed, 0, 0, need);
@@ -888,10 +1196,7 @@ sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row,
         }
         clear_tiles(S, tiles);
     } else {
-        if (f.at >= 0) tau = rank_list<false>(S, listed, 0, f.before, need);
-        for (int t = threadIdx.x; t < tiles; t += SB) S.tile[t] = W->tile[t];
-        if (threadIdx.x == 0) S.pick = W->last;
-        __syncthreads();
+        if (f.at >= 0) tau = rank_bin(S, listed, 0, f.before, need);
     }
     list_to_tiles(S, listed, tau, m);
     if (threadIdx.x < 64) token_of_tiles(S, row, V, mass, tau, uniform[r], S.pick - 1, amax, out + r);
@@ -900,16 +1205,38 @@ sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row,
 // Bytes of workspace a row needs of n rows of V logits; 0: none, the rows are not cut into chunks.  They are where few rows leave
 // the chip idle and a row is long enough to outweigh three more launches.  In chunks against one workgroup a row, us, with top-p
 // alone, with top-k 50 and with neither (which of them rows ask for is only known on the device):
-//   32,768:  1 row 31 / 37, 26 / 23, 18 / 19;  8 rows 34 / 38, 28 / 24, 18 / 20;  32 rows 36 / 38, 30 / 24, 19 / 20
-//   49,152:  8 rows 36 / 50, 27 / 28, 19 / 25;  32 rows 40 / 51, 32 / 28, 21 / 26;  64 rows 47 / 50, 36 / 29, 24 / 27
-//   73,448:  1 row 33 / 65, 25 / 34, 19 / 34;  32 rows 47 / 68, 35 / 34, 25 / 35;  64 rows 55 / 68, 42 / 34, 29 / 35
-//   122,753: 5 rows 42 / 102, 28 / 45, 21 / 51;  32 rows 60 / 108, 39 / 45, 30 / 56;  64 rows 66 / 113, 44 / 49, 34 / 61;
-//            96 rows 80 / 116, 55 / 50, 43 / 62
+//   32,768:  1 row 31 / 37, 26 / 15, 18 / 20;  8 rows 34 / 38, 28 / 17, 18 / 20;  32 rows 36 / 38, 30 / 17, 19 / 20  (chunks: before their
+//            kernels were made shorter)
+//   49,152:  8 rows 27 / 49, 26 / 17, 17 / 26;  32 rows 32 / 50, 31 / 18, 20 / 26;  64 rows 47 / 52, 36 / 18, 24 / 28
+//   73,448:  1 row 26 / 65, 24 / 19, 17 / 34;  32 rows 39 / 68, 35 / 20, 22 / 35;  64 rows 55 / 69, 42 / 20, 29 / 36
+//   122,753: 5 rows 30 / 103, 26 / 24, 17 / 56;  32 rows 45 / 105, 41 / 25, 25 / 56;  64 rows 53 / 111, 43 / 27, 32 / 62;
+//            96 rows 80 / 115, 55 / 29, 43 / 63
+// A caller who knows that every row asks for a top-k of at most FEW_K gives no workspace and has them by one workgroup each.
 #define CHUNKS_FROM 40960
 #define CHUNKS_MANY_FROM 98304      // ... with more than 32 rows, up to 64
 extern "C" long ilm_sample_ws(int n, int V) {
     if (V <= CHUNKS_FROM || n > (V > CHUNKS_MANY_FROM ? 64 : 32)) return 0;
     return (long)(sizeof(RowWork) + sizeof(u64) * ((V + 255) / 256) + 15) / 16 * 16;
+}
+
+// The largest top-k that a row is served with in one reading (top_k_of_few)
+extern "C" int ilm_sample_few_k() { return FEW_K; }
+
+static inline uint64_t mix64(uint64_t x) {   // splitmix64's finaliser
+    x += 0x9E3779B97F4A7C15ull;
+    x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+    x = (x ^ (x >> 27)) * 0x94D2049BB133111Bull;
+    return x ^ (x >> 31);
+}
+
+// On the host: out[i] = the uniform number of (seeds[i], keys[i], indices[i]), n of each; `seeds` null: `seed` for all
+extern "C" int ilm_uniforms(float* out, const uint64_t* seeds, uint64_t seed, const uint64_t* keys, const uint64_t* indices, int n) {
+    ILM_REQUIRE(n >= 0 && (n == 0 || (out != nullptr && keys != nullptr && indices != nullptr)), "uniforms: bad arguments, n=%d", n);
+    for (int i = 0; i < n; ++i) {
+        const uint64_t x = mix64(mix64(mix64(seeds != nullptr ? seeds[i] : seed) ^ keys[i]) ^ indices[i]);
+        out[i] = (float)(x >> 40) / 16777216.0f;
+    }
+    return 0;
 }
 
 // `ws`: n * ilm_sample_ws(n, V) bytes, 16-byte aligned, or null: every row by one workgroup

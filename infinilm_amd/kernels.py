@@ -870,12 +870,40 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
             raise KernelError(f"{nm} must be float32 with one entry a row")
     if top_k.numel() != n:
         raise KernelError("top_k must have one entry a row")
+    return _sample(logits, temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(), uniform.data_ptr(), False)
+
+
+def sample_packed(logits: torch.Tensor, params: torch.Tensor, few: bool = False) -> torch.Tensor:
+    """`sample` with the rows' parameters one after the other in one float32 tensor [4, rows]: temperature, top_k (the bits of
+    an int32), top_p, u.  `few`: every row asks for a top-k of 2 to `ilm_sample_few_k()` (or is greedy), so one reading of a row by one
+    workgroup gives its token and long rows need not be cut into chunks."""
+    _dev(logits, params)
+    if logits.dtype != F32 or logits.dim() != 2 or logits.stride(1) != 1:
+        raise KernelError("sample takes float32 rows")
+    n = logits.shape[0]
+    if params.dtype != F32 or params.numel() != 4 * n or not params.is_contiguous():
+        raise KernelError("the rows' parameters are float32, four a row")
+    p = params.data_ptr()
+    return _sample(logits, p, p + 4 * n, p + 8 * n, p + 12 * n, few)
+
+
+def _sample(logits: torch.Tensor, temperature: int, top_k: int, top_p: int, uniform: int, few: bool) -> torch.Tensor:
+    n, V = logits.shape
     out = torch.empty((n,), dtype=torch.int32, device=logits.device)
-    per_row = _lib().ilm_sample_ws(n, V)
+    per_row = 0 if few else _lib().ilm_sample_ws(n, V)
     ws = torch.empty((n * per_row,), dtype=torch.uint8, device=logits.device) if per_row else None
-    _run("ilm_sample", out.data_ptr(), logits.data_ptr(), temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(),
-         uniform.data_ptr(), _ptr(ws), n, V, logits.stride(0), _stream())
+    _run("ilm_sample", out.data_ptr(), logits.data_ptr(), temperature, top_k, top_p, uniform, _ptr(ws), n, V, logits.stride(0), _stream())
     return out
+
+
+def sample_few_k() -> int:
+    return _lib().ilm_sample_few_k()
+
+
+def uniforms(out: int, seeds: Optional[int], seed: int, keys: int, indices: int, n: int) -> None:
+    """Host addresses: float32 out[n] = the uniform numbers of (seeds[i], keys[i], indices[i]), each 64 bits; no `seeds`: `seed` for all."""
+    if _lib().ilm_uniforms(out, seeds, seed, keys, indices, n) != 0:
+        raise KernelError(_libmod.last_error())
 
 
 # ---- operands in fragment order (csrc/frag.h): the products of a decode step ------------------------------

@@ -1052,3 +1052,39 @@ def test_argmax_and_sampling(K):
     top = set(torch.topk(logits[0], 3).indices.tolist())
     for u in (0.01, 0.4, 0.99):
         assert run(1.5, 3, 1.0, u, logits[:1])[0] in top
+
+
+@pytest.mark.parametrize("V", [4095, 4096, 4099, 40003, 122753])
+@pytest.mark.parametrize("name", ["normal", "few values", "mostly masked", "close together", "sorted", "NaN", "infinity"])
+def test_sampling_top_k_of_few(K, name, V):
+    """A top-k that one reading of a row may give, at the ends of its range and of the lists it takes, beside rows that it leaves to the
+    histograms: the plain distribution's intervals (within 1e-6, see test_sampling_where_thresholds_are_hard), and where NaN and infinities leave
+    none, the tokens that rows in chunks give."""
+    g = torch.Generator().manual_seed(V + 1)
+    row = {"normal": lambda: torch.randn(V, generator=g) * 2,
+           "few values": lambda: torch.randint(0, 40, (V,), generator=g).float(),
+           "mostly masked": lambda: torch.where(torch.rand(V, generator=g) < 0.99, -math.inf, torch.randn(V, generator=g)),
+           "close together": lambda: 3.0 + torch.randn(V, generator=g) * 1e-4,
+           "sorted": lambda: torch.randn(V, generator=g).sort().values,
+           "NaN": lambda: torch.where(torch.rand(V, generator=g) < 0.1, math.nan, torch.randn(V, generator=g)),
+           "infinity": lambda: torch.randn(V, generator=g)}[name]()
+    if name == "infinity":
+        row[V // 3], row[V // 2] = math.inf, -math.inf
+    most = K.sample_few_k()
+    us = [0.0, 0.3, 0.71, 1.0 - 2.0 ** -24]
+    n = len(us)
+    mk = lambda v, dt: torch.tensor(v, dtype=dt, device=DEV)
+    rows = row.expand(n, V).contiguous().to(DEV)
+    for k in (2, 3, 50, 63, 64, 65, 128, most, most + 1):
+        for p in (1.0, 0.9, 1e-3):
+            prm = torch.cat([mk([0.8] * n, torch.float32), mk([k] * n, torch.int32).view(torch.float32), mk([p] * n, torch.float32), mk(us, torch.float32)])
+            one, cut = K.sample_packed(rows, prm, few=True).tolist(), K.sample_packed(rows, prm).tolist()
+            assert one == cut
+            if name in ("NaN", "infinity"):
+                assert all(row[t] == row[t] for t in one)
+                continue
+            dist = P.plain_sample_distribution(row, 0.8, k, p)
+            cdf = torch.cumsum(dist, 0)
+            for u, tok in zip(us, one):
+                assert 0 <= tok < V and dist[tok] > 0, f"token {tok} is outside the kept set (k={k}, p={p})"
+                assert float(cdf[tok] - dist[tok]) - 1e-6 <= u <= float(cdf[tok]) + 1e-6
