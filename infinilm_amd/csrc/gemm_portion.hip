@@ -1,0 +1,327 @@
+// bfloat16 products of portions of prompts, C[M,N] = X[M,K] W[N,K]^T (+ bias), where the outputs make about one round of tiles over the
+// chip: beyond that the vendor library's tiles win, which keep the matrix cores busier (1.4 PFLOP/s against 1.2 at 2048 x 32768 x
+// 4096).  K in steps of 64, whose rows of X and W go from memory into LDS without passing through registers, NS stages deep; the
+// second half of a stage is read while the first is multiplied, and the next stage's first half while the second is.
+//
+// What bounds it: with one tile a compute unit a chain of K / 64 stages (0.28 us each for 128 x 64 outputs, of which the matrix cores are
+// busy 0.1), the start and the end.  So tiles are chosen to fill the chip once (kernels.py), stages are as many as LDS holds, and the results
+// leave through LDS in whole lines (eight bytes a lane straight from the sums: 2048 x 1024 x 1024 10.9 us, now 9.1; 2048 x 8192 x 1024 49.8, now 34.9).
+//
+// Three forms: the product alone; act(gate) * up of a feed-forward's first product (the rows of W are taken so that a lane holds gate
+// and up of the same outputs); and the fused q | k | v projection with rotation and the write into the paged cache.  us, against the vendor
+// library's product (and the kernel after it):
+//   product   2048 x 1024 x 1024  9.1 / 10.7, x 4096 23.9 / 25.9; 1000 x 2048 x 2048 13.6 / 16.5; 300 x 1024 x 1024 5.6 / 7.1; 100 x 8192 x 1024 6.5 / 9.8
+//   gate, up  2048 x 8192 x 1024 40.0 / 42.5; 1000 rows 23.6 / 27.7; 300 rows 12.6 / 17.4; 100 rows 9.2 / 12.4
+//   q, k, v   2048 x 1280 x 1024 18.7 / 20.1; 1000 rows 11.2 / 15.2; 300 rows 7.5 / 10.2; 300 x 4608 x 4096 23.8 / 27.7
+// An output's sum runs over K in steps of 32 from the first on, whatever the form and the tile.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((address_space(3))) void* lds_ptr;
+
+#define GP_BK 64   // k a stage: a row is one 128-byte line
+
+enum { GP_PLAIN = 0, GP_GLU = 1, GP_ROPE = 2 };
+
+struct GpArgs {
+    const bf16* X;
+    const bf16* W;
+    const bf16* bias;
+    bf16* C;
+    int M, N, K;        // N: output columns a row of C (GLU: W has 2 N rows)
+    int lda, ldw, ldc;
+    int m_tiles, n_tiles;
+    int glu;
+    // rope
+    const int* pos;
+    const float* cosT;
+    const float* sinT;
+    bf16* kc;
+    bf16* vc;
+    const int* slots;
+    int nh, nkv, d, page;
+};
+
+__device__ __forceinline__ f32x4 gp_mfma(uint4 a, uint4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// The row of W that stands at place j of tile nt
+template <int BN, int WN, int EPI>
+__device__ __forceinline__ int gp_w_row(const GpArgs& A, int nt, int j) {
+    if (EPI == GP_PLAIN) {
+        const int n = nt * BN + j;
+        return n < A.N ? n : A.N - 1;
+    }
+    const int seg = j / WN, jj = j % WN, second = jj / (WN / 2), p = nt * (BN / 2) + seg * (WN / 2) + jj % (WN / 2);
+    if (EPI == GP_GLU) return (p < A.N ? p : A.N - 1) + second * A.N;
+    const int half = A.d / 2, pairs = A.N / 2, pc = p < pairs ? p : pairs - 1;
+    return pc / half * A.d + pc % half + second * half;
+}
+
+template <int BM, int BN, int WM, int WN, int NS, int EPI>
+__global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64, 2)
+gemm_portion_kernel(const GpArgs A) {
+    constexpr int NW = (BM / WM) * (BN / WN), ROWS = BM + BN, GROUPS = ROWS / 8, PER = GROUPS / NW, TM = WM / 16, TN = WN / 16;
+    static_assert(GROUPS % NW == 0 && (BN / 8) % NW == 0, "whole loads");
+    constexpr int OUT = EPI == GP_GLU ? BN / 2 : BN, PITCH = OUT + 8;   // columns a tile gives, elements between its rows in LDS
+    constexpr int STAGES = NS * ROWS * GP_BK, STAGED = EPI == GP_ROPE ? 0 : BM * PITCH;
+    __shared__ __align__(16) bf16 lds[STAGES > STAGED ? STAGES : STAGED];   // [stage][rows of W, then rows of X][64]; at the end the tile's results
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, q = lane >> 4;
+    int mt, nt;
+    {
+        const int total = A.m_tiles * A.n_tiles, per = total >> 3, rem = total & 7, xcd = blockIdx.x & 7;
+        const int id = xcd * per + (xcd < rem ? xcd : rem) + ((int)blockIdx.x >> 3);
+        mt = id % A.m_tiles;
+        nt = id / A.m_tiles;
+    }
+    const int m0 = mt * BM;
+    const int wn = wave % (BN / WN), wm = wave / (BN / WN);
+
+    const int lrow = lane >> 3, piece = (lane & 7) ^ lrow;
+    uint32_t from[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int row = (wave + NW * i) * 8 + lrow;
+        if (NW * i < BN / 8) {
+            from[i] = (uint32_t)gp_w_row<BN, WN, EPI>(A, nt, row) * ((uint32_t)A.ldw * 2u) + piece * 16;
+        } else {
+            const int m = m0 + row - BN;
+            from[i] = (uint32_t)(m < A.M ? m : A.M - 1) * ((uint32_t)A.lda * 2u) + piece * 16;
+        }
+    }
+    const char* wb = reinterpret_cast<const char*>(A.W);
+    const char* xb = reinterpret_cast<const char*>(A.X);
+    // (The compiler waits for all loads into LDS before it reads any of it, so these are written out and waited for by number.  They have no
+    // register to deliver to, and nothing else here uses m0.)
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)(&lds[0]) + (uint32_t)wave * 1024;
+    auto issue = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + (uint32_t)(buf * ROWS * 128 + NW * i * 1024)),
+                         "v"(from[i]), "s"(NW * i < BN / 8 ? wb : xb)
+                         : "memory");
+        wb += GP_BK * 2;
+        xb += GP_BK * 2;
+    };
+    f32x4 acc[TN][TM];
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int g = 0; g < TM; ++g) acc[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int stages = A.K / GP_BK;
+    const int sw = r & 7;
+    uint4 a[2][TN], b[2][TM];
+    auto read = [&](int s, int buf) {
+        const uint4* base = reinterpret_cast<const uint4*>(&lds[0]) + buf * (ROWS * 8) + ((s * 4 + q) ^ sw);
+        const uint4* ws = base + (wn * WN + r) * 8;
+        const uint4* xs = base + (BN + wm * WM + r) * 8;
+#pragma unroll
+        for (int t = 0; t < TN; ++t) a[s][t] = ws[t * 128];
+#pragma unroll
+        for (int g = 0; g < TM; ++g) b[s][g] = xs[g * 128];
+    };
+    auto multiply = [&](int s) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < TM; ++g)
+#pragma unroll
+            for (int t = 0; t < TN; ++t) acc[t][g] = gp_mfma(a[s][t], b[s][g], acc[t][g]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int ahead = stages < NS ? stages : NS;
+    for (int i = 0; i < ahead; ++i) issue(i);
+    if (stages > NS - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * PER) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0);
+    int buf = 0, st = 0;
+    for (; st + NS < stages; ++st) {
+        read(1, buf);
+        multiply(0);
+        // stage st + 1 has landed (this wave's part), and this wave is done with stage st's buffer
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * PER) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        issue(buf);
+        buf = buf + 1 == NS ? 0 : buf + 1;
+        read(0, buf);
+        multiply(1);
+    }
+    for (; st + 1 < stages; ++st) {
+        read(1, buf);
+        multiply(0);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        buf = buf + 1 == NS ? 0 : buf + 1;
+        read(0, buf);
+        multiply(1);
+    }
+    read(1, buf);
+    multiply(0);
+    multiply(1);
+    // acc[t][g][e] of lane (r, q): row wm WM + 16 g + r of the tile, place wn WN + 16 t + 4 q + e
+    if (EPI == GP_ROPE) {
+        const int half = A.d / 2, pairs = A.N / 2;
+#pragma unroll
+        for (int g = 0; g < TM; ++g) {
+            const int m = m0 + wm * WM + g * 16 + r;
+            if (m >= A.M) continue;
+            const int p_m = A.pos[m], slot = A.slots != nullptr ? A.slots[m] : -1;
+#pragma unroll
+            for (int t = 0; t < TN / 2; ++t) {
+                const int pair = nt * (BN / 2) + wn * (WN / 2) + t * 16 + 4 * q;   // (16 pairs from a multiple of 16 on: one head's)
+                if (pair >= pairs) continue;
+                const int hs = pair / half, i0 = pair % half;
+                float v[2][4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        v[h][e] = to_f32(from_f32<bf16>(acc[t + h * (TN / 2)][g][e] + (A.bias != nullptr ? to_f32(A.bias[hs * A.d + h * half + i0 + e]) : 0.f)));
+                if (hs >= A.nh + A.nkv) {   // values, cached transposed
+                    if (slot < 0) continue;
+                    bf16* dst = A.vc + ((size_t)(slot / A.page) * A.nkv + (hs - A.nh - A.nkv)) * A.d * A.page + (slot % A.page);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        dst[(size_t)(i0 + e) * A.page] = from_f32<bf16>(v[0][e]);
+                        dst[(size_t)(i0 + half + e) * A.page] = from_f32<bf16>(v[1][e]);
+                    }
+                    continue;
+                }
+                const float4 cs = *reinterpret_cast<const float4*>(A.cosT + (size_t)p_m * half + i0);
+                const float4 sn = *reinterpret_cast<const float4*>(A.sinT + (size_t)p_m * half + i0);
+                const float c4[4] = {cs.x, cs.y, cs.z, cs.w}, s4[4] = {sn.x, sn.y, sn.z, sn.w};
+                bf16 o[2][4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    o[0][e] = from_f32<bf16>(v[0][e] * c4[e] - v[1][e] * s4[e]);
+                    o[1][e] = from_f32<bf16>(v[1][e] * c4[e] + v[0][e] * s4[e]);
+                }
+                bf16* dst;
+                if (hs < A.nh) dst = A.C + (size_t)m * A.ldc + (size_t)hs * A.d + i0;
+                else if (slot >= 0) dst = A.kc + (((size_t)(slot / A.page) * A.nkv + (hs - A.nh)) * A.page + (slot % A.page)) * A.d + i0;
+                else continue;
+                *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(o[0]);
+                *reinterpret_cast<uint2*>(dst + half) = *reinterpret_cast<const uint2*>(o[1]);
+            }
+        }
+        return;
+    }
+    // The results go to memory through LDS, whole lines of a row at a time
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < TM; ++g) {
+        const int row = wm * WM + g * 16 + r;
+#pragma unroll
+        for (int t = 0; t < (EPI == GP_GLU ? TN / 2 : TN); ++t) {
+            const int col = wn * (EPI == GP_GLU ? WN / 2 : WN) + t * 16 + 4 * q;
+            bf16 o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (EPI == GP_GLU) {
+                    float vg = acc[t][g][e], vu = acc[t + TN / 2][g][e];
+                    if (A.bias != nullptr) {
+                        const int n = nt * OUT + col + e, ne = n < A.N ? n : A.N - 1;
+                        vg += to_f32(A.bias[ne]);
+                        vu += to_f32(A.bias[ne + A.N]);
+                    }
+                    // (gate and up rounded to bfloat16 first, as the product's kernel alone stores them)
+                    o[e] = from_f32<bf16>(glu_act(to_f32(from_f32<bf16>(vg)), A.glu) * to_f32(from_f32<bf16>(vu)));
+                } else {
+                    float v = acc[t][g][e];
+                    if (A.bias != nullptr) {
+                        const int n = nt * OUT + col + e;
+                        v += to_f32(A.bias[n < A.N ? n : A.N - 1]);
+                    }
+                    o[e] = from_f32<bf16>(v);
+                }
+            }
+            *reinterpret_cast<uint2*>(&lds[row * PITCH + col]) = *reinterpret_cast<const uint2*>(o);
+        }
+    }
+    __syncthreads();
+    constexpr int P8 = OUT / 8;   // 16-byte pieces a row
+    const bool vec = (A.ldc & 7) == 0 && ((uintptr_t)A.C & 15) == 0;
+#pragma unroll 4
+    for (int i = tid; i < BM * P8; i += NW * 64) {
+        const int row = i / P8, m = m0 + row, n = nt * OUT + i % P8 * 8;
+        if (m >= A.M) break;
+        const bf16* from = &lds[row * PITCH + i % P8 * 8];
+        bf16* dst = A.C + (size_t)m * A.ldc + n;
+        if (vec && n + 7 < A.N) {
+            *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(from);
+        } else {
+            for (int e = 0; e < 8; ++e)
+                if (n + e < A.N) dst[e] = from[e];
+        }
+    }
+}
+
+// tile: 1: 64 x 64 outputs (gate, up: 64 x 128 rows of W), 2: 128 x 64, 3: 128 x 128, 4: 256 x 128, 5: 256 x 256
+#define GP_RUN(BM_, BN_, WM_, WN_, NS_, EPI_, NCOLS_)                                                       \
+    {                                                                                                       \
+        a.m_tiles = (a.M + BM_ - 1) / BM_;                                                                  \
+        a.n_tiles = ((NCOLS_) + BN_ - 1) / BN_;                                                             \
+        ILM_REQUIRE((long long)a.m_tiles * a.n_tiles < (1ll << 31), "gemm_portion: too many tiles");        \
+        gemm_portion_kernel<BM_, BN_, WM_, WN_, NS_, EPI_>                                                  \
+            <<<a.m_tiles * a.n_tiles, (BM_ / WM_) * (BN_ / WN_) * 64, 0, stream>>>(a);                      \
+    }
+
+static int gp_check(const char* what, int M, int rows, int K, const void* X, int lda, const void* W, int ldw) {
+    ILM_REQUIRE(M > 0 && rows > 0 && K > 0 && K % GP_BK == 0, "%s: bad sizes M=%d rows of W=%d K=%d (K in steps of 64)", what, M, rows, K);
+    ILM_REQUIRE(lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K, "%s: K=%d lda=%d ldw=%d", what, K, lda, ldw);
+    ILM_REQUIRE(((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0, "%s: operands must be 16-byte aligned", what);
+    // (a row's place is 32 bits of bytes)
+    ILM_REQUIRE((long long)M * lda < (1ll << 31) && (long long)rows * ldw < (1ll << 31), "%s: operands beyond 4 GiB", what);
+    return 0;
+}
+
+// C [M, ldc] = X W^T + bias (`glu` < 0: W has N rows), or act(X Wg^T + bg) * (X Wu^T + bu), W = [Wg; Wu] of 2 N rows, `glu` the gate's activation
+extern "C" int ilm_gemm_portion(void* C, int ldc, const void* X, int lda, const void* W, int ldw, const void* bias, int M, int N, int K,
+                                int glu, int tile, hipStream_t stream) {
+    if (gp_check("gemm_portion", M, glu < 0 ? N : 2 * N, K, X, lda, W, ldw)) return -1;
+    ILM_REQUIRE(ldc >= N && N < (1 << 30), "gemm_portion: N=%d ldc=%d", N, ldc);
+    GpArgs a = {};
+    a.X = (const bf16*)X; a.W = (const bf16*)W; a.bias = (const bf16*)bias; a.C = (bf16*)C;
+    a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldw = ldw; a.ldc = ldc; a.glu = glu;
+    if (glu < 0) {
+        ILM_REQUIRE(tile >= 1 && tile <= 3, "gemm_portion: there is no tile %d", tile);
+        if (tile == 1) GP_RUN(64, 64, 32, 32, 4, GP_PLAIN, N)
+        else if (tile == 2) GP_RUN(128, 64, 32, 32, 3, GP_PLAIN, N)
+        else GP_RUN(128, 128, 64, 32, 4, GP_PLAIN, N)
+    } else {
+        ILM_REQUIRE(tile == 1 || tile == 4 || tile == 5, "gemm_portion: there is no tile %d", tile);
+        if (tile == 1) GP_RUN(64, 128, 32, 64, 3, GP_GLU, 2 * N)
+        else if (tile == 4) GP_RUN(256, 128, 64, 64, 3, GP_GLU, 2 * N)
+        else GP_RUN(256, 256, 128, 64, 2, GP_GLU, 2 * N)
+    }
+    ILM_LAUNCH_CHECK("gemm_portion");
+    return 0;
+}
+
+// Q [M, ldq] receives the rotated query heads; k (rotated) and v go to the cache slots (slots may be
+// null: nothing is cached; a slot below 0: that token is not).  W [(nh + 2 nkv) d, ldw] holds the q, k, v rows in this order.
+extern "C" int ilm_gemm_portion_rope(void* Q, int ldq, const void* X, int lda, const void* W, int ldw, const void* bias,
+                                     int M, int K, const void* pos, const void* cosT, const void* sinT, void* kc, void* vc,
+                                     const void* slots, int nh, int nkv, int d, int page, int tile, hipStream_t stream) {
+    ILM_REQUIRE(nh > 0 && nkv >= 0 && d > 0 && d % 32 == 0 && (long long)(nh + 2 * nkv) * d < (1 << 30),
+                "gemm_portion_rope: %d + 2 x %d heads of %d", nh, nkv, d);
+    if (gp_check("gemm_portion_rope", M, (nh + 2 * nkv) * d, K, X, lda, W, ldw)) return -1;
+    ILM_REQUIRE(ldq >= nh * d && ldq % 4 == 0 && ((uintptr_t)Q & 7) == 0, "gemm_portion_rope: ldq=%d", ldq);
+    ILM_REQUIRE(pos != nullptr && ((uintptr_t)cosT & 15) == 0 && ((uintptr_t)sinT & 15) == 0, "gemm_portion_rope: tables must be 16-byte aligned");
+    ILM_REQUIRE(slots == nullptr || (page > 0 && kc != nullptr && vc != nullptr && ((uintptr_t)kc & 7) == 0), "gemm_portion_rope: cache missing");
+    ILM_REQUIRE(tile == 1 || tile == 2, "gemm_portion_rope: there is no tile %d", tile);
+    GpArgs a = {};
+    a.X = (const bf16*)X; a.W = (const bf16*)W; a.bias = (const bf16*)bias; a.C = (bf16*)Q;
+    a.M = M; a.N = (nh + 2 * nkv) * d; a.K = K; a.lda = lda; a.ldw = ldw; a.ldc = ldq;
+    a.pos = (const int*)pos; a.cosT = (const float*)cosT; a.sinT = (const float*)sinT; a.kc = (bf16*)kc; a.vc = (bf16*)vc;
+    a.slots = (const int*)slots; a.nh = nh; a.nkv = nkv; a.d = d; a.page = page;
+    if (tile == 1) GP_RUN(64, 64, 32, 32, 4, GP_ROPE, a.N)
+    else GP_RUN(128, 64, 32, 32, 3, GP_ROPE, a.N)
+    ILM_LAUNCH_CHECK("gemm_portion_rope");
+    return 0;
+}

@@ -227,7 +227,12 @@ def qkv_rope_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]
     if not (USE_QKV_ROPE and not FORCE_BASIC and x.dtype == BF16 and w.dtype == BF16 and _few_rows(M, K) and rd == d and d % 32 == 0
             and K % 8 == 0 and K <= 8192 and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0
             and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
-        return None
+        # a portion of a prompt (rows beyond the few), where its tiles make about one round
+        tile = 0
+        if (USE_QKV_ROPE and x.dtype == BF16 and M > FRAG_MAX_ROWS and rd == d and d % 32 == 0 and _portion_operands_ok(x, w)
+                and cos.data_ptr() % 16 == 0 and sin.data_ptr() % 16 == 0):
+            tile = _portion_tile("rope", M, w.shape[0], K, x.device)
+        return _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d, tile) if tile else None
     return _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)
 
 
@@ -240,7 +245,7 @@ def qkv_rope_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
     return _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)
 
 
-def _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d):
+def _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d, tile=0):
     M, K = x.shape
     _dev(x, w, bias, positions, cos, sin, k_cache, v_cache, slots)
     _i32(positions, "positions")
@@ -258,10 +263,71 @@ def _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv,
             raise KernelError("cache tensors missing or of another dtype than the activations")
         page = _check_cache(k_cache, v_cache, nkv, d)
     q = torch.empty((M, nh * d), dtype=x.dtype, device=x.device)
-    _run("ilm_gemm_qkv_rope" if x.dtype == BF16 else "ilm_gemm_f32_rope", q.data_ptr(), q.stride(0), x.data_ptr(), x.stride(0),
-         w.data_ptr(), w.stride(0), _ptr(bias), M, K, positions.data_ptr(), cos.data_ptr(), sin.data_ptr(), _ptr(k_cache) if slots is not None else None,
-         _ptr(v_cache) if slots is not None else None, _ptr(slots), nh, nkv, d, page, _stream())
+    args = (q.data_ptr(), q.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), _ptr(bias), M, K, positions.data_ptr(),
+            cos.data_ptr(), sin.data_ptr(), _ptr(k_cache) if slots is not None else None, _ptr(v_cache) if slots is not None else None,
+            _ptr(slots), nh, nkv, d, page)
+    if tile:
+        _run("ilm_gemm_portion_rope", *args, tile, _stream())
+    else:
+        _run("ilm_gemm_qkv_rope" if x.dtype == BF16 else "ilm_gemm_f32_rope", *args, _stream())
     return q
+
+
+USE_PORTION = os.environ.get("INFINILM_AMD_PORTION", "1") == "1"   # 0: portions' products by the vendor library
+
+
+def _portion_tile(form: str, M: int, rows: int, K: int, device) -> int:
+    """The tile with which a portion's product (gemm_portion.hip) is faster than the vendor library's (and the kernel after it), 0 for
+    none: `form` "plain", "glu" or "rope", `rows` of W.  The line lies where the tiles come to more than a round over the chip: the library's
+    larger tiles then use it better, and a smaller tile's second round costs as much as the first.
+
+    plain: the smallest tile of which one round does (64 x 64, 128 x 64, 128 x 128).  K up to 4096: 2048 x 2048 x 8192 75.2 us against 75.7,
+    600 x 4096 x 16384 130 / 126; and with fewer than half of the units busy up to 2048, as the library cuts a long K (300 x 1024 x 4096, 80 tiles,
+    14.2 / 13.8; 700 x 1024 x 4096, 176 tiles, 14.8 / 17.8).  Two rounds: 700 x 8192 x 1024 18.2 / 18.0, 2048 x 12288 x 2048 106 / 100.
+    glu: K up to 1024 (1000 x 12288 x 2048 57.9 / 56.0, 400 rows 34.5 / 35.1).  A round of the large tiles that leaves less than a quarter of
+    the chip idle, else the small ones up to three rounds (two share a unit): 700 x 8192 x 1024 19.9 / 23.1, 300 rows 12.6 / 17.4.
+    rope: five quarters of a round (tiles end unevenly): 2048 x 1280 x 1024, 320 tiles, 18.7 / 20.1; 300 x 4608 x 4096, 216 tiles, 23.8 / 27.7;
+    more lose: 2047 x 4608 x 4096 119 / 79, 2048 x 6912 x 2304 128 / 117."""
+    if not USE_PORTION or K % 64:
+        return 0
+    cus = _num_cus(device)
+    count = lambda bm, bn: -(-M // bm) * -(-rows // bn)
+    if form == "glu":
+        if K > 1024:
+            return 0
+        for tile, bm, bn in ((5, 256, 256), (4, 256, 128)):
+            if 4 * count(bm, bn) > 3 * cus and count(bm, bn) <= cus:
+                return tile
+        return 1 if count(64, 128) <= 3 * cus else 0
+    if K > 4096:
+        return 0
+    if form == "rope":
+        return next((tile for tile, bm in ((1, 64), (2, 128)) if 4 * count(bm, 64) <= 5 * cus), 0)
+    for tile, bm, bn in ((1, 64, 64), (2, 128, 64), (3, 128, 128)):
+        n = count(bm, bn)
+        if n <= cus:
+            return tile if 2 * n > cus or K <= 2048 else 0
+    return 0
+
+
+def _portion_operands_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    return (_mfma_operands_ok(x, w, x.shape[1]) and not FORCE_BASIC and x.shape[0] * x.stride(0) < 1 << 31 and w.shape[0] * w.stride(0) < 1 << 31)
+
+
+def portion_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, tile: int) -> torch.Tensor:
+    """out = x w^T (+ bias) by gemm_portion.hip, all bfloat16."""
+    _run("ilm_gemm_portion", out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), _ptr(bias), x.shape[0],
+         w.shape[0], x.shape[1], -1, tile, _stream())
+    return out
+
+
+def portion_glu(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], act: str, tile: int) -> torch.Tensor:
+    """act(x Wg^T + bg) * (x Wu^T + bu), W = [Wg; Wu], by gemm_portion.hip."""
+    M, I = x.shape[0], w.shape[0] // 2
+    out = torch.empty((M, I), dtype=BF16, device=x.device)
+    _run("ilm_gemm_portion", out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), _ptr(bias), M, I, x.shape[1],
+         glu_code(act), tile, _stream())
+    return out
 
 
 GLU_ACTIVATIONS = {"silu": 0, "gelu_tanh": 1}    # activations of a gated feed-forward's gate (glu_act in common.h)
@@ -422,6 +488,11 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, 
         _run("ilm_gemm_skinny", out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K, a.stride(0),
              w.stride(0), out.stride(0), float(alpha), 0, _DT[out_dtype], SKINNY_VARIANT, _stream())
         return out
+    # a portion of a prompt whose outputs make about one round of tiles over the chip
+    if fast and aligned and alpha == 1.0 and out_dtype == BF16 and M > 64 and not few and _portion_operands_ok(a, w):
+        tile = _portion_tile("plain", M, N, K, a.device)
+        if tile:
+            return portion_gemm(a, w, bias, out, tile)
     if M > 16 and fast and bias is not None and alpha == 1.0 and out_dtype == BF16 and USE_LIBRARY_GEMM:
         # many rows with a bias: the vendor library's product with the bias row as its addend
         with _timed("library_gemm"):
@@ -634,7 +705,16 @@ def gateup_swiglu_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Te
             and (resident or tall) and K % 8 == 0 and w.shape[0] % 2 == 0 and w.shape[1] == K
             and x.stride(1) == 1 and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0):
-        return None
+        # a portion of a prompt, or more decoded tokens than the kernels above take
+        tile = 0
+        if USE_GATEUP_SWIGLU and row_ss is None and M > 32 and w.shape[0] % 2 == 0 and _portion_operands_ok(x, w):
+            tile = _portion_tile("glu", M, w.shape[0], K, x.device)
+        if not tile:
+            return None
+        _dev(x, w, bias)
+        if bias is not None and (bias.shape != (w.shape[0],) or bias.dtype != BF16 or not bias.is_contiguous()):
+            raise KernelError("bias does not fit the fused gate/up projection")
+        return portion_glu(x, w, bias, act, tile)
     _dev(x, w, bias)
     I = w.shape[0] // 2
     if bias is not None and (bias.shape != (2 * I,) or bias.dtype != BF16 or not bias.is_contiguous()):

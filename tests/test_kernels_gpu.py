@@ -1088,3 +1088,88 @@ def test_sampling_top_k_of_few(K, name, V):
             for u, tok in zip(us, one):
                 assert 0 <= tok < V and dist[tok] > 0, f"token {tok} is outside the kept set (k={k}, p={p})"
                 assert float(cdf[tok] - dist[tok]) - 1e-6 <= u <= float(cdf[tok]) + 1e-6
+
+
+BF16 = torch.bfloat16
+PORTION_SIZES = [(33, 8, 64), (64, 200, 128), (65, 1000, 192), (127, 129, 256), (128, 64, 320), (129, 257, 448), (300, 520, 1024), (513, 1032, 576)]
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K_", PORTION_SIZES)
+def test_portion_product(K, M, N, K_, bias):
+    """Every tile at edges of rows, outputs and stages (fewer stages than the kernel holds, just as many, more), into rows of any stride.
+    An output is a float sum (off by at most K 2^-24 of the sum of its terms' sizes) rounded to bfloat16 (2^-8 of it)."""
+    g = torch.Generator().manual_seed(M * 31 + N)
+    x, w = (torch.randn(s, generator=g).to(BF16).to(DEV) for s in ((M, K_ + 8), (N, K_ + 16)))
+    x, w = x[:, 8:], w[:, :K_]
+    b = torch.randn(N, generator=g).to(BF16).to(DEV) if bias else None
+    want = x.double() @ w.double().T + (b.double() if bias else 0.0)
+    size = x.double().abs() @ w.double().abs().T + (b.double().abs() if bias else 0.0)
+    first = None
+    for tile in (1, 2, 3):
+        for pad in (0, 3, 8):
+            c = torch.full((M, N + pad), 7.0, dtype=BF16, device=DEV)
+            K.portion_gemm(x, w, b, c[:, :N], tile)
+            assert torch.equal(c[:, N:], torch.full_like(c[:, N:], 7.0))
+            err = (c[:, :N].double() - want).abs()
+            assert bool((err <= want.abs() * 2.0 ** -8 + size * K_ * 2.0 ** -23).all()), (tile, pad)
+            first = c[:, :N].clone() if first is None else first
+            assert torch.equal(c[:, :N], first), (tile, pad)     # one order of sums, whatever the tile
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("M,N,K_", PORTION_SIZES)
+def test_portion_gate_and_up(K, M, N, K_, act):
+    """The same sums as the product's, and the activation kernel's results on them."""
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn((M, K_), generator=g).to(BF16).to(DEV), (torch.randn((2 * N, K_), generator=g) / math.sqrt(K_)).to(BF16).to(DEV)
+    for b in (None, torch.randn(2 * N, generator=g).to(BF16).to(DEV)):
+        want = K.swiglu(K.portion_gemm(x, w, b, torch.empty((M, 2 * N), dtype=BF16, device=DEV), 1), act)
+        for tile in (1, 4, 5):
+            assert torch.equal(K.portion_glu(x, w, b, act, tile), want), tile
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(3, 1, 32), (4, 2, 64), (5, 5, 96), (8, 2, 128)])
+@pytest.mark.parametrize("M", [65, 130, 333])
+def test_portion_qkv(K, M, nh, nkv, d):
+    """The product's sums, and what the rotation's kernel makes of them, in the queries' rows and in the cache; tokens without a slot
+    write nothing.  The two kernels may round a rotated value differently by its last bit (a sum of two products, contracted or not)."""
+    g = torch.Generator().manual_seed(M + d)
+    K_, page, pages = 192, 16, M // 16 + 2
+    N = (nh + 2 * nkv) * d
+    x, w = torch.randn((M, K_), generator=g).to(BF16).to(DEV), (torch.randn((N, K_), generator=g) / math.sqrt(K_)).to(BF16).to(DEV)
+    cos, sin = (torch.randn((500, d // 2), generator=g).to(DEV) for _ in range(2))
+    pos = torch.randint(0, 500, (M,), generator=g, dtype=torch.int32).to(DEV)
+    slots = torch.randperm(page * pages, generator=g)[:M].to(torch.int32)
+    slots[::7] = -1
+    slots = slots.to(DEV)
+    for b in (None, torch.randn(N, generator=g).to(BF16).to(DEV)):
+        rows = K.portion_gemm(x, w, b, torch.empty((M, N), dtype=BF16, device=DEV), 1)
+        kc, vc = torch.zeros((pages, nkv, page, d), dtype=BF16, device=DEV), torch.zeros((pages, nkv, d, page), dtype=BF16, device=DEV)
+        K.rope_kvwrite(rows, pos, cos, sin, kc, vc, slots, nh, nkv, d, d)
+        for tile in (1, 2):
+            for s in (slots, None):
+                kc2, vc2 = torch.zeros_like(kc), torch.zeros_like(vc)
+                q = K._qkv_rope(x, w, b, pos, cos, sin, kc2, vc2, s, nh, nkv, d, tile)
+                near = lambda a, c: bool(((a.double() - c.double()).abs() <= c.double().abs() * 2.0 ** -7 + 1e-6).all())
+                assert near(q, rows[:, :nh * d])
+                if s is None:
+                    assert not kc2.any() and not vc2.any()
+                else:
+                    assert near(kc2, kc) and torch.equal(vc2, vc)
+
+
+def test_portion_rule(K):
+    """The rule takes what the kernels take: K in steps of 64, one round of tiles, and the public entry points go there and give
+    the library path's results to rounding."""
+    dev = torch.device(DEV)
+    assert K._portion_tile("plain", 2048, 1024, 1000, dev) == 0 and K._portion_tile("glu", 300, 8192, 2048, dev) == 0
+    for M, N, K_ in ((2048, 1024, 1024), (300, 1024, 1024), (65, 8192, 1024), (600, 4096, 2048)):
+        tile = K._portion_tile("plain", M, N, K_, dev)
+        assert tile in (1, 2, 3)
+        g = torch.Generator(device=DEV).manual_seed(M)
+        x, w = torch.randn((M, K_), generator=g, device=DEV).to(BF16), torch.randn((N, K_), generator=g, device=DEV).to(BF16)
+        want = x.float() @ w.float().T
+        got = K.gemm(x, w)
+        assert torch.equal(got, K.portion_gemm(x, w, None, torch.empty_like(got), tile))
+        assert float((got.float() - want).norm() / want.norm()) < 2.0 ** -8
