@@ -12,7 +12,7 @@
 // library's product (and the kernel after it):
 //   product   2048 x 1024 x 1024  9.1 / 10.7, x 4096 23.9 / 25.9; 1000 x 2048 x 2048 13.6 / 16.5; 300 x 1024 x 1024 5.6 / 7.1; 100 x 8192 x 1024 6.5 / 9.8
 //   gate, up  2048 x 8192 x 1024 40.0 / 42.5; 1000 rows 23.6 / 27.7; 300 rows 12.6 / 17.4; 100 rows 9.2 / 12.4
-//   q, k, v   2048 x 1280 x 1024 18.7 / 20.1; 1000 rows 11.2 / 15.2; 300 rows 7.5 / 10.2; 300 x 4608 x 4096 23.8 / 27.7
+//   q, k, v   2048 x 1280 x 1024 18.7 / 20.1; 1000 rows 10.6 / 15.1; 300 rows 7.3 / 10.3; 300 x 4608 x 4096 23.8 / 27.7
 // An output's sum runs over K in steps of 32 from the first on, whatever the form and the tile.
 #include "common.h"
 
@@ -66,7 +66,7 @@ gemm_portion_kernel(const GpArgs A) {
     constexpr int NW = (BM / WM) * (BN / WN), ROWS = BM + BN, GROUPS = ROWS / 8, PER = GROUPS / NW, TM = WM / 16, TN = WN / 16;
     static_assert(GROUPS % NW == 0 && (BN / 8) % NW == 0, "whole loads");
     constexpr int OUT = EPI == GP_GLU ? BN / 2 : BN, PITCH = OUT + 8;   // columns a tile gives, elements between its rows in LDS
-    constexpr int STAGES = NS * ROWS * GP_BK, STAGED = EPI == GP_ROPE ? 0 : BM * PITCH;
+    constexpr int STAGES = NS * ROWS * GP_BK, STAGED = BM * PITCH;
     __shared__ __align__(16) bf16 lds[STAGES > STAGED ? STAGES : STAGED];   // [stage][rows of W, then rows of X][64]; at the end the tile's results
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, q = lane >> 4;
     int mt, nt;
@@ -165,15 +165,16 @@ gemm_portion_kernel(const GpArgs A) {
     multiply(1);
     // acc[t][g][e] of lane (r, q): row wm WM + 16 g + r of the tile, place wn WN + 16 t + 4 q + e
     if (EPI == GP_ROPE) {
+        // (values go straight into their transposed cache; queries and keys through LDS, first halves of pairs ahead of second halves)
         const int half = A.d / 2, pairs = A.N / 2;
+        __syncthreads();
 #pragma unroll
         for (int g = 0; g < TM; ++g) {
-            const int m = m0 + wm * WM + g * 16 + r;
-            if (m >= A.M) continue;
-            const int p_m = A.pos[m], slot = A.slots != nullptr ? A.slots[m] : -1;
+            const int row = wm * WM + g * 16 + r, m = m0 + row < A.M ? m0 + row : A.M - 1;
+            const int p_m = A.pos[m], slot = A.slots != nullptr && m0 + row < A.M ? A.slots[m] : -1;
 #pragma unroll
             for (int t = 0; t < TN / 2; ++t) {
-                const int pair = nt * (BN / 2) + wn * (WN / 2) + t * 16 + 4 * q;   // (16 pairs from a multiple of 16 on: one head's)
+                const int place = wn * (WN / 2) + t * 16 + 4 * q, pair = nt * (BN / 2) + place;   // (16 pairs from a multiple of 16 on: one head's)
                 if (pair >= pairs) continue;
                 const int hs = pair / half, i0 = pair % half;
                 float v[2][4];
@@ -182,7 +183,7 @@ gemm_portion_kernel(const GpArgs A) {
 #pragma unroll
                     for (int h = 0; h < 2; ++h)
                         v[h][e] = to_f32(from_f32<bf16>(acc[t + h * (TN / 2)][g][e] + (A.bias != nullptr ? to_f32(A.bias[hs * A.d + h * half + i0 + e]) : 0.f)));
-                if (hs >= A.nh + A.nkv) {   // values, cached transposed
+                if (hs >= A.nh + A.nkv) {
                     if (slot < 0) continue;
                     bf16* dst = A.vc + ((size_t)(slot / A.page) * A.nkv + (hs - A.nh - A.nkv)) * A.d * A.page + (slot % A.page);
 #pragma unroll
@@ -201,13 +202,24 @@ gemm_portion_kernel(const GpArgs A) {
                     o[0][e] = from_f32<bf16>(v[0][e] * c4[e] - v[1][e] * s4[e]);
                     o[1][e] = from_f32<bf16>(v[1][e] * c4[e] + v[0][e] * s4[e]);
                 }
-                bf16* dst;
-                if (hs < A.nh) dst = A.C + (size_t)m * A.ldc + (size_t)hs * A.d + i0;
-                else if (slot >= 0) dst = A.kc + (((size_t)(slot / A.page) * A.nkv + (hs - A.nh)) * A.page + (slot % A.page)) * A.d + i0;
-                else continue;
-                *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(o[0]);
-                *reinterpret_cast<uint2*>(dst + half) = *reinterpret_cast<const uint2*>(o[1]);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) *reinterpret_cast<uint2*>(&lds[row * PITCH + h * (BN / 2) + place]) = *reinterpret_cast<const uint2*>(o[h]);
             }
+        }
+        __syncthreads();
+        constexpr int P8 = BN / 8;
+        for (int i = tid; i < BM * P8; i += NW * 64) {   // (eight pairs from a multiple of eight on are one head's)
+            const int row = i / P8, m = m0 + row, h = i % P8 / (P8 / 2), place = i % (P8 / 2) * 8, pair = nt * (BN / 2) + place;
+            if (m >= A.M) break;
+            const int hs = pair / half, at = pair % half + h * half;
+            if (pair >= pairs || hs >= A.nh + A.nkv) continue;
+            bf16* dst = A.C + (size_t)m * A.ldc + (size_t)hs * A.d + at;
+            if (hs >= A.nh) {
+                const int slot = A.slots != nullptr ? A.slots[m] : -1;
+                if (slot < 0) continue;
+                dst = A.kc + (((size_t)(slot / A.page) * A.nkv + (hs - A.nh)) * A.page + (slot % A.page)) * A.d + at;
+            }
+            *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(&lds[row * PITCH + h * (BN / 2) + place]);
         }
         return;
     }
@@ -311,9 +323,9 @@ extern "C" int ilm_gemm_portion_rope(void* Q, int ldq, const void* X, int lda, c
     ILM_REQUIRE(nh > 0 && nkv >= 0 && d > 0 && d % 32 == 0 && (long long)(nh + 2 * nkv) * d < (1 << 30),
                 "gemm_portion_rope: %d + 2 x %d heads of %d", nh, nkv, d);
     if (gp_check("gemm_portion_rope", M, (nh + 2 * nkv) * d, K, X, lda, W, ldw)) return -1;
-    ILM_REQUIRE(ldq >= nh * d && ldq % 4 == 0 && ((uintptr_t)Q & 7) == 0, "gemm_portion_rope: ldq=%d", ldq);
+    ILM_REQUIRE(ldq >= nh * d && ldq % 8 == 0 && ((uintptr_t)Q & 15) == 0, "gemm_portion_rope: ldq=%d", ldq);
     ILM_REQUIRE(pos != nullptr && ((uintptr_t)cosT & 15) == 0 && ((uintptr_t)sinT & 15) == 0, "gemm_portion_rope: tables must be 16-byte aligned");
-    ILM_REQUIRE(slots == nullptr || (page > 0 && kc != nullptr && vc != nullptr && ((uintptr_t)kc & 7) == 0), "gemm_portion_rope: cache missing");
+    ILM_REQUIRE(slots == nullptr || (page > 0 && kc != nullptr && vc != nullptr && ((uintptr_t)kc & 15) == 0), "gemm_portion_rope: cache missing");
     ILM_REQUIRE(tile == 1 || tile == 2, "gemm_portion_rope: there is no tile %d", tile);
     GpArgs a = {};
     a.X = (const bf16*)X; a.W = (const bf16*)W; a.bias = (const bf16*)bias; a.C = (bf16*)Q;

@@ -74,6 +74,7 @@ _SIGNATURES = {
     "ilm_softcap": [_P, _L, _F, _P],
     "ilm_moe_route": [_P, _P, _P, _I, _I, _I, _I, _I, _F, _P],
     "ilm_moe_route_groups": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P],
+    "ilm_moe_plan_few": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _I, _I, _I, _P],
     "ilm_moe_sort": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "ilm_moe_gemm": [_P, _I, _P, _I, _P, _I, _P, _P, _L, _I, _P, _P, _I, _I, _I, _I, _F, _F, _I, _I, _I, _I, _I, _P],
     "ilm_moe_combine": [_P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _P, _P, _I, _I, _P],
@@ -149,6 +150,8 @@ def load(verbose: bool = True) -> ctypes.CDLL:
     lib.ilm_delta_chunk_ws.argtypes = [c_int, c_int]
     lib.ilm_sample_ws.restype = c_long
     lib.ilm_sample_ws.argtypes = [c_int, c_int]
+    lib.ilm_moe_plan_few_ok.restype = c_int
+    lib.ilm_moe_plan_few_ok.argtypes = [c_int, c_int, c_int]
     lib.ilm_sample_few_k.restype = c_int
     lib.ilm_sample_few_k.argtypes = []
     lib.ilm_attn_static_init.restype = c_int

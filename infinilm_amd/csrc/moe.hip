@@ -192,10 +192,10 @@ extern "C" int ilm_moe_route_groups(void* ids, void* wts, const void* z, const v
 }
 
 // ---- ordering by expert --------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(1024)
-moe_sort_kernel(int* __restrict__ offsets, int* __restrict__ perm, int* __restrict__ inv, int* __restrict__ tiles, int* __restrict__ n_tiles,
-                const int* __restrict__ ids, int P, int E, int max_tiles, int tile_rows) {
-    __shared__ int cnt[MOE_MAX_E], cur[MOE_MAX_E], tbase[MOE_MAX_E];
+// The pairs' order by expert, by a block of 1024: `ids` the pairs' experts (in memory or in LDS)
+__device__ __forceinline__ void moe_sort(int* __restrict__ offsets, int* __restrict__ perm, int* __restrict__ inv, int* __restrict__ tiles,
+                                         int* __restrict__ n_tiles, const int* ids, int P, int E, int max_tiles, int tile_rows, int* cnt, int* cur,
+                                         int* tbase) {
     const int tid = threadIdx.x;
     for (int e = tid; e < E; e += 1024) cnt[e] = 0;
     __syncthreads();
@@ -238,7 +238,101 @@ moe_sort_kernel(int* __restrict__ offsets, int* __restrict__ perm, int* __restri
     }
 }
 
+__global__ void __launch_bounds__(1024)
+moe_sort_kernel(int* __restrict__ offsets, int* __restrict__ perm, int* __restrict__ inv, int* __restrict__ tiles, int* __restrict__ n_tiles,
+                const int* __restrict__ ids, int P, int E, int max_tiles, int tile_rows) {
+    __shared__ int cnt[MOE_MAX_E], cur[MOE_MAX_E], tbase[MOE_MAX_E];
+    moe_sort(offsets, perm, inv, tiles, n_tiles, ids, P, E, max_tiles, tile_rows, cnt, cur, tbase);
+}
+
+// moe_route_groups_kernel and moe_sort_kernel in one, for few tokens and at most 64 experts: a wave a token and a lane an expert, so a choice is a
+// reduction in registers, and the order is made by the same block from LDS.  The same scores, choices and weights, bit for bit.  Decode steps of 16
+// tokens, 16 experts in 4 groups, top 2: 8.7 us against 9.0 and
+// 4.5 and the gap between them, all of it latency.
+#define MOE_FEW_TOKENS 64
+#define MOE_FEW_PAIRS 512
+__global__ void __launch_bounds__(1024)
+moe_plan_few_kernel(int* __restrict__ ids, float* __restrict__ wts, const float* __restrict__ z, const float* __restrict__ corr, int T_, int E, int top,
+                    int z_stride, int groups, int keep, float wscale, int* __restrict__ offsets, int* __restrict__ perm, int* __restrict__ inv,
+                    int* __restrict__ tiles, int* __restrict__ n_tiles, int sorted, int max_tiles, int tile_rows) {
+    __shared__ int cnt[64], cur[64], tbase[64], chosen[MOE_FEW_PAIRS];
+    const int lane = threadIdx.x & 63, size = E / groups, mine = lane < E ? lane / size : groups;
+    const float c = corr != nullptr && lane < E ? corr[lane] : 0.f;
+    // the lane with the largest v among those with a number, ties to the lower one; `fallback` if there is none (rows of NaN)
+    auto take = [&](float v, bool in, int fallback) {
+        float best = -INFINITY;
+        int bi = 0x7fffffff;
+        if (in && v >= -INFINITY) {
+            best = v;
+            bi = lane;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const float ov = __shfl_xor(best, o, 64);
+            const int oi = __shfl_xor(bi, o, 64);
+            if (ov > best || (ov == best && oi < bi)) {
+                best = ov;
+                bi = oi;
+            }
+        }
+        return bi == 0x7fffffff ? fallback : bi;
+    };
+    for (int t = threadIdx.x >> 6; t < T_; t += 16) {
+        const float zl = lane < E ? z[(size_t)t * z_stride + lane] : -INFINITY;
+        const float zmax = wave_max(zl);
+        const float ex = lane < E ? expf(zl - zmax) : 0.f;
+        const float score = ex / wave_sum(ex);
+        float v = score + c;
+        if (groups > 1 && keep < groups) {
+            float b = -INFINITY;    // lane g: the largest of group g
+            for (int i = 0; i < size; ++i) b = fmaxf(b, __shfl(v, (lane < groups ? lane : 0) * size + i, 64));
+            unsigned long long kept = 0;
+            for (int k = 0; k < keep; ++k) {
+                const int g = take(b, lane < groups, k);
+                kept |= 1ull << g;
+                if (lane == g) b = -INFINITY;
+            }
+            if (lane < E && !((kept >> mine) & 1ull)) v = -INFINITY;
+        }
+        float sum = 0.f;
+        for (int s = 0; s < top; ++s) {
+            const int e = take(v, lane < E, s);
+            const float sc = __shfl(score, e, 64);
+            sum += sc;
+            if (lane == 0) {
+                ids[(size_t)t * top + s] = e;
+                chosen[t * top + s] = e;
+                wts[(size_t)t * top + s] = sc;
+            }
+            if (lane == e) v = -INFINITY;
+        }
+        if (lane == 0)
+            for (int s = 0; s < top; ++s) wts[(size_t)t * top + s] = wts[(size_t)t * top + s] / (sum + 1e-20f) * wscale;
+    }
+    __syncthreads();
+    moe_sort(offsets, perm, inv, tiles, n_tiles, chosen, T_ * top, sorted, max_tiles, tile_rows, cnt, cur, tbase);
+}
+
 extern "C" int ilm_moe_tile_rows() { return MOE_TM; }
+
+// Whether ilm_moe_plan_few takes a step
+extern "C" int ilm_moe_plan_few_ok(int T_, int E, int top) { return T_ > 0 && T_ <= MOE_FEW_TOKENS && E <= 64 && T_ * top <= MOE_FEW_PAIRS; }
+
+// ilm_moe_route_groups (float32 correction) over E experts and ilm_moe_sort over the first `sorted` of them
+extern "C" int ilm_moe_plan_few(void* ids, void* wts, const void* z, const void* corr, int T_, int E, int top, int z_stride, int groups, int keep,
+                                float wscale, void* offsets, void* perm, void* inv, void* tiles, void* n_tiles, int sorted, int max_tiles,
+                                int tile_rows, hipStream_t stream) {
+    ILM_REQUIRE(E > 0 && top > 0 && top <= E && ilm_moe_plan_few_ok(T_, E, top), "moe_plan_few: %d tokens, %d experts, top %d", T_, E, top);
+    ILM_REQUIRE(groups > 0 && E % groups == 0 && keep > 0 && keep <= groups && top <= keep * (E / groups),
+                "moe_plan_few: %d of %d groups of %d experts, top %d", keep, groups, E, top);
+    const int P = T_ * top, need = P / tile_rows + (sorted < P ? sorted : P);
+    ILM_REQUIRE(sorted > 0 && sorted <= E && (tile_rows == MOE_TM || tile_rows == MOE_BM) && max_tiles >= (need < P ? need : P),
+                "moe_plan_few: %d tiles of %d rows do not hold %d pairs of %d experts", max_tiles, tile_rows, P, sorted);
+    moe_plan_few_kernel<<<1, 1024, 0, stream>>>((int*)ids, (float*)wts, (const float*)z, (const float*)corr, T_, E, top, z_stride, groups, keep, wscale,
+                                                (int*)offsets, (int*)perm, (int*)inv, (int*)tiles, (int*)n_tiles, sorted, max_tiles, tile_rows);
+    ILM_LAUNCH_CHECK("moe_plan_few");
+    return 0;
+}
 
 extern "C" int ilm_moe_sort(void* offsets, void* perm, void* inv, void* tiles, void* n_tiles, const void* ids, int P, int E,
                             int max_tiles, int tile_rows, hipStream_t stream) {

@@ -230,7 +230,8 @@ def qkv_rope_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor]
         # a portion of a prompt (rows beyond the few), where its tiles make about one round
         tile = 0
         if (USE_QKV_ROPE and x.dtype == BF16 and M > FRAG_MAX_ROWS and rd == d and d % 32 == 0 and _portion_operands_ok(x, w)
-                and cos.data_ptr() % 16 == 0 and sin.data_ptr() % 16 == 0):
+                and cos.data_ptr() % 16 == 0 and sin.data_ptr() % 16 == 0
+                and (slots is None or (k_cache is not None and k_cache.data_ptr() % 16 == 0))):
             tile = _portion_tile("rope", M, w.shape[0], K, x.device)
         return _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d, tile) if tile else None
     return _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)
@@ -2143,7 +2144,10 @@ def moe_route(logits: torch.Tensor, experts: int, top: int, big_tiles_ok: bool =
     plan.top, plan.pairs = int(top), P
     plan.ids = torch.empty((T, top), dtype=torch.int32, device=dev)
     plan.weights = torch.empty((T, top), dtype=F32, device=dev)
-    if grouped:
+    few = grouped and bool(_lib().ilm_moe_plan_few_ok(T, total, int(top)))     # (choice and order in one kernel, below)
+    if few:
+        pass
+    elif grouped:
         _run("ilm_moe_route_groups", plan.ids.data_ptr(), plan.weights.data_ptr(), logits.data_ptr(), _ptr(correction), 0, T, total, int(top),
              logits.stride(0), int(groups), int(keep), float(weight_scale), _stream())
     else:
@@ -2157,6 +2161,11 @@ def moe_route(logits: torch.Tensor, experts: int, top: int, big_tiles_ok: bool =
     plan.inv = book[experts + 1 + P:experts + 1 + 2 * P]
     plan.tiles = book[experts + 1 + 2 * P:experts + 1 + 2 * P + 3 * plan.max_tiles]
     plan.n_tiles = book[-1:]
+    if few:
+        _run("ilm_moe_plan_few", plan.ids.data_ptr(), plan.weights.data_ptr(), logits.data_ptr(), _ptr(correction), T, total, int(top),
+             logits.stride(0), int(groups), int(keep), float(weight_scale), plan.offsets.data_ptr(), plan.perm.data_ptr(), plan.inv.data_ptr(),
+             plan.tiles.data_ptr(), plan.n_tiles.data_ptr(), int(experts), plan.max_tiles, plan.tile_rows, _stream())
+        return plan
     _run("ilm_moe_sort", plan.offsets.data_ptr(), plan.perm.data_ptr(), plan.inv.data_ptr(), plan.tiles.data_ptr(), plan.n_tiles.data_ptr(),
          plan.ids.data_ptr(), P, int(experts), plan.max_tiles, plan.tile_rows, _stream())
     return plan

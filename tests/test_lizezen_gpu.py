@@ -721,3 +721,37 @@ def test_long_decoding(tmp_path):
     rows = [runner.step([StepEntry("a", [toks[i]], [0])]).cpu()[0] for i in range(10, 510)]
     _close(torch.stack(rows), want[10:], TOL["float32"], "500 decoded tokens")
     runner.cache.check()
+
+
+@pytest.mark.parametrize("T,E,ident,top,groups,keep", [(1, 1, 0, 1, 1, 1), (16, 14, 2, 2, 4, 2), (17, 5, 0, 3, 1, 1), (64, 56, 8, 8, 8, 5), (33, 60, 4, 2, 64, 2),
+                                                       (40, 63, 0, 7, 3, 1), (64, 12, 0, 4, 3, 3)])
+def test_choice_and_order_of_few_tokens(K, T, E, ident, top, groups, keep):
+    """Choice and order by one kernel against the two kernels that more tokens take: experts and weights bit for bit, rows of NaN and
+    of equal logits among them, and the same pairs in every expert's stretch of the order."""
+    from infinilm_amd.csrc import lib
+    L = lib.load()
+    total, g = E + ident, torch.Generator().manual_seed(T + E)
+    z, corr = torch.randn((T, total + 1), generator=g).to(DEV), (0.3 * torch.randn(total, generator=g)).to(DEV)
+    z[T // 2] = 0.25
+    if T > 2:
+        z[T - 1] = math.nan
+    assert L.ilm_moe_plan_few_ok(T, total, top)
+    for c in (corr, torch.zeros_like(corr)):
+        plan = K.moe_route(z, E, top, softmax=True, weight_scale=1.7, identity=ident, correction=c, groups=groups, keep=keep, normalise=True)
+        P, s = T * top, torch.cuda.current_stream().cuda_stream
+        ids, wts = torch.empty((T, top), dtype=torch.int32, device=DEV), torch.empty((T, top), dtype=torch.float32, device=DEV)
+        assert L.ilm_moe_route_groups(ids.data_ptr(), wts.data_ptr(), z.data_ptr(), c.data_ptr(), 0, T, total, top, z.stride(0), groups, keep, 1.7, s) == 0
+        assert torch.equal(plan.ids, ids) and torch.equal(plan.weights.nan_to_num(-1.0), wts.nan_to_num(-1.0))
+        off, perm, inv = (torch.full((n,), -7, dtype=torch.int32, device=DEV) for n in (E + 1, P, P))
+        tiles, n_tiles = torch.full((3 * plan.max_tiles,), -7, dtype=torch.int32, device=DEV), torch.zeros(1, dtype=torch.int32, device=DEV)
+        assert L.ilm_moe_sort(off.data_ptr(), perm.data_ptr(), inv.data_ptr(), tiles.data_ptr(), n_tiles.data_ptr(), ids.data_ptr(), P, E,
+                              plan.max_tiles, plan.tile_rows, s) == 0
+        assert torch.equal(plan.offsets, off) and torch.equal(plan.n_tiles, n_tiles)
+        n = 3 * int(n_tiles)
+        assert torch.equal(plan.tiles[:n], tiles[:n])
+        o = off.tolist()
+        for e in range(E):
+            assert sorted(plan.perm[o[e]:o[e + 1]].tolist()) == sorted(perm[o[e]:o[e + 1]].tolist())
+        flat = plan.ids.flatten()
+        placed = plan.inv >= 0
+        assert torch.equal(placed, flat < E) and torch.equal(plan.perm[plan.inv[placed].long()].long(), placed.nonzero().flatten())
