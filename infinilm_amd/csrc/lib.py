@@ -32,6 +32,7 @@ _SIGNATURES = {
     "ilm_gemm_tall": [_P, _I, _L, _I, _I, _I, _P, _I, _I, _I, _I, _P, _I, _I, _P],
     "ilm_gemm_tall_swiglu": [_P, _I, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
     "ilm_gemm_qkv_rope": [_P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
+    "ilm_gemm_qkv_rope_sum": [_P, _I, _P, _P, _P, _I, _L, _F, _P, _I, _F, _F, _P, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "ilm_frag_pack_weight": [_P, _P, _P, _I, _I, _I, _I, _P],
     "ilm_frag_pack_rows": [_P, _P, _I, _I, _I, _P],
     "ilm_frag_unpack_rows": [_P, _P, _I, _I, _I, _P],

@@ -246,23 +246,30 @@ def qkv_rope_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
     return _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)
 
 
-def _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d, tile=0):
-    M, K = x.shape
-    _dev(x, w, bias, positions, cos, sin, k_cache, v_cache, slots)
+def _qkv_rope_checks(w, bias, dtype, M, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d) -> int:
+    """What the fused projections assume of their operands; the cache's page size (0 without slots)."""
     _i32(positions, "positions")
-    if w.shape != ((nh + 2 * nkv) * d, K) or positions.numel() != M:
-        raise KernelError(f"fused projection {tuple(w.shape)} does not fit {nh}+2*{nkv} heads of {d} over {K}")
-    if bias is not None and (bias.shape != (w.shape[0],) or bias.dtype != x.dtype or not bias.is_contiguous()):
+    if w.shape[0] != (nh + 2 * nkv) * d or positions.numel() != M:
+        raise KernelError(f"fused projection {tuple(w.shape)} does not fit {nh}+2*{nkv} heads of {d}")
+    if bias is not None and (bias.shape != (w.shape[0],) or bias.dtype != dtype or not bias.is_contiguous()):
         raise KernelError("bias does not fit the fused projection")
     if cos.dtype != F32 or sin.dtype != F32 or cos.shape != sin.shape or cos.shape[1] != d // 2 \
             or not cos.is_contiguous() or not sin.is_contiguous():
         raise KernelError(f"rotation tables must be float32 [positions, {d // 2}], got {tuple(cos.shape)}")
-    page = 0
-    if slots is not None:
-        _i32(slots, "slots")
-        if k_cache is None or v_cache is None or k_cache.dtype != x.dtype or v_cache.dtype != x.dtype:
-            raise KernelError("cache tensors missing or of another dtype than the activations")
-        page = _check_cache(k_cache, v_cache, nkv, d)
+    if slots is None:
+        return 0
+    _i32(slots, "slots")
+    if k_cache is None or v_cache is None or k_cache.dtype != dtype or v_cache.dtype != dtype:
+        raise KernelError("cache tensors missing or of another dtype than the activations")
+    return _check_cache(k_cache, v_cache, nkv, d)
+
+
+def _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d, tile=0):
+    M, K = x.shape
+    _dev(x, w, bias, positions, cos, sin, k_cache, v_cache, slots)
+    if w.shape[1] != K:
+        raise KernelError(f"fused projection {tuple(w.shape)} does not fit rows of {K}")
+    page = _qkv_rope_checks(w, bias, x.dtype, M, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)
     q = torch.empty((M, nh * d), dtype=x.dtype, device=x.device)
     args = (q.data_ptr(), q.stride(0), x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), _ptr(bias), M, K, positions.data_ptr(),
             cos.data_ptr(), sin.data_ptr(), _ptr(k_cache) if slots is not None else None, _ptr(v_cache) if slots is not None else None,
@@ -272,6 +279,38 @@ def _qkv_rope(x, w, bias, positions, cos, sin, k_cache, v_cache, slots, nh, nkv,
     else:
         _run("ilm_gemm_qkv_rope" if x.dtype == BF16 else "ilm_gemm_f32_rope", *args, _stream())
     return q
+
+
+QKV_SUM_PARTS = 8       # most parts of a branch that the projection sums itself
+
+
+def _qkv_sum_rows(M: int, K: int) -> bool:
+    """Whether a workgroup of the fused projection takes M rows of K to form with 256 numbers a wave (eight waves, sixteen from K 3,073 on)."""
+    return M <= 16 and K % 256 == 0 and M * K <= (4096 if K > 3072 else 2048)
+
+
+def qkv_rope_sum(residual: torch.Tensor, parts: torch.Tensor, alpha: float, norm_w: torch.Tensor, w_offset: float, eps: float, w: torch.Tensor,
+                 bias: Optional[torch.Tensor], positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: Optional[torch.Tensor],
+                 v_cache: Optional[torch.Tensor], slots: Optional[torch.Tensor], nh: int, nkv: int, d: int, rd: int):
+    """`add_rmsnorm` (parts [P, M, K] float32) and `qkv_rope_gemm` in one kernel: (rotated q, the residual rows with the branch in them, a tensor
+    of their own), or None where it does not apply.  Every workgroup forms the rows for itself, so for one or two of them
+    (gemm_qkv_rope.hip has both sides' times)."""
+    M, K = residual.shape
+    if not (USE_QKV_ROPE and not FORCE_BASIC and w.dtype == BF16 and _qkv_sum_rows(M, K) and rd == d and d % 32 == 0
+            and residual.dtype == F32 and residual.is_contiguous() and parts.dtype == F32 and parts.dim() == 3 and parts.is_contiguous()
+            and tuple(parts.shape[1:]) == (M, K) and 1 <= parts.shape[0] <= QKV_SUM_PARTS and norm_w.shape == (K,) and norm_w.is_contiguous()
+            and norm_w.dtype in (BF16, F32) and w.shape == ((nh + 2 * nkv) * d, K) and w.stride(1) == 1 and w.stride(0) % 8 == 0
+            and w.data_ptr() % 16 == 0 and residual.data_ptr() % 16 == 0 and parts.data_ptr() % 16 == 0):
+        return None
+    _dev(residual, parts, norm_w, w, bias, positions, cos, sin, k_cache, v_cache, slots)
+    page = _qkv_rope_checks(w, bias, BF16, M, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)
+    q = torch.empty((M, nh * d), dtype=BF16, device=w.device)
+    new = torch.empty_like(residual)
+    _run("ilm_gemm_qkv_rope_sum", q.data_ptr(), q.stride(0), residual.data_ptr(), new.data_ptr(), parts.data_ptr(), parts.shape[0], parts.stride(0),
+         float(alpha), norm_w.data_ptr(), _dt(norm_w), float(w_offset), float(eps), w.data_ptr(), w.stride(0), _ptr(bias), M, K, positions.data_ptr(),
+         cos.data_ptr(), sin.data_ptr(), _ptr(k_cache) if slots is not None else None, _ptr(v_cache) if slots is not None else None, _ptr(slots),
+         nh, nkv, d, page, _stream())
+    return q, new
 
 
 USE_PORTION = os.environ.get("INFINILM_AMD_PORTION", "1") == "1"   # 0: portions' products by the vendor library

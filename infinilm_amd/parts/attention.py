@@ -117,11 +117,18 @@ class GQAttention(Mixer):
         fn = getattr(self.position, "takes_frag", None)
         return bool(fn is not None and not self.gated and not self.values_are_keys and fn(rows, self.qkv, self.nh, self.nkv, self.d))
 
-    def forward(self, x, batch, cache_view, tail=None):
+    def project_pending(self, pending, batch, cache_view):
+        fn = getattr(self.position, "project_pending", None)
+        if fn is None or self.gated or self.values_are_keys:
+            return None
+        self.position.check(batch)
+        return fn(pending, self.qkv, batch, cache_view, self.nh, self.nkv, self.d)
+
+    def forward(self, x, batch, cache_view, tail=None, projected=None):
         pe = self.position
         pe.check(batch)
-        qkv = None
-        if batch.taps is None and not self.gated and not self.values_are_keys:   # (a dump of the rotated rows needs them in one piece)
+        qkv = projected
+        if qkv is None and batch.taps is None and not self.gated and not self.values_are_keys:   # (a dump of the rotated rows needs them in one piece)
             qkv = pe.project_encode_store(x, self.qkv, batch, cache_view, self.nh, self.nkv, self.d)
         if qkv is None:
             rows = self.qkv.forward(x)

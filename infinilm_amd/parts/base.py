@@ -254,6 +254,19 @@ class NormTail:
 
 
 @dataclass
+class PendingNorm:
+    """A norm whose rows are not formed yet: those of `stream` with the float32 parts that are still due to it.  A mixer that forms them inside
+    its own projection puts the sum back into the stream (`settled`)."""
+    stream: "ResidualStream"
+    weight: torch.Tensor
+    weight_offset: float
+    eps: float
+
+    def settled(self, residual: torch.Tensor) -> None:
+        self.stream.residual, self.stream.pending, self.stream.pending_scale = residual, None, 1.0
+
+
+@dataclass
 class DeferredNorm:
     """A norm's output up to one number a row: `x` = residual * weight in the activations' dtype, and
     partial sums of squares of the residual's rows (`sumsq` [tiles, 32]), from which the consumer
@@ -277,7 +290,8 @@ class Norm(Part):
 
 
 class Mixer(Part):
-    """`takes_tail`: forward accepts `tail=NormTail` and may answer with a DeferredNorm."""
+    """`takes_tail`: forward accepts `tail=NormTail` and may answer with a DeferredNorm.  A mixer with `project_pending(pending, batch,
+    cache_view)` may form its rows from a `PendingNorm` itself: what it returns (None: it does not) goes to forward as `projected`."""
     takes_tail = False
     # True: forward takes every index from the batch's device tensors also in steps that hold portions of prompts
     # (never from the host copies `h_*`), so that such steps can be recorded and replayed for other requests

@@ -13,6 +13,7 @@ import torch
 from .. import kernels
 from ..config.spec import LayerSpec
 from .base import BuildContext, DeferredNorm, HyperStreams, Param, Part, ResidualStream, join_name
+from .norm import RMSNorm
 from .registry import ARRANGEMENTS, build_feed_forward, build_mixer, build_norm, register_arrangement
 
 
@@ -46,7 +47,15 @@ class PreNormBlock:
     def forward(self, stream: ResidualStream, batch, cache_view) -> None:
         # a decode step of many rows: the mixer may take its rows in fragment order, which the norm then writes
         rows = stream.residual.shape[0]
-        if (batch.taps is None and getattr(self.norm1, "takes_frag_request", False)
+        # very few rows: the mixer's projection may form the normed rows itself, without the norm's kernel
+        projected = None
+        if batch.taps is None and isinstance(self.norm1, RMSNorm) and isinstance(stream, ResidualStream) and hasattr(self.mixer, "project_pending"):
+            pending = self.norm1.pending(stream)
+            if pending is not None:
+                projected = self.mixer.project_pending(pending, batch, cache_view)
+        if projected is not None:
+            x = None
+        elif (batch.taps is None and getattr(self.norm1, "takes_frag_request", False)
                 and getattr(self.mixer, "takes_frag", lambda rows: False)(rows)):
             x = self.norm1.forward(stream, frag=True)
         else:
@@ -56,10 +65,13 @@ class PreNormBlock:
         # (see NormTail).  Not while intermediate values are dumped: they are taken between the kernels.
         tail = None
         if self.mixer.takes_tail and batch.taps is None:
-            tail = self.norm2.tail(stream, self.residual_scale, x.shape[0])
-            if tail is not None and not self.ffn.takes_deferred(x.shape[0]):
+            tail = self.norm2.tail(stream, self.residual_scale, rows)
+            if tail is not None and not self.ffn.takes_deferred(rows):
                 tail = None
-        y = self.mixer.forward(x, batch, cache_view) if tail is None else self.mixer.forward(x, batch, cache_view, tail=tail)
+        more = {} if tail is None else {"tail": tail}
+        if projected is not None:
+            more["projected"] = projected
+        y = self.mixer.forward(x, batch, cache_view, **more)
         if isinstance(y, DeferredNorm):
             x = y
         else:

@@ -12,7 +12,7 @@ from typing import Dict
 import torch
 
 from .. import kernels
-from .base import BuildContext, HyperStreams, Norm, NormTail, Param, ResidualStream
+from .base import BuildContext, HyperStreams, Norm, NormTail, Param, PendingNorm, ResidualStream
 from .registry import register_norm
 
 
@@ -47,6 +47,14 @@ class RMSNorm(Norm):
         if stream.pending is not None or self.dtype != torch.bfloat16 or rows > kernels.TAIL_MAX_ROWS:
             return None
         return NormTail(stream.residual, float(scale), self.weight, self.eps)
+
+    def pending(self, stream: ResidualStream):
+        """The norm of rows that a product's float32 parts are still due to, for a mixer that forms them itself; None where there is none."""
+        h = stream.pending
+        if (self.dtype != torch.bfloat16 or h is None or h.dim() != 3 or stream.more or stream.pending_norm is not None
+                or stream.pending_gate is not None):
+            return None
+        return PendingNorm(stream, self.weight, self.weight_offset, self.eps)
 
     def forward(self, stream: ResidualStream, frag: bool = False):
         """`frag`: the consumer takes its rows in fragment order (`kernels.FragRows`)."""

@@ -154,6 +154,15 @@ class RotaryEmbedding(PositionEncoding):
         fused = kernels.qkv_rope_f32 if x.dtype == torch.float32 else kernels.qkv_rope_gemm
         return fused(x, proj.weight, proj.bias, batch.positions, self.cos, self.sin, view.k, view.v, view.slots, nh, nkv, d, self.rotary_dim)
 
+    def project_pending(self, pending, proj, batch, view, nh, nkv, d):
+        s = pending.stream
+        out = kernels.qkv_rope_sum(s.residual, s.pending, s.pending_scale, pending.weight, pending.weight_offset, pending.eps, proj.weight, proj.bias,
+                                   batch.positions, self.cos, self.sin, view.k, view.v, view.slots, nh, nkv, d, self.rotary_dim)
+        if out is None:
+            return None
+        pending.settled(out[1])
+        return out[0]
+
     def encode_and_store(self, qkv, batch, view, nh, nkv, d):
         kernels.rope_kvwrite(qkv, batch.positions, self.cos, self.sin, view.k, view.v, view.slots, nh, nkv, d,
                              self.rotary_dim)
@@ -172,6 +181,9 @@ class NoPositionEncoding(RotaryEmbedding):
         return False
 
     def project_encode_store(self, x, proj, batch, view, nh, nkv, d):
+        return None
+
+    def project_pending(self, pending, proj, batch, view, nh, nkv, d):
         return None
 
 

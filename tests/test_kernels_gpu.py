@@ -1173,3 +1173,38 @@ def test_portion_rule(K):
         got = K.gemm(x, w)
         assert torch.equal(got, K.portion_gemm(x, w, None, torch.empty_like(got), tile))
         assert float((got.float() - want).norm() / want.norm()) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("M,K_,nh,nkv,d,parts", [(1, 256, 2, 1, 32, 1), (1, 1024, 16, 2, 64, 4), (2, 1024, 5, 1, 64, 8), (1, 2048, 16, 2, 64, 2), (8, 256, 3, 3, 96, 3),
+                                                 (1, 3328, 4, 4, 64, 3), (1, 4096, 32, 2, 128, 4), (2, 768, 6, 2, 128, 5)])
+def test_qkv_projection_that_forms_its_rows(K, M, K_, nh, nkv, d, parts):
+    """Against the norm's kernel and the projection one after the other.  The new residual rows are the same sums; the norm's sum of squares
+    is taken in another order (some 2^-22 of it), which can turn a normed value's last bit (2^-8), and by that an output by at
+    most 2^-8 of a thousandth or so of its terms: held to 2^-6 of the largest output of a row."""
+    g = torch.Generator().manual_seed(M * K_ + d)
+    page, pages, N = 16, 4, (nh + 2 * nkv) * d
+    r, h = torch.randn((M, K_), generator=g).to(DEV) * 3, torch.randn((parts, M, K_), generator=g).to(DEV)
+    w = (torch.randn((N, K_), generator=g) / math.sqrt(K_)).to(BF16).to(DEV)
+    nw = (1 + 0.1 * torch.randn(K_, generator=g)).to(DEV)
+    b = torch.randn(N, generator=g).to(BF16).to(DEV)
+    cos, sin = (torch.randn((64, d // 2), generator=g).to(DEV) for _ in range(2))
+    pos = torch.randint(0, 64, (M,), generator=g, dtype=torch.int32).to(DEV)
+    slots = torch.randperm(page * pages, generator=g)[:M].to(torch.int32).to(DEV)
+    if M > 2:
+        slots[1] = -1
+    for nw_, off, bias in ((nw, 0.0, None), (nw.to(BF16), 1.0, b)):
+        c1, c2 = ([torch.zeros((pages, nkv, page, d), dtype=BF16, device=DEV), torch.zeros((pages, nkv, d, page), dtype=BF16, device=DEV)] for _ in range(2))
+        before = r.clone()
+        q, new = K.qkv_rope_sum(r, h, 0.7, nw_, off, 1e-5, w, bias, pos, cos, sin, *c1, slots, nh, nkv, d, d)
+        assert torch.equal(r, before)
+        want = r.clone()
+        x = K.add_rmsnorm(want, h, nw_, 0.7, 1e-5, BF16, weight_offset=off)
+        assert float((new - want).abs().max()) <= 2.0 ** -22 * float(want.abs().max() + h.abs().sum(0).max())
+        ref = K.qkv_rope_gemm(x, w, bias, pos, cos, sin, *c2, slots, nh, nkv, d, d)
+        for got, exp in ((q, ref), (c1[0], c2[0]), (c1[1], c2[1])):
+            assert float((got.float() - exp.float()).abs().max()) <= 2.0 ** -6 * float(exp.float().abs().max())
+            assert torch.equal(got == 0, exp == 0) or float(((got == 0) != (exp == 0)).float().mean()) < 1e-3
+    more = torch.zeros((parts, 9, K_), device=DEV)      # (more rows than a workgroup forms)
+    assert K.qkv_rope_sum(more[0], more, 1.0, nw, 0.0, 1e-5, w, None, pos, cos, sin, None, None, None, nh, nkv, d, d) is None
+    assert K.qkv_rope_sum(r[:, :K_ - 8].contiguous(), h[:, :, :K_ - 8].contiguous(), 1.0, nw[:K_ - 8], 0.0, 1e-5, w[:, :K_ - 8].contiguous(), None, pos, cos, sin,
+                          None, None, None, nh, nkv, d, d) is None
