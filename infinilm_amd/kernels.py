@@ -837,7 +837,7 @@ def bound_rows(rows: int) -> int:
     return b
 
 
-def attention_chunks(max_total_len: int, page: int, pairs: int, device) -> tuple:
+def attention_chunks(max_total_len: int, page: int, pairs: int, device, head_dim: int = 128) -> tuple:
     """(keys a chunk, chunks) of the chunked single-token attention for `pairs` = tokens x head groups.
 
     A chunk is a whole number of steps of ATT_STEP keys.  Few tokens: one step a chunk (latency
@@ -874,8 +874,20 @@ def attention_chunks(max_total_len: int, page: int, pairs: int, device) -> tuple
             if 2 <= n <= steps and (cost(n), -n) < (cost(best), -best):
                 best = n
         per_chunk = best
+    # Heads of up to 64: a step is half as long (1.15 us beside a workgroup's other 6) and the chunks' merge cheap, so shorter chunks, as long
+    # as they are at most 16 and come to at most four workgroups a unit.  16 heads of 64 over 2, all contexts alike / between a sixth
+    # and the whole, against the rule above: 32 tokens of 1,900 keys 11.0 us with 128 a chunk (512: 12.9); 48 of 1,000 9.2 / 9.0 with
+    # 128 (384: 11.5 / 10.6), of 1,900 15.2 / 12.9 with 256 (512: 17.7 / 15.6), of 3,800 20.0 / 19.6 with 512 (1024: 27.1 / 26.6); 64 of 500 9.0 / 8.0
+    # with 128 (384: 11.1 / 10.1), of 8,000 40.6 with 1024 (2048: 46.9); 96 of 1,000 15.4 / 13.2 with 256 (512: 18.4 / 15.1).
+    if head_dim <= 64:
+        short = 1
+        while short < per_chunk and (-(-steps // short) > 16 or workgroups(short) > 4 * cus):
+            short *= 2
+        per_chunk = min(per_chunk, short)
     while -(-steps // per_chunk) > ATT_MAX_CHUNKS:
         per_chunk += 1
+    # as many chunks of more equal length: 64 tokens of 500 keys at the 8B head shape 13.3 us in chunks of 2 + 2 steps, 15.8 in 3 + 1
+    per_chunk = -(-steps // -(-steps // per_chunk))
     span = per_chunk * ATT_STEP
     return span, -(-max_total_len // span)
 
@@ -930,7 +942,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             _i32(single_rows, "single_rows")
             rows, n_single = single_rows, single_rows.numel()
         # (the tokens counted as the recorded steps round them, so that an eager step and a replayed one cut alike)
-        span, nsplit = attention_chunks(int(max_total_len), page, bound_rows(n_single) * nkv * (-(-(nh // nkv) // 16)), q.device)
+        span, nsplit = attention_chunks(int(max_total_len), page, bound_rows(n_single) * nkv * (-(-(nh // nkv) // 16)), q.device, d)
         ws_acc = ws_ml = None
         if nsplit > 1 and (span, nsplit) != (ATT_STEP, 2):   # (two chunks of one step meet inside a workgroup)
             # partial results of the rows served here (not of every token of the step)
