@@ -405,7 +405,8 @@ def gather_rows(x: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
 
 _LIBRARY_F32_OUT = [True]   # cleared when torch.mm refuses out_dtype
 KSPLIT_SPAN = 4096  # K range of one part of the K-split few-rows product (ilm_gemm_ksplit_max_k(1))
-KSPLIT_FEW_SPAN = 1024   # ... and with up to 16 rows of up to KSPLIT_SPAN
+KSPLIT_FEW_SPAN = 1024   # ... and with up to 16 rows of up to KSPLIT_FEW_MAX
+KSPLIT_FEW_MAX = 8192
 # Rows up to which the products keep X in registers (16 or 32; 32 only for K up to 4096 a workgroup)
 FEW_ROWS = int(os.environ.get("INFINILM_AMD_FEW_ROWS", "32"))
 
@@ -483,15 +484,16 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, 
             _run("ilm_gemm_rows64", parts.data_ptr(), N, M * N, kb, w.data_ptr(), w.stride(0), M, N, K, a.data_ptr(),
                  a.stride(0), 0, _stream())
         return parts
-    # Up to 16 rows and 4,096 k: parts of 1,024 k, which give a small matrix as many workgroups as the chip takes and every wave
+    # Up to 16 rows and 8,192 k: parts of 1,024 k, which give a small matrix as many workgroups as the chip takes and every wave
     # a short chain of loads (8 rows: 1024 x 4096 4.6 us against 8.6 with all of K in one workgroup, 1024 x 2048 3.9 / 5.4,
-    # 2048 x 2048 4.5 / 5.9, 2304 x 2304 5.8 / 7.4, 4096 x 4096 8.3 / 10.2).  The upper end is where the parts of 4,096 begin, whose
-    # number callers count on, and no measurement's: 8 rows of 2048 x 8192 12.5 us in two parts, 7.7 in eight (with the
-    # norm that sums them 16.1 / 13.9), 2048 x 12288 14.0 / 12.1 (17.9 / 16.2), 4096 x 8192 20.9 / 13.3 (25.9 / 17.8), 4096 x 16384
-    # 27.1 / 25.0 (31.4 / 30.7).  One size is left that K whole serves better: 256 tiles of W, a tile a unit, and 2,049 to 3,072 k, whose
-    # three parts of 170 workgroups take a second round (with the norm 4096 x 3072 10.4 us whole, 11.2 in three parts, 10.7 in
-    # four for 1 row, 11.6, 12.1 and 11.6 for 8; but 5120 x 3072 16.8, 12.9 and 15.0).
-    span = KSPLIT_FEW_SPAN if M <= 16 and K <= KSPLIT_SPAN else KSPLIT_SPAN
+    # 2048 x 2048 4.5 / 5.9, 2304 x 2304 5.8 / 7.4, 4096 x 4096 8.3 / 10.2; against two parts of up to 4,096, with the norm that sums them: 1024 x 8192
+    # 9.2 us / 11.9, 2048 x 8192 11.9 / 16.1, 4096 x 8192 17.8 / 25.3, 2304 x 5760 12.5 / 17.3, 2048 x 6144 11.6 / 12.7).  The upper end is
+    # where the parts come to more than the eight that `qkv_rope_sum` takes: beyond, the gain is small (with the norm 2048 x 12288 17.9 us in three
+    # parts, 16.2 in twelve, 4096 x 16384 31.4 in four, 30.7 in sixteen).  One size is left that K whole serves better: 256 tiles of W, a tile a
+    # unit, and 2,049 to 3,072 k, whose three parts of 170 workgroups take a second round (with the norm 4096 x 3072 10.4 us whole, 11.2 in
+    # three parts, 10.7 in four for 1 row, 11.6, 12.1 and 11.6 for 8; but 5120 x 3072 16.8, 12.9 and 15.0).
+    # (From 4,096 k on for matrices of 1,024 rows or more, the range that was measured; narrower ones keep parts of 4,096.)
+    span = KSPLIT_FEW_SPAN if M <= 16 and (K <= KSPLIT_SPAN or (K <= KSPLIT_FEW_MAX and N >= 1024)) else KSPLIT_SPAN
     if fast and aligned and plain and allow_parts and out is None and M <= max(16, FEW_ROWS) and K > span and USE_KSPLIT:
         kb = -(-K // span)
         parts = torch.empty((kb, M, N), dtype=F32, device=a.device)

@@ -1208,3 +1208,17 @@ def test_qkv_projection_that_forms_its_rows(K, M, K_, nh, nkv, d, parts):
     assert K.qkv_rope_sum(more[0], more, 1.0, nw, 0.0, 1e-5, w, None, pos, cos, sin, None, None, None, nh, nkv, d, d) is None
     assert K.qkv_rope_sum(r[:, :K_ - 8].contiguous(), h[:, :, :K_ - 8].contiguous(), 1.0, nw[:K_ - 8], 0.0, 1e-5, w[:, :K_ - 8].contiguous(), None, pos, cos, sin,
                           None, None, None, nh, nkv, d, d) is None
+
+
+@pytest.mark.parametrize("M,N,K_,parts", [(8, 1024, 8192, 8), (16, 2304, 5760, 6), (1, 4099, 4104, 5), (3, 1030, 8200, 3), (2, 1023, 8192, 2)])
+def test_gemm_few_rows_in_short_parts_of_a_long_k(K, M, N, K_, parts):
+    """Either side of where K beyond 4,096 is cut into parts of 1,024: the parts' float sum against float64, as in
+    test_gemm_few_rows_in_short_parts, and the norm that sums them."""
+    a, w = _rand((M, K_), 60, torch.bfloat16), _rand((N, K_), 61, torch.bfloat16)
+    got = K.gemm(a.to(DEV), w.to(DEV), allow_parts=True)
+    assert got.dtype == torch.float32 and got.shape == (parts, M, N)
+    want = P.plain_linear(a.to(F64), w.to(F64))
+    _close(got.sum(0), want, 2e-6 * math.sqrt(K_))
+    r = torch.zeros((M, N), dtype=torch.float32, device=DEV)
+    K.add_rmsnorm(r, got, torch.ones(N, dtype=torch.bfloat16, device=DEV), 1.0, 1e-6, torch.bfloat16)
+    _close(r, want, 2e-6 * math.sqrt(K_))
