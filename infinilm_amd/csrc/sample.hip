@@ -402,7 +402,7 @@ __device__ __forceinline__ uint32_t rank_list(SampleLds& S, int n, uint32_t leas
 // rank_list of one bin's elements, which lie even over a short range of keys: a long list falls into 2,048 steps of that range, one or two
 // elements a step, and the step that holds the threshold is ranked by every wave for itself (one histogram instead of radix's three:
 // 5 rows of 122,753, top-p 0.95, about 390 listed: the kernel that ends in it
-// 14.3 -> 10.6 us)
+// 14.3 -> 10.6 us).  Rows by one workgroup keep radix: inlined there too, this code cost short lists 0.3 us and gave long ones nothing
 #define STEP_MAX 64
 __device__ __forceinline__ uint32_t rank_bin(SampleLds& S, int n, uint32_t least, u64 base, double need) {
     if (n <= RANK_MAX) return rank_list<false>(S, n, least, base, need);
@@ -648,7 +648,7 @@ __device__ __noinline__ void sample_row(SampleLds& S, const float* row, int V, f
                 // (a bin of ties has one key, as a rule, which the first of radix_bin's passes finds)
                 const int n = TIES ? LIST_CAP + 1
                                    : collect(row, V, S, mass, [&](float l) { return okey(l) >= tau && bin_of(l, mx, per) == bin; });
-                tp = n <= LIST_CAP ? rank_bin(S, n, tau, base, need) : radix_bin<false>(row, V, S, mass, bin, per, tau, base, need);
+                tp = n <= LIST_CAP ? rank_list<false>(S, n, tau, base, need) : radix_bin<false>(row, V, S, mass, bin, per, tau, base, need);
             }
         }
         if (!(pp > 0.f)) tp = okey(mx);
