@@ -1222,3 +1222,13 @@ def test_gemm_few_rows_in_short_parts_of_a_long_k(K, M, N, K_, parts):
     r = torch.zeros((M, N), dtype=torch.float32, device=DEV)
     K.add_rmsnorm(r, got, torch.ones(N, dtype=torch.bfloat16, device=DEV), 1.0, 1e-6, torch.bfloat16)
     _close(r, want, 2e-6 * math.sqrt(K_))
+
+
+def test_a_top_k_that_is_no_int(K):
+    """Rows whose top-k is a float, or beyond 32 bits, beside others: the tokens of the whole number, and of the whole vocabulary."""
+    from infinilm_amd import SamplingParams
+    from infinilm_amd.sampling import Sampler
+    logits = torch.randn((3, 5000), generator=torch.Generator().manual_seed(3)).to(DEV)
+    rows = lambda ks: [(SamplingParams(top_k=k, top_p=0.9), i, 4) for i, k in enumerate(ks)]
+    want = Sampler(5).sample(logits, rows([50, 4, 0]))
+    assert Sampler(5).sample(logits, rows([50.0, 4.5, 2 ** 31])) == want

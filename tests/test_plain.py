@@ -329,3 +329,13 @@ def test_uniform_numbers_of_something_else_than_whole_numbers_are_refused(n, bad
         columns[place][n // 2] = bad
         with pytest.raises(TypeError):
             uniforms_for(*columns)
+
+
+@pytest.mark.parametrize("top_k,kept", [([50.0, 3], [50, 3]), ([7, 2.5, 0], [7, 2, 0]), ([2 ** 31, 2 ** 40, 1], [2 ** 31 - 1, 2 ** 31 - 1, 1]),
+                                        ([math.inf, 5], [2 ** 31 - 1, 5]), ([True, 4], [1, 4])])
+def test_one_requests_top_k_does_not_fail_the_others(top_k, kept):
+    """Whatever number `SamplingParams` takes as a top-k reaches the kernels as an int32."""
+    from infinilm_amd import SamplingParams
+    from infinilm_amd.sampling.sampler import _int32s
+
+    assert _int32s([SamplingParams(top_k=k).top_k for k in top_k]).tolist() == kept
