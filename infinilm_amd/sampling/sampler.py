@@ -9,6 +9,7 @@ it was preempted.
 """
 from __future__ import annotations
 
+import operator
 from array import array
 from typing import List, Sequence, Tuple
 
@@ -39,7 +40,7 @@ def _words(values: Sequence[int]) -> array:
     try:
         return array("Q", values)
     except OverflowError:     # negative ones wrap, and of numbers of more than 64 bits the lowest count
-        return array("Q", [v & _MASK for v in values])
+        return array("Q", [operator.index(v) & _MASK for v in values])
 
 
 def _int32s(values: Sequence[int]) -> array:

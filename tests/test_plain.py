@@ -339,3 +339,15 @@ def test_one_requests_top_k_does_not_fail_the_others(top_k, kept):
     from infinilm_amd.sampling.sampler import _int32s
 
     assert _int32s([SamplingParams(top_k=k).top_k for k in top_k]).tolist() == kept
+
+
+@pytest.mark.parametrize("n", [1, 24, 40])
+def test_uniform_numbers_of_numpy_whole_numbers(n):
+    """Negative ones wrap as Python's do."""
+    import numpy as np
+    from infinilm_amd.sampling.sampler import uniform_for, uniforms_for
+
+    rows = [(-3 - i, -(1 << 62) + i, i - 5) for i in range(n)]
+    for kind in (np.int64, np.array):
+        columns = [kind(c) if kind is np.array else [kind(v) for v in c] for c in zip(*rows)]
+        assert uniforms_for(*columns).tolist() == [uniform_for(*r) for r in rows]
