@@ -64,10 +64,13 @@ def _uniforms_into(out: int, seeds: Sequence[int], request_keys: Sequence[int], 
 
 
 def uniforms_for(seeds: Sequence[int], request_keys: Sequence[int], indices: Sequence[int]) -> np.ndarray:
-    """`uniform_for` of every row."""
+    """`uniform_for` of every row; one by one where there is no native library (they are numbers of the host, and need no GPU)."""
     out = np.empty((len(seeds),), dtype=np.float32)
     if len(seeds):
-        _uniforms_into(out.ctypes.data, list(seeds), request_keys, indices)
+        try:
+            _uniforms_into(out.ctypes.data, list(seeds), request_keys, indices)
+        except (OSError, RuntimeError):
+            out[:] = [uniform_for(*map(operator.index, row)) for row in zip(seeds, request_keys, indices)]
     return out
 
 

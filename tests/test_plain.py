@@ -351,3 +351,17 @@ def test_uniform_numbers_of_numpy_whole_numbers(n):
     for kind in (np.int64, np.array):
         columns = [kind(c) if kind is np.array else [kind(v) for v in c] for c in zip(*rows)]
         assert uniforms_for(*columns).tolist() == [uniform_for(*r) for r in rows]
+
+
+def test_uniform_numbers_without_the_native_library(monkeypatch):
+    from infinilm_amd import kernels
+    from infinilm_amd.sampling.sampler import uniform_for, uniforms_for
+
+    def none():
+        raise RuntimeError("no library")
+
+    monkeypatch.setattr(kernels, "_lib", none)
+    rows = [(5 - i, 1 << i, i) for i in range(40)]
+    assert uniforms_for(*zip(*rows)).tolist() == [uniform_for(*r) for r in rows]
+    with pytest.raises(TypeError):
+        uniforms_for([1, 2.5], [0, 1], [0, 1])
