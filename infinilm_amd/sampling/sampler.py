@@ -82,7 +82,16 @@ class Sampler:
         # has run)
         self._staging = [None, None]
         self._copied = [None, None]
+        self._copied_on = [-1, -1]
         self._turn = 0
+
+    def _record(self, t: int) -> None:
+        """Marks the end of buffer t's copy.  An event belongs to the device that it was first recorded on, and the next
+        logits may lie on another."""
+        device = torch.cuda.current_device()
+        if self._copied[t] is None or self._copied_on[t] != device:
+            self._copied[t], self._copied_on[t] = torch.cuda.Event(), device
+        self._copied[t].record()
 
     def sample(self, logits: torch.Tensor, rows: Sequence[Tuple[SamplingParams, int, int]]) -> List[int]:
         """`rows[i]` = (params, request key, index of the token being generated) for logits[i]."""
@@ -106,8 +115,6 @@ class Sampler:
         t = self._turn = self._turn ^ 1
         if self._copied[t] is not None:
             self._copied[t].synchronize()
-        elif dev.type == "cuda":
-            self._copied[t] = torch.cuda.Event()
         if self._staging[t] is None or self._staging[t][0].numel() < 4 * n:
             buf = torch.empty((4 * max(n, 64),), dtype=torch.float32, pin_memory=dev.type == "cuda")
             self._staging[t] = (buf, memoryview(buf.numpy()).cast("B"), buf.data_ptr())
@@ -121,5 +128,5 @@ class Sampler:
         d = torch.empty((4 * n,), dtype=torch.float32, device=dev)
         d.copy_(buf[:4 * n], non_blocking=True)
         if dev.type == "cuda":
-            self._copied[t].record()
+            self._record(t)
         return kernels.sample_packed(logits, d, few=0 < min(top_k) and max(top_k) <= kernels.sample_few_k())

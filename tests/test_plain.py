@@ -365,3 +365,31 @@ def test_uniform_numbers_without_the_native_library(monkeypatch):
     assert uniforms_for(*zip(*rows)).tolist() == [uniform_for(*r) for r in rows]
     with pytest.raises(TypeError):
         uniforms_for([1, 2.5], [0, 1], [0, 1])
+
+
+def test_a_sampler_moves_between_devices(monkeypatch):
+    """Its events are recorded on the device at hand; one that stays on its device keeps them."""
+    from infinilm_amd.sampling import Sampler
+
+    class Event:
+        made = 0
+
+        def __init__(self):
+            self.device = None
+            Event.made += 1
+
+        def record(self):
+            if self.device not in (None, torch.cuda.current_device()):
+                raise RuntimeError("Event device does not match recording stream's device")
+            self.device = torch.cuda.current_device()
+
+    at = [0]
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: at[0])
+    s = Sampler()
+    for device, made in ((0, 2), (0, 2), (1, 4), (0, 6)):
+        at[0] = device
+        for t in (0, 1):
+            s._record(t)
+            assert s._copied[t].device == device
+        assert Event.made == made
