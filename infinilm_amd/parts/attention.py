@@ -119,7 +119,8 @@ class GQAttention(Mixer):
 
     def project_pending(self, pending, batch, cache_view):
         fn = getattr(self.position, "project_pending", None)
-        if fn is None or self.gated or self.values_are_keys:
+        # (a mixer made from this one whose forward is its own is called as ever)
+        if fn is None or self.gated or self.values_are_keys or type(self).forward is not GQAttention.forward:
             return None
         self.position.check(batch)
         return fn(pending, self.qkv, batch, cache_view, self.nh, self.nkv, self.d)

@@ -51,6 +51,8 @@ class RMSNorm(Norm):
     def pending(self, stream: ResidualStream):
         """The norm of rows that a product's float32 parts are still due to, for a mixer that forms them itself; None where there is none."""
         h = stream.pending
+        if type(self).forward is not RMSNorm.forward:    # (a norm made from this one norms its own way)
+            return None
         if (self.dtype != torch.bfloat16 or h is None or h.dim() != 3 or stream.more or stream.pending_norm is not None
                 or stream.pending_gate is not None):
             return None

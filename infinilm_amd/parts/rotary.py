@@ -155,6 +155,8 @@ class RotaryEmbedding(PositionEncoding):
         return fused(x, proj.weight, proj.bias, batch.positions, self.cos, self.sin, view.k, view.v, view.slots, nh, nkv, d, self.rotary_dim)
 
     def project_pending(self, pending, proj, batch, view, nh, nkv, d):
+        if type(self).project_encode_store is not RotaryEmbedding.project_encode_store:   # (an encoding made from this one projects its own way)
+            return None
         s = pending.stream
         out = kernels.qkv_rope_sum(s.residual, s.pending, s.pending_scale, pending.weight, pending.weight_offset, pending.eps, proj.weight, proj.bias,
                                    batch.positions, self.cos, self.sin, view.k, view.v, view.slots, nh, nkv, d, self.rotary_dim)
@@ -181,9 +183,6 @@ class NoPositionEncoding(RotaryEmbedding):
         return False
 
     def project_encode_store(self, x, proj, batch, view, nh, nkv, d):
-        return None
-
-    def project_pending(self, pending, proj, batch, view, nh, nkv, d):
         return None
 
 
