@@ -94,14 +94,14 @@ gemm_portion_kernel(const GpArgs A) {
     const char* wb = reinterpret_cast<const char*>(A.W);
     const char* xb = reinterpret_cast<const char*>(A.X);
     // (The compiler waits for all loads into LDS before it reads any of it, so these are written out and waited for by number.  They have no
-    // register to deliver to, and nothing else here uses m0.)
+    // register to deliver to.)
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)(&lds[0]) + (uint32_t)wave * 1024;
     auto issue = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < PER; ++i)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds0 + (uint32_t)(buf * ROWS * 128 + NW * i * 1024)),
                          "v"(from[i]), "s"(NW * i < BN / 8 ? wb : xb)
-                         : "memory");
+                         : "m0", "memory");
         wb += GP_BK * 2;
         xb += GP_BK * 2;
     };
