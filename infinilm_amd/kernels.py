@@ -407,6 +407,7 @@ _LIBRARY_F32_OUT = [True]   # cleared when torch.mm refuses out_dtype
 KSPLIT_SPAN = 4096  # K range of one part of the K-split few-rows product (ilm_gemm_ksplit_max_k(1))
 KSPLIT_FEW_SPAN = 1024   # ... and with up to 16 rows of up to KSPLIT_FEW_MAX
 KSPLIT_FEW_MAX = 8192
+KSPLIT_FEW_MAX_N = 8192  # ... and outputs: widest row of which the norm that sums the parts holds a piece a thread (ilm_add_rmsnorm)
 # Rows up to which the products keep X in registers (16 or 32; 32 only for K up to 4096 a workgroup)
 FEW_ROWS = int(os.environ.get("INFINILM_AMD_FEW_ROWS", "32"))
 
@@ -417,6 +418,24 @@ def _few_rows(M: int, K: int) -> bool:
     beside the W fragments in flight."""
     groups = max(1, min(FEW_ROWS // 16, 8192 // max(K, 4096)))
     return M <= 16 * groups
+
+
+def _few_span(M: int, N: int, K: int) -> int:
+    """K of one part of a few-rows product on its way into the residual sum (K up to it: no parts).
+
+    Up to 16 rows, 8,192 outputs and 8,192 k: parts of 1,024 k, which give a small matrix as many workgroups as the chip takes and every wave
+    a short chain of loads (8 rows: 1024 x 4096 4.6 us against 8.6 with all of K in one workgroup, 1024 x 2048 3.9 / 5.4,
+    2048 x 2048 4.5 / 5.9, 2304 x 2304 5.8 / 7.4, 4096 x 4096 8.3 / 10.2; against two parts of up to 4,096, with the norm that sums them: 1024 x 8192
+    9.2 us / 11.9, 2048 x 8192 11.9 / 16.1, 4096 x 8192 17.8 / 25.3, 8192 x 8192 36.5 / 43.7, 2304 x 5760 12.5 / 17.3, 2048 x 6144 11.6 / 12.7).  More
+    outputs lose what is won, and more: the norm reads the parts of such rows one after the other (8 rows with the norm: 8200 x 4096 64.5 us against
+    46.2 whole, 12288 x 4096 94.0 / 63.2; 8200 x 8192 107 / 67.3 in two parts, 12288 x 8192 162 / 99.9).  The upper end of K is
+    where the parts come to more than the eight that `qkv_rope_sum` takes: beyond, the gain is small (with the norm 2048 x 12288 17.9 us in three
+    parts, 16.2 in twelve, 4096 x 16384 31.4 in four, 30.7 in sixteen).  One size is left that K whole serves better: 256 tiles of W, a tile a
+    unit, and 2,049 to 3,072 k, whose three parts of 170 workgroups take a second round (with the norm 4096 x 3072 10.4 us whole, 11.2 in
+    three parts, 10.7 in four for 1 row, 11.6, 12.1 and 11.6 for 8; but 5120 x 3072 16.8, 12.9 and 15.0).  (From 4,096 k on for matrices of 1,024
+    rows or more, the range that was measured; narrower ones keep parts of 4,096.)"""
+    short = M <= 16 and N <= KSPLIT_FEW_MAX_N and (K <= KSPLIT_SPAN or (K <= KSPLIT_FEW_MAX and N >= 1024))
+    return KSPLIT_FEW_SPAN if short else KSPLIT_SPAN
 
 
 def _f32_few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -484,16 +503,7 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, 
             _run("ilm_gemm_rows64", parts.data_ptr(), N, M * N, kb, w.data_ptr(), w.stride(0), M, N, K, a.data_ptr(),
                  a.stride(0), 0, _stream())
         return parts
-    # Up to 16 rows and 8,192 k: parts of 1,024 k, which give a small matrix as many workgroups as the chip takes and every wave
-    # a short chain of loads (8 rows: 1024 x 4096 4.6 us against 8.6 with all of K in one workgroup, 1024 x 2048 3.9 / 5.4,
-    # 2048 x 2048 4.5 / 5.9, 2304 x 2304 5.8 / 7.4, 4096 x 4096 8.3 / 10.2; against two parts of up to 4,096, with the norm that sums them: 1024 x 8192
-    # 9.2 us / 11.9, 2048 x 8192 11.9 / 16.1, 4096 x 8192 17.8 / 25.3, 2304 x 5760 12.5 / 17.3, 2048 x 6144 11.6 / 12.7).  The upper end is
-    # where the parts come to more than the eight that `qkv_rope_sum` takes: beyond, the gain is small (with the norm 2048 x 12288 17.9 us in three
-    # parts, 16.2 in twelve, 4096 x 16384 31.4 in four, 30.7 in sixteen).  One size is left that K whole serves better: 256 tiles of W, a tile a
-    # unit, and 2,049 to 3,072 k, whose three parts of 170 workgroups take a second round (with the norm 4096 x 3072 10.4 us whole, 11.2 in
-    # three parts, 10.7 in four for 1 row, 11.6, 12.1 and 11.6 for 8; but 5120 x 3072 16.8, 12.9 and 15.0).
-    # (From 4,096 k on for matrices of 1,024 rows or more, the range that was measured; narrower ones keep parts of 4,096.)
-    span = KSPLIT_FEW_SPAN if M <= 16 and (K <= KSPLIT_SPAN or (K <= KSPLIT_FEW_MAX and N >= 1024)) else KSPLIT_SPAN
+    span = _few_span(M, N, K)
     if fast and aligned and plain and allow_parts and out is None and M <= max(16, FEW_ROWS) and K > span and USE_KSPLIT:
         kb = -(-K // span)
         parts = torch.empty((kb, M, N), dtype=F32, device=a.device)
