@@ -849,8 +849,9 @@ def bound_rows(rows: int) -> int:
     return b
 
 
-def attention_chunks(max_total_len: int, page: int, pairs: int, device, head_dim: int = 128) -> tuple:
-    """(keys a chunk, chunks) of the chunked single-token attention for `pairs` = tokens x head groups.
+def attention_chunks(max_total_len: int, page: int, pairs: int, device, head_dim: int = 128, reach: int = 0) -> tuple:
+    """(keys a chunk, chunks) of the chunked single-token attention for `pairs` = tokens x head groups; `reach`: the window (below 0: less the
+    length of a token's own chunk), 0 for none.
 
     A chunk is a whole number of steps of ATT_STEP keys.  Few tokens: one step a chunk (latency
     counts, the chip is not full anyway).  Up to four steps as long as the launch still has a
@@ -891,15 +892,22 @@ def attention_chunks(max_total_len: int, page: int, pairs: int, device, head_dim
     # and the whole, against the rule above: 32 tokens of 1,900 keys 11.0 us with 128 a chunk (512: 12.9); 48 of 1,000 9.2 / 9.0 with
     # 128 (384: 11.5 / 10.6), of 1,900 15.2 / 12.9 with 256 (512: 17.7 / 15.6), of 3,800 20.0 / 19.6 with 512 (1024: 27.1 / 26.6); 64 of 500 9.0 / 8.0
     # with 128 (384: 11.1 / 10.1), of 8,000 40.6 with 1024 (2048: 46.9); 96 of 1,000 15.4 / 13.2 with 256 (512: 18.4 / 15.1).
-    if head_dim <= 64:
+    # Contexts that the rule above leaves whole stay so up to 2,048 keys, as chunks would bring a merge that costs more than they save (8 heads of 64,
+    # 64 tokens: 500 keys 15.8 us whole, 17.9 in two, 1,900 keys 42.6 / 45.7, 3,800 keys 102.7 / 93.7; 128 tokens of 300 keys, 16 heads over 2, 7.3, in
+    # three 9.2), and under a window always.  A window shorter than the chunk ends inside it whatever its length: 48 tokens of up to 3,800 keys,
+    # window 256, 10.8 us in four chunks, 12.2 in eight; window 1024 20.1 / 17.7.
+    if head_dim <= 64 and (steps > per_chunk or (steps > 16 and reach == 0)):
         short = 1
         while short < per_chunk and (-(-steps // short) > 16 or workgroups(short) > 4 * cus):
             short *= 2
-        per_chunk = min(per_chunk, short)
+        if reach == 0 or short * ATT_STEP <= abs(reach):
+            per_chunk = min(per_chunk, short)
     while -(-steps // per_chunk) > ATT_MAX_CHUNKS:
         per_chunk += 1
-    # as many chunks of more equal length: 64 tokens of 500 keys at the 8B head shape 13.3 us in chunks of 2 + 2 steps, 15.8 in 3 + 1
-    per_chunk = -(-steps // -(-steps // per_chunk))
+    # As many chunks of more equal length: 64 tokens of 500 keys at the 8B head shape 13.1 us in chunks of 2 + 2 steps, 15.5 in 3 + 1.  Not
+    # under a window, which moves: there 11.7 us against 10.0 (window 256).
+    if reach == 0:
+        per_chunk = -(-steps // -(-steps // per_chunk))
     span = per_chunk * ATT_STEP
     return span, -(-max_total_len // span)
 
@@ -954,7 +962,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             _i32(single_rows, "single_rows")
             rows, n_single = single_rows, single_rows.numel()
         # (the tokens counted as the recorded steps round them, so that an eager step and a replayed one cut alike)
-        span, nsplit = attention_chunks(int(max_total_len), page, bound_rows(n_single) * nkv * (-(-(nh // nkv) // 16)), q.device, d)
+        span, nsplit = attention_chunks(int(max_total_len), page, bound_rows(n_single) * nkv * (-(-(nh // nkv) // 16)), q.device, d, reach)
         ws_acc = ws_ml = None
         if nsplit > 1 and (span, nsplit) != (ATT_STEP, 2):   # (two chunks of one step meet inside a workgroup)
             # partial results of the rows served here (not of every token of the step)

@@ -17,3 +17,13 @@ def chip(monkeypatch):
                                         (16, 32768, 5120, 4096)])
 def test_parts_of_a_few_rows_product(M, N, k, span):
     assert K._few_span(M, N, k) == span
+
+
+@pytest.mark.parametrize("keys,pairs,d,reach,cut", [
+    (500, 512, 64, 0, (512, 1)), (300, 256, 64, 0, (384, 1)), (1900, 512, 64, 0, (2048, 1)), (3800, 512, 64, 0, (2048, 2)),   # whole contexts
+    (3800, 96, 64, 0, (512, 8)), (3800, 96, 64, 256, (1024, 4)), (3800, 96, 64, -256, (1024, 4)), (3800, 96, 64, 1024, (512, 8)),  # and windows
+    (8000, 512, 64, 1024, (8192, 1)), (500, 128, 128, 0, (256, 2)), (500, 128, 128, 256, (384, 2)), (1900, 64, 64, 0, (128, 15)),
+    (4096, 16, 128, 0, (256, 16)), (4096, 128, 128, 0, (1024, 4))])
+def test_chunks_of_the_decode_attention(keys, pairs, d, reach, cut):
+    span, chunks = K.attention_chunks(keys, 64, pairs, DEV, d, reach)
+    assert (span, chunks) == cut and span * (chunks - 1) < keys <= span * chunks
