@@ -105,6 +105,32 @@ gemm_portion_kernel(const GpArgs A) {
         wb += GP_BK * 2;
         xb += GP_BK * 2;
     };
+    // The lane's outputs' biases, asked for ahead of the stages: behind them their way through memory cost 0.8 to 1.9 us (65 x 1024 x 1024
+    // 6.2 us, now 5.5, as without a bias and as the library's product with its addend; 2048 x 2048 x 1536 19.8, now 16.3, library 17.6).  With tiles
+    // of 256 x 256, whose sums leave no registers for them, right after the stages.
+    constexpr bool EARLY = TM * TN <= 16;
+    bf16 bs[TN][4];
+    auto load_bias = [&]() {
+        if (A.bias == nullptr) return;
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            const int tt = t % (TN / 2), second = t / (TN / 2);   // (gate, up and pairs: the second half of the t are the other of the same outputs)
+            int n;
+            if (EPI == GP_ROPE) {
+                const int half = A.d / 2, pairs = A.N / 2, p = nt * (BN / 2) + wn * (WN / 2) + tt * 16 + 4 * q, pc = p < pairs ? p : 0;
+                n = pc / half * A.d + pc % half + second * half;
+            } else {
+                n = EPI == GP_GLU ? nt * OUT + wn * (WN / 2) + tt * 16 + 4 * q : nt * OUT + wn * WN + t * 16 + 4 * q;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int at = EPI == GP_ROPE ? n + e : n + e < A.N ? n + e : A.N - 1;
+                bs[t][e] = A.bias[EPI == GP_GLU ? at + second * A.N : at];
+            }
+        }
+    };
+    if (EARLY) load_bias();
+    auto biased = [&](float v, int t, int e) { return A.bias != nullptr ? v + to_f32(bs[t][e]) : v; };
     f32x4 acc[TN][TM];
 #pragma unroll
     for (int t = 0; t < TN; ++t)
@@ -163,6 +189,7 @@ gemm_portion_kernel(const GpArgs A) {
     read(1, buf);
     multiply(0);
     multiply(1);
+    if (!EARLY) load_bias();
     // acc[t][g][e] of lane (r, q): row wm WM + 16 g + r of the tile, place wn WN + 16 t + 4 q + e
     if (EPI == GP_ROPE) {
         // (values go straight into their transposed cache; queries and keys through LDS, first halves of pairs ahead of second halves)
@@ -181,8 +208,7 @@ gemm_portion_kernel(const GpArgs A) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int h = 0; h < 2; ++h)
-                        v[h][e] = to_f32(from_f32<bf16>(acc[t + h * (TN / 2)][g][e] + (A.bias != nullptr ? to_f32(A.bias[hs * A.d + h * half + i0 + e]) : 0.f)));
+                    for (int h = 0; h < 2; ++h) v[h][e] = to_f32(from_f32<bf16>(biased(acc[t + h * (TN / 2)][g][e], t + h * (TN / 2), e)));
                 if (hs >= A.nh + A.nkv) {
                     if (slot < 0) continue;
                     bf16* dst = A.vc + ((size_t)(slot / A.page) * A.nkv + (hs - A.nh - A.nkv)) * A.d * A.page + (slot % A.page);
@@ -235,21 +261,11 @@ gemm_portion_kernel(const GpArgs A) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 if (EPI == GP_GLU) {
-                    float vg = acc[t][g][e], vu = acc[t + TN / 2][g][e];
-                    if (A.bias != nullptr) {
-                        const int n = nt * OUT + col + e, ne = n < A.N ? n : A.N - 1;
-                        vg += to_f32(A.bias[ne]);
-                        vu += to_f32(A.bias[ne + A.N]);
-                    }
+                    const float vg = biased(acc[t][g][e], t, e), vu = biased(acc[t + TN / 2][g][e], t + TN / 2, e);
                     // (gate and up rounded to bfloat16 first, as the product's kernel alone stores them)
                     o[e] = from_f32<bf16>(glu_act(to_f32(from_f32<bf16>(vg)), A.glu) * to_f32(from_f32<bf16>(vu)));
                 } else {
-                    float v = acc[t][g][e];
-                    if (A.bias != nullptr) {
-                        const int n = nt * OUT + col + e;
-                        v += to_f32(A.bias[n < A.N ? n : A.N - 1]);
-                    }
-                    o[e] = from_f32<bf16>(v);
+                    o[e] = from_f32<bf16>(biased(acc[t][g][e], t, e));
                 }
             }
             *reinterpret_cast<uint2*>(&lds[row * PITCH + col]) = *reinterpret_cast<const uint2*>(o);
