@@ -322,8 +322,12 @@ def _portion_tile(form: str, M: int, rows: int, K: int, device) -> int:
     larger tiles then use it better, and a smaller tile's second round costs as much as the first.
 
     plain: the smallest tile of which one round does (64 x 64, 128 x 64, 128 x 128).  K up to 4096: 2048 x 2048 x 8192 75.2 us against 75.7,
-    600 x 4096 x 16384 130 / 126; and with fewer than half of the units busy up to 2048, as the library cuts a long K (300 x 1024 x 4096, 80 tiles,
-    14.2 / 13.8; 700 x 1024 x 4096, 176 tiles, 14.8 / 17.8).  Two rounds: 700 x 8192 x 1024 18.2 / 18.0, 2048 x 12288 x 2048 106 / 100.
+    600 x 4096 x 16384 130 / 126; and with fewer than half of the units busy up to 2048, with fewer than an eighth up to 1024, as the library cuts a
+    long K (300 x 1024 x 4096, 80 tiles, 14.2 / 13.8; 700 x 1024 x 4096, 176 tiles, 14.8 / 17.8; 65 x 512 x 2048, 16 tiles, 7.9 / 5.4, x 1024 5.3 / 5.3).
+    Two rounds: 700 x 8192 x 1024 18.2 / 18.0, 2048 x 12288 x 2048 106 / 100.  Few outputs of many rows, where the library's tiles waste nothing: 2048 x
+    512 x 2048, 256 tiles, 12.6 / 11.7, x 1024 8.0 / 9.4; by larger tiles 8192 x 512 x 1024 14.4 / 13.7, x 512 9.9 / 11.3, 2048 x 768 x 3072 19.7 / 19.2.
+    Fewer outputs than a tile's 64: 1000 x 16 x 512 4.3 / 3.9, x 256 3.7 / 3.7, but 128 x 16 x 512 4.3 / 6.8.  Rows that are no multiple of 8 leave an element
+    at a time, which the larger tiles feel: 923 x 3853 x 2304 26.9 / 25.5, 137 x 8717 x 640 11.6 / 9.2; the small one 249 x 2381 x 2880 12.4 / 18.5.
     glu: K up to 1024 (1000 x 12288 x 2048 57.9 / 56.0, 400 rows 34.5 / 35.1).  A round of the large tiles that leaves less than a quarter of
     the chip idle, else the small ones up to three rounds (two share a unit): 700 x 8192 x 1024 19.9 / 23.1, 300 rows 12.6 / 17.4.
     rope: five quarters of a round (tiles end unevenly): 2048 x 1280 x 1024, 320 tiles, 18.7 / 20.1; 300 x 4608 x 4096, 216 tiles, 23.8 / 27.7;
@@ -346,7 +350,13 @@ def _portion_tile(form: str, M: int, rows: int, K: int, device) -> int:
     for tile, bm, bn in ((1, 64, 64), (2, 128, 64), (3, 128, 128)):
         n = count(bm, bn)
         if n <= cus:
-            return tile if 2 * n > cus or K <= 2048 else 0
+            if K > (1024 if 8 * n < cus else 2048 if 2 * n <= cus else 4096):
+                return 0
+            if rows < 64 and K > (512 if M <= 128 else 256):
+                return 0
+            if rows < 768 and (K > 512 if tile > 1 else K > 1024 and 4 * n > 3 * cus):
+                return 0
+            return 0 if tile > 1 and (rows % 8 or (rows < 1024 and K > 1536)) else tile
     return 0
 
 

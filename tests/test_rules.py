@@ -27,3 +27,14 @@ def test_parts_of_a_few_rows_product(M, N, k, span):
 def test_chunks_of_the_decode_attention(keys, pairs, d, reach, cut):
     span, chunks = K.attention_chunks(keys, 64, pairs, DEV, d, reach)
     assert (span, chunks) == cut and span * (chunks - 1) < keys <= span * chunks
+
+
+@pytest.mark.parametrize("M,N,k,tile", [
+    (2048, 1024, 1024, 2), (300, 1024, 1024, 1), (65, 8192, 1024, 1), (600, 4096, 2048, 3), (2048, 1024, 4096, 2), (700, 1024, 4096, 1),
+    (2048, 1024, 1000, 0), (2048, 2048, 8192, 0), (700, 8192, 1024, 0), (300, 1024, 4096, 0),        # stages, a long K, two rounds, half of the units
+    (65, 512, 1024, 1), (65, 512, 2048, 0), (512, 256, 1536, 1), (65, 1024, 2048, 1),                # an eighth
+    (2048, 512, 2048, 0), (2048, 512, 1024, 1), (1000, 512, 2048, 1), (8192, 512, 1024, 0), (8192, 512, 512, 3), (2048, 768, 3072, 0), (2048, 768, 1536, 2),
+    (1000, 16, 512, 0), (1000, 16, 256, 1), (128, 16, 512, 1), (128, 16, 1024, 0),                   # few outputs
+    (923, 3853, 2304, 0), (137, 8717, 640, 0), (249, 2381, 2880, 1)])                                # odd rows
+def test_portions_products(M, N, k, tile):
+    assert K._portion_tile("plain", M, N, k, DEV) == tile
