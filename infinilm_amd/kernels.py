@@ -330,8 +330,10 @@ def _portion_tile(form: str, M: int, rows: int, K: int, device) -> int:
     at a time, which the larger tiles feel: 923 x 3853 x 2304 26.9 / 25.5, 137 x 8717 x 640 11.6 / 9.2; the small one 249 x 2381 x 2880 12.4 / 18.5.
     glu: K up to 1024 (1000 x 12288 x 2048 57.9 / 56.0, 400 rows 34.5 / 35.1).  A round of the large tiles that leaves less than a quarter of
     the chip idle, else the small ones up to three rounds (two share a unit): 700 x 8192 x 1024 19.9 / 23.1, 300 rows 12.6 / 17.4.
-    rope: five quarters of a round (tiles end unevenly): 2048 x 1280 x 1024, 320 tiles, 18.7 / 20.1; 300 x 4608 x 4096, 216 tiles, 23.8 / 27.7;
-    more lose: 2047 x 4608 x 4096 119 / 79, 2048 x 6912 x 2304 128 / 117."""
+    rope: five quarters of a round (tiles end unevenly): 2048 x 1280 x 1024, 320 tiles, 18.4 / 19.9; 256 x 4608 x 4096, 288 tiles, 25.0 / 38.0; 300 x
+    4608 x 4096, 216 tiles, 23.8 / 27.7; more lose: 2047 x 4608 x 4096 119 / 79, 2048 x 6912 x 2304 128 / 117.  Tiles of 128 rows only up to a round where
+    K is long, as the library cuts it, or short, as the tiles' ends weigh: 512 x 4608 x 4096, 288 tiles, 36.9 / 34.4, 300 x 6144 x 4096 37.0 / 31.9, 1400 x
+    1536 x 512, 264 tiles, 17.7 / 16.8; but 2041 x 1280 x 2048, 320 tiles, 24.7 / 26.0."""
     if not USE_PORTION or K % 64:
         return 0
     cus = _num_cus(device)
@@ -346,7 +348,9 @@ def _portion_tile(form: str, M: int, rows: int, K: int, device) -> int:
     if K > 4096:
         return 0
     if form == "rope":
-        return next((tile for tile, bm in ((1, 64), (2, 128)) if 4 * count(bm, 64) <= 5 * cus), 0)
+        if 4 * count(64, 64) <= 5 * cus:
+            return 1
+        return 2 if count(128, 64) <= cus or (4 * count(128, 64) <= 5 * cus and 512 < K <= 2048) else 0
     for tile, bm, bn in ((1, 64, 64), (2, 128, 64), (3, 128, 128)):
         n = count(bm, bn)
         if n <= cus:

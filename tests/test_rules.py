@@ -38,3 +38,10 @@ def test_chunks_of_the_decode_attention(keys, pairs, d, reach, cut):
     (923, 3853, 2304, 0), (137, 8717, 640, 0), (249, 2381, 2880, 1)])                                # odd rows
 def test_portions_products(M, N, k, tile):
     assert K._portion_tile("plain", M, N, k, DEV) == tile
+
+
+@pytest.mark.parametrize("M,N,k,tile", [
+    (1024, 1280, 1024, 1), (256, 4608, 4096, 1), (300, 4608, 4096, 2), (2048, 1280, 1024, 2), (2041, 1280, 2048, 2), (256, 6912, 2304, 2),
+    (512, 4608, 4096, 0), (505, 4608, 3584, 0), (300, 6144, 4096, 0), (1400, 1536, 512, 0), (1280, 1536, 512, 2), (2048, 6912, 2304, 0)])
+def test_portions_projections_with_rotation(M, N, k, tile):
+    assert K._portion_tile("rope", M, N, k, DEV) == tile
