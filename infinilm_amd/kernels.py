@@ -328,8 +328,11 @@ def _portion_tile(form: str, M: int, rows: int, K: int, device) -> int:
     512 x 2048, 256 tiles, 12.6 / 11.7, x 1024 8.0 / 9.4; by larger tiles 8192 x 512 x 1024 14.4 / 13.7, x 512 9.9 / 11.3, 2048 x 768 x 3072 19.7 / 19.2.
     Fewer outputs than a tile's 64: 1000 x 16 x 512 4.3 / 3.9, x 256 3.7 / 3.7, but 128 x 16 x 512 4.3 / 6.8.  Rows that are no multiple of 8 leave an element
     at a time, which the larger tiles feel: 923 x 3853 x 2304 26.9 / 25.5, 137 x 8717 x 640 11.6 / 9.2; the small one 249 x 2381 x 2880 12.4 / 18.5.
+    Of drawn sizes that the rule takes seven in 198 lose (3 to 10 %, where the library has a tile that fits: 339 x 7616 x 2560 27.0 / 24.4), and the mean is 1.27 times as fast.
     glu: K up to 1024 (1000 x 12288 x 2048 57.9 / 56.0, 400 rows 34.5 / 35.1).  A round of the large tiles that leaves less than a quarter of
-    the chip idle, else the small ones up to three rounds (two share a unit): 700 x 8192 x 1024 19.9 / 23.1, 300 rows 12.6 / 17.4.
+    the chip idle and of its rows empty, else the small ones up to three rounds (two share a unit): 700 x 8192 x 1024 19.9 / 23.1, 300 rows 12.6 / 17.4;
+    300 x 16384 x 768, whose 256 tiles of 256 rows are two fifths empty, 19.3 with them, 17.5 with 640 small ones, 20.4.  Not a few tiles of a
+    small W, whose chain of stages alone is longer than the library's two kernels: 65 x 1024 x 1024 8.6 / 7.8, 200 rows 8.6 / 10.7, 65 x 2048 x 1024 8.8 / 10.3.
     rope: five quarters of a round (tiles end unevenly): 2048 x 1280 x 1024, 320 tiles, 18.4 / 19.9; 256 x 4608 x 4096, 288 tiles, 25.0 / 38.0; 300 x
     4608 x 4096, 216 tiles, 23.8 / 27.7; more lose: 2047 x 4608 x 4096 119 / 79, 2048 x 6912 x 2304 128 / 117.  Tiles of 128 rows only up to a round where
     K is long, as the library cuts it, or short, as the tiles' ends weigh: 512 x 4608 x 4096, 288 tiles, 36.9 / 34.4, 300 x 6144 x 4096 37.0 / 31.9, 1400 x
@@ -342,8 +345,10 @@ def _portion_tile(form: str, M: int, rows: int, K: int, device) -> int:
         if K > 1024:
             return 0
         for tile, bm, bn in ((5, 256, 256), (4, 256, 128)):
-            if 4 * count(bm, bn) > 3 * cus and count(bm, bn) <= cus:
+            if 4 * count(bm, bn) > 3 * cus and count(bm, bn) <= cus and 4 * M > 3 * bm * -(-M // bm):
                 return tile
+        if rows < 2048 and K >= 768 and 8 * count(64, 128) < cus:
+            return 0
         return 1 if count(64, 128) <= 3 * cus else 0
     if K > 4096:
         return 0

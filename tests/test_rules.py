@@ -45,3 +45,10 @@ def test_portions_products(M, N, k, tile):
     (512, 4608, 4096, 0), (505, 4608, 3584, 0), (300, 6144, 4096, 0), (1400, 1536, 512, 0), (1280, 1536, 512, 2), (2048, 6912, 2304, 0)])
 def test_portions_projections_with_rotation(M, N, k, tile):
     assert K._portion_tile("rope", M, N, k, DEV) == tile
+
+
+@pytest.mark.parametrize("M,N,k,tile", [
+    (300, 8192, 1024, 1), (700, 8192, 1024, 1), (1000, 8192, 1024, 4), (2048, 8192, 1024, 5), (300, 16384, 768, 1), (500, 16384, 768, 4),
+    (65, 1024, 1024, 0), (130, 1536, 768, 1), (33, 512, 1024, 0), (200, 1024, 1024, 1), (65, 2048, 1024, 1), (65, 512, 512, 1), (400, 12288, 2048, 0)])
+def test_portions_gate_and_up(M, N, k, tile):
+    assert K._portion_tile("glu", M, N, k, DEV) == tile
