@@ -687,11 +687,10 @@ __device__ __noinline__ void sample_row(SampleLds& S, const float* row, int V, f
 // elements reach, and few more do (of independent numbers 56 for k = 50, 532 for 224).  So the row is read once for the maxima, at one
 // instruction an element instead of some 40 for bins, the bound is found by one wave bit by bit in registers, and only threads with an element
 // that reaches it read theirs again.  64 rows of 73,448, top-k 50, top-p 0.9: 35 us ->
-// 20, top-k 200 45 -> 36, 5 rows of 122,753, top-k 50 46 -> 24.
+// 20, top-k 200 45 -> 36; 5 rows of 122,753, top-k 50 24, in chunks 26 (46 by one workgroup with histograms).
 #define FEW_K 224
 #define FEW_GROUPS (SB / 4)
 #define FEW_FROM (4 * SB)   // vocabulary from which every thread has elements
-#define FEW_TIES 64     // groups beyond k at the bound from which a row is left to the histograms (rows of ties)
 
 // Threshold and token of a list of up to 64 E elements that holds all of the top-k: by the first wave, E elements a lane, each weighed
 // against all (rank_list, top_p_of_list and token_of_list in one wave, without their barriers: some 12 us for a list of 60)
@@ -772,7 +771,67 @@ __device__ __forceinline__ void token_of_few(const SampleLds& S, int n, int k, f
     if (lane == 0) *out = (int)pick;
 }
 
-// The row's top-k of 2 to FEW_K; false: the list does not hold it (ties, masked rows, NaN)
+// The token of a row whose top-k ends in ties: kept are the n listed elements, fewer than k, and all of key `at` below them.  One more reading of the row, an
+// instruction or two an element, gives the tiles' masses (5 rows of 122,753 equal numbers, top-p 0.9: 47 us, by histograms 217, in chunks 176)
+#define TIE_TILES 8
+__device__ __noinline__ void token_of_ties(SampleLds& S, const float* row, int V, Mass mass, uint32_t at, int n, float pp, float uniform, int* out) {
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, m = tile_groups(V), tiles = (V + 256 * m - 1) / (256 * m);
+    const u64 tie = mass(key_to_float(at));
+    const bool whole = ((uintptr_t)row & 15) == 0;
+    u64 total = 0;
+    for (int t0 = w; t0 < tiles; t0 += TIE_TILES * SNW) {
+        int ties[TIE_TILES] = {};
+        u64 more[TIE_TILES] = {};
+        for (int g = 0; g < m; ++g) {
+            float l[TIE_TILES][4];   // of as many tiles at once: a tile's way through memory is longer than its work
+#pragma unroll
+            for (int u = 0; u < TIE_TILES; ++u) {
+                const int i0 = ((t0 + u * SNW) * m + g) * 256 + 4 * lane;
+                if (whole && i0 + 3 < V) {
+                    const float4 v = *reinterpret_cast<const float4*>(row + i0);
+                    l[u][0] = v.x, l[u][1] = v.y, l[u][2] = v.z, l[u][3] = v.w;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) l[u][e] = row[i0 + e < V ? i0 + e : V - 1];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < TIE_TILES; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bool in = ((t0 + u * SNW) * m + g) * 256 + 4 * lane + e < V;
+                    const uint32_t key = okey(l[u][e]);
+                    ties[u] += __popcll(__builtin_amdgcn_ballot_w64(in && key == at));
+                    if (in && key > at && l[u][e] == l[u][e]) more[u] += mass(l[u][e]);
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < TIE_TILES; ++u) {
+            const int t = t0 + u * SNW;
+            if (t >= tiles) break;
+            const u64 sum = (u64)ties[u] * tie + (__builtin_amdgcn_ballot_w64(more[u] > 0) != 0ull ? wave_sum_u64(more[u]) : 0ull);
+            if (lane == 0) {
+                S.tile[t] = sum;
+                total += sum;
+            }
+        }
+    }
+    uint32_t tau = at;
+    if (pp < 1.0f) {
+        total = block_sum_u64<SB>(total, S.red);
+        const uint32_t tp = pp > 0.f ? rank_list<false>(S, n, 0, 0, (double)pp * (double)total) : okey(mass.mx);
+        tau = tp > at ? tp : at;
+    }
+    if (tau > at) {
+        clear_tiles(S, tiles);
+        list_to_tiles(S, n, tau, m);
+    } else {
+        __syncthreads();
+    }
+    if (w == 0) token_of_tiles(S, row, V, mass, tau, uniform, -1, 0, out);
+}
+
+// The row's top-k of 2 to FEW_K; false: the list does not hold it (an infinite maximum with ties, many elements a thread that reach the bound)
 __device__ __forceinline__ bool top_k_of_few(SampleLds& S, const float* row, int V, float temp, int k, float pp, float uniform, int cut, int* out) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     uint32_t* group = reinterpret_cast<uint32_t*>(S.hist);      // [FEW_GROUPS]; behind them the waves' results
@@ -808,20 +867,28 @@ __device__ __forceinline__ bool top_k_of_few(SampleLds& S, const float* row, int
             const uint32_t v = __shfl_xor(top, o, 64);
             top = v > top ? v : top;
         }
+        const int reached = reach(at);    // (by all lanes: behind the branch a ballot counts the first lane's groups alone)
         if (lane == 0) {
             bound[0] = at;
             bound[1] = top;
-            bound[2] = (uint32_t)reach(at);
+            bound[2] = (uint32_t)reached;
         }
     }
     __syncthreads();
     const uint32_t at = bound[0];
     const float mx = key_to_float(bound[1]);
-    if ((int)bound[2] > k + FEW_TIES) return false;
     const Mass mass = {mx, 1.0f / temp, cut};
-    if (okey(most) >= at)
+    // Every group at the bound: ties, more perhaps than the list holds (255 of 256 stand for some 1,400 elements where they lie anywhere)
+    const bool ties = bound[2] == FEW_GROUPS;
+    // At a bound without mass (a mask that leaves fewer than k groups, or a bound far below the maximum) and at one of ties only what lies above is listed:
+    // where that comes to fewer than k, the first adds nothing that could be drawn, and the second all of its ties
+    const u64 tie = mass(key_to_float(at));
+    const bool above = temp > 0.f && mass(mx) > 0 && (ties || tie == 0);
+    if (ties && !above) return false;
+    const uint32_t least = above ? at + 1 : at;
+    if (okey(most) >= least)
         over_row<SB>(row, V, [&](int i, float l) {
-            if (okey(l) >= at && l == l) {
+            if (okey(l) >= least && l == l) {
                 const int to = atomicAdd(&S.listed, 1);
                 if (to < LIST_CAP) {
                     S.list.key[to] = okey(l);
@@ -832,7 +899,11 @@ __device__ __forceinline__ bool top_k_of_few(SampleLds& S, const float* row, int
         });
     __syncthreads();
     const int n = S.listed;
-    if (n < k || n > LIST_CAP) return false;
+    if (n > LIST_CAP || (n < k && !above)) return false;
+    if (n < k && tie > 0) {
+        token_of_ties(S, row, V, mass, at, n, pp, uniform, out);
+        return true;
+    }
     if (n > 128) {
         uint32_t tau = rank_list<true>(S, n, 0, 0, (double)k);
         if (pp < 1.0f) {

@@ -1232,3 +1232,58 @@ def test_a_top_k_that_is_no_int(K):
     rows = lambda ks: [(SamplingParams(top_k=k, top_p=0.9), i, 4) for i, k in enumerate(ks)]
     want = Sampler(5).sample(logits, rows([50, 4, 0]))
     assert Sampler(5).sample(logits, rows([50.0, 4.5, 2 ** 31])) == want
+
+
+@pytest.mark.parametrize("V", [4096, 40003, 122753])
+@pytest.mark.parametrize("name", ["masked to 60", "masked to 3", "finite mask", "all equal", "two values", "zeros of both signs", "cold", "ties and a mask", "steps", "NaN and a mask"])
+def test_sampling_top_k_of_few_that_ends_in_ties_or_in_a_mask(K, name, V):
+    """The bound of a top-k of few where nothing above it reaches k: elements that no number can draw below, or ties, whose whole number is kept.
+    The plain distribution's intervals (within 1e-6, see test_sampling_where_thresholds_are_hard), and the tokens that rows in chunks give."""
+    g = torch.Generator().manual_seed(V + 2)
+    row = torch.randn(V, generator=g) * 2
+    some = torch.randperm(V, generator=g)
+    temp = 0.02 if name == "cold" else 0.8
+    if name == "masked to 60":
+        row[some[60:]] = -math.inf
+    elif name == "masked to 3":
+        row[some[3:]] = -math.inf
+    elif name == "finite mask":
+        row[some[60:]] = -3e38
+    elif name == "all equal":
+        row[:] = 1.25
+    elif name == "two values":
+        row[:] = -1.0
+        row[some[:30]] = 0.5
+    elif name == "zeros of both signs":
+        row = -row.abs() - 1
+        row[some[:500]] = 0.0
+        row[some[500:1000]] = -0.0
+    elif name == "ties and a mask":
+        row[some[2000:]] = -math.inf
+        row[some[:2000]] = torch.randint(0, 3, (2000,), generator=g).float()
+    elif name == "steps":
+        row = (row * 2).round() / 2
+    elif name == "NaN and a mask":
+        row[some[100:]] = -math.inf
+        row[some[:40]] = math.nan
+    us = [0.0, 0.3, 0.71, 1.0 - 2.0 ** -24]
+    mk = lambda v, dt: torch.tensor(v, dtype=dt, device=DEV)
+    rows = row.expand(4, V).contiguous().to(DEV)
+    for k in (2, 50, 100, 191, 192, K.sample_few_k()):
+        for p in (1.0, 0.9, 1e-3):
+            prm = torch.cat([mk([temp] * 4, torch.float32), mk([k] * 4, torch.int32).view(torch.float32), mk([p] * 4, torch.float32), mk(us, torch.float32)])
+            one = K.sample_packed(rows, prm, few=True).tolist()
+            assert one == K.sample_packed(rows, prm).tolist()
+            if name == "NaN and a mask":
+                assert all(row[t] == row[t] and row[t] > -math.inf for t in one)
+                continue
+            if name == "zeros of both signs":      # (their keys differ, so where a top-k ends among them it ends at the sign)
+                if k > 500:
+                    continue
+                dist = P.plain_sample_distribution(torch.where((row == 0) & (torch.signbit(row)), -1.0, row), temp, k, p)
+            else:
+                dist = P.plain_sample_distribution(row, temp, k, p)
+            cdf = torch.cumsum(dist, 0)
+            for u, tok in zip(us, one):
+                assert 0 <= tok < V and dist[tok] > 0, f"token {tok} is outside the kept set (k={k}, p={p})"
+                assert float(cdf[tok] - dist[tok]) - 1e-6 <= u <= float(cdf[tok]) + 1e-6
