@@ -1282,7 +1282,7 @@ sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row,
 //   73,448:  1 row 26 / 65, 24 / 19, 17 / 34;  32 rows 39 / 68, 35 / 20, 22 / 35;  64 rows 55 / 69, 42 / 20, 29 / 36
 //   122,753: 5 rows 30 / 103, 26 / 24, 17 / 56;  32 rows 45 / 105, 41 / 25, 25 / 56;  64 rows 53 / 111, 43 / 27, 32 / 62;
 //            96 rows 80 / 115, 55 / 29, 43 / 63
-// A caller who knows that every row asks for a top-k of at most FEW_K gives no workspace and has them by one workgroup each.
+// A caller who knows that every row asks for a top-k of at most FEW_K may give no workspace and have them by one workgroup each (the rule: kernels.sample_one_reading).
 #define CHUNKS_FROM 40960
 #define CHUNKS_MANY_FROM 98304      // ... with more than 32 rows, up to 64
 extern "C" long ilm_sample_ws(int n, int V) {

@@ -129,4 +129,4 @@ class Sampler:
         d.copy_(buf[:4 * n], non_blocking=True)
         if dev.type == "cuda":
             self._record(t)
-        return kernels.sample_packed(logits, d, few=0 < min(top_k) and max(top_k) <= kernels.sample_few_k())
+        return kernels.sample_packed(logits, d, few=0 < min(top_k) and kernels.sample_one_reading(n, logits.shape[1], max(top_k)))
