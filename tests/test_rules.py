@@ -60,3 +60,9 @@ def test_portions_gate_and_up(M, N, k, tile):
     (8, 152064, 64, False), (16, 122753, 160, True), (12, 152064, 160, False), (32, 122753, 224, True), (64, 152064, 224, True), (64, 152064, 225, False)])
 def test_route_of_a_small_top_k(n, V, k, one):
     assert K.sample_one_reading(n, V, k) == one
+
+
+@pytest.mark.parametrize("M,k,taken", [(1, 2048, True), (2, 1024, True), (8, 256, True), (1, 3328, True), (1, 4096, True), (1, 2304, False), (1, 3072, False),
+                                       (2, 2048, False), (1, 1000, False), (1, 4352, False), (9, 256, False)])
+def test_rows_that_the_projection_forms(M, k, taken):
+    assert K._qkv_sum_rows(M, k) == taken
