@@ -370,7 +370,9 @@ def _portion_tile(form: str, M: int, rows: int, K: int, device) -> int:
 
 
 def _portion_operands_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    return (_mfma_operands_ok(x, w, x.shape[1]) and not FORCE_BASIC and x.shape[0] * x.stride(0) < 1 << 31 and w.shape[0] * w.stride(0) < 1 << 31)
+    """(Rows that share memory, as an expanded one's do, stay with the library.)"""
+    return (_mfma_operands_ok(x, w, x.shape[1]) and not FORCE_BASIC and min(x.stride(0), w.stride(0)) >= x.shape[1]
+            and x.shape[0] * x.stride(0) < 1 << 31 and w.shape[0] * w.stride(0) < 1 << 31)
 
 
 def portion_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, tile: int) -> torch.Tensor:

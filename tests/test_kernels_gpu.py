@@ -1287,3 +1287,24 @@ def test_sampling_top_k_of_few_that_ends_in_ties_or_in_a_mask(K, name, V):
             for u, tok in zip(us, one):
                 assert 0 <= tok < V and dist[tok] > 0, f"token {tok} is outside the kept set (k={k}, p={p})"
                 assert float(cdf[tok] - dist[tok]) - 1e-6 <= u <= float(cdf[tok]) + 1e-6
+
+
+@pytest.mark.parametrize("shared", ["x", "w"])
+def test_products_of_rows_that_share_memory(K, shared):
+    """One row for all (an expanded tensor), at sizes whose portions have a kernel of their own: the product, gate/up with its activation and
+    q/k/v with rotation give what the rows one by one give, or leave the call to who takes it.  (Tolerance: bfloat16 results.)"""
+    g = torch.Generator().manual_seed(9)
+    M, N, k = 300, 1024, 1024
+    x, w = torch.randn((M, k), generator=g).to(BF16).to(DEV), (torch.randn((N, k), generator=g) / 32).to(BF16).to(DEV)
+    x, w = (x[:1].expand(M, k), w) if shared == "x" else (x, w[:1].expand(N, k))
+    want = x.float() @ w.float().T
+    assert float((K.gemm(x, w).float() - want).abs().max()) <= 2.0 ** -7 * float(want.abs().max())
+    y = K.gateup_swiglu_gemm(x, w, None)
+    if y is not None:
+        want_y = torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:]
+        assert float((y.float() - want_y).abs().max()) <= 2.0 ** -6 * float(want_y.abs().max())
+    pos = torch.zeros(M, dtype=torch.int32, device=DEV)
+    cos, sin = torch.ones((4, 32), device=DEV), torch.zeros((4, 32), device=DEV)
+    q = K.qkv_rope_gemm(x, w, None, pos, cos, sin, None, None, None, 12, 2, 64, 64)
+    if q is not None:
+        assert float((q.float() - want[:, :768]).abs().max()) <= 2.0 ** -7 * float(want.abs().max())
