@@ -219,9 +219,10 @@ USE_QKV_ROPE = os.environ.get("INFINILM_AMD_QKV_ROPE", "1") == "1"
 def qkv_rope_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], positions: torch.Tensor,
                   cos: torch.Tensor, sin: torch.Tensor, k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor],
                   slots: Optional[torch.Tensor], nh: int, nkv: int, d: int, rd: int) -> Optional[torch.Tensor]:
-    """The fused projection x w^T (+ bias) of a few rows, q and k rotated and k, v written to the cache
-    in the product's epilogue.  Returns the rotated q [T, nh*d], or None where the fused kernel does
-    not apply (more than 32 rows, float32, a partly rotated or odd-sized head): the caller then
+    """The fused projection x w^T (+ bias), q and k rotated and k, v written to the cache in the product's
+    epilogue: of a few rows (up to 32), and of portions of prompts (more than 64 rows) whose tiles make about one
+    round over the chip (`_portion_tile`).  Returns the rotated q [T, nh*d], or None where no fused kernel
+    applies (33 to 64 rows, more than a round, float32, a partly rotated or odd-sized head): the caller then
     runs the projection and `rope_kvwrite` one after the other."""
     M, K = x.shape
     if not (USE_QKV_ROPE and not FORCE_BASIC and x.dtype == BF16 and w.dtype == BF16 and _few_rows(M, K) and rd == d and d % 32 == 0
@@ -751,10 +752,11 @@ def gateup_resident_ok(rows: int, w: torch.Tensor) -> bool:
 def gateup_swiglu_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor],
                        row_ss: Optional[torch.Tensor] = None, eps: float = 0.0, frag_w=None,
                        act: str = "silu") -> Optional[torch.Tensor]:
-    """act(x Wg^T + bg) * (x Wu^T + bu) for few rows in bfloat16, W = [Wg; Wu]: the fused gate/up
-    projection with the SwiGLU in its epilogue, [M, I] (up to 32 rows with X in registers; 17 to 208 with chunks
-    of X in LDS where the outputs fill the chip).  None where no kernel applies (more rows, few outputs,
-    float32): the caller then runs the projection and the activation.  `row_ss`: x is what `gemm_tail` left (residual * norm weight) and row_ss its
+    """act(x Wg^T + bg) * (x Wu^T + bu) in bfloat16, W = [Wg; Wu]: the fused gate/up projection with the SwiGLU in its
+    epilogue, [M, I] (up to 32 rows with X in registers; 17 to 208 with chunks of X in LDS where the outputs
+    fill the chip; other numbers of rows from 33 on and K up to 1024 in tiles, where those make a round or a few
+    over the chip: `_portion_tile`).  None where no kernel applies (larger products, float32): the caller then runs
+    the projection and the activation.  `row_ss`: x is what `gemm_tail` left (residual * norm weight) and row_ss its
     partial sums of squares: the rows' division by sqrt(mean square + eps) happens in this kernel's
     epilogue (only the kernel with X in registers does that: `gateup_resident_ok`)."""
     M, K = x.shape

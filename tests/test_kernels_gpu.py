@@ -1173,6 +1173,25 @@ def test_portion_rule(K):
         got = K.gemm(x, w)
         assert torch.equal(got, K.portion_gemm(x, w, None, torch.empty_like(got), tile))
         assert float((got.float() - want).norm() / want.norm()) < 2.0 ** -8
+    # gate/up and q/k/v: the forms that end in what their next kernel did, against the product and that kernel (see test_portion_qkv on the rotation)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    for M in (300, 700):
+        x, w = torch.randn((M, 1024), generator=g, device=DEV).to(BF16), (torch.randn((8192, 1024), generator=g, device=DEV) / 32).to(BF16)
+        assert K._portion_tile("glu", M, 8192, 1024, dev)
+        y = K.gateup_swiglu_gemm(x, w, None)
+        assert y is not None and torch.equal(y, K.swiglu(K.portion_gemm(x, w, None, torch.empty((M, 8192), dtype=BF16, device=DEV), 1), "silu"))
+    for M in (300, 1000, 2048):
+        x, w = torch.randn((M, 1024), generator=g, device=DEV).to(BF16), (torch.randn((1280, 1024), generator=g, device=DEV) / 32).to(BF16)
+        pos, slots = torch.arange(M, dtype=torch.int32, device=DEV), torch.arange(M, dtype=torch.int32, device=DEV)
+        cos, sin = torch.rand((M, 32), generator=g, device=DEV), torch.rand((M, 32), generator=g, device=DEV)
+        caches = [(torch.zeros((M // 16 + 1, 2, 16, 64), dtype=BF16, device=DEV), torch.zeros((M // 16 + 1, 2, 64, 16), dtype=BF16, device=DEV)) for _ in range(2)]
+        assert K._portion_tile("rope", M, 1280, 1024, dev)
+        q = K.qkv_rope_gemm(x, w, None, pos, cos, sin, *caches[0], slots, 16, 2, 64, 64)
+        rows = K.portion_gemm(x, w, None, torch.empty((M, 1280), dtype=BF16, device=DEV), 1)
+        K.rope_kvwrite(rows, pos, cos, sin, *caches[1], slots, 16, 2, 64, 64)
+        assert q is not None and torch.equal(caches[0][1], caches[1][1])
+        for got, want in ((q, rows[:, :1024]), (caches[0][0], caches[1][0])):
+            assert bool(((got.double() - want.double()).abs() <= want.double().abs() * 2.0 ** -7 + 1e-6).all())
 
 
 @pytest.mark.parametrize("M,K_,nh,nkv,d,parts", [(1, 256, 2, 1, 32, 1), (1, 1024, 16, 2, 64, 4), (2, 1024, 5, 1, 64, 8), (1, 2048, 16, 2, 64, 2), (8, 256, 3, 3, 96, 3),
