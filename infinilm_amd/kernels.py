@@ -7,6 +7,7 @@ library or a CPU tensor is an error.
 """
 from __future__ import annotations
 
+import functools
 import os
 from typing import Optional
 
@@ -1071,7 +1072,9 @@ def _sample(logits: torch.Tensor, temperature: int, top_k: int, top_p: int, unif
     return out
 
 
+@functools.lru_cache(maxsize=None)
 def sample_few_k() -> int:
+    """The largest top-k that a row is served with in one reading (the library's constant)."""
     return _lib().ilm_sample_few_k()
 
 

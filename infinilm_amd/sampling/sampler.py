@@ -85,13 +85,11 @@ class Sampler:
         self._copied_on = [-1, -1]
         self._turn = 0
 
-    def _record(self, t: int) -> None:
-        """Marks the end of buffer t's copy.  An event belongs to the device that it was first recorded on, and the next
-        logits may lie on another."""
-        device = torch.cuda.current_device()
-        if self._copied[t] is None or self._copied_on[t] != device:
+    def _event(self, t: int, device: int):
+        """The event of buffer t's copy.  It belongs to the device that it was first recorded on, and the next logits may lie on another."""
+        if self._copied_on[t] != device:
             self._copied[t], self._copied_on[t] = torch.cuda.Event(), device
-        self._copied[t].record()
+        return self._copied[t]
 
     def sample(self, logits: torch.Tensor, rows: Sequence[Tuple[SamplingParams, int, int]]) -> List[int]:
         """`rows[i]` = (params, request key, index of the token being generated) for logits[i]."""
@@ -128,5 +126,5 @@ class Sampler:
         d = torch.empty((4 * n,), dtype=torch.float32, device=dev)
         d.copy_(buf[:4 * n], non_blocking=True)
         if dev.type == "cuda":
-            self._record(t)
+            self._event(t, dev.index).record()
         return kernels.sample_packed(logits, d, few=0 < min(top_k) and kernels.sample_one_reading(n, logits.shape[1], max(top_k)))

@@ -390,6 +390,6 @@ def test_a_sampler_moves_between_devices(monkeypatch):
     for device, made in ((0, 2), (0, 2), (1, 4), (0, 6)):
         at[0] = device
         for t in (0, 1):
-            s._record(t)
+            s._event(t, device).record()
             assert s._copied[t].device == device
         assert Event.made == made
