@@ -248,7 +248,7 @@ moe_sort_kernel(int* __restrict__ offsets, int* __restrict__ perm, int* __restri
 // moe_route_groups_kernel and moe_sort_kernel in one, for few tokens and at most 64 experts: a wave a token and a lane an expert, so a choice is a
 // reduction in registers, and the order is made by the same block from LDS.  The same scores, choices and weights, bit for bit.  Decode steps of 16
 // tokens, 16 experts in 4 groups, top 2: 8.7 us against 9.0 and
-// 4.5 and the gap between them, all of it latency.
+// 4.5 and the gap between them, all of it latency.  More tokens take turns and lose (kernels.MOE_PLAN_TOKENS has both sides).
 #define MOE_FEW_TOKENS 64
 #define MOE_FEW_PAIRS 512
 __global__ void __launch_bounds__(1024)

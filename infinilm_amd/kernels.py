@@ -2225,6 +2225,12 @@ class ExpertPlan:
     __slots__ = ("ids", "weights", "perm", "inv", "tiles", "n_tiles", "offsets", "max_tiles", "top", "pairs", "tile_rows")
 
 
+# Tokens up to which experts are chosen and the pairs ordered in one kernel (ilm_moe_plan_few): a wave a token in its one block; more take turns there, where
+# two kernels spread over the chip.  us in two kernels against one: 16 experts in 4 groups, top 2: 1 token 9.8 / 6.5, 16 11.2 / 7.7, 24 11.3 / 10.4, 32 11.4 / 11.5,
+# 64 11.7 / 19.1; 64 experts, top 8: 16 tokens 16.4 / 13.9, 24 16.5 / 19.4, 64 16.9 / 35.9
+MOE_PLAN_TOKENS = 16
+
+
 def moe_route(logits: torch.Tensor, experts: int, top: int, big_tiles_ok: bool = False, softmax: bool = False,
               weight_scale: float = 1.0, identity: int = 0, correction: Optional[torch.Tensor] = None, groups: int = 1, keep: int = 1,
               normalise: bool = False) -> ExpertPlan:
@@ -2252,7 +2258,7 @@ def moe_route(logits: torch.Tensor, experts: int, top: int, big_tiles_ok: bool =
     plan.top, plan.pairs = int(top), P
     plan.ids = torch.empty((T, top), dtype=torch.int32, device=dev)
     plan.weights = torch.empty((T, top), dtype=F32, device=dev)
-    few = grouped and bool(_lib().ilm_moe_plan_few_ok(T, total, int(top)))     # (choice and order in one kernel, below)
+    few = grouped and T <= MOE_PLAN_TOKENS and bool(_lib().ilm_moe_plan_few_ok(T, total, int(top)))     # (choice and order in one kernel, below)
     if few:
         pass
     elif grouped:

@@ -755,3 +755,29 @@ def test_choice_and_order_of_few_tokens(K, T, E, ident, top, groups, keep):
         flat = plan.ids.flatten()
         placed = plan.inv >= 0
         assert torch.equal(placed, flat < E) and torch.equal(plan.perm[plan.inv[placed].long()].long(), placed.nonzero().flatten())
+
+
+@pytest.mark.parametrize("T,total,top,groups,keep", [(16, 16, 2, 4, 2), (17, 64, 8, 8, 4), (33, 60, 4, 4, 2), (64, 64, 8, 1, 1)])
+def test_choice_and_order_by_the_entry_itself(K, T, total, top, groups, keep):
+    """One token a wave and more, whose waves take turns, whatever number of tokens the rule sends there; rows of NaN and infinities among them."""
+    from infinilm_amd.csrc import lib
+    L, P, s = lib.load(), T * top, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator().manual_seed(T)
+    z, c = torch.randn((T, total), generator=g), (0.3 * torch.randn(total, generator=g)).to(DEV)
+    z[torch.rand((T, total), generator=g) < 0.05] = -math.inf
+    z[T // 3, ::5] = math.nan
+    z[T // 2, 1] = math.inf
+    z = z.to(DEV)
+    new = lambda n: torch.full((n,), -7, dtype=torch.int32, device=DEV)
+    got, want = [[new(P), torch.zeros(P, device=DEV), new(total + 1), new(P), new(P), new(3 * P), new(1)] for _ in range(2)]
+    assert L.ilm_moe_plan_few(got[0].data_ptr(), got[1].data_ptr(), z.data_ptr(), c.data_ptr(), T, total, top, total, groups, keep, 1.5,
+                              *(t.data_ptr() for t in got[2:]), total, P, L.ilm_moe_tile_rows(), s) == 0
+    assert L.ilm_moe_route_groups(want[0].data_ptr(), want[1].data_ptr(), z.data_ptr(), c.data_ptr(), 0, T, total, top, total, groups, keep, 1.5, s) == 0
+    assert L.ilm_moe_sort(*(t.data_ptr() for t in want[2:]), want[0].data_ptr(), P, total, P, L.ilm_moe_tile_rows(), s) == 0
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1].nan_to_num(-1.0), want[1].nan_to_num(-1.0))
+    assert torch.equal(got[2], want[2]) and torch.equal(got[6], want[6])
+    n = 3 * int(want[6])
+    assert torch.equal(got[5][:n], want[5][:n])
+    at = got[2].tolist()
+    for e in range(total):
+        assert sorted(got[3][at[e]:at[e + 1]].tolist()) == sorted(want[3][at[e]:at[e + 1]].tolist())

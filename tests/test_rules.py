@@ -66,3 +66,16 @@ def test_route_of_a_small_top_k(n, V, k, one):
                                        (2, 2048, False), (1, 1000, False), (1, 4352, False), (9, 256, False)])
 def test_rows_that_the_projection_forms(M, k, taken):
     assert K._qkv_sum_rows(M, k) == taken
+
+
+@pytest.mark.parametrize("T,one", [(1, True), (16, True), (17, False), (64, False)])
+def test_experts_are_chosen_and_ordered_in_one_kernel_for_few_tokens(monkeypatch, T, one):
+    from types import SimpleNamespace
+
+    called = []
+    monkeypatch.setattr(K, "_dev", lambda *a: None)
+    monkeypatch.setattr(K, "_stream", lambda: 0)
+    monkeypatch.setattr(K, "_lib", lambda: SimpleNamespace(ilm_moe_plan_few_ok=lambda *a: 1, ilm_moe_tile_rows=lambda: 16, ilm_moe_big_tile_rows=lambda: 128))
+    monkeypatch.setattr(K, "_run", lambda name, *a, **k: called.append(name))
+    K.moe_route(torch.zeros(T, 16), 16, 2, softmax=True, groups=4, keep=2, correction=torch.zeros(16), normalise=True)
+    assert called == (["ilm_moe_plan_few"] if one else ["ilm_moe_route_groups", "ilm_moe_sort"])
