@@ -291,6 +291,13 @@ def _qkv_sum_rows(M: int, K: int) -> bool:
     return M <= 16 and K % 256 == 0 and M * K <= (4096 if K > 3072 else 2048)
 
 
+def _qkv_sum_parts(M: int, K: int, N: int, parts: int) -> bool:
+    """Whether every workgroup's reading of so many parts is worth the norm's kernel: beyond four, with every wave's place taken by several rows, not over
+    many outputs, whose workgroups all read them (8 parts: 2 rows of 1,024 over 3,072 outputs 8.8 us against 8.2 with the norm's kernel, over 1,280 7.2
+    / 7.3, 4 parts 7.8 / 8.3; 4 rows of 512 over 4,608 8.5 / 8.1; 8 rows of 256 7.7 / 7.9; 1 row of 2,048 11.3 / 12.0)."""
+    return parts <= 4 or M == 1 or M * K <= 1024 or K <= 256 or N < 2048
+
+
 def qkv_rope_sum(residual: torch.Tensor, parts: torch.Tensor, alpha: float, norm_w: torch.Tensor, w_offset: float, eps: float, w: torch.Tensor,
                  bias: Optional[torch.Tensor], positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_cache: Optional[torch.Tensor],
                  v_cache: Optional[torch.Tensor], slots: Optional[torch.Tensor], nh: int, nkv: int, d: int, rd: int):
@@ -302,7 +309,8 @@ def qkv_rope_sum(residual: torch.Tensor, parts: torch.Tensor, alpha: float, norm
             and residual.dtype == F32 and residual.is_contiguous() and parts.dtype == F32 and parts.dim() == 3 and parts.is_contiguous()
             and tuple(parts.shape[1:]) == (M, K) and 1 <= parts.shape[0] <= QKV_SUM_PARTS and norm_w.shape == (K,) and norm_w.is_contiguous()
             and norm_w.dtype in (BF16, F32) and w.shape == ((nh + 2 * nkv) * d, K) and w.stride(1) == 1 and w.stride(0) % 8 == 0
-            and w.data_ptr() % 16 == 0 and residual.data_ptr() % 16 == 0 and parts.data_ptr() % 16 == 0):
+            and w.data_ptr() % 16 == 0 and residual.data_ptr() % 16 == 0 and parts.data_ptr() % 16 == 0
+            and _qkv_sum_parts(M, K, w.shape[0], parts.shape[0])):
         return None
     _dev(residual, parts, norm_w, w, bias, positions, cos, sin, k_cache, v_cache, slots)
     page = _qkv_rope_checks(w, bias, BF16, M, positions, cos, sin, k_cache, v_cache, slots, nh, nkv, d)

@@ -68,6 +68,12 @@ def test_rows_that_the_projection_forms(M, k, taken):
     assert K._qkv_sum_rows(M, k) == taken
 
 
+@pytest.mark.parametrize("M,k,N,parts,taken", [(1, 2048, 6144, 8, True), (2, 1024, 1280, 8, True), (2, 1024, 3072, 4, True), (2, 1024, 3072, 8, False),
+                                               (4, 512, 4608, 5, False), (8, 256, 6144, 8, True), (4, 256, 6144, 8, True)])
+def test_parts_that_the_projection_sums(M, k, N, parts, taken):
+    assert K._qkv_sum_parts(M, k, N, parts) == taken
+
+
 @pytest.mark.parametrize("T,one", [(1, True), (16, True), (17, False), (64, False)])
 def test_experts_are_chosen_and_ordered_in_one_kernel_for_few_tokens(monkeypatch, T, one):
     from types import SimpleNamespace
