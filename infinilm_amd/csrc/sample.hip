@@ -687,47 +687,30 @@ __device__ __noinline__ void sample_row(SampleLds& S, const float* row, int V, f
 // elements reach, and few more do (of independent numbers 56 for k = 50, 532 for 224).  So the row is read once for the maxima, at one
 // instruction an element instead of some 40 for bins, the bound is found by one wave bit by bit in registers, and only threads with an element
 // that reaches it read theirs again.  64 rows of 73,448, top-k 50, top-p 0.9: 35 us ->
-// 20, top-k 200 45 -> 36; 5 rows of 122,753, top-k 50 24, in chunks 26 (46 by one workgroup with histograms).
+// 20, top-k 100 25, top-k 200 45 -> 36; 5 rows of 122,753, top-k 50 24, in chunks 26 (46 by one workgroup with histograms).
 #define FEW_K 224
 #define FEW_GROUPS (SB / 4)
 #define FEW_FROM (4 * SB)   // vocabulary from which every thread has elements
+#define FEW_WAVE 64       // listed elements that one wave ranks, an element a lane
 
-// Threshold and token of a list of up to 64 E elements that holds all of the top-k: by the first wave, E elements a lane, each weighed
-// against all (rank_list, top_p_of_list and token_of_list in one wave, without their barriers: some 12 us for a list of 60)
-template <int E>
+// Threshold and token of a list of up to 64 elements that holds all of the top-k: by the first wave, an element a lane, each weighed
+// against all (rank_list, top_p_of_list and token_of_list in one wave, without their barriers: some 12 us for a list of 60).  Two elements a lane
+// lose to the block: 8 rows of 4,096, k 60 15.4 us against 13.3, k 100 21.4 / 16.3, 8 rows of 73,448, k 100 29.2 / 25.0.
 __device__ __forceinline__ void token_of_few(const SampleLds& S, int n, int k, float pp, float uniform, int* out) {
     const int lane = threadIdx.x & 63;
-    uint32_t key[E];
-    int index[E];
-    u64 mass[E];
-    int count[E];
-    u64 above[E];    // mass of the elements with keys from this one's on
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int i = e * 64 + lane;
-        key[e] = i < n ? S.list.key[i] : 0u;
-        index[e] = i < n ? S.list.index[i] : -1;
-        mass[e] = i < n ? S.list.mass[i] : 0ull;
-        count[e] = 0;
-        above[e] = 0;
-    }
+    const uint32_t key = lane < n ? S.list.key[lane] : 0u;
+    const int index = lane < n ? S.list.index[lane] : -1;
+    const u64 mass = lane < n ? S.list.mass[lane] : 0ull;
+    int count = 0;
+    u64 above = 0;    // mass of the elements with keys from this one's on
 #pragma unroll 4
     for (int j = 0; j < n; ++j) {
         const uint32_t kj = S.list.key[j];
-        const u64 mj = S.list.mass[j];
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            count[e] += kj >= key[e] ? 1 : 0;
-            above[e] += kj >= key[e] ? mj : 0ull;
-        }
+        const u64 mj = S.list.mass[j];    // (read whether or not it counts: loads behind a condition wait one after the other)
+        count += kj >= key ? 1 : 0;
+        above += kj >= key ? mj : 0ull;
     }
-    auto largest = [&](auto of) {    // (of: a key, or 0)
-        uint32_t best = 0;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const uint32_t v = of(e);
-            best = v > best ? v : best;
-        }
+    auto largest = [&](uint32_t best) {    // (of a key a lane, or 0)
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
             const uint32_t v = __shfl_xor(best, o, 64);
@@ -735,39 +718,29 @@ __device__ __forceinline__ void token_of_few(const SampleLds& S, int n, int k, f
         }
         return best;
     };
-    auto kept = [&](uint32_t tau) {    // mass of the elements from tau on
-        u64 sum = 0;
-#pragma unroll
-        for (int e = 0; e < E; ++e) sum += key[e] >= tau ? mass[e] : 0ull;
-        return wave_sum_u64(sum);
-    };
-    uint32_t tau = largest([&](int e) { return count[e] >= k ? key[e] : 0u; });
+    auto kept = [&](uint32_t tau) { return wave_sum_u64(key >= tau ? mass : 0ull); };    // mass of the elements from tau on
+    uint32_t tau = largest(count >= k ? key : 0u);
     u64 total = kept(tau);
     if (pp < 1.0f) {
         const double need = (double)pp * (double)total;
-        const uint32_t tp = !(pp > 0.f) ? largest([&](int e) { return key[e]; })
-                            : total > 0 ? largest([&](int e) { return key[e] >= tau && (double)above[e] >= need ? key[e] : 0u; })
-                                        : 0u;
+        const uint32_t tp = largest(!(pp > 0.f) || (total > 0 && key >= tau && (double)above >= need) ? key : 0u);
         if (tp > tau) {
             tau = tp;
             total = kept(tau);
         }
     }
     const double target = (double)uniform * (double)total;
-    u64 run[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) run[e] = 0;
+    u64 run = 0;
 #pragma unroll 4
     for (int j = 0; j < n; ++j) {
         const int ij = S.list.index[j];
         const u64 mj = S.list.key[j] >= tau ? S.list.mass[j] : 0ull;
-#pragma unroll
-        for (int e = 0; e < E; ++e) run[e] += ij <= index[e] ? mj : 0ull;
+        run += ij <= index ? mj : 0ull;
     }
-    uint32_t pick = 0;    // the first index that passes the target (as its complement), else the last kept one
-    pick = largest([&](int e) { return key[e] >= tau && mass[e] > 0 && target < (double)run[e] ? ~(uint32_t)index[e] : 0u; });
+    // the first index that passes the target (as its complement), else the last kept one
+    uint32_t pick = largest(key >= tau && mass > 0 && target < (double)run ? ~(uint32_t)index : 0u);
     if (pick != 0) pick = ~pick;
-    else pick = largest([&](int e) { return index[e] >= 0 && key[e] >= tau ? (uint32_t)index[e] + 1u : 0u; }) - 1u;
+    else pick = largest(index >= 0 && key >= tau ? (uint32_t)index + 1u : 0u) - 1u;
     if (lane == 0) *out = (int)pick;
 }
 
@@ -904,7 +877,7 @@ __device__ __forceinline__ bool top_k_of_few(SampleLds& S, const float* row, int
         token_of_ties(S, row, V, mass, at, n, pp, uniform, out);
         return true;
     }
-    if (n > 128) {
+    if (n > FEW_WAVE) {
         uint32_t tau = rank_list<true>(S, n, 0, 0, (double)k);
         if (pp < 1.0f) {
             const uint32_t tp = pp > 0.f ? top_p_of_list(S, n, tau, pp) : okey(mx);
@@ -919,8 +892,7 @@ __device__ __forceinline__ bool top_k_of_few(SampleLds& S, const float* row, int
             if (w == 0) token_of_tiles(S, row, V, mass, tau, uniform, S.pick - 1, 0, out);
         }
     } else if (w == 0) {
-        if (n <= 64) token_of_few<1>(S, n, k, pp, uniform, out);
-        else token_of_few<2>(S, n, k, pp, uniform, out);
+        token_of_few(S, n, k, pp, uniform, out);
     }
     return true;
 }

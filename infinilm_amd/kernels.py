@@ -1087,14 +1087,19 @@ def sample_few_k() -> int:
 
 
 def sample_one_reading(n: int, V: int, k: int) -> bool:
-    """Whether n rows of V, all of a top-k up to `k`, go to one workgroup each (`few` of `sample_packed`) and not in chunks.  A workgroup's list and its
-    ranking grow with k, and its reading with V; chunks take as long whatever V, up to 8 rows, longer from 12 rows on and with every row more.  us
-    in chunks against one workgroup, top-p 0.9:
-      1 to 8 rows:  65,536: k 128 26.0 / 25.6, 192 31.7 / 34.0;  73,448: k 64 23.9 / 22.6, 128 29.5 / 27.7, 160 32.1 / 34.2;  98,000: k 50 23.9 / 20.1, 64 24.5
-                    / 23.4, 96 25.6 / 29.9;  122,753: k 50 24.4 / 22.8, 64 26.2 / 27.0, 96 29.0 / 32.4, 192 33.0 / 39.2;  152,064: k 32 24.9 / 25.0, 64 26.2 / 29.7
-      12, 16 rows:  122,753: k 96 32.5 / 32.4, 160 38.7 / 38.1;  152,064: k 80 33.8 / 32.8, 160 38.9 / 41.6
-      32 rows:      122,753: k 96 42.7 / 33.2, 224 49.5 / 42.8;  152,064: k 224 50.8 / 45.0"""
-    return k <= sample_few_k() and (n >= 24 or (V - 40960) * k <= (4_500_000 if n < 12 else 13_500_000))
+    """Whether n rows of V, all of a top-k up to `k`, go to one workgroup each (`few` of `sample_packed`) and not in chunks.  A workgroup's reading grows
+    with V, and its list and ranking with k, fastest beyond 96; chunks take as long whatever V, up to 8 rows, longer from 12 rows on and with every
+    row more.  us in chunks against one workgroup, top-p 0.9:
+      1 to 8 rows:  65,536: k 128 25.9 / 25.7, 192 31.9 / 34.0;  73,448: k 64 23.8 / 19.9, 128 29.4 / 27.9, 160 32.2 / 33.7;  98,000: k 96 25.6 / 23.3, 112 26.1
+                    / 27.4;  122,753: k 50 24.4 / 23.0, 96 26.3 / 26.3, 112 26.3 / 29.4, 192 32.5 / 39.2;  152,064: k 16 23.1 / 24.0, 50 23.9 / 26.0
+      12, 16 rows:  122,753: k 96 32.4 / 28.6, 160 38.7 / 38.2;  152,064: k 96 32.2 / 30.3, 112 32.9 / 33.2, 160 39.0 / 41.7
+      32 rows:      122,753: k 96 42.4 / 29.4, 224 49.9 / 43.0;  152,064: k 224 50.5 / 45.4"""
+    if k > sample_few_k():
+        return False
+    if n >= 24:
+        return True
+    room = (V - 40960) * k
+    return room <= 13_500_000 if n >= 12 else V <= 131072 and (k <= 96 or room <= 4_500_000)
 
 
 def uniforms(out: int, seeds: Optional[int], seed: int, keys: int, indices: int, n: int) -> None:

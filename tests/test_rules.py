@@ -56,7 +56,7 @@ def test_portions_gate_and_up(M, N, k, tile):
 
 @pytest.mark.parametrize("n,V,k,one", [
     (1, 32768, 224, True), (64, 73448, 50, True), (5, 49152, 224, True), (1, 65536, 128, True), (1, 65536, 192, False), (2, 73448, 128, True),
-    (8, 73448, 160, False), (1, 98000, 64, True), (4, 98000, 96, False), (5, 122753, 50, True), (5, 122753, 100, False), (1, 122753, 200, False),
+    (8, 73448, 160, False), (4, 98000, 96, True), (1, 98000, 112, False), (5, 122753, 50, True), (1, 122753, 96, True), (1, 152064, 16, False), (5, 122753, 100, False), (1, 122753, 200, False),
     (8, 152064, 64, False), (16, 122753, 160, True), (12, 152064, 160, False), (32, 122753, 224, True), (64, 152064, 224, True), (64, 152064, 225, False)])
 def test_route_of_a_small_top_k(n, V, k, one):
     assert K.sample_one_reading(n, V, k) == one
