@@ -457,7 +457,8 @@ def _few_span(M: int, N: int, K: int) -> int:
     Up to 16 rows, 8,192 outputs and 8,192 k: parts of 1,024 k, which give a small matrix as many workgroups as the chip takes and every wave
     a short chain of loads (8 rows: 1024 x 4096 4.6 us against 8.6 with all of K in one workgroup, 1024 x 2048 3.9 / 5.4,
     2048 x 2048 4.5 / 5.9, 2304 x 2304 5.8 / 7.4, 4096 x 4096 8.3 / 10.2; against two parts of up to 4,096, with the norm that sums them: 1024 x 8192
-    9.2 us / 11.9, 2048 x 8192 11.9 / 16.1, 4096 x 8192 17.8 / 25.3, 8192 x 8192 36.5 / 43.7, 2304 x 5760 12.5 / 17.3, 2048 x 6144 11.6 / 12.7).  More
+    9.2 us / 11.9, 2048 x 8192 11.9 / 16.1, 4096 x 8192 17.8 / 25.3, 8192 x 8192 36.5 / 43.7, 2304 x 5760 12.5 / 17.3, 2048 x 6144 11.6 / 12.7; other
+    norms gain less, and there, where two parts give every unit one workgroup, lose 0.6 us: 1 row with a layer norm 13.3 / 12.7).  More
     outputs lose what is won, and more: the norm reads the parts of such rows one after the other (8 rows with the norm: 8200 x 4096 64.5 us against
     46.2 whole, 12288 x 4096 94.0 / 63.2; 8200 x 8192 107 / 67.3 in two parts, 12288 x 8192 162 / 99.9).  The upper end of K is
     where the parts come to more than the eight that `qkv_rope_sum` takes: beyond, the gain is small (with the norm 2048 x 12288 17.9 us in three
