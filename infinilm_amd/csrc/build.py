@@ -121,17 +121,20 @@ def build(verbose: bool = True) -> str:
             s = pending.pop(0)
             obj = os.path.join(out_dir, s[:-4] + f".{os.getpid()}.o")
             cmd = [hipcc] + HIPCC_FLAGS + ["-I", HERE, "-c", os.path.join(HERE, s), "-o", obj]
-            p = subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, env=env, cwd=out_dir)
-            running.append((s, obj, p))
+            said = tempfile.TemporaryFile()   # (a pipe that nobody reads meanwhile stops a compiler with many warnings for good)
+            p = subprocess.Popen(cmd, stdout=said, stderr=subprocess.STDOUT, env=env, cwd=out_dir)
+            running.append((s, obj, p, said))
         still = []
-        for s, obj, p in running:
+        for s, obj, p, said in running:
             rc = p.poll()
             if rc is None:
-                still.append((s, obj, p))
+                still.append((s, obj, p, said))
                 continue
-            out = p.stdout.read().decode(errors="replace")
+            said.seek(0)
+            out = said.read().decode(errors="replace")
+            said.close()
             if rc != 0:
-                for _, _, q in running:
+                for _, _, q, _ in running:
                     if q is not p and q.poll() is None:
                         q.kill()
                 raise RuntimeError(f"infinilm_amd: hipcc failed on {s}:\n{out}")
@@ -143,7 +146,7 @@ def build(verbose: bool = True) -> str:
         if running:
             time.sleep(0.2)
             if verbose and time.time() - last > 10:
-                _say("still compiling " + ", ".join(s for s, _, _ in running) + f" ({time.time() - t0:.0f} s)")
+                _say("still compiling " + ", ".join(s for s, _, _, _ in running) + f" ({time.time() - t0:.0f} s)")
                 last = time.time()
     tmp_lib = os.path.join(out_dir, f".{LIB_NAME}.{os.getpid()}")
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-fno-gpu-rdc"] + sorted(objs) + ["-o", tmp_lib]
