@@ -17,36 +17,16 @@
 // tile, which is the B-side layout of the second product (V^T tile of 16 dims x 4 keys on the A side,
 // values transposed in the cache: 16 bytes are four consecutive keys of one dim): no exchange between lanes.
 // Needs head sizes in steps of 16 up to 256, pages that are multiples of 4 keys, 16-byte aligned rows.
-#include "common.h"
-
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
-#define FA_CHUNK 128
-#define FA_TILES (FA_CHUNK / 16)
-#define FA_WS_PAD 4   // a partial result is d outputs, its maximum, its sum and two unused floats (16-byte rows)
-
-__device__ __forceinline__ f32x4 fa_mfma(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// (M, L, ACC) <- fold of (M, L, ACC) and a chunk's (m, l, acc): explicit multiply-adds, the same in both
-// launch shapes and in the fold kernel
-__device__ __forceinline__ void fa_fold_scales(float& M, float& L, float m, float l, float& a, float& b) {
-    const float Mn = fmaxf(M, m);
-    a = expf(M - Mn);
-    b = expf(m - Mn);
-    L = fmaf(L, a, l * b);
-    M = Mn;
-}
+#include "attn_f32.h"
 
 // DT: head size / 16.  !SPLIT: gridDim.z == 1 and the wave walks all chunks; SPLIT: blockIdx.z is the
 // chunk and the partial result goes to ws[((t * nh + h) * gridDim.z + chunk) * (d + FA_WS_PAD)].
-// P16: pages hold whole tiles of 16 keys.
+// `rows`: the launch's tokens, -1 for none; null: all.  P16: pages hold whole tiles of 16 keys.
 template <int DT, bool SPLIT, bool P16>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DT <= 8 ? 2 : 1)))
 attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __restrict__ qp, const float* __restrict__ kc,
                 const float* __restrict__ vc, const int* __restrict__ block_tables, const int* __restrict__ seg,
-                const int* __restrict__ pos, int nh, int nkv, int nsub, int page, int max_blocks, int q_stride,
+                const int* __restrict__ pos, const int* __restrict__ rows, int nh, int nkv, int nsub, int page, int max_blocks, int q_stride,
                 int out_stride, float scale, int reach, float softcap) {
     constexpr int d = DT * 16;
     // tiles of keys (and of values) in flight: two, or one where the running result of the wave that walks all
@@ -57,7 +37,9 @@ attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __
     // 2 heads of 128 31.3 (36.6).  Four tiles in flight with the values started before the softmax spilled at four waves a
     // SIMD and was slower.
     constexpr int NB = (!SPLIT && DT > 6) ? 1 : 2;
-    const int t = blockIdx.x, lane = threadIdx.x, r = lane & 15, q = lane >> 4;
+    const int t = rows != nullptr ? rows[blockIdx.x] : blockIdx.x;
+    if (t < 0) return;
+    const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
     const int G = nh / nkv;
     const int kvh = blockIdx.y / nsub, sub = blockIdx.y % nsub;
     const int heads = (G - sub * 16 < 16) ? G - sub * 16 : 16;
@@ -297,13 +279,20 @@ attn_f32_fold_kernel(float* __restrict__ out, const float* __restrict__ ws, cons
     if (dim < d) orow[dim] = ACC * (1.0f / L);
 }
 
+int fa_fold(float* out, const float* ws, const int* pos, int T, int nh, int d, int nchunks, int out_stride, int reach, hipStream_t stream) {
+    attn_f32_fold_kernel<<<dim3(T, nh), 64 * ((d + 63) / 64), 0, stream>>>(out, ws, pos, nh, d, nchunks, out_stride, reach);
+    ILM_LAUNCH_CHECK("attn_f32_fold");
+    return 0;
+}
+
 extern "C" int ilm_attn_f32_chunk() { return FA_CHUNK; }
 extern "C" int ilm_attn_f32_ws_row(int d) { return d + FA_WS_PAD; }
 
-// ws: null (one wave walks all chunks of its token), or float [T][nh][nchunks][d + 4] with
+// rows: the T tokens this call serves (-1: none), null for tokens 0 .. T - 1.  fold: the step's tokens, T without `rows`.
+// ws: null (one wave walks all chunks of its token), or float [fold][nh][nchunks][d + 4] with
 // nchunks >= ceil((largest position + 1) / ilm_attn_f32_chunk()): one wave a chunk, then the fold.
 extern "C" int ilm_attn_f32(void* out, void* ws, int nchunks, const void* q, const void* kc, const void* vc,
-                            const void* block_tables, const void* seg, const void* pos, int T_, int nh, int nkv, int d,
+                            const void* block_tables, const void* seg, const void* pos, const void* rows, int T_, int fold, int nh, int nkv, int d,
                             int page, int max_blocks, int q_stride, int out_stride, float scale, int reach, float softcap,
                             hipStream_t stream) {
     ILM_REQUIRE(T_ > 0 && nh > 0 && nkv > 0 && d > 0 && page > 0 && max_blocks > 0, "attn_f32: bad sizes");
@@ -314,12 +303,13 @@ extern "C" int ilm_attn_f32(void* out, void* ws, int nchunks, const void* q, con
                     && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 15) == 0 && (ws == nullptr || ((uintptr_t)ws & 15) == 0),
                 "attn_f32: rows must be 16-byte aligned");
     ILM_REQUIRE(ws == nullptr || (nchunks >= 1 && nchunks <= 65535), "attn_f32: %d chunks", nchunks);
+    ILM_REQUIRE(rows != nullptr || fold == T_, "attn_f32: %d tokens of %d", T_, fold);
     const int G = nh / nkv, nsub = (G + 15) / 16;
     ILM_REQUIRE((long long)nkv * nsub <= 65535 && nh <= 65535, "attn_f32: too many heads");
     dim3 grid(T_, nkv * nsub, ws != nullptr ? nchunks : 1);
     const bool p16 = page % 16 == 0;
 #define FA_ARGS (float*)out, (float*)ws, (const float*)q, (const float*)kc, (const float*)vc, (const int*)block_tables, \
-                (const int*)seg, (const int*)pos, nh, nkv, nsub, page, max_blocks, q_stride, out_stride, scale, reach, softcap
+                (const int*)seg, (const int*)pos, (const int*)rows, nh, nkv, nsub, page, max_blocks, q_stride, out_stride, scale, reach, softcap
 #define FA_CASE(DT_)                                                                        \
     case DT_:                                                                               \
         if (ws != nullptr && p16) attn_f32_kernel<DT_, true, true><<<grid, 64, 0, stream>>>(FA_ARGS);  \
@@ -335,10 +325,6 @@ extern "C" int ilm_attn_f32(void* out, void* ws, int nchunks, const void* q, con
 #undef FA_CASE
 #undef FA_ARGS
     ILM_LAUNCH_CHECK("attn_f32");
-    if (ws != nullptr) {
-        attn_f32_fold_kernel<<<dim3(T_, nh), 64 * ((d + 63) / 64), 0, stream>>>((float*)out, (const float*)ws, (const int*)pos, nh, d, nchunks,
-                                                              out_stride, reach);
-        ILM_LAUNCH_CHECK("attn_f32_fold");
-    }
+    if (ws != nullptr) return fa_fold((float*)out, (const float*)ws, (const int*)pos, fold, nh, d, nchunks, out_stride, reach, stream);
     return 0;
 }

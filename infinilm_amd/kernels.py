@@ -26,7 +26,14 @@ BASIC_SPLIT = os.environ.get("INFINILM_AMD_BASIC_SPLIT", "1") == "1"   # 0: alwa
 BASIC_SPLIT_WAVES = 4096   # (token, head) pairs up to which the plain kernel takes one wave a chunk
 F32_ATTN_CHUNK = 128   # keys a chunk of the 32-bit matrix-core attention (ilm_attn_f32_chunk())
 F32_ATTN_SPLIT = os.environ.get("INFINILM_AMD_F32_ATTN_SPLIT", "1") == "1"   # 0: always one wave a (token, head group)
-F32_ATTN_SPLIT_WAVES = 2048   # (token, head group) pairs up to which it takes one wave a chunk
+F32_ATTN_TILE_HEADS = (64, 128)   # head sizes of the kernel that takes portions in tiles of tokens (ilm_attn_f32_tile_ok())
+# (token, head group) pairs beyond which portions take it.  Below, a wave a token and chunk fills the chip as well or better, and single tokens beside
+# the portion need no launch of their own: 128 tokens of 32 heads of 128 over 2 19.7 us, in tiles 20.3; 300 38.4 / 34.1; 210 and three single ones of up
+# to 900 keys 31.4 / 40.1; 200 of 16 heads of 64 over 2 16.7 / 18.8, 300 23.0 / 19.6; 17 of 36 heads of 64 8.6 / 9.5, 40 11.7 / 11.4, 300 133 / 31.
+F32_ATTN_TILE_MIN = int(os.environ.get("INFINILM_AMD_F32_ATTN_TILE_MIN", "512"))
+# Waves up to which these kernels take one (a workgroup) a chunk.  In tiles, split / whole: 800 tokens of 32 heads of 128 over 2 (1,600 waves) 98 / 108 us,
+# 1,200 (2,400) 184 / 165; 300 of 36 heads of 64 (1,368) 31 / 34, 500 (2,268) 61 / 56; 300 at the end of 2,000 keys 140 / 222 and 168 / 214
+F32_ATTN_SPLIT_WAVES = 2048
 # INFINILM_AMD_BASIC=1 runs the plain kernels everywhere (for telling a kernel's fault from the engine's)
 FORCE_BASIC = os.environ.get("INFINILM_AMD_BASIC", "0") == "1"
 SKINNY_VARIANT = int(os.environ.get("INFINILM_AMD_SKINNY_VARIANT", "0"))  # 0: the kernel chooses
@@ -1010,15 +1017,31 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     if (q.dtype == F32 and not FORCE_BASIC and d % 16 == 0 and d <= 256 and page % 4 == 0 and q.stride(0) % 4 == 0
             and q.data_ptr() % 16 == 0 and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0):
         # the 32-bit path: the group's heads side by side on the float matrix instruction.  Few tokens (decoding):
-        # one wave a chunk of keys and a fold; many: one wave a token that walks its chunks.  The same bits.
+        # one wave a chunk of keys and a fold; many: one wave a token that walks its chunks; portions of prompts: tiles of
+        # tokens that share their keys through LDS.  The same bits.
+        G = nh // nkv
+        groups = nkv * -(-G // 16)
+        rows, n_single, waves = None, T, T * groups
+        tiled = 0
+        if (tiles is not None and tiles.numel() > 0 and T * groups > F32_ATTN_TILE_MIN and d in F32_ATTN_TILE_HEADS and page % 16 == 0):
+            _i32(tiles, "tiles")
+            tiled = tiles.numel() // 2
+            waves = tiled * groups * (8 if G > 8 else 4 if G > 4 else 2 if G > 2 else 1)
+            rows, n_single = single_rows, 0 if single_rows is None else single_rows.numel()
+            if n_single:
+                _i32(single_rows, "single_rows")
         ws, nchunks = None, 1
-        waves = T * nkv * -(-(nh // nkv) // 16)
         if F32_ATTN_SPLIT and waves <= F32_ATTN_SPLIT_WAVES and bound > F32_ATTN_CHUNK:
             nchunks = -(-bound // F32_ATTN_CHUNK)
             ws = torch.empty((T * nh * nchunks * (d + 4),), dtype=F32, device=q.device)
-        _run("ilm_attn_f32", out.data_ptr(), _ptr(ws), nchunks, q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-             block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr(), T, nh, nkv, d, page,
-             block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
+        if tiled:
+            _run("ilm_attn_f32_tile", out.data_ptr(), _ptr(ws), nchunks, q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                 block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr(), tiles.data_ptr(), tiled, 0 if n_single else T, nh, nkv, d,
+                 page, block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
+        if n_single:
+            _run("ilm_attn_f32", out.data_ptr(), _ptr(ws), nchunks, q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                 block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr(), _ptr(rows), n_single, T, nh, nkv, d, page,
+                 block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
         return out
     # The plain kernel.  Few tokens over long contexts (decoding): one wave a chunk of keys and a fold of the
     # partial results, instead of one wave a head; the bits are the same (see attn_basic.hip).

@@ -39,6 +39,8 @@ def test_constants_mirrored_in_python_equal_the_library(K):
     assert L.ilm_attn_mfma_step() == K.ATT_STEP
     assert L.ilm_attn_basic_chunk() == K.BASIC_CHUNK
     assert L.ilm_attn_f32_chunk() == K.F32_ATTN_CHUNK and L.ilm_attn_f32_ws_row(128) == 132
+    assert L.ilm_attn_f32_tile_tokens() == K.ATT_TILE_TOKENS
+    assert all(bool(L.ilm_attn_f32_tile_ok(d, 16)) == (d in K.F32_ATTN_TILE_HEADS) for d in range(16, 272, 16))
     assert L.ilm_gemm_ksplit_max_k(1) == K.KSPLIT_SPAN
     assert L.ilm_gemm_rows64_span() == K.ROWS64_SPAN
 
@@ -763,6 +765,45 @@ def test_attention_float32_short_contexts(K, monkeypatch, nh, nkv, d, window):
             outs.append(out.cpu())
     assert all(torch.equal(o, outs[0]) for o in outs[1:])
     _close(outs[0], want, 3e-6)
+
+
+@pytest.mark.parametrize("nh,nkv,d,page", [(32, 2, 128, 64), (17, 1, 64, 16), (10, 2, 64, 48), (12, 2, 128, 16), (4, 1, 128, 32), (3, 3, 64, 64),
+                                           (4, 2, 128, 16)])
+@pytest.mark.parametrize("window", [0, 100, 21])
+def test_attention_float32_tiles_of_tokens_give_the_same_bits(K, monkeypatch, nh, nkv, d, page, window):
+    """Portions whose tokens share their keys through LDS: every number of heads a wave and of tokens a tile, tiles that end on either side of a
+    chunk, beside single tokens, against the kernel that takes tokens one by one."""
+    case = dict(lens=[1, 2, 16, 17, 40, 128, 131, 300, 700, 523], qlens=[1, 2, 9, 17, 8, 3, 7, 300, 1, 12], window=window, seed=13)
+    monkeypatch.setattr(K, "F32_ATTN_TILE_MIN", 1 << 30)
+    alone, want = _attention_case(K, torch.float32, nh, nkv, d, page, **case)
+    monkeypatch.setattr(K, "F32_ATTN_TILE_MIN", 0)
+    for split in (True, False):
+        monkeypatch.setattr(K, "F32_ATTN_SPLIT", split)
+        tiles, _ = _attention_case(K, torch.float32, nh, nkv, d, page, **case)
+        assert torch.equal(tiles.cpu(), alone.cpu())
+    _close(tiles, want, 3e-6)
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(9, 1, 64), (5, 1, 128), (3, 1, 64), (2, 2, 128)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_attention_float32_tiles_keep_later_values_from_earlier_tokens(K, monkeypatch, nh, nkv, d, bad):
+    """A value that is not finite reaches the tokens that see it and no other of the tile; what lies in the page behind the last token is not read."""
+    n, first, page = 150, 101, 64
+    k, v, q = (_rand((m, h, d), s, torch.float32) for m, h, s in ((n, nkv, 1), (n, nkv, 2), (n - first, nh, 3)))
+    v[125, 0, 5] = bad
+    kc, vc, bt = _paged([k], [v], page, 4, 4, torch.float32)
+    for i in range(n, 192):
+        kc[bt[0, i // page], :, i % page] = bad
+        vc[bt[0, i // page], :, :, i % page] = bad
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    tiles = i32([[a, min(8, n - first - a)] for a in range(0, n - first, 8)])
+    outs = []
+    for most in (0, 1 << 30):
+        monkeypatch.setattr(K, "F32_ATTN_TILE_MIN", most)
+        outs.append(K.paged_attention(q.reshape(-1, nh * d).to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), i32([0] * (n - first)), i32(list(range(first, n))),
+                                      nh, nkv, d, 0.1, max_total_len=n, tiles=tiles).cpu())
+    assert torch.isfinite(outs[0][:125 - first]).all() and not torch.isfinite(outs[0][125 - first:, 5]).any()
+    assert torch.equal(torch.nan_to_num(outs[0], nan=7e30), torch.nan_to_num(outs[1], nan=7e30))
 
 
 def test_attention_float32_refuses_a_bound_below_a_position_loudly(K):
