@@ -10,38 +10,47 @@
 // runs beside the other's matrix work.  2,048 rows against the kernel on v_mfma_f32_16x16x4_f32 that this one replaced (tiles of
 // 128 x 128, 106 TFLOP/s at most): 32768 x 4096 2.86 ms against 5.20 (192 TFLOP/s, of which the matrix cores are busy half
 // the time), 4096 x 16384 1.42 against 2.67, 1024 x 1024 44 us against 106; 300 x 4608 x 4096 142 us against 416.
+// Tiles beyond whole rounds over the chip left most of it idle (288 tiles of 2048 x 4608 on 256 units: two rounds, the second an eighth full;
+// 300 x 4608 54 tiles): their eight slices of K go to as many workgroups, and a second kernel adds the slices' sums, 128 KB each, in their
+// order.  us, the best whole form before: 2048 x 4608 x 4096 578 -> 405, 300 x 4608 x 4096 144 -> 102, 100 x 4096 x 16384 391 -> 166, 2048 x 1024
+// x 4096 162 -> 106, 1024 x 2304 x 5760 262 -> 192.
 // K must be a multiple of 4 and rows 16-byte aligned.
 #include "f32_split.h"
 
-// BM x BN outputs a workgroup (rows of X, rows of W), WM x WN a wave
-template <int BM, int BN, int WM, int WN>
+
+// Tiles whose K is cut: those from number `first` on, `slices` slices of K each, which `parts` workgroups a tile share.  Every slice's
+// sum leaves for a workspace and gemm_f32_sum_kernel adds them in their order, so the bits are those of a whole tile.
+struct FtCut {
+    int first, slices, parts;
+};
+
+// Workgroups go to the 8 XCDs round-robin: those of one XCD take the m tiles of one n tile one after the
+// other, so a tile of W is fetched into one L2 only.
+__device__ __forceinline__ void ft_place(int id, int m_tiles, int n_tiles, int& mt, int& nt) {
+    const int full = (n_tiles / 8) * 8 * m_tiles;   // n tiles in whole rounds of 8
+    if (id < full) {
+        const int xcd = id & 7, local = id >> 3;
+        mt = local % m_tiles;
+        nt = (local / m_tiles) * 8 + xcd;
+    } else {
+        const int rest = id - full;
+        mt = rest % m_tiles;
+        nt = (n_tiles / 8) * 8 + rest / m_tiles;
+    }
+}
+
+// BM x BN outputs a workgroup (rows of X, rows of W), WM x WN a wave.  CUT: some slices, whose sums leave one by one
+template <int BM, int BN, int WM, int WN, bool CUT>
 __global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64)
 gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const float* __restrict__ W,
                      const float* __restrict__ bias, int M, int N, int K, int lda, int ldw, int ldc, float alpha,
-                     int m_tiles, int n_tiles, int vec_store) {
+                     int m_tiles, int n_tiles, int vec_store, float* __restrict__ ws, const FtCut cut) {
     constexpr int NW = (BM / WM) * (BN / WN), NT = NW * 64, ROWS = BM + BN;
     constexpr int LOADS = ROWS * 8 / NT, W_LOADS = BN * 8 / NT, TM = WM / 16, TN = WN / 16;
     static_assert(ROWS * 8 % NT == 0 && BN * 8 % NT == 0, "whole loads");
     // [stage][group of 16 rows (of W, then of X)][piece][slot]
     __shared__ __align__(16) uint4 lds[2][ROWS / 16][3][64];
-    // Workgroups go to the 8 XCDs round-robin: those of one XCD take the m tiles of one n tile one after the
-    // other, so a tile of W is fetched into one L2 only.
-    int mt, nt;
-    {
-        const int id = blockIdx.x;
-        const int full = (n_tiles / 8) * 8 * m_tiles;   // n tiles in whole rounds of 8
-        if (id < full) {
-            const int xcd = id & 7, local = id >> 3;
-            mt = local % m_tiles;
-            nt = (local / m_tiles) * 8 + xcd;
-        } else {
-            const int rest = id - full;
-            mt = rest % m_tiles;
-            nt = (n_tiles / 8) * 8 + rest / m_tiles;
-        }
-    }
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, q = lane >> 4;
-    const int n0 = nt * BN, m0 = mt * BM;
     const int wn = (wave % (BN / WN)) * TN, wm = BN / 16 + (wave / (BN / WN)) * TM;   // the wave's first row groups
     const bool early = wave < NW / 2;
 
@@ -51,16 +60,23 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
 
     // a thread stages 16 bytes (piece tid % 8 of a row's 128) of LOADS rows: tid / 8 + i * NT / 8
     const int lrow = tid >> 3, lk4 = tid & 7;
-    const float4* wsrc = reinterpret_cast<const float4*>(W + (size_t)n0 * ldw);
-    const float4* xsrc = reinterpret_cast<const float4*>(X + (size_t)m0 * lda);
     // (in 16 bytes: a row of the tile, the tile's last row inside the matrix; rows beyond are that one again)
     const uint32_t w4 = ldw >> 2, x4 = lda >> 2;
     uint32_t wfrom = lrow * w4, xfrom = lrow * x4;
-    const uint32_t wlast = (uint32_t)min(N - 1 - n0, BN - 1) * w4, xlast = (uint32_t)min(M - 1 - m0, BM - 1) * x4;
     const int put = (lrow >> 4) * 384 + f3_slot(lrow & 15, lk4 & 3) * 2 + (lk4 >> 2);   // in 8 bytes
     const int get = f3_slot(r, q);
     float4 reg[LOADS];
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    f32x4 acc[TN][TM], total[CUT ? 1 : TN][CUT ? 1 : TM];
+    const int tile = CUT ? cut.first + (int)blockIdx.x / cut.parts : blockIdx.x, part = CUT ? blockIdx.x % cut.parts : 0;
+    const int slice0 = CUT ? part * cut.slices / cut.parts : 0;
+    const int st0 = slice0 * per, st1 = CUT ? min((part + 1) * cut.slices / cut.parts * per, stages) : stages;
+    int mt, nt;
+    ft_place(tile, m_tiles, n_tiles, mt, nt);
+    const int n0 = nt * BN, m0 = mt * BM;
+    const float4* wsrc = reinterpret_cast<const float4*>(W + (size_t)n0 * ldw);
+    const float4* xsrc = reinterpret_cast<const float4*>(X + (size_t)m0 * lda);
+    const uint32_t wlast = (uint32_t)min(N - 1 - n0, BN - 1) * w4, xlast = (uint32_t)min(M - 1 - m0, BM - 1) * x4;
     auto fetch = [&](int st) {
         const int k4 = st * 8 + lk4, k4c = k4 < k4_last ? k4 : k4_last;
         asm volatile("" : "+v"(wfrom), "+v"(xfrom));   // the rows' offsets are made here each time: outside the loop they would take LOADS registers
@@ -82,32 +98,40 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
         }
     };
 
-    f32x4 acc[TN][TM], total[TN][TM];
+    // a slice's sums, as the waves hold them: [cut tile][slice][wave][t][g][lane]
+    auto leave = [&](int slice) {
+        f32x4* to = reinterpret_cast<f32x4*>(ws) + (((size_t)(tile - cut.first) * cut.slices + slice) * NW + wave) * (TN * TM * 64) + lane;
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+            for (int g = 0; g < TM; ++g) to[(t * TM + g) * 64] = acc[t][g];
+    };
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
         for (int g = 0; g < TM; ++g) {
             acc[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
-            total[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (!CUT) total[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
 
-    fetch(0);
-    store(0);
-    fetch(1);
+    fetch(st0);
+    store(st0);
+    fetch(st0 + 1);
     __syncthreads();
-    int in_slice = 0;
-    for (int st = 0; st < stages; ++st) {
-        if (early && st + 1 < stages) {
+    int in_slice = 0, slice = slice0;
+    for (int st = st0; st < st1; ++st) {
+        if (early && st + 1 < st1) {
             store(st + 1);
             fetch(st + 2);
         }
         if (in_slice == per) {   // a slice ends: its sum joins the total, the next starts from zero
             in_slice = 0;
+            if (CUT) leave(slice++);
 #pragma unroll
             for (int t = 0; t < TN; ++t)
 #pragma unroll
                 for (int g = 0; g < TM; ++g) {
-                    total[t][g] += acc[t][g];
+                    if (!CUT) total[t][g] += acc[t][g];
                     acc[t][g] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
         }
@@ -130,11 +154,15 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
                 f3_step(a, b, acc, t0, g);
             }
         }
-        if (!early && st + 1 < stages) {
+        if (!early && st + 1 < st1) {
             store(st + 1);
             fetch(st + 2);
         }
         __syncthreads();
+    }
+    if (CUT) {
+        leave(slice);
+        return;
     }
     unsigned long long open = 0;   // outputs to be computed again: bit (g * TN + t) * 4 + e
     static_assert(TM * TN * 4 <= 64, "a bit an output");
@@ -147,7 +175,7 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
         for (int t = 0; t < TN; ++t) {
             const int n = n0 + (wn + t) * 16 + 4 * q;
             if (n >= N) continue;
-            f32x4 v = total[t][g] + acc[t][g];
+            f32x4 v = total[CUT ? 0 : t][CUT ? 0 : g] + acc[t][g];
             float o[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -187,38 +215,139 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
     }
 }
 
-// `tile`: 0 the rule below, 1 .. 3 one of the three shapes (for measurements and tests)
-extern "C" int ilm_gemm_f32_tile(void* C, const void* X, const void* W, const void* bias, int M, int N, int K,
-                                 int lda, int ldw, int ldc, float alpha, int tile, hipStream_t stream) {
-    ILM_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32_tile: bad sizes M=%d N=%d K=%d", M, N, K);
+// Cut tiles: the slices' sums in ascending order.  A thread takes the four outputs that a lane of the tile's workgroup held together.
+template <int BM, int BN, int WM, int WN>
+__global__ void __launch_bounds__(256)
+gemm_f32_sum_kernel(float* __restrict__ C, const float* __restrict__ ws, const float* __restrict__ X, const float* __restrict__ W,
+                    const float* __restrict__ bias, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int m_tiles, int n_tiles,
+                    int vec_store, const FtCut cut) {
+    constexpr int TM = WM / 16, TN = WN / 16, EACH = BM * BN / 4;   // threads a tile
+    const int tile = cut.first + blockIdx.x / (EACH / 256);
+    const int i = blockIdx.x % (EACH / 256) * 256 + threadIdx.x, lane = i & 63, r = lane & 15, q = lane >> 4;
+    const int g = i / 64 % TM, t = i / (64 * TM) % TN, wave = i / (64 * TM * TN);
+    const f32x4* from = reinterpret_cast<const f32x4*>(ws) + (size_t)(tile - cut.first) * cut.slices * EACH + i;
+    f32x4 s[F3_SLICES];
+#pragma unroll
+    for (int k = 0; k < F3_SLICES; ++k) s[k] = from[(size_t)(k < cut.slices ? k : 0) * EACH];
+    f32x4 v = s[0];
+#pragma unroll
+    for (int k = 1; k < F3_SLICES; ++k)
+        if (k < cut.slices) v += s[k];
+    int mt, nt;
+    ft_place(tile, m_tiles, n_tiles, mt, nt);
+    const int m = mt * BM + (wave / (BN / WN) * TM + g) * 16 + r, n = nt * BN + (wave % (BN / WN) * TN + t) * 16 + 4 * q;
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const bool live = m < M && n + e < N;
+        float x = f3_settle(v[e], live, X, W, m, n + e, K, lda, ldw);
+        if (bias != nullptr && live) x += bias[n + e];
+        o[e] = alpha * x;
+    }
+    if (m >= M || n >= N) return;
+    float* dst = C + (size_t)m * ldc + n;
+    if (vec_store && n + 3 < N) {
+        *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[e] = o[e];
+    }
+}
+
+// Which of the three tiles, or 4: the first, with the tiles beyond whole rounds cut (`parts` workgroups a tile)
+static int ft_form(int M, int N, int K, int slices, int* parts) {
+    // What ends soonest, by what a round of each takes (us at K 4096, measured on 256 units: the ratios count).  128 x
+    // 256 and 128 x 128 run one a unit, 325 and 197 a round; of 64 x 64 three share a unit: 95 alone, 142 two of them,
+    // 66 each when many follow one another.  2048 x 4096 outputs: 368, 405 and 529 us; 300 x 4608: 324, 197 and 142.
+    const long long cus = ilm_num_cus();
+    auto count = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const long long n1 = count(128, 256), t1 = 325 * ((n1 + cus - 1) / cus), t2 = 197 * ((count(128, 128) + cus - 1) / cus);
+    const long long n3 = count(64, 64), t3 = n3 <= cus ? 95 : n3 <= 2 * cus ? 142 : 66 * n3 / cus + 10;
+    const int form = t1 <= t2 && t1 <= t3 ? 1 : t2 <= t3 ? 2 : 3;
+    const long long rest = n1 % cus;
+    if (rest == 0 || slices < 2) return form;
+    // Cut: rounds of workgroups of some slices each and 3 us for the start of a round, then the sum, 4 us and 0.03 a slice of a tile (128 KB, written and
+    // read).  By this rule / measured, and the best whole form: 2048 x 4608 x 4096 380 / 405 (578), 1024 x 4608 x 4096 257 / 248 (325), 300 x 4608
+    // x 4096 104 / 102 (144), 100 x 4608 x 4096 52 / 53 (102), 1024 x 4096 x 4096 209 / 210 (202), 2048 x 2304 x 2304 168 / 164 (182),
+    // 1024 x 2304 x 2304 99 / 96 (109), 2048 x 1024 x 1024 46 / 47 (42), 1024 x 6912 x 2304 237 / 245 (193), 1300 x 2048 x 12288 400 / 396 (568).
+    const double unit = 325. / 4096 * K / slices;
+    double best = 0.;
+    for (int p = 2; p <= slices; ++p) {
+        const double t = (double)((rest * p + cus - 1) / cus) * (unit * ((slices + p - 1) / p) + 3.);
+        if (p == 2 || t < best) best = t, *parts = p;
+    }
+    best += n1 / cus * 325. / 4096 * K + 4. + 0.03 * (double)(rest * slices);
+    return best < (form == 1 ? t1 : form == 2 ? t2 : t3) / 4096. * K ? 4 : form;
+}
+static int ft_slices(int K) {
+    const int steps = (K + F3_STEP - 1) / F3_STEP, per = (steps + F3_SLICES - 1) / F3_SLICES;
+    return (steps + per - 1) / per;
+}
+static int ft_rest(int M, int N) { return (int)((long long)((M + 127) / 128) * ((N + 255) / 256) % ilm_num_cus()); }
+
+static int ft_check(const char* name, const void* X, const void* W, int M, int N, int K, int lda, int ldw, int ldc) {
+    ILM_REQUIRE(M > 0 && N > 0 && K > 0, "%s: bad sizes M=%d N=%d K=%d", name, M, N, K);
     ILM_REQUIRE(K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && lda >= K && ldw >= K && ldc >= N,
-                "gemm_f32_tile: K=%d lda=%d ldw=%d ldc=%d", K, lda, ldw, ldc);
-    ILM_REQUIRE(((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0, "gemm_f32_tile: operands must be 16-byte aligned");
-    ILM_REQUIRE(lda < (1 << 24) && ldw < (1 << 24), "gemm_f32_tile: rows of %d and %d floats", lda, ldw);   // (offsets inside a tile take 32 bits)
-    ILM_REQUIRE(tile >= 0 && tile <= 3, "gemm_f32_tile: there is no tile %d", tile);
-    const int vec_store = (ldc % 4 == 0 && ((uintptr_t)C & 15) == 0) ? 1 : 0;
-#define FT_RUN(BM_, BN_, WM_, WN_)                                                                                          \
-    {                                                                                                                       \
-        const int m_tiles = (M + BM_ - 1) / BM_, n_tiles = (N + BN_ - 1) / BN_;                                             \
-        ILM_REQUIRE((long long)m_tiles * n_tiles < (1ll << 31), "gemm_f32_tile: too many tiles");                           \
-        gemm_f32_tile_kernel<BM_, BN_, WM_, WN_><<<m_tiles * n_tiles, (BM_ / WM_) * (BN_ / WN_) * 64, 0, stream>>>(         \
-            (float*)C, (const float*)X, (const float*)W, (const float*)bias, M, N, K, lda, ldw, ldc, alpha, m_tiles,        \
-            n_tiles, vec_store);                                                                                            \
-    }
-    if (tile == 0) {
-        // The tile that ends soonest, by what a round of each takes (us at K 4096, measured on 256 units: the ratios count).  128 x
-        // 256 and 128 x 128 run one a unit, 325 and 197 a round; of 64 x 64 three share a unit: 95 alone, 142 two of them,
-        // 66 each when many follow one another.  2048 x 4096 outputs: 368, 405 and 529 us; 300 x 4608: 324, 197 and 142.
-        const long long cus = ilm_num_cus();
-        auto count = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-        const long long t1 = 325 * ((count(128, 256) + cus - 1) / cus), t2 = 197 * ((count(128, 128) + cus - 1) / cus);
-        const long long n3 = count(64, 64), t3 = n3 <= cus ? 95 : n3 <= 2 * cus ? 142 : 66 * n3 / cus + 10;
-        tile = t1 <= t2 && t1 <= t3 ? 1 : t2 <= t3 ? 2 : 3;
-    }
-    if (tile == 1) FT_RUN(128, 256, 64, 64)
-    else if (tile == 2) FT_RUN(128, 128, 64, 32)
-    else FT_RUN(64, 64, 32, 32)
-#undef FT_RUN
-    ILM_LAUNCH_CHECK("gemm_f32_tile");
+                "%s: K=%d lda=%d ldw=%d ldc=%d", name, K, lda, ldw, ldc);
+    ILM_REQUIRE(((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0, "%s: operands must be 16-byte aligned", name);
+    ILM_REQUIRE(lda < (1 << 24) && ldw < (1 << 24), "%s: rows of %d and %d floats", name, lda, ldw);   // (offsets inside a tile take 32 bits)
+    ILM_REQUIRE((long long)((M + 63) / 64) * ((N + 63) / 64) < (1ll << 31), "%s: too many tiles", name);
     return 0;
 }
+#define FT_ARGS (float*)C, (const float*)X, (const float*)W, (const float*)bias, M, N, K, lda, ldw, ldc, alpha
+#define FT_RUN(BM_, BN_, WM_, WN_, CUT_, BLOCKS_)                                                                       \
+    {                                                                                                                   \
+        const int m_tiles = (M + BM_ - 1) / BM_, n_tiles = (N + BN_ - 1) / BN_;                                         \
+        gemm_f32_tile_kernel<BM_, BN_, WM_, WN_, CUT_><<<BLOCKS_, (BM_ / WM_) * (BN_ / WN_) * 64, 0, stream>>>(         \
+            FT_ARGS, m_tiles, n_tiles, vec_store, (float*)ws, cut);                                                     \
+        ILM_LAUNCH_CHECK("gemm_f32_tile");                                                                              \
+    }
+
+// `tile`: 0 the rule above, 1 .. 3 one of the three shapes (for measurements and tests)
+extern "C" int ilm_gemm_f32_tile(void* C, const void* X, const void* W, const void* bias, int M, int N, int K,
+                                 int lda, int ldw, int ldc, float alpha, int tile, hipStream_t stream) {
+    if (ft_check("gemm_f32_tile", X, W, M, N, K, lda, ldw, ldc) != 0) return -1;
+    ILM_REQUIRE(tile >= 0 && tile <= 3, "gemm_f32_tile: there is no tile %d", tile);
+    const int vec_store = (ldc % 4 == 0 && ((uintptr_t)C & 15) == 0) ? 1 : 0;
+    int parts;
+    void* ws = nullptr;
+    const FtCut cut = {};
+    if (tile == 0) tile = ft_form(M, N, K, 1, &parts);   // (of the whole forms)
+    if (tile == 1) FT_RUN(128, 256, 64, 64, false, m_tiles * n_tiles)
+    else if (tile == 2) FT_RUN(128, 128, 64, 32, false, m_tiles * n_tiles)
+    else FT_RUN(64, 64, 32, 32, false, m_tiles * n_tiles)
+    return 0;
+}
+
+// Floats of the workspace that the form with cut tiles takes, or 0 where one of the others ends sooner
+extern "C" long ilm_gemm_f32_cut_ws(int M, int N, int K) {
+    int parts;
+    if (M <= 0 || N <= 0 || K <= 0 || ft_form(M, N, K, ft_slices(K), &parts) != 4) return 0;
+    return (long)ft_rest(M, N) * ft_slices(K) * 128 * 256;
+}
+
+// The same product with the tiles beyond whole rounds cut into their slices of K.  ws: ws_floats floats, at least as many as slices of such tiles hold.
+// `parts`: workgroups a tile, 0 the rule's.
+extern "C" int ilm_gemm_f32_cut(void* C, const void* X, const void* W, const void* bias, int M, int N, int K, int lda, int ldw, int ldc,
+                                float alpha, int parts, void* ws, long ws_floats, hipStream_t stream) {
+    if (ft_check("gemm_f32_cut", X, W, M, N, K, lda, ldw, ldc) != 0) return -1;
+    const int slices = ft_slices(K), rest = ft_rest(M, N), m_tiles = (M + 127) / 128, n_tiles = (N + 255) / 256;
+    int rule = slices;
+    ft_form(M, N, K, slices, &rule);
+    if (parts == 0) parts = rule;
+    ILM_REQUIRE(parts >= 1 && parts <= slices, "gemm_f32_cut: %d workgroups for %d slices", parts, slices);
+    ILM_REQUIRE(rest > 0 && ws != nullptr && ((uintptr_t)ws & 15) == 0 && ws_floats >= (long)rest * slices * 128 * 256,
+                "gemm_f32_cut: %d tiles of %d slices, a workspace of %ld floats", rest, slices, ws_floats);
+    const int vec_store = (ldc % 4 == 0 && ((uintptr_t)C & 15) == 0) ? 1 : 0;
+    const FtCut cut = {m_tiles * n_tiles - rest, slices, parts};
+    if (cut.first > 0) FT_RUN(128, 256, 64, 64, false, cut.first)
+    FT_RUN(128, 256, 64, 64, true, rest * parts)
+    gemm_f32_sum_kernel<128, 256, 64, 64><<<rest * (128 * 256 / 1024), 256, 0, stream>>>(
+        (float*)C, (const float*)ws, (const float*)X, (const float*)W, (const float*)bias, M, N, K, lda, ldw, ldc, alpha, m_tiles, n_tiles, vec_store,
+        cut);
+    ILM_LAUNCH_CHECK("gemm_f32_sum");
+    return 0;
+}
+#undef FT_RUN
+#undef FT_ARGS

@@ -605,6 +605,12 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, 
     if pieces and F32_FEW_ROWS > 0:
         # the 32-bit path's many rows (portions of prompts): tiles on the same products, every
         # output summed in the few-rows kernel's order, so a row's bits do not depend on the rows around it
+        need = _lib().ilm_gemm_f32_cut_ws(M, N, K)
+        if need:   # tiles that would fill a part of a round over the chip: their K over several workgroups, summed in the same order
+            ws = torch.empty((need,), dtype=F32, device=a.device)
+            _run("ilm_gemm_f32_cut", out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K, a.stride(0), w.stride(0), out.stride(0),
+                 float(alpha), 0, ws.data_ptr(), need, _stream())
+            return out
         _run("ilm_gemm_f32_tile", out.data_ptr(), a.data_ptr(), w.data_ptr(), _ptr(bias), M, N, K, a.stride(0),
              w.stride(0), out.stride(0), float(alpha), 0, _stream())
         return out

@@ -330,6 +330,36 @@ def test_gemm_float32_in_pieces(K, M, N, K_):
         assert torch.equal(c, out), f"tile {tile}"
 
 
+@pytest.mark.parametrize("M,N,K_", [(65, 63, 36), (127, 257, 68), (129, 1030, 260), (300, 513, 1028), (130, 255, 2052), (200, 301, 8192), (1100, 8200, 132)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_gemm_float32_cut_tiles_give_the_same_bits(K, M, N, K_, odd):
+    """Tiles whose slices of K go to several workgroups, as many as there are slices and fewer, few slices and eight, alone and after a round of whole
+    tiles, with a bias, a factor and rows that cannot be stored four at a time; infinities, NaNs and sums that the pieces cannot give among them."""
+    from infinilm_amd.csrc import lib
+    L = lib.load()
+    g = torch.Generator().manual_seed(M + N + odd)
+    a, w, bias = torch.randn((M, K_), generator=g), torch.randn((N, K_), generator=g), torch.randn((N,), generator=g)
+    if odd:
+        a[M // 3, 3], a[M // 2, K_ - 1], a[M - 1] = math.inf, math.nan, a[M - 1] * 2.0 ** -80
+        w[N // 2, 5], w[N - 1, :2], a[0, :2] = -math.inf, torch.tensor([3e38, -3e38]), torch.tensor([3.0, 3.0])
+    a, w, bias = a.to(DEV), w.to(DEV), bias.to(DEV)
+    steps = -(-K_ // 32)
+    slices = -(-steps // (-(-steps // 8)))
+    ld = N + (3 if odd else 0)
+    args = (a.data_ptr(), w.data_ptr(), bias.data_ptr(), M, N, K_, K_, K_, ld, 0.5)
+    ws = torch.empty(((-(-M // 128)) * (-(-N // 256)) * slices * 128 * 256,), device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    want = torch.full((M, ld), 7.0, device=DEV)
+    assert L.ilm_gemm_f32_tile(want.data_ptr(), *args, 1, stream) == 0
+    assert not odd or not torch.isfinite(want).all()
+    for parts in sorted({0, 1, 2, min(3, slices), slices}):
+        c = torch.full((M, ld), 7.0, device=DEV)
+        assert L.ilm_gemm_f32_cut(c.data_ptr(), *args, parts, ws.data_ptr(), ws.numel(), stream) == 0
+        _same(c, want)
+    assert L.ilm_gemm_f32_cut(c.data_ptr(), *args, slices + 1, ws.data_ptr(), ws.numel(), stream) != 0
+    assert L.ilm_gemm_f32_cut(c.data_ptr(), *args, 0, ws.data_ptr(), 100, stream) != 0
+
+
 @pytest.mark.parametrize("M", [1, 40, 130])
 @pytest.mark.parametrize("K_", [4, 32, 1028, 4096])
 def test_gemm_float32_operands_of_one_mantissa(K, M, K_):
