@@ -32,6 +32,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 #define MOE_BGROUP 4 // row tiles of that kernel that walk the output slices together
 #define MOE_TN 64
 #define MOE_KS 64
+#define MOE_FEW_K 4096   // longest rows of the few-rows kernel: 16 k-steps of 32 for each of 8 waves
 #define MOE_LD (MOE_KS + 8)   // bf16 elements a row of a tile in LDS (144 bytes)
 
 __device__ __forceinline__ float moe_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
@@ -503,6 +504,126 @@ moe_gemm_mfma_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict_
 }
 
 
+// bfloat16 on the matrix cores, few rows an expert (decoded tokens): bound by reading the experts' matrices once.  Block: 8 waves that split K; a
+// workgroup keeps a tile's rows (16 MG at a time) of its wave's K in registers and walks tiles of 16 rows of W (GLU: of gate and up), the
+// next one's loads in flight while the waves' sums meet in LDS, in wave order.  No barrier between loads, where the kernel above has two
+// every 64 k.  
+// us, with the kernel above and now, 2 of 14 experts a token: gate/up 2048 x 2048 1 token 23.8 / 9.6, 4 33.1 / 27.2, 16 49.8 / 44.4 (4.5 TB/s), 32 56.9 /
+// 51.5; down 19.7 / 6.0, 24.5 / 13.9, 31.3 / 23.2, 32.5 / 26.9; 16 of 2 of 16 experts 4096 x 4096 207 / 186 and 112 / 96.  Not below K 1024 (512: 26.6 /
+// 33.4), where the waves' sums meet more often than they multiply.  One workgroup a unit where a wave's part of K takes more than 128 registers.
+template <bool GLU, int KSTEPS, int MG>
+__global__ void __launch_bounds__(512, KSTEPS * MG <= 4 ? 4 : 2)
+moe_gemm_few_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict__ X, int ldx, const int* __restrict__ perm, int top,
+                    const float* __restrict__ pair_w, const bf16* __restrict__ W, size_t w_expert, int ldw, const int* __restrict__ tiles,
+                    const int* __restrict__ n_tiles, int N, int K, float limit, float alpha, int act, int ks) {
+    // D pieces of W (16 rows' part of a wave) in flight beside the one that is multiplied: gate and up rows where registers allow and both are
+    // long (45.2 -> 44.4 us; plain tiles in twos 23.2 -> 23.6).  EACH: pieces an output tile
+    constexpr int D = GLU && KSTEPS == 8 ? 2 : 1, EACH = GLU ? 2 : 1;
+    __shared__ float part[2][MG][8][64][4];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const int nt_all = (N + 15) / 16, et_all = *n_tiles;
+    if (et_all <= 0) return;
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+    const int k8_last = (K >> 3) - 1;
+    int k8c[KSTEPS];
+    bool kok[KSTEPS];
+#pragma unroll
+    for (int u = 0; u < KSTEPS; ++u) {
+        const int k8 = (wave * ks + u) * 4 + q;
+        kok[u] = u < ks && k8 <= k8_last;
+        k8c[u] = kok[u] ? k8 : (u == 0 ? k8_last : k8c[0]);
+    }
+    const bool ragged = ks < KSTEPS || K != 256 * ks;   // (then some lanes hold a number twice: zeros for the matrix cores, as an infinity times zero is none)
+    // the workgroups of an expert tile share its tiles of W (more expert tiles than workgroups: each takes several)
+    const int sharers = (int)gridDim.x > et_all ? (int)gridDim.x / et_all : 1, share = blockIdx.x / et_all;
+    if (share >= sharers || share >= nt_all) return;
+    const int et = threadIdx.x < 256 * MG ? threadIdx.x : 0, eg = et >> 8, e = et & 3, l = (et & 255) >> 2;
+    const int m = eg * 16 + (l & 15);
+    int buf = 0;
+#pragma unroll 1
+    for (int tile = blockIdx.x % et_all; tile < et_all; tile += gridDim.x) {
+        const int place0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+        const bf16* We = W + (size_t)tiles[3 * tile] * w_expert;
+        auto w_row = [&](int t, int hf) -> const uint4* {
+            const int n = t * 16 + r < N ? t * 16 + r : N - 1;
+            return reinterpret_cast<const uint4*>(We + (size_t)(n + hf * N) * ldw);
+        };
+#pragma unroll 1
+        for (int row0 = 0; row0 < rows; row0 += 16 * MG) {   // (up to 16 MG tokens: once)
+            uint4 a[D][KSTEPS], xf[MG][KSTEPS];
+            auto load = [&](uint4 (&to)[KSTEPS], int t, int hf) {
+                const uint4* wp = w_row(t, hf);
+#pragma unroll
+                for (int u = 0; u < KSTEPS; ++u) to[u] = wp[k8c[u]];
+            };
+            load(a[0], share, 0);
+            if (D == 2) load(a[D - 1], share, 1);
+#pragma unroll
+            for (int g = 0; g < MG; ++g) {
+                const bool has = row0 + g * 16 + r < rows;
+                const int place = place0 + (has ? row0 + g * 16 + r : 0);
+                int row = place;
+                float w = 1.0f;
+                if (GLU || perm != nullptr) {
+                    const int pair = perm != nullptr ? perm[place] : place;
+                    row = pair / top;
+                    if (GLU && pair_w != nullptr) w = pair_w[pair];
+                }
+                const uint4* xp = reinterpret_cast<const uint4*>(X + (size_t)row * ldx);
+#pragma unroll
+                for (int u = 0; u < KSTEPS; ++u) {
+                    uint4 v = xp[k8c[u]];
+                    if (GLU && pair_w != nullptr) v = moe_scale8(v, w);
+                    xf[g][u] = kok[u] && has ? v : zero;
+                }
+            }
+#pragma unroll 1
+            for (int nt = share; nt < nt_all; nt += sharers) {
+                const int n = nt * 16 + (l >> 4) * 4 + e;
+                float gate = 0.f;
+#pragma unroll
+                for (int v = 0; v < EACH; ++v) {
+                    f32x4 acc[MG];
+#pragma unroll
+                    for (int g = 0; g < MG; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if (ragged) {
+#pragma unroll
+                        for (int u = 0; u < KSTEPS; ++u)
+                            if (!kok[u]) a[v % D][u] = zero;
+                    }
+#pragma unroll
+                    for (int u = 0; u < KSTEPS; ++u)
+#pragma unroll
+                        for (int g = 0; g < MG; ++g)
+                            acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[v % D][u]), __builtin_bit_cast(bf16x8, xf[g][u]),
+                                                                             acc[g], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    // the piece D further on
+                    const int next = v + D < EACH ? nt : nt + sharers;
+                    if (next < nt_all) load(a[v % D], next, (v + D) % EACH);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int g = 0; g < MG; ++g) *reinterpret_cast<f32x4*>(&part[buf][g][wave][lane][0]) = acc[g];
+                    __syncthreads();
+                    float s = 0.f;
+#pragma unroll
+                    for (int w = 0; w < 8; ++w) s += part[buf][eg][w][l][e];
+                    buf ^= 1;   // (the other buffer's readers passed this barrier)
+                    if (GLU && v == 0) {
+                        gate = s;
+                        continue;
+                    }
+                    if (threadIdx.x < 256 * MG && n < N && row0 + m < rows) {
+                        if (GLU) s = moe_glu(gate, s, limit, alpha, act);
+                        else if (act == MOE_ACT_RELU2) { s = fmaxf(s, 0.f); s *= s; }
+                        out[(size_t)(place0 + row0 + m) * ld_out + n] = from_f32<bf16>(s);
+                    }
+                }
+            }
+        }
+    }
+}
+
 // bfloat16 on the matrix cores, many rows an expert.  Block: 2 x WN waves; tile: up to 128 rows of one expert x 64 WN rows of W
 // (GLU: the gate rows and the up rows of 32 WN outputs; else 64 WN outputs); wave (wm, wn) owns 64 rows x 64 rows of W (GLU:
 // gate and up of 32 outputs, so the activation has both in one thread): 16 products for 8 fragment reads a k-step.  WN = 4
@@ -751,9 +872,10 @@ moe_gemm_plain_kernel(T* __restrict__ out, int ld_out, const T* __restrict__ X, 
     }
 }
 
+// few_rows: most rows an expert has (the step's tokens), where that is at most 32 and the caller knows it; else 0
 extern "C" int ilm_moe_gemm(void* out, int ld_out, const void* X, int ldx, const void* perm, int top, const void* pair_w, const void* W,
                             long w_expert, int ldw, const void* tiles, const void* n_tiles, int max_tiles, int N, int K, int glu,
-                            float limit, float alpha, int act, int dtype, int force_plain, int tile_rows, int wide_mode, hipStream_t stream) {
+                            float limit, float alpha, int act, int dtype, int force_plain, int tile_rows, int wide_mode, int few_rows, hipStream_t stream) {
     ILM_REQUIRE(act == MOE_ACT_NONE || act == (glu ? MOE_ACT_SILU : MOE_ACT_RELU2), "moe_gemm: activation %d (0: none, 1: the square of relu, in the plain form, "
                 "2: silu, in the GLU form)", act);
     ILM_REQUIRE(tile_rows == MOE_TM || tile_rows == MOE_BM, "moe_gemm: tiles of %d rows (%d or %d)", tile_rows, MOE_TM, MOE_BM);
@@ -775,6 +897,21 @@ extern "C" int ilm_moe_gemm(void* out, int ld_out, const void* X, int ldx, const
         else if (glu) moe_gemm_mfma128_kernel<true, 2><<<big, 256, 0, stream>>>(MOE_ARGS(bf16), n_slices);
         else if (wide) moe_gemm_mfma128_kernel<false, 4><<<big, 512, 0, stream>>>(MOE_ARGS(bf16), n_slices);
         else moe_gemm_mfma128_kernel<false, 2><<<big, 256, 0, stream>>>(MOE_ARGS(bf16), n_slices);
+    } else if (dtype == ILM_DTYPE_BF16 && aligned && !force_plain && few_rows > 0 && few_rows <= 32 && K >= 1024 && K <= MOE_FEW_K) {
+        const long items = (long)max_tiles * ((N + 15) / 16);
+        const int ks = ((K + 31) / 32 + 7) / 8, most = (ks <= 4 ? 2 : 1) * ilm_num_cus();
+        const dim3 few((int)(items < most ? items : most));
+#define MOE_FEW(KS_, MG_)                                                                                    \
+    {                                                                                                        \
+        if (glu) moe_gemm_few_kernel<true, KS_, MG_><<<few, 512, 0, stream>>>(MOE_ARGS(bf16), ks);           \
+        else moe_gemm_few_kernel<false, KS_, MG_><<<few, 512, 0, stream>>>(MOE_ARGS(bf16), ks);              \
+    }
+        if (few_rows <= 16) {
+            if (ks <= 4) MOE_FEW(4, 1) else if (ks <= 8) MOE_FEW(8, 1) else MOE_FEW(16, 1)
+        } else {
+            if (ks <= 4) MOE_FEW(4, 2) else if (ks <= 8) MOE_FEW(8, 2) else MOE_FEW(16, 2)
+        }
+#undef MOE_FEW
     } else if (tile_rows != MOE_TM) {
         ILM_REQUIRE(false, "moe_gemm: tiles of %d rows are the bfloat16 matrix-core kernel's alone", tile_rows);
     } else if (dtype == ILM_DTYPE_BF16 && aligned && !force_plain) {

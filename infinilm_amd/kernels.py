@@ -2260,6 +2260,7 @@ MOE_FORCE_PLAIN = os.environ.get("INFINILM_AMD_MOE_PLAIN", "0") == "1"   # 1: th
 # 1: the plain form's few-rows kernel takes two blocks of 64 outputs a workgroup for large matrices (faster while a step's loads
 # were in flight over one step's products only, 175 -> 149 us; with two sets of load registers one block is: 132 against 135 us)
 MOE_PLAIN_PAIR = os.environ.get("INFINILM_AMD_MOE_PLAIN_PAIR", "0") == "1"
+MOE_FEW_TOKENS = int(os.environ.get("INFINILM_AMD_MOE_FEW_TOKENS", "32"))   # tokens up to which the kernel that keeps their rows in registers runs (at most 32)
 MOE_WIDE = int(os.environ.get("INFINILM_AMD_MOE_WIDE", "0"))   # 1: tiles of 256 rows of W in the many-rows kernel wherever the outputs fill one (measured slower at the shapes tried)
 
 
@@ -2346,10 +2347,12 @@ def moe_gemm(x: torch.Tensor, w: torch.Tensor, plan: ExpertPlan, glu: bool, limi
     if act not in (("none", "silu") if glu else ("none", "relu2")):
         raise KernelError(f"the experts' plain product takes no activation or relu2, the gated one none or silu, got {act!r}")
     out = torch.empty((plan.pairs, N), dtype=x.dtype, device=x.device)
+    tokens = plan.pairs // plan.top     # (and so the most rows of an expert)
     _run("ilm_moe_gemm", out.data_ptr(), N, x.data_ptr(), x.stride(0), plan.perm.data_ptr() if (glu or gather) else None, plan.top,
          plan.weights.data_ptr() if glu and weighted else None,
          w.data_ptr(), Nw * K, K, plan.tiles.data_ptr(), plan.n_tiles.data_ptr(), plan.max_tiles, N, K, int(bool(glu)), float(limit),
-         float(alpha), {"none": 0, "relu2": 1, "silu": 2}[act], _dt(x), int(MOE_FORCE_PLAIN), plan.tile_rows, int(MOE_WIDE) | (2 if MOE_PLAIN_PAIR else 0), _stream(), label="ilm_moe_gemm (gate/up)" if glu else ("ilm_moe_gemm (up)" if gather else "ilm_moe_gemm (down)"))
+         float(alpha), {"none": 0, "relu2": 1, "silu": 2}[act], _dt(x), int(MOE_FORCE_PLAIN), plan.tile_rows, int(MOE_WIDE) | (2 if MOE_PLAIN_PAIR else 0),
+         tokens if tokens <= MOE_FEW_TOKENS else 0, _stream(), label="ilm_moe_gemm (gate/up)" if glu else ("ilm_moe_gemm (up)" if gather else "ilm_moe_gemm (down)"))
     return out
 
 

@@ -1398,3 +1398,45 @@ def test_products_of_rows_that_share_memory(K, shared):
     q = K.qkv_rope_gemm(x, w, None, pos, cos, sin, None, None, None, 12, 2, 64, 64)
     if q is not None:
         assert float((q.float() - want[:, :768]).abs().max()) <= 2.0 ** -7 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("T,E,top,K_,N", [(1, 3, 1, 1024, 1), (1, 600, 2, 1032, 40), (5, 4, 3, 1536, 17), (16, 5, 2, 2048, 200), (16, 2, 2, 2056, 33), (17, 3, 2, 2048, 48),
+                                          (32, 2, 1, 1024, 31), (32, 40, 4, 4096, 16), (9, 2, 1, 4096, 100)])
+def test_experts_of_few_rows(K, T, E, top, K_, N):
+    """Experts whose rows stay in registers, in all forms of their products, against float64: more experts than workgroups of a share and than
+    workgroups, tiles of W that end inside one, K that leaves waves part of their steps.  The result is rounded to bfloat16 (2^-9 of it), the
+    float sums before that are good to 2^-24 sqrt(K) of a sum of magnitude one, and a gate's activation passes on at most 1.1 times that: 2^-8 covers both.
+    An infinite number in W reaches its own output alone."""
+    g = torch.Generator().manual_seed(T * 31 + K_ + N)
+    plan = K.moe_route(torch.randn((T, E), generator=g).to(DEV), E, top)
+    perm, ids = plan.perm.cpu().long(), plan.ids.cpu().long().flatten()
+    token, expert, weight = perm // top, ids[perm], plan.weights.cpu().flatten()[perm]
+    x = torch.randn((T, K_), generator=g).to(BF16)
+    w = (torch.randn((E, 2 * N, K_), generator=g) / math.sqrt(K_)).to(BF16)
+    w[expert[0], 0, K_ - 1] = math.inf
+    xd, wd = x.to(DEV), w.to(DEV)
+    wp = wd[:, :N].contiguous()
+    assert T <= K.MOE_FEW_TOKENS
+
+    def product(rows, form):
+        return torch.stack([w[e, :N if form == "plain" else 2 * N].to(F64) @ r for e, r in zip(expert.tolist(), rows.to(F64))])
+
+    def glu(rows, limit):
+        z = product(rows, "glu")
+        a, b = z[:, :N], z[:, N:]
+        if limit is None:
+            return a * torch.sigmoid(a) * b
+        a, b = a.clamp(max=limit), b.clamp(-limit, limit)
+        return a * torch.sigmoid(1.702 * a) * (b + 1)
+
+    rows = x[token]
+    scaled = (rows.float() * weight[:, None]).to(BF16)
+    order = rows.to(DEV)
+    for got, want in ((K.moe_gemm(xd, wd, plan, True, act="silu", weighted=False), glu(rows, None)), (K.moe_gemm(xd, wd, plan, True, 0.8), glu(scaled, 0.8)),
+                      (K.moe_gemm(order, wp, plan, False), product(rows, "plain")),
+                      (K.moe_gemm(xd, wp, plan, False, gather=True, act="relu2"), product(rows, "plain").clamp(min=0) ** 2)):
+        got = got.cpu()
+        whole = torch.isfinite(want)
+        assert whole.sum() >= want.numel() - 2 * T and torch.isfinite(got.float())[whole].all()
+        torch.testing.assert_close(got.to(F64)[~whole], want[~whole], equal_nan=True)
+        _close(torch.where(whole, got.to(F64), 0.0), torch.where(whole, want, 0.0), 2.0 ** -8)
