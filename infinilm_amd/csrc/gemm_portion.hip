@@ -10,7 +10,7 @@
 // Three forms: the product alone; act(gate) * up of a feed-forward's first product (the rows of W are taken so that a lane holds gate
 // and up of the same outputs); and the fused q | k | v projection with rotation and the write into the paged cache.  us, against the vendor
 // library's product (and the kernel after it):
-//   product   2048 x 1024 x 1024  9.1 / 10.7, x 4096 23.9 / 25.9; 1000 x 2048 x 2048 13.6 / 16.5; 300 x 1024 x 1024 5.6 / 7.1; 100 x 8192 x 1024 6.5 / 9.8
+//   product   2048 x 1024 x 1024  9.1 / 10.7, x 4096 22.3 / 25.9; 1000 x 2048 x 2048 13.6 / 16.5; 300 x 1024 x 1024 5.6 / 7.1; 100 x 8192 x 1024 6.5 / 9.8
 //   gate, up  2048 x 8192 x 1024 40.0 / 42.5; 1000 rows 23.6 / 27.7; 300 rows 12.6 / 17.4; 100 rows 9.2 / 12.4
 //   q, k, v   2048 x 1280 x 1024 18.7 / 20.1; 1000 rows 10.6 / 15.1; 300 rows 7.3 / 10.3; 300 x 4608 x 4096 23.8 / 27.7
 // An output's sum runs over K in steps of 32 from the first on, whatever the form and the tile.
@@ -31,7 +31,7 @@ struct GpArgs {
     bf16* C;
     int M, N, K;        // N: output columns a row of C (GLU: W has 2 N rows)
     int lda, ldw, ldc;
-    int m_tiles, n_tiles;
+    int m_tiles, n_tiles, group;   // group: m tiles that the n tiles are walked with
     int glu;
     // rope
     const int* pos;
@@ -73,8 +73,10 @@ gemm_portion_kernel(const GpArgs A) {
     {
         const int total = A.m_tiles * A.n_tiles, per = total >> 3, rem = total & 7, xcd = blockIdx.x & 7;
         const int id = xcd * per + (xcd < rem ? xcd : rem) + ((int)blockIdx.x >> 3);
-        mt = id % A.m_tiles;
-        nt = id / A.m_tiles;
+        const int band = id / (A.group * A.n_tiles), first = band * A.group, rows = A.m_tiles - first < A.group ? A.m_tiles - first : A.group;
+        const int at = id - first * A.n_tiles;
+        mt = first + at % rows;
+        nt = at / rows;
     }
     const int m0 = mt * BM;
     const int wn = wave % (BN / WN), wm = wave / (BN / WN);
@@ -289,12 +291,27 @@ gemm_portion_kernel(const GpArgs A) {
     }
 }
 
+// M tiles that are walked together before the next n tile.  An XCD takes an eighth of the tiles, consecutive ones, and fetches their rows of X and W into
+// its own L2: with all m tiles together all of X for each (2048 x 1024 x 4096 in tiles of 128 x 64: 134 MB in all, 67 MB where four m tiles are
+// walked with eight n tiles: 24.1 -> 22.4 us; 1000 x 1024 x 4096 15.2 -> 14.6).  But then a row of W is fetched by several: only where at most two
+// thirds of the rows are left (1000 x 2304 x 2304, four fifths, 18.0 -> 18.8), and not for q, k and v (2048 x 1280 x 1024, a round and a
+// quarter, in a model's step 16.1 -> 17.6).
+static int gp_group(int m_tiles, int n_tiles, int bm, int bn) {
+    const long long per = ((long long)m_tiles * n_tiles + 7) / 8;
+    auto rows = [&](int g) { return (long long)g * bm + (per + g - 1) / g * bn; };
+    int best = m_tiles;
+    for (int g = 1; g < m_tiles && (long long)(g - 1) * bm < rows(best); ++g)
+        if (rows(g) < rows(best)) best = g;
+    return 3 * rows(best) <= 2 * rows(m_tiles) ? best : m_tiles;
+}
+
 // tile: 1: 64 x 64 outputs (gate, up: 64 x 128 rows of W), 2: 128 x 64, 3: 128 x 128, 4: 256 x 128, 5: 256 x 256
 #define GP_RUN(BM_, BN_, WM_, WN_, NS_, EPI_, NCOLS_)                                                       \
     {                                                                                                       \
         a.m_tiles = (a.M + BM_ - 1) / BM_;                                                                  \
         a.n_tiles = ((NCOLS_) + BN_ - 1) / BN_;                                                             \
         ILM_REQUIRE((long long)a.m_tiles * a.n_tiles < (1ll << 31), "gemm_portion: too many tiles");        \
+        a.group = EPI_ == GP_PLAIN ? gp_group(a.m_tiles, a.n_tiles, BM_, BN_) : a.m_tiles;                  \
         gemm_portion_kernel<BM_, BN_, WM_, WN_, NS_, EPI_>                                                  \
             <<<a.m_tiles * a.n_tiles, (BM_ / WM_) * (BN_ / WN_) * 64, 0, stream>>>(a);                      \
     }
@@ -318,8 +335,9 @@ extern "C" int ilm_gemm_portion(void* C, int ldc, const void* X, int lda, const 
     a.M = M; a.N = N; a.K = K; a.lda = lda; a.ldw = ldw; a.ldc = ldc; a.glu = glu;
     if (glu < 0) {
         ILM_REQUIRE(tile >= 1 && tile <= 3, "gemm_portion: there is no tile %d", tile);
+        // (128 x 64: one workgroup a unit by the rule, so five stages; three, 2048 x 1024 x 4096 22.9 us, now 22.3; in a model's step 30 -> 27)
         if (tile == 1) GP_RUN(64, 64, 32, 32, 4, GP_PLAIN, N)
-        else if (tile == 2) GP_RUN(128, 64, 32, 32, 3, GP_PLAIN, N)
+        else if (tile == 2) GP_RUN(128, 64, 32, 32, 5, GP_PLAIN, N)
         else GP_RUN(128, 128, 64, 32, 4, GP_PLAIN, N)
     } else {
         ILM_REQUIRE(tile == 1 || tile == 4 || tile == 5, "gemm_portion: there is no tile %d", tile);

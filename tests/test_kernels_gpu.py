@@ -1440,3 +1440,15 @@ def test_experts_of_few_rows(K, T, E, top, K_, N):
         assert whole.sum() >= want.numel() - 2 * T and torch.isfinite(got.float())[whole].all()
         torch.testing.assert_close(got.to(F64)[~whole], want[~whole], equal_nan=True)
         _close(torch.where(whole, got.to(F64), 0.0), torch.where(whole, want, 0.0), 2.0 ** -8)
+
+
+@pytest.mark.parametrize("tile,M,N,K_", [(1, 1100, 1220, 64), (1, 1990, 700, 128), (2, 2041, 1000, 64), (2, 4000, 330, 192), (3, 4000, 1100, 64), (1, 130, 2000, 64)])
+def test_portion_product_walks_its_tiles_in_bands(K, tile, M, N, K_):
+    """Products whose tiles are walked in bands of several rows of tiles, the last band lower than the others: every output once.  float sums of products of
+    bfloat16 (2^-24 sqrt(K) of the norm of the addends) and one rounding to bfloat16, 2^-9: 2^-8 of the largest."""
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn((M, K_), generator=g).to(BF16).to(DEV), torch.randn((N, K_), generator=g).to(BF16).to(DEV)
+    out = torch.full((M, N), math.nan, dtype=BF16, device=DEV)
+    K.portion_gemm(x, w, None, out, tile)
+    want = x.to(F64) @ w.to(F64).T
+    assert float((out.to(F64) - want).abs().max()) < 2.0 ** -8 * float(want.abs().max())
