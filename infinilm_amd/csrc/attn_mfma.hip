@@ -467,26 +467,33 @@ attn_merge_kernel(bf16* __restrict__ out, const float* __restrict__ ws_acc, cons
 
 // ------------------------------------------------------------------------------------------------
 // Tiles of up to ATT_TT consecutive tokens of one request (portions of prompts): the 4 waves of a
-// workgroup take 2 tokens each and share every 64-key tile of K and V through LDS (the next tile is
+// workgroup take 2 tokens (or groups of tokens) each and share every 64-key tile of K and V through LDS (the next tile is
 // already on its way: into registers, or, for heads of 128 and pages that hold whole tiles, straight
 // into a second pair of LDS buffers), so a tile is read from the cache once per 8 tokens x 16 heads.  No key chunks and no
 // workspace: one workgroup walks all keys its tokens see, in ascending order of absolute key
 // index, 32 at a time.
 // ------------------------------------------------------------------------------------------------
 #define ATT_TT 8
-#define ATT_NT 2
 #define ATT_TK 64        // keys per tile
 #define ATT_BT_LDS 2048  // block-table entries kept in LDS
 #define ATT_LAZY 8.0f    // the exponent's reference point follows the maximum in steps of at least this
 
 __device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
-template <int D16, bool PAGE64, bool WF>   // WF: see attn_mfma_kernel
+// WF: see attn_mfma_kernel.  The 16 columns of the matrix instruction are CT tokens x 16 / CT heads, and a wave takes NT such groups.  9 to 16 heads: a token a
+// group, two groups a wave.  5 to 8: two tokens a group, one group a wave, so a tile of 8 tokens costs half the instructions that it costs with half of
+// the columns empty (2,048 tokens of 16 heads of 64 over 2 42.5 -> 33.1 us, of 128 55.6 -> 42.8, 37 tokens 7.2 -> 5.9; two groups a wave and 16 tokens a
+// workgroup 40.6, 52.3 and 7.8, better only for thousands of tokens over long contexts: 3,000 over 6,000 keys 144 against 175, 247 before).  Up to four:
+// four tokens a group, and a workgroup takes two neighbouring tiles, 16 tokens, where they are a run of a request (36 heads of 64, 2,048 tokens
+// 366 -> 121 us; 32 of 128 over 8 152 -> 59; 300 tokens 18.9 -> 9.2 and 13.9 -> 10.6).
+template <int D16, bool PAGE64, bool WF, int CT>
 __global__ void __launch_bounds__(256, 2)
 attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16* __restrict__ kc,
                  const bf16* __restrict__ vc, const int* __restrict__ block_tables, const int* __restrict__ seg,
                  const int* __restrict__ pos, const int* __restrict__ tiles, int nh, int nkv, int page,
-                 int max_blocks, int q_stride, int out_stride, float scale_log2e, float capq, int reach, int pair_base) {
+                 int max_blocks, int q_stride, int out_stride, float scale_log2e, float capq, int reach, int pair_base, int n_tiles) {
+    constexpr int NT = CT == 1 ? 2 : 1, HW = 16 / CT;   // HW: heads a group
+    constexpr bool PAIR = 4 * NT * CT > ATT_TT;
     constexpr int D = D16 * 16;
     constexpr int KS = (D + 31) / 32;
     // K rows [key][d] and V rows [d][key] in LDS, read in 16-byte pieces by 16 rows x 4 lane groups.
@@ -517,19 +524,34 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
     // compute unit), workgroups w and w + pair_base land on the same unit (workgroups go to the
     // eight dies in turn and to a die's units in turn): the second of them then takes the items
     // from the short end, so that every unit holds a long and a short one.
-    const int n_items = gridDim.x * gridDim.y;
-    const int w = blockIdx.y * gridDim.x + blockIdx.x;
-    const int item = (pair_base > 0 && w >= pair_base) ? n_items - 1 - (w - pair_base) : w;
-    const int tile_id = gridDim.x - 1 - item / gridDim.y;
+    // (PAIR: the items are pairs of tiles, the work of the pairs' first tiles; behind them come the second tiles, which have something to do only where the
+    // two are no run)
+    const int n_lead = PAIR ? (n_tiles + 1) / 2 : n_tiles;
+    const int n_items = n_lead * gridDim.y;
+    int w = blockIdx.y * gridDim.x + blockIdx.x;
+    const bool second = PAIR && w >= n_items;
+    if (second) w -= n_items;
+    const int item = (!second && pair_base > 0 && w >= pair_base) ? n_items - 1 - (w - pair_base) : w;
+    const int lead = n_lead - 1 - item / gridDim.y;
     const int by = item % gridDim.y;
-    const int t0 = tiles[2 * tile_id], ntok = tiles[2 * tile_id + 1];
+    int t0, ntok;
+    if (!PAIR) {
+        t0 = tiles[2 * lead];
+        ntok = tiles[2 * lead + 1];
+    } else {
+        const int other = 2 * lead + 1 < n_tiles ? 2 * lead + 1 : 2 * lead;
+        const int ta = tiles[4 * lead], na = tiles[4 * lead + 1], tb = tiles[2 * other], nb = other > 2 * lead ? tiles[2 * other + 1] : 0;
+        const bool run = na == ATT_TT && nb > 0 && tb == ta + ATT_TT && seg[tb] == seg[ta];
+        t0 = second ? tb : ta;
+        ntok = second ? (run ? 0 : nb) : (run ? na + nb : na);
+    }
     if (ntok <= 0) return;   // a tile of no tokens: what fills up the list of a recorded step (the whole workgroup leaves)
     const int G = nh / nkv;
     const int HG = (G + 15) / 16;
     const int kvh = by / HG, hg = by % HG;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, qg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: what depends on it stays in SGPRs
-    const int hcol = hg * 16 + r;
+    const int hcol = hg * 16 + r % HW;
     const bool head_ok = hcol < G;
     const int head = kvh * G + (head_ok ? hcol : G - 1);
     const int p_first = pos[t0], p_last = p_first + ntok - 1;
@@ -545,15 +567,19 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
     auto page_of = [&](int key) -> int { return bt_in_lds ? bt_s[key / page - blk_first] : bt[key / page]; };
 
     // this wave's tokens
-    int tok[ATT_NT], pj[ATT_NT], loj[ATT_NT];
-    bool tok_ok[ATT_NT];
-    uint4 qf[ATT_NT][KS];
+    int tok[NT], pj[NT], loj[NT];
+    bool tok_ok[NT];
+    uint4 qf[NT][KS];
+    // the first and last position of the wave's tokens, and the first keys they see
+    auto pos_of = [&](int i) { return p_first + (i < ntok ? i : ntok - 1); };
+    const int pw_first = pos_of(wave * (NT * CT)), pw_last = pos_of(wave * (NT * CT) + NT * CT - 1);
+    const int lw_first = first_key(pw_first, reach), lw_last = first_key(pw_last, reach);
 #pragma unroll
-    for (int j = 0; j < ATT_NT; ++j) {
-        const int i = wave * ATT_NT + j;
+    for (int j = 0; j < NT; ++j) {
+        const int i = wave * (NT * CT) + j * CT + (CT > 1 ? r / HW : 0);
         tok_ok[j] = i < ntok;
         tok[j] = t0 + (tok_ok[j] ? i : ntok - 1);
-        pj[j] = p_first + (tok_ok[j] ? i : ntok - 1);
+        pj[j] = pos_of(i);
         loj[j] = first_key(pj[j], reach);
         const bf16* qrow = q + (size_t)tok[j] * q_stride + (size_t)head * D;
 #pragma unroll
@@ -563,11 +589,11 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
             qf[j][ks] = dofs < D ? v : zero4;
         }
     }
-    f32x4 acc[ATT_NT][D16], lacc[ATT_NT];   // lacc: every element holds the column's sum of p
-    float mc[ATT_NT];                        // reference point of the exponent: (a past maximum) * scale * log2(e)
+    f32x4 acc[NT][D16], lacc[NT];   // lacc: every element holds the column's sum of p
+    float mc[NT];                        // reference point of the exponent: (a past maximum) * scale * log2(e)
     const uint4 ones4 = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);   // bfloat16 1.0
 #pragma unroll
-    for (int j = 0; j < ATT_NT; ++j) {
+    for (int j = 0; j < NT; ++j) {
         mc[j] = NEG_BIG;
         lacc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -710,7 +736,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
     // the matrix instructions of another to run beside them.
     auto fast_tile = [&](int kb) {
         uint4 kf0[2][KS], kf1[2][KS];
-        f32x4 s0[ATT_NT][2], s1[ATT_NT][2];
+        f32x4 s0[NT][2], s1[NT][2];
 #pragma unroll
         for (int tau = 0; tau < 2; ++tau)
 #pragma unroll
@@ -718,7 +744,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
 #pragma unroll
         for (int tau = 0; tau < 2; ++tau)
 #pragma unroll
-            for (int j = 0; j < ATT_NT; ++j) {
+            for (int j = 0; j < NT; ++j) {
                 s0[j][tau] = f32x4{0.f, 0.f, 0.f, 0.f};
                 s1[j][tau] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
@@ -727,7 +753,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
 #pragma unroll
             for (int tau = 0; tau < 2; ++tau)
 #pragma unroll
-                for (int j = 0; j < ATT_NT; ++j) s0[j][tau] = mfma16(kf0[tau][ks], qf[j][ks], s0[j][tau]);
+                for (int j = 0; j < NT; ++j) s0[j][tau] = mfma16(kf0[tau][ks], qf[j][ks], s0[j][tau]);
         __builtin_amdgcn_sched_barrier(0);   // the next fragments take the registers of these
 #pragma unroll
         for (int tau = 0; tau < 2; ++tau)
@@ -737,15 +763,15 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
 #define ATT_FOLLOW(S_, PRE_)                                                                               \
         {                                                                                                  \
             /* scores become exponents relative to the reference point, in place */                       \
-            float lm[ATT_NT];                                                                              \
+            float lm[NT];                                                                              \
             bool over = false;                                                                             \
             if (capq > 0.f) {                                                                              \
                 const float icapq = 1.0f / capq;                                                           \
-                _Pragma("unroll") for (int j = 0; j < ATT_NT; ++j)                                         \
+                _Pragma("unroll") for (int j = 0; j < NT; ++j)                                         \
                     _Pragma("unroll") for (int tau = 0; tau < 2; ++tau)                                    \
                         _Pragma("unroll") for (int e = 0; e < 4; ++e) S_[j][tau][e] = att_cap(S_[j][tau][e], capq, icapq); \
             }                                                                                              \
-            _Pragma("unroll") for (int j = 0; j < ATT_NT; ++j) {                                           \
+            _Pragma("unroll") for (int j = 0; j < NT; ++j) {                                           \
                 const bool unset = mc[j] < 0.5f * NEG_BIG;   /* no key seen yet: exponents relative to 0 */ \
                 const float nm = unset ? 0.f : -mc[j];                                                     \
                 _Pragma("unroll") for (int tau = 0; tau < 2; ++tau)                                        \
@@ -756,7 +782,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
             }                                                                                              \
             if (__builtin_amdgcn_ballot_w64(over) != 0ull) {                                               \
                 PRE_                                                                                       \
-                _Pragma("unroll") for (int j = 0; j < ATT_NT; ++j) {                                       \
+                _Pragma("unroll") for (int j = 0; j < NT; ++j) {                                       \
                     float mx = lm[j];                                                                      \
                     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));                                                \
                     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));                                                \
@@ -789,18 +815,18 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
         }
         ATT_FOLLOW(s0, )
         // scores of the second sub-tile on the matrix cores, p of the first on the vector units
-        uint4 pf0[ATT_NT], pf1[ATT_NT], pl0[WF ? ATT_NT : 1], pl1[WF ? ATT_NT : 1];
+        uint4 pf0[NT], pf1[NT], pl0[WF ? NT : 1], pl1[WF ? NT : 1];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
             for (int tau = 0; tau < 2; ++tau)
 #pragma unroll
-                for (int j = 0; j < ATT_NT; ++j) s1[j][tau] = mfma16(kf1[tau][ks], qf[j][ks], s1[j][tau]);
+                for (int j = 0; j < NT; ++j) s1[j][tau] = mfma16(kf1[tau][ks], qf[j][ks], s1[j][tau]);
             if (ks == 0) ATT_PQ(s0, 0, 0, 0, x, y)
             if (ks == 1 || KS == 1) ATT_PQ(s0, 0, 1, 0, z, w)
-            if (ks == 2 || (KS <= 2 && ks == KS - 1)) ATT_PQ(s0, 1, 0, 0, x, y)
-            if (ks == KS - 1) ATT_PQ(s0, 1, 1, 0, z, w)
+            if (NT == 2 && (ks == 2 || (KS <= 2 && ks == KS - 1))) ATT_PQ(s0, NT - 1, 0, 0, x, y)
+            if (NT == 2 && ks == KS - 1) ATT_PQ(s0, NT - 1, 1, 0, z, w)
             __builtin_amdgcn_sched_barrier(0);
         }
         // the next tile leaves for the registers only now: until here they held score fragments
@@ -809,18 +835,18 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
         // (should the reference point move now, the first sub-tile's products, made with the old one,
         // are added first, and the interleaved block below adds zeros in their place)
         ATT_FOLLOW(s1, {
-            _Pragma("unroll") for (int j = 0; j < ATT_NT; ++j) {
+            _Pragma("unroll") for (int j = 0; j < NT; ++j) {
                 lacc[j] = mfma16(ones4, pf0[j], lacc[j]);
                 if (WF) lacc[j] = mfma16(ones4, pl0[WF ? j : 0], lacc[j]);
             }
             _Pragma("unroll") for (int db = 0; db < D16; ++db) {
                 const uint4 v = *reinterpret_cast<const uint4*>(&Vs[v_at(db * 16 + r, qg)]);
-                _Pragma("unroll") for (int j = 0; j < ATT_NT; ++j) {
+                _Pragma("unroll") for (int j = 0; j < NT; ++j) {
                     acc[j][db] = mfma16(v, pf0[j], acc[j][db]);
                     if (WF) acc[j][db] = mfma16(v, pl0[WF ? j : 0], acc[j][db]);
                 }
             }
-            _Pragma("unroll") for (int j = 0; j < ATT_NT; ++j) {
+            _Pragma("unroll") for (int j = 0; j < NT; ++j) {
                 pf0[j] = zero4;
                 if (WF) pl0[WF ? j : 0] = zero4;
             }
@@ -831,7 +857,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
         for (int db = 0; db < DH; ++db) vf[db] = *reinterpret_cast<const uint4*>(&Vs[v_at(db * 16 + r, qg)]);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < ATT_NT; ++j) {
+        for (int j = 0; j < NT; ++j) {
             lacc[j] = mfma16(ones4, pf0[j], lacc[j]);
             if (WF) lacc[j] = mfma16(ones4, pl0[WF ? j : 0], lacc[j]);
         }
@@ -842,15 +868,15 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
                 const int db = h * DH + i;
                 if (db < D16) {
 #pragma unroll
-                    for (int j = 0; j < ATT_NT; ++j) {
+                    for (int j = 0; j < NT; ++j) {
                         acc[j][db] = mfma16(vf[i], pf0[j], acc[j][db]);
                         if (WF) acc[j][db] = mfma16(vf[i], pl0[WF ? j : 0], acc[j][db]);
                     }
                 }
                 if (h == 0 && i == 0) ATT_PQ(s1, 0, 0, 1, x, y)
                 if (h == 0 && i == DH - 1) ATT_PQ(s1, 0, 1, 1, z, w)
-                if (h == 1 && i == 0) ATT_PQ(s1, 1, 0, 1, x, y)
-                if (h == 1 && i == DH - 1) ATT_PQ(s1, 1, 1, 1, z, w)
+                if (NT == 2 && h == 1 && i == 0) ATT_PQ(s1, NT - 1, 0, 1, x, y)
+                if (NT == 2 && h == 1 && i == DH - 1) ATT_PQ(s1, NT - 1, 1, 1, z, w)
                 __builtin_amdgcn_sched_barrier(0);
             }
             // the next half: second half of this sub-tile, then the first of the other
@@ -861,7 +887,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
             }
         }
 #pragma unroll
-        for (int j = 0; j < ATT_NT; ++j) {
+        for (int j = 0; j < NT; ++j) {
             lacc[j] = mfma16(ones4, pf1[j], lacc[j]);
             if (WF) lacc[j] = mfma16(ones4, pl1[WF ? j : 0], lacc[j]);
         }
@@ -872,7 +898,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
                 const int db = h * DH + i;
                 if (db < D16) {
 #pragma unroll
-                    for (int j = 0; j < ATT_NT; ++j) {
+                    for (int j = 0; j < NT; ++j) {
                         acc[j][db] = mfma16(vf[i], pf1[j], acc[j][db]);
                         if (WF) acc[j][db] = mfma16(vf[i], pl1[WF ? j : 0], acc[j][db]);
                     }
@@ -896,11 +922,11 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
         // work on the second while the vector units do the softmax of the first.
         constexpr int NSUB = ATT_TK / 32;
         bool any[NSUB];
-        f32x4 s[NSUB][ATT_NT][2];
+        f32x4 s[NSUB][NT][2];
 #pragma unroll
         for (int sub = 0; sub < NSUB; ++sub) {
             const int kbs = kb + sub * 32;
-            any[sub] = kbs <= pj[ATT_NT - 1] && kbs + 32 > loj[0];   // wave-uniform
+            any[sub] = kbs <= pw_last && kbs + 32 > lw_first;   // wave-uniform
             if (!any[sub]) continue;
             uint4 kf[2][KS];
 #pragma unroll
@@ -914,7 +940,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
                                       : zero4;
                 }
 #pragma unroll
-                for (int j = 0; j < ATT_NT; ++j) s[sub][j][tau] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < NT; ++j) s[sub][j][tau] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
             // four independent accumulator chains (2 key tiles x 2 tokens), interleaved over d
 #pragma unroll
@@ -922,7 +948,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
 #pragma unroll
                 for (int tau = 0; tau < 2; ++tau)
 #pragma unroll
-                    for (int j = 0; j < ATT_NT; ++j) s[sub][j][tau] = mfma16(kf[tau][ks], qf[j][ks], s[sub][j][tau]);
+                    for (int j = 0; j < NT; ++j) s[sub][j][tau] = mfma16(kf[tau][ks], qf[j][ks], s[sub][j][tau]);
         }
 #pragma unroll
         for (int sub = 0; sub < NSUB; ++sub) {
@@ -934,11 +960,11 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
             // and on most sub-tiles no lane talks to another.  The row sums come out of the matrix
             // cores with the values (a row of ones), from the same rounded p.  Sub-tiles that every
             // token of the wave sees whole (all but the diagonal and a window's edge) skip the masks.
-            const bool full = kbs + 31 <= pj[0] && kbs >= loj[ATT_NT - 1];   // wave-uniform
-            float sv[ATT_NT][8], lm[ATT_NT];
+            const bool full = kbs + 31 <= pw_first && kbs >= lw_last;   // wave-uniform
+            float sv[NT][8], lm[NT];
             bool over = false;
 #pragma unroll
-            for (int j = 0; j < ATT_NT; ++j) {
+            for (int j = 0; j < NT; ++j) {
 #pragma unroll
                 for (int tau = 0; tau < 2; ++tau)
 #pragma unroll
@@ -957,7 +983,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
             }
             if (__builtin_amdgcn_ballot_w64(over) != 0ull) {
 #pragma unroll
-                for (int j = 0; j < ATT_NT; ++j) {
+                for (int j = 0; j < NT; ++j) {
                     float mx = lm[j];
                     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
                     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
@@ -973,9 +999,9 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
                         for (int e = 0; e < 4; ++e) acc[j][db][e] *= corr;
                 }
             }
-            uint4 pf[ATT_NT], pl[WF ? ATT_NT : 1];
+            uint4 pf[NT], pl[WF ? NT : 1];
 #pragma unroll
-            for (int j = 0; j < ATT_NT; ++j) {
+            for (int j = 0; j < NT; ++j) {
                 float pe[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) pe[i] = __builtin_amdgcn_exp2f(fmaf(sv[j][i], scale_log2e, -mc[j]));
@@ -1003,7 +1029,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
                 const uint4 v = *reinterpret_cast<const uint4*>(&Vs[v_at(db * 16 + r, sub * 4 + qg)]);
                 const uint4 vf = (PAGE64 || vok) ? v : zero4;   // PAGE64: the tile's own page, finite, times p = 0
 #pragma unroll
-                for (int j = 0; j < ATT_NT; ++j) {
+                for (int j = 0; j < NT; ++j) {
                     acc[j][db] = mfma16(vf, pf[j], acc[j][db]);
                     if (WF) acc[j][db] = mfma16(vf, pl[WF ? j : 0], acc[j][db]);
                 }
@@ -1032,7 +1058,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
     }
     if (!head_ok) return;
 #pragma unroll
-    for (int j = 0; j < ATT_NT; ++j) {
+    for (int j = 0; j < NT; ++j) {
         if (!tok_ok[j]) continue;
         const float inv = 1.0f / lacc[j][0];
         bf16* orow = out + (size_t)tok[j] * out_stride + (size_t)head * D;
@@ -1063,27 +1089,36 @@ extern "C" int ilm_attn_tile(void* out, const void* q, const void* kc, const voi
                 "attn_tile: q and out rows must be 16-byte / 8-byte aligned");
     const int G = nh / nkv, HG = (G + 15) / 16;
     ILM_REQUIRE(nkv * HG <= 65535, "attn_tile: grid too large");
-    dim3 grid(n_tiles, nkv * HG);
+    const int ct = G > 8 ? 1 : G > 4 ? 2 : 4;
+    const bool pair = ct == 4;
+    dim3 grid(pair ? (n_tiles + 1) / 2 * 2 : n_tiles, nkv * HG);
     const float sl2 = scale * 1.4426950408889634f;
     const float capq = softcap > 0.f ? softcap / scale : 0.f;
     const int cus = ilm_num_cus();
-    const long long n_items = (long long)n_tiles * nkv * HG;
+    const long long n_items = (long long)(pair ? (n_tiles + 1) / 2 : n_tiles) * nkv * HG;
     const int pair_base = (n_items > cus && n_items <= 2 * cus) ? cus : 0;
 #define AT_ARGS (bf16*)out, (const bf16*)q, (const bf16*)kc, (const bf16*)vc, (const int*)block_tables, (const int*)seg, \
-                (const int*)pos, (const int*)tiles, nh, nkv, page, max_blocks, q_stride, out_stride, sl2, capq, reach, pair_base
-#define AT_CASE(D16)                                                                   \
-    case D16:                                                                          \
-        if (float_weights) {                                                           \
-            if (page % ATT_TK == 0) attn_tile_kernel<D16, true, true><<<grid, 256, 0, stream>>>(AT_ARGS);  \
-            else attn_tile_kernel<D16, false, true><<<grid, 256, 0, stream>>>(AT_ARGS);    \
-        } else if (page % ATT_TK == 0) attn_tile_kernel<D16, true, false><<<grid, 256, 0, stream>>>(AT_ARGS);  \
-        else attn_tile_kernel<D16, false, false><<<grid, 256, 0, stream>>>(AT_ARGS);   \
+                (const int*)pos, (const int*)tiles, nh, nkv, page, max_blocks, q_stride, out_stride, sl2, capq, reach, pair_base, n_tiles
+#define AT_RUN(D16, P64, WF_)                                                                          \
+    {                                                                                                  \
+        if (ct == 1) attn_tile_kernel<D16, P64, WF_, 1><<<grid, 256, 0, stream>>>(AT_ARGS);            \
+        else if (ct == 2) attn_tile_kernel<D16, P64, WF_, 2><<<grid, 256, 0, stream>>>(AT_ARGS);       \
+        else attn_tile_kernel<D16, P64, WF_, 4><<<grid, 256, 0, stream>>>(AT_ARGS);                    \
+    }
+#define AT_CASE(D16)                                            \
+    case D16:                                                   \
+        if (float_weights) {                                    \
+            if (page % ATT_TK == 0) AT_RUN(D16, true, true)     \
+            else AT_RUN(D16, false, true)                       \
+        } else if (page % ATT_TK == 0) AT_RUN(D16, true, false) \
+        else AT_RUN(D16, false, false)                          \
         break
     switch (d / 16) {
         AT_CASE(1); AT_CASE(2); AT_CASE(3); AT_CASE(4); AT_CASE(5); AT_CASE(6); AT_CASE(7); AT_CASE(8);
         default: ILM_REQUIRE(false, "attn_tile: head size %d", d);
     }
 #undef AT_CASE
+#undef AT_RUN
 #undef AT_ARGS
     ILM_LAUNCH_CHECK("attn_tile");
     return 0;

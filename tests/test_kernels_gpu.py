@@ -947,6 +947,25 @@ def test_attention_bfloat16_two_chunks_in_one_workgroup(K, monkeypatch, nh, nkv,
         assert torch.equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("nh,nkv,d,page", [(1, 1, 64, 16), (4, 2, 128, 64), (8, 2, 16, 64), (3, 1, 96, 64), (5, 1, 128, 64), (12, 2, 64, 64), (16, 2, 48, 16), (8, 1, 128, 32),
+                                           (9, 1, 64, 64)])
+@pytest.mark.parametrize("window", [0, 64, 37])
+def test_attention_bfloat16_tiles_of_few_heads(K, monkeypatch, nh, nkv, d, page, window):
+    """Columns that hold one, two and four tokens: tiles that pair with the next one of their request and such that do not (a tile cut short, another
+    request's, the last of an odd number), portions that end on either side of a key tile; with a softcap and float weights too."""
+    attention = K.paged_attention
+    case = dict(lens=[8, 9, 64, 65, 130, 40, 300, 17, 7, 200], qlens=[8, 9, 16, 63, 24, 5, 130, 1, 7, 33], seed=70 + d + nh, window=window)
+    out, want = _attention_case(K, torch.bfloat16, nh, nkv, d, page, **case)
+    _close(out, want, 1.2e-2)
+    outs = []
+    for tiles in (True, False):     # in tiles and one by one, under a softcap
+        def both(*a, tiles=None, single_rows=None, _on=tiles, **k):
+            return attention(*a, tiles=tiles if _on else None, single_rows=single_rows if _on else None, softcap=3.0, float_weights=True, **k)
+        monkeypatch.setattr(K, "paged_attention", both)
+        outs.append(_attention_case(K, torch.bfloat16, nh, nkv, d, page, **case)[0])
+    _close(outs[0], outs[1], 1.2e-2)
+
+
 def test_attention_bfloat16_with_a_block_table_beyond_lds(K):
     """33,000 keys in pages of 16: more block-table entries than the tile kernel keeps in LDS, and
     the most chunks the single-token kernel cuts a context into."""
