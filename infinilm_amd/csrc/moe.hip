@@ -556,8 +556,6 @@ moe_gemm_few_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict__
 #pragma unroll
                 for (int u = 0; u < KSTEPS; ++u) to[u] = wp[k8c[u]];
             };
-            load(a[0], share, 0);
-            if (D == 2) load(a[D - 1], share, 1);
 #pragma unroll
             for (int g = 0; g < MG; ++g) {
                 const bool has = row0 + g * 16 + r < rows;
@@ -577,6 +575,8 @@ moe_gemm_few_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict__
                     xf[g][u] = kok[u] && has ? v : zero;
                 }
             }
+            load(a[0], share, 0);
+            if (D == 2) load(a[D - 1], share, 1);
 #pragma unroll 1
             for (int nt = share; nt < nt_all; nt += sharers) {
                 const int n = nt * 16 + (l >> 4) * 4 + e;
