@@ -58,6 +58,7 @@ _SIGNATURES = {
     "ilm_attn_tile": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _F, _I, _P],
     "ilm_argmax": [_P, _P, _I, _I, _I, _P],
     "ilm_sample": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+    "ilm_sample_host": [_P, _P, _P, _P, _P, _P, c_uint64, _P, _P, _P, _I, _I, _I, _P],
     "ilm_uniforms": [_P, _P, c_uint64, _P, _P, _I],
     "ilm_unary": [_P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "ilm_lin_prep": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P],
@@ -157,6 +158,8 @@ def load(verbose: bool = True) -> ctypes.CDLL:
     lib.ilm_sample_ws.argtypes = [c_int, c_int]
     lib.ilm_moe_plan_few_ok.restype = c_int
     lib.ilm_moe_plan_few_ok.argtypes = [c_int, c_int, c_int]
+    lib.ilm_sample_host_rows.restype = c_int
+    lib.ilm_sample_host_rows.argtypes = []
     lib.ilm_sample_few_k.restype = c_int
     lib.ilm_sample_few_k.argtypes = []
     lib.ilm_attn_static_init.restype = c_int

@@ -29,6 +29,8 @@
 // result depends on no order of atomics, and finer than sums of floats.
 #include "common.h"
 
+#include <string.h>
+
 #include <type_traits>
 
 #define SB 1024
@@ -897,15 +899,47 @@ __device__ __forceinline__ bool top_k_of_few(SampleLds& S, const float* row, int
     return true;
 }
 
+// ---- what each row asks for: in device memory (N 0), or up to N rows' in the launch itself, which saves the copy ahead of it and the buffer that such a
+// copy reads.  A kernel's first argument, so it lies where the kernel's arguments begin; read there, as an array among arguments that is
+// indexed by the row would be copied into scratch memory first.
+template <int N>
+struct RowSettings {
+    float temperature[N];
+    int top_k[N];
+    float top_p[N], uniform[N];
+};
+template <>
+struct RowSettings<0> {
+    const float* temperature;
+    const int* top_k;
+    const float *top_p, *uniform;
+};
+struct Settings {
+    float temperature;
+    int top_k;
+    float top_p, uniform;
+};
+template <int N>
+__device__ __forceinline__ Settings settings_of(const RowSettings<N>& rows, int r) {
+    if constexpr (N == 0) {
+        return {rows.temperature[r], rows.top_k[r], rows.top_p[r], rows.uniform[r]};
+    } else {
+        typedef const __attribute__((address_space(4))) RowSettings<N>* Args;
+        const Args a = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+        return {a->temperature[r], a->top_k[r], a->top_p[r], a->uniform[r]};
+    }
+}
+
+template <int N>
 __global__ void __launch_bounds__(SB)
-sample_kernel(int* __restrict__ out, const float* __restrict__ logits, const float* __restrict__ temperature,
-              const int* __restrict__ top_k, const float* __restrict__ top_p,
-              const float* __restrict__ uniform, int V, int stride, int cut) {
+sample_kernel(const RowSettings<N> rows, int* __restrict__ out, const float* __restrict__ logits, int V, int stride, int cut) {
     __shared__ SampleLds S;
-    const int r = blockIdx.x, k = top_k[r];
+    const int r = blockIdx.x;
+    const Settings set = settings_of<N>(rows, r);
+    const int k = set.top_k;
     const float* row = logits + (size_t)r * stride;
-    const float temp = temperature[r];
-    if (k > 1 && k <= FEW_K && k < V && V >= FEW_FROM && temp != 0.0f && top_k_of_few(S, row, V, temp, k, top_p[r], uniform[r], cut, out + r)) return;
+    const float temp = set.temperature;
+    if (k > 1 && k <= FEW_K && k < V && V >= FEW_FROM && temp != 0.0f && top_k_of_few(S, row, V, temp, k, set.top_p, set.uniform, cut, out + r)) return;
     const RowMax m = block_argmax<SB>(row, V, sample_of(row[(size_t)threadIdx.x * V / SB]), S.meet);
     const float mx = m.value;
     const int amax = m.index == 0x7fffffff ? 0 : m.index;
@@ -914,8 +948,8 @@ sample_kernel(int* __restrict__ out, const float* __restrict__ logits, const flo
         return;
     }
     const float per = bins_per(mx, m.seen.low, 1.0f / temp);
-    if (m.seen.ties * TIE_SHARE > SB) sample_row<true>(S, row, V, mx, amax, temp, k, top_p[r], uniform[r], cut, out + r, per, 0, 0);
-    else sample_row<false>(S, row, V, mx, amax, temp, k, top_p[r], uniform[r], cut, out + r, per, 0, 0);
+    if (m.seen.ties * TIE_SHARE > SB) sample_row<true>(S, row, V, mx, amax, temp, k, set.top_p, set.uniform, cut, out + r, per, 0, 0);
+    else sample_row<false>(S, row, V, mx, amax, temp, k, set.top_p, set.uniform, cut, out + r, per, 0, 0);
 }
 
 // ---- rows in chunks ----------------------------------------------------------------------------------------
@@ -991,14 +1025,16 @@ __device__ __forceinline__ int row_max(const RowWork* W, int chunks, float* mx, 
     return bi == 0x7fffffff ? 0 : bi;
 }
 
+template <int N>
 __global__ void __launch_bounds__(CHUNK_THREADS)
-sample_hist_kernel(char* __restrict__ ws, size_t ws_row, const float* __restrict__ logits, const float* __restrict__ temperature,
-                   const int* __restrict__ top_k, const float* __restrict__ top_p, int V, int stride, int cut) {
+sample_hist_kernel(const RowSettings<N> rows, char* __restrict__ ws, size_t ws_row, const float* __restrict__ logits, int V, int stride, int cut) {
     __shared__ u64 hist[NBINS];
     __shared__ u64 red[CHUNK_THREADS / 64];
-    const int r = blockIdx.y, k = top_k[r];
+    const int r = blockIdx.y;
+    const Settings set = settings_of<N>(rows, r);
+    const int k = set.top_k;
     RowWork* W = reinterpret_cast<RowWork*>(ws + (size_t)r * ws_row);
-    const float temp = temperature[r], pp = top_p[r];
+    const float temp = set.temperature, pp = set.top_p;
     const bool count = k > 0 && k < V;
     if (temp == 0.0f || k == 1 || (!count && !(pp < 1.0f))) return;
     float mx, low;
@@ -1076,18 +1112,20 @@ __device__ __forceinline__ Found row_threshold(const u64 (&mine)[NBINS / NT], u6
     return f;
 }
 
+template <int N>
 __global__ void __launch_bounds__(CHUNK_THREADS)
-sample_list_kernel(char* __restrict__ ws, size_t ws_row, const float* __restrict__ logits, const float* __restrict__ temperature,
-                   const int* __restrict__ top_k, const float* __restrict__ top_p, int V, int stride, int cut) {
+sample_list_kernel(const RowSettings<N> rows, char* __restrict__ ws, size_t ws_row, const float* __restrict__ logits, int V, int stride, int cut) {
     __shared__ u64 red[CHUNK_THREADS / 64];
     __shared__ Found shared;
     __shared__ uint32_t keys[LIST_CAP];   // the chunk's listed elements: a place in the row's list costs a round trip through memory, so a chunk asks
     __shared__ int indices[LIST_CAP];     // once for all of its own
     __shared__ int own, from, last;
-    const int r = blockIdx.y, k = top_k[r];
+    const int r = blockIdx.y;
+    const Settings set = settings_of<N>(rows, r);
+    const int k = set.top_k;
     RowWork* W = reinterpret_cast<RowWork*>(ws + (size_t)r * ws_row);
     const float* row = logits + (size_t)r * stride;
-    const float temp = temperature[r], pp = top_p[r];
+    const float temp = set.temperature, pp = set.top_p;
     const bool count = k > 0 && k < V;
     if (temp == 0.0f || k == 1) return;
     if (threadIdx.x == 0) own = 0, last = 0;
@@ -1180,15 +1218,17 @@ sample_list_kernel(char* __restrict__ ws, size_t ws_row, const float* __restrict
     }
 }
 
+template <int N>
 __global__ void __launch_bounds__(SB)
-sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row, int chunks, const float* __restrict__ logits,
-                    const float* __restrict__ temperature, const int* __restrict__ top_k, const float* __restrict__ top_p,
-                    const float* __restrict__ uniform, int V, int stride, int cut) {
+sample_token_kernel(const RowSettings<N> rows, int* __restrict__ out, char* __restrict__ ws, size_t ws_row, int chunks, const float* __restrict__ logits,
+                    int V, int stride, int cut) {
     __shared__ SampleLds S;
-    const int r = blockIdx.x, k = top_k[r];
+    const int r = blockIdx.x;
+    const Settings set = settings_of<N>(rows, r);
+    const int k = set.top_k;
     RowWork* W = reinterpret_cast<RowWork*>(ws + (size_t)r * ws_row);
     const float* row = logits + (size_t)r * stride;
-    const float temp = temperature[r], pp = top_p[r];
+    const float temp = set.temperature, pp = set.top_p;
     const bool count = k > 0 && k < V;
     float mx, low;
     bool ties;
@@ -1210,8 +1250,8 @@ sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row,
             tau = count ? radix_bin<true>(row, V, S, mass, f.at, per, 0, f.before, need)
                         : radix_bin<false>(row, V, S, mass, f.at, per, 0, f.before, need);
         }
-        if (ties) sample_row<true>(S, row, V, mx, amax, temp, k, pp, uniform[r], cut, out + r, per, known, tau);
-        else sample_row<false>(S, row, V, mx, amax, temp, k, pp, uniform[r], cut, out + r, per, known, tau);
+        if (ties) sample_row<true>(S, row, V, mx, amax, temp, k, pp, set.uniform, cut, out + r, per, known, tau);
+        else sample_row<false>(S, row, V, mx, amax, temp, k, pp, set.uniform, cut, out + r, per, known, tau);
         return;
     }
     for (int i = threadIdx.x; i < listed; i += SB) {
@@ -1234,7 +1274,7 @@ sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row,
             if (tp > tau) tau = tp;
         }
         if (listed <= RANK_MAX) {
-            token_of_list(S, listed, tau, uniform[r], amax, out + r);
+            token_of_list(S, listed, tau, set.uniform, amax, out + r);
             return;
         }
         clear_tiles(S, tiles);
@@ -1242,7 +1282,7 @@ sample_token_kernel(int* __restrict__ out, char* __restrict__ ws, size_t ws_row,
         if (f.at >= 0) tau = rank_bin(S, listed, 0, f.before, need);
     }
     list_to_tiles(S, listed, tau, m);
-    if (threadIdx.x < 64) token_of_tiles(S, row, V, mass, tau, uniform[r], S.pick - 1, amax, out + r);
+    if (threadIdx.x < 64) token_of_tiles(S, row, V, mass, tau, set.uniform, S.pick - 1, amax, out + r);
 }
 
 // Bytes of workspace a row needs of n rows of V logits; 0: none, the rows are not cut into chunks.  They are where few rows leave
@@ -1282,18 +1322,13 @@ extern "C" int ilm_uniforms(float* out, const uint64_t* seeds, uint64_t seed, co
     return 0;
 }
 
-// `ws`: n * ilm_sample_ws(n, V) bytes, 16-byte aligned, or null: every row by one workgroup
-extern "C" int ilm_sample(void* out, const void* logits, const void* temperature, const void* top_k,
-                          const void* top_p, const void* uniform, void* ws, int n, int V, int stride,
-                          hipStream_t stream) {
-    ILM_REQUIRE(n > 0 && V > 0 && stride >= V, "sample: bad sizes n=%d V=%d stride=%d", n, V, stride);
-    ILM_REQUIRE(((uintptr_t)ws & 15) == 0, "sample: the workspace must be 16-byte aligned");
+template <int N>
+static int sample_rows(const RowSettings<N>& rows, void* out, const void* logits, void* ws, int n, int V, int stride, hipStream_t stream) {
     int cut = 0;   // V elements of at most 2^43 each: below 2^64 up to a vocabulary of 2^20
     while ((long long)V >> (20 + cut)) ++cut;
     const size_t ws_row = (size_t)ilm_sample_ws(n, V);
     if (ws == nullptr || ws_row == 0) {
-        sample_kernel<<<n, SB, 0, stream>>>((int*)out, (const float*)logits, (const float*)temperature, (const int*)top_k,
-                                            (const float*)top_p, (const float*)uniform, V, stride, cut);
+        sample_kernel<N><<<n, SB, 0, stream>>>(rows, (int*)out, (const float*)logits, V, stride, cut);
         ILM_LAUNCH_CHECK("sample");
         return 0;
     }
@@ -1305,12 +1340,46 @@ extern "C" int ilm_sample(void* out, const void* logits, const void* temperature
     const dim3 grid(chunks, n);
     char* w = (char*)ws;
     sample_max_kernel<<<grid, CHUNK_THREADS, 0, stream>>>(w, ws_row, (const float*)logits, V, stride);
-    sample_hist_kernel<<<grid, CHUNK_THREADS, 0, stream>>>(w, ws_row, (const float*)logits, (const float*)temperature, (const int*)top_k,
-                                                           (const float*)top_p, V, stride, cut);
-    sample_list_kernel<<<grid, CHUNK_THREADS, 0, stream>>>(w, ws_row, (const float*)logits, (const float*)temperature, (const int*)top_k,
-                                                           (const float*)top_p, V, stride, cut);
-    sample_token_kernel<<<n, SB, 0, stream>>>((int*)out, w, ws_row, chunks, (const float*)logits, (const float*)temperature,
-                                              (const int*)top_k, (const float*)top_p, (const float*)uniform, V, stride, cut);
+    sample_hist_kernel<N><<<grid, CHUNK_THREADS, 0, stream>>>(rows, w, ws_row, (const float*)logits, V, stride, cut);
+    sample_list_kernel<N><<<grid, CHUNK_THREADS, 0, stream>>>(rows, w, ws_row, (const float*)logits, V, stride, cut);
+    sample_token_kernel<N><<<n, SB, 0, stream>>>(rows, (int*)out, w, ws_row, chunks, (const float*)logits, V, stride, cut);
     ILM_LAUNCH_CHECK("sample");
     return 0;
+}
+static int sample_check(int n, int V, int stride, const void* ws) {
+    ILM_REQUIRE(n > 0 && V > 0 && stride >= V, "sample: bad sizes n=%d V=%d stride=%d", n, V, stride);
+    ILM_REQUIRE(((uintptr_t)ws & 15) == 0, "sample: the workspace must be 16-byte aligned");
+    return 0;
+}
+
+// `ws`: n * ilm_sample_ws(n, V) bytes, 16-byte aligned, or null: every row by one workgroup
+extern "C" int ilm_sample(void* out, const void* logits, const void* temperature, const void* top_k,
+                          const void* top_p, const void* uniform, void* ws, int n, int V, int stride,
+                          hipStream_t stream) {
+    if (sample_check(n, V, stride, ws) != 0) return -1;
+    const RowSettings<0> rows = {(const float*)temperature, (const int*)top_k, (const float*)top_p, (const float*)uniform};
+    return sample_rows<0>(rows, out, logits, ws, n, V, stride, stream);
+}
+
+// The same with what the rows ask for at host addresses, read before the call returns (a recorded call keeps it), for up to ilm_sample_host_rows() rows;
+// the uniform numbers from seeds (null: `seed` for all), keys and indices as ilm_uniforms forms them.  64 rows of 73,448 with a top-k of 50 through the
+// sampler 32.7 -> 21.6 us a call, 5 of 122,753 with top-p 35.9 -> 29.5 (a copy of 2 us and what waits for it less, and 12 us less on the host).
+extern "C" int ilm_sample_host_rows() { return 192; }   // (16 bytes a row, within the 4 KB that a launch's arguments may take)
+extern "C" int ilm_sample_host(void* out, const void* logits, const float* temperature, const int* top_k, const float* top_p, const uint64_t* seeds,
+                               uint64_t seed, const uint64_t* keys, const uint64_t* indices, void* ws, int n, int V, int stride, hipStream_t stream) {
+    if (sample_check(n, V, stride, ws) != 0) return -1;
+    ILM_REQUIRE(n <= ilm_sample_host_rows(), "sample_host: %d rows", n);
+#define SAMPLE_HOST(N_)                                                                        \
+    {                                                                                          \
+        RowSettings<N_> rows;                                                                  \
+        memcpy(rows.temperature, temperature, n * sizeof(float));                              \
+        memcpy(rows.top_k, top_k, n * sizeof(int));                                            \
+        memcpy(rows.top_p, top_p, n * sizeof(float));                                          \
+        if (ilm_uniforms(rows.uniform, seeds, seed, keys, indices, n) != 0) return -1;         \
+        return sample_rows<N_>(rows, out, logits, ws, n, V, stride, stream);                   \
+    }
+    if (n <= 16) SAMPLE_HOST(16)
+    if (n <= 64) SAMPLE_HOST(64)
+    SAMPLE_HOST(192)
+#undef SAMPLE_HOST
 }

@@ -1101,6 +1101,26 @@ def sample_packed(logits: torch.Tensor, params: torch.Tensor, few: bool = False)
     return _sample(logits, p, p + 4 * n, p + 8 * n, p + 12 * n, few)
 
 
+SAMPLE_HOST_ROWS = 192      # most rows whose settings travel with the launch (ilm_sample_host_rows())
+
+
+def sample_host(logits: torch.Tensor, temperature, top_k, top_p, seeds, seed: int, keys, indices, few: bool = False) -> torch.Tensor:
+    """`sample` with what the rows ask for in host arrays (`array`: "f", "i", "f"), at most SAMPLE_HOST_ROWS of them, read before this returns; the uniform
+    numbers from `seeds` (None: `seed` for all), keys and indices (`array` "Q").  `few` as in `sample_packed`."""
+    _dev(logits)
+    if logits.dtype != F32 or logits.dim() != 2 or logits.stride(1) != 1:
+        raise KernelError("sample takes float32 rows")
+    n, V = logits.shape
+    if n > SAMPLE_HOST_ROWS or not len(temperature) == len(top_k) == len(top_p) == len(keys) == len(indices) == n or (seeds is not None and len(seeds) != n):
+        raise KernelError(f"settings, a key and an index for each of {n} rows (at most {SAMPLE_HOST_ROWS})")
+    out = torch.empty((n,), dtype=torch.int32, device=logits.device)
+    per_row = 0 if few else _lib().ilm_sample_ws(n, V)
+    ws = torch.empty((n * per_row,), dtype=torch.uint8, device=logits.device) if per_row else None
+    _run("ilm_sample_host", out.data_ptr(), logits.data_ptr(), temperature.buffer_info()[0], top_k.buffer_info()[0], top_p.buffer_info()[0],
+         None if seeds is None else seeds.buffer_info()[0], seed, keys.buffer_info()[0], indices.buffer_info()[0], _ptr(ws), n, V, logits.stride(0), _stream())
+    return out
+
+
 def _sample(logits: torch.Tensor, temperature: int, top_k: int, top_p: int, uniform: int, few: bool) -> torch.Tensor:
     n, V = logits.shape
     out = torch.empty((n,), dtype=torch.int32, device=logits.device)

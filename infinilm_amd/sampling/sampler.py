@@ -106,6 +106,15 @@ class Sampler:
             raise ValueError("no rows to sample")
         if all(p.greedy for p, _, _ in rows):
             return kernels.argmax(logits)
+        params, keys, indices = zip(*rows)
+        top_k = [p.top_k for p in params]
+        few = 0 < min(top_k) and kernels.sample_one_reading(n, logits.shape[1], max(top_k))
+        temperature, top_p = array("f", [p.temperature for p in params]), array("f", [p.top_p for p in params])
+        seeds = [self.seed if p.seed is None else p.seed for p in params]
+        if n <= kernels.SAMPLE_HOST_ROWS:      # they travel with the launch
+            one = seeds.count(seeds[0]) == n
+            return kernels.sample_host(logits, temperature, _int32s(top_k), top_p, None if one else _words(seeds), _words(seeds[:1])[0], _words(keys),
+                                       _words(indices), few)
         # temperature, top_k, top_p and the uniform numbers in one pinned buffer and one copy that
         # queues behind the step (a copy from pageable memory would make the host wait for the step
         # and the device wait for four copies)
@@ -117,14 +126,12 @@ class Sampler:
             buf = torch.empty((4 * max(n, 64),), dtype=torch.float32, pin_memory=dev.type == "cuda")
             self._staging[t] = (buf, memoryview(buf.numpy()).cast("B"), buf.data_ptr())
         buf, raw, at = self._staging[t]
-        params, keys, indices = zip(*rows)
-        top_k = [p.top_k for p in params]
-        raw[0:4 * n] = memoryview(array("f", [p.temperature for p in params])).cast("B")
+        raw[0:4 * n] = memoryview(temperature).cast("B")
         raw[4 * n:8 * n] = memoryview(_int32s(top_k)).cast("B")
-        raw[8 * n:12 * n] = memoryview(array("f", [p.top_p for p in params])).cast("B")
-        _uniforms_into(at + 12 * n, [self.seed if p.seed is None else p.seed for p in params], keys, indices)
+        raw[8 * n:12 * n] = memoryview(top_p).cast("B")
+        _uniforms_into(at + 12 * n, seeds, keys, indices)
         d = torch.empty((4 * n,), dtype=torch.float32, device=dev)
         d.copy_(buf[:4 * n], non_blocking=True)
         if dev.type == "cuda":
             self._event(t, dev.index).record()
-        return kernels.sample_packed(logits, d, few=0 < min(top_k) and kernels.sample_one_reading(n, logits.shape[1], max(top_k)))
+        return kernels.sample_packed(logits, d, few=few)

@@ -40,6 +40,7 @@ def test_constants_mirrored_in_python_equal_the_library(K):
     assert L.ilm_attn_basic_chunk() == K.BASIC_CHUNK
     assert L.ilm_attn_f32_chunk() == K.F32_ATTN_CHUNK and L.ilm_attn_f32_ws_row(128) == 132
     assert L.ilm_attn_f32_tile_tokens() == K.ATT_TILE_TOKENS
+    assert L.ilm_sample_host_rows() == K.SAMPLE_HOST_ROWS
     assert all(bool(L.ilm_attn_f32_tile_ok(d, 16)) == (d in K.F32_ATTN_TILE_HEADS) for d in range(16, 272, 16))
     assert L.ilm_gemm_ksplit_max_k(1) == K.KSPLIT_SPAN
     assert L.ilm_gemm_rows64_span() == K.ROWS64_SPAN
@@ -1471,3 +1472,35 @@ def test_portion_product_walks_its_tiles_in_bands(K, tile, M, N, K_):
     K.portion_gemm(x, w, None, out, tile)
     want = x.to(F64) @ w.to(F64).T
     assert float((out.to(F64) - want).abs().max()) < 2.0 ** -8 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 192, 193])
+@pytest.mark.parametrize("V", [3000, 50000])
+def test_sampling_with_the_rows_settings_in_the_launch(K, n, V):
+    """Settings that travel with the launch, for every size of that form and the first beyond it, and the sampler that uses it: the tokens of settings in
+    device memory, by one workgroup a row and in chunks; launched twice and recorded, so that no launch sees another's."""
+    from array import array
+    from infinilm_amd.sampling import Sampler, SamplingParams
+    from infinilm_amd.sampling.sampler import uniforms_for
+    g = torch.Generator().manual_seed(n + V)
+    logits = (2.0 * torch.randn((n, V), generator=g)).to(DEV)
+    settings = [(0.5 + i % 5 * 0.2, (0, 1, 20, 400)[i % 4], (1.0, 0.9, 0.3)[i % 3], 1000 + i * (1 << 40), i) for i in range(n)]
+    t, k, p, keys, index = (list(x) for x in zip(*settings))
+    prm = torch.cat([torch.tensor(t), torch.tensor(k, dtype=torch.int32).view(torch.float32), torch.tensor(p),
+                     torch.from_numpy(uniforms_for([9] * n, keys, index))]).to(DEV)
+    want = K.sample_packed(logits, prm)
+    if n <= K.SAMPLE_HOST_ROWS:
+        args = (array("f", t), array("i", k), array("f", p))
+        one = K.sample_host(logits, *args, None, 9, array("Q", keys), array("Q", index))
+        other = K.sample_host(logits, array("f", [1.0] * n), array("i", [1] * n), args[2], array("Q", [3] * n), 0, array("Q", keys), array("Q", index))
+        assert torch.equal(one, want) and torch.equal(other, K.argmax(logits))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            rec = K.sample_host(logits, *args, array("Q", [9] * n), 0, array("Q", keys), array("Q", index))
+        args[0][0] = 77.0
+        for _ in range(3):
+            rec.fill_(-1)
+            graph.replay()
+            assert torch.equal(rec, want)
+    rows = [(SamplingParams(temperature=a, top_k=b, top_p=c), d, e) for a, b, c, d, e in settings]
+    assert torch.equal(Sampler(9).sample_device(logits, rows), want)
