@@ -341,7 +341,10 @@ extern "C" int ilm_gemm_portion(void* C, int ldc, const void* X, int lda, const 
         else GP_RUN(128, 128, 64, 32, 4, GP_PLAIN, N)
     } else {
         ILM_REQUIRE(tile == 1 || tile == 4 || tile == 5, "gemm_portion: there is no tile %d", tile);
-        if (tile == 1) GP_RUN(64, 128, 32, 64, 3, GP_GLU, 2 * N)
+        // (beyond two a unit two stages instead of three, so that three share one: 700 x 6144 x 1024, 528 tiles, 18.7 -> 15.3 us, 700 x 8192 x 1024, 704,
+        // 18.9 -> 17.1; up to two a unit the third stage is worth more: 700 x 4096 x 768, 352, 10.8 / 11.2, 37 x 8192 x 1024 8.7 / 11.5)
+        if (tile == 1 && (long long)((M + 63) / 64) * ((N + 63) / 64) > 2 * ilm_num_cus()) GP_RUN(64, 128, 32, 64, 2, GP_GLU, 2 * N)
+        else if (tile == 1) GP_RUN(64, 128, 32, 64, 3, GP_GLU, 2 * N)
         else if (tile == 4) GP_RUN(256, 128, 64, 64, 3, GP_GLU, 2 * N)
         else GP_RUN(256, 256, 128, 64, 2, GP_GLU, 2 * N)
     }

@@ -1504,3 +1504,13 @@ def test_sampling_with_the_rows_settings_in_the_launch(K, n, V):
             assert torch.equal(rec, want)
     rows = [(SamplingParams(temperature=a, top_k=b, top_p=c), d, e) for a, b, c, d, e in settings]
     assert torch.equal(Sampler(9).sample_device(logits, rows), want)
+
+
+@pytest.mark.parametrize("M,N,K_", [(1100, 2050, 64), (700, 3072, 192), (700, 2048, 320)])
+def test_portion_gate_and_up_beyond_two_tiles_a_unit(K, M, N, K_):
+    """Two stages in LDS instead of three, with one stage of K, three and five, against the product and the activation apart: the same bits."""
+    g = torch.Generator().manual_seed(M + N + K_)
+    x, w = torch.randn((M, K_), generator=g).to(BF16).to(DEV), torch.randn((2 * N, K_), generator=g).to(BF16).to(DEV)
+    assert -(-M // 64) * -(-N // 64) > 2 * K._num_cus(torch.device(DEV)) or N == 2048
+    got = K.portion_glu(x, w, None, "silu", 1)
+    assert torch.equal(got, K.swiglu(K.portion_gemm(x, w, None, torch.empty((M, 2 * N), dtype=BF16, device=DEV), 1), "silu"))
