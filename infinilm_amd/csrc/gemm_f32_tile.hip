@@ -7,7 +7,8 @@
 // So a tile of 128 x 256 with 64 x 64 outputs a wave where there are enough of them for the chip, smaller ones
 // else.  The pieces of two stages of 32 k lie in LDS (147 KB), in fragment order.  Half of the waves cut
 // the next stage before they multiply, the other half after: two waves share a SIMD, and one's vector work
-// runs beside the other's matrix work.  2,048 rows against the kernel on v_mfma_f32_16x16x4_f32 that this one replaced (tiles of
+// runs beside the other's matrix work (the one that multiplies goes ahead, s_setprio: 2048 x 4608 x 4096 405 -> 395 us, 4096 x 16384 1,380 -> 1,340,
+// 32768 x 4096 2,795 -> 2,760).  2,048 rows against the kernel on v_mfma_f32_16x16x4_f32 that this one replaced (tiles of
 // 128 x 128, 106 TFLOP/s at most): 32768 x 4096 2.86 ms against 5.20 (192 TFLOP/s, of which the matrix cores are busy half
 // the time), 4096 x 16384 1.42 against 2.67, 1024 x 1024 44 us against 106; 300 x 4608 x 4096 142 us against 416.
 // Tiles beyond whole rounds over the chip left most of it idle (288 tiles of 2048 x 4608 on 256 units: two rounds, the second an eighth full;
@@ -138,6 +139,7 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
         ++in_slice;
         // two tiles of W at a time: all of a wave's W fragments would take the registers that its sums need (LDS has room
         // for the second reading of X)
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int t0 = 0; t0 < TN; t0 += 2) {
             asm volatile("" ::: "memory");   // (X's fragments are read again, not kept)
@@ -154,6 +156,7 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
                 f3_step(a, b, acc, t0, g);
             }
         }
+        __builtin_amdgcn_s_setprio(0);
         if (!early && st + 1 < st1) {
             store(st + 1);
             fetch(st + 2);
