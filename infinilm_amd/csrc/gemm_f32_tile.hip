@@ -40,12 +40,17 @@ __device__ __forceinline__ void ft_place(int id, int m_tiles, int n_tiles, int& 
     }
 }
 
-// BM x BN outputs a workgroup (rows of X, rows of W), WM x WN a wave.  CUT: some slices, whose sums leave one by one
-template <int BM, int BN, int WM, int WN, bool CUT>
+// BM x BN outputs a workgroup (rows of X, rows of W), WM x WN a wave.  CUT: some slices, whose sums leave one by one.
+// GLU: W = [gate; up] of N outputs each, a tile's groups of 16 rows in turn from either, so that a lane holds gate and up of the same outputs and
+// writes act(gate) * up, the bits of the product and the activation kernel one after the other, which write the sums (268 MB for 2048 x 32768) and
+// read them again.  us, apart / here: 2048 x 32768 x 4096 3,000 / 2,880, 2048 x 8192 x 1024 216 / 199, 1024 x 11520 x 2304 324 / 312, in cut tiles 1300 x
+// 32768 x 4096 2,046 / 1,982, 300 x 32768 x 4096 596 / 587.  (The matrix whose rows a wave fetches is the same for all of its lanes: as an offset a lane it cost a
+// register, which went to scratch memory in the loop, 2,840 beside 2,877 apart.)
+template <int BM, int BN, int WM, int WN, bool CUT, bool GLU>
 __global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64)
 gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const float* __restrict__ W,
                      const float* __restrict__ bias, int M, int N, int K, int lda, int ldw, int ldc, float alpha,
-                     int m_tiles, int n_tiles, int vec_store, float* __restrict__ ws, const FtCut cut) {
+                     int m_tiles, int n_tiles, int vec_store, float* __restrict__ ws, const FtCut cut, int act) {
     constexpr int NW = (BM / WM) * (BN / WN), NT = NW * 64, ROWS = BM + BN;
     constexpr int LOADS = ROWS * 8 / NT, W_LOADS = BN * 8 / NT, TM = WM / 16, TN = WN / 16;
     static_assert(ROWS * 8 % NT == 0 && BN * 8 % NT == 0, "whole loads");
@@ -63,7 +68,10 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
     const int lrow = tid >> 3, lk4 = tid & 7;
     // (in 16 bytes: a row of the tile, the tile's last row inside the matrix; rows beyond are that one again)
     const uint32_t w4 = ldw >> 2, x4 = lda >> 2;
-    uint32_t wfrom = lrow * w4, xfrom = lrow * x4;
+    // (GLU: a wave's rows are all of gate or all of up; NT / 8 rows of the tile on are NT / 16 rows on of the same)
+    const int up = GLU ? wave >> 1 & 1 : 0;
+    const uint32_t w_each = (GLU ? NT / 16 : NT / 8) * w4;
+    uint32_t wfrom = (GLU ? (lrow >> 5) * 16 + (lrow & 15) : lrow) * w4, xfrom = lrow * x4;
     const int put = (lrow >> 4) * 384 + f3_slot(lrow & 15, lk4 & 3) * 2 + (lk4 >> 2);   // in 8 bytes
     const int get = f3_slot(r, q);
     float4 reg[LOADS];
@@ -74,15 +82,15 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
     const int st0 = slice0 * per, st1 = CUT ? min((part + 1) * cut.slices / cut.parts * per, stages) : stages;
     int mt, nt;
     ft_place(tile, m_tiles, n_tiles, mt, nt);
-    const int n0 = nt * BN, m0 = mt * BM;
-    const float4* wsrc = reinterpret_cast<const float4*>(W + (size_t)n0 * ldw);
+    const int n0 = nt * (GLU ? BN / 2 : BN), m0 = mt * BM;
+    const float4* wsrc = reinterpret_cast<const float4*>(W + (size_t)(n0 + up * N) * ldw);
     const float4* xsrc = reinterpret_cast<const float4*>(X + (size_t)m0 * lda);
-    const uint32_t wlast = (uint32_t)min(N - 1 - n0, BN - 1) * w4, xlast = (uint32_t)min(M - 1 - m0, BM - 1) * x4;
+    const uint32_t wlast = (uint32_t)min(N - 1 - n0, (GLU ? BN / 2 : BN) - 1) * w4, xlast = (uint32_t)min(M - 1 - m0, BM - 1) * x4;
     auto fetch = [&](int st) {
         const int k4 = st * 8 + lk4, k4c = k4 < k4_last ? k4 : k4_last;
         asm volatile("" : "+v"(wfrom), "+v"(xfrom));   // the rows' offsets are made here each time: outside the loop they would take LOADS registers
 #pragma unroll
-        for (int i = 0; i < W_LOADS; ++i) reg[i] = wsrc[min(wfrom + i * (NT / 8) * w4, wlast) + (uint32_t)k4c];
+        for (int i = 0; i < W_LOADS; ++i) reg[i] = wsrc[min(wfrom + i * w_each, wlast) + (uint32_t)k4c];
 #pragma unroll
         for (int i = W_LOADS; i < LOADS; ++i) reg[i] = xsrc[min(xfrom + (i - W_LOADS) * (NT / 8) * x4, xlast) + (uint32_t)k4c];
     };
@@ -169,6 +177,65 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
     }
     unsigned long long open = 0;   // outputs to be computed again: bit (g * TN + t) * 4 + e
     static_assert(TM * TN * 4 <= 64, "a bit an output");
+    if constexpr (GLU) {
+        // acc[2 p][g][e] and acc[2 p + 1][g][e] of lane (r, q): gate and up of row m0 + 16 (wm's group + g) + r, output n0 + 16 (wn / 2 + p) + 4 q + e.
+        // Where one of the two is to be computed again the other waits in its place in C; where both are, their product as it is (a NaN stays)
+        auto biased = [&](float v, int n) { return bias != nullptr ? v + bias[n] : v; };
+#pragma unroll
+        for (int g = 0; g < TM; ++g) {
+            const int m = m0 + (wm - BN / 16 + g) * 16 + r;
+            if (m >= M) continue;
+#pragma unroll
+            for (int t = 0; t < TN; t += 2) {
+                const int n = n0 + (wn + t) * 8 + 4 * q;
+                if (n >= N) continue;
+                const f32x4 vg = total[t][g] + acc[t][g], vu = total[t + 1][g] + acc[t + 1][g];
+                float o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (n + e >= N) continue;
+                    const bool og = f3_unsaid(vg[e]), ou = f3_unsaid(vu[e]);
+                    if (og) open |= 1ull << ((g * TN + t) * 4 + e);
+                    if (ou) open |= 1ull << ((g * TN + t + 1) * 4 + e);
+                    const float gate = biased(vg[e], n + e), u = biased(vu[e], N + n + e);
+                    o[e] = og && !ou ? u : (ou && !og ? gate : glu_act(gate, act) * u);
+                }
+                float* dst = C + (size_t)m * ldc + n;
+                if (vec_store && n + 3 < N) {
+                    *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e < N) dst[e] = o[e];
+                }
+            }
+        }
+        for (unsigned long long lanes; (lanes = __builtin_amdgcn_ballot_w64(open != 0ull)) != 0ull;) {
+            const int owner = __builtin_ctzll(lanes);
+            const bool mine = lane == owner;
+            const int bit = __builtin_amdgcn_readlane(open != 0ull ? __builtin_ctzll(open) : 0, owner), g = bit / (4 * TN);
+            const int first = bit - ((bit >> 2) & 1) * 4;   // the gate's bit; up's is four on
+            const int which = __builtin_amdgcn_readlane((int)(open >> first & 0x11ull), owner);
+            const int m = m0 + (wm - BN / 16 + g) * 16 + (owner & 15);
+            const int n = n0 + (wn + first / 4 % TN) * 8 + 4 * (owner >> 4) + (first & 3);
+            const float* x = X + (size_t)m * lda;
+            if (f3_has_nan(x, K)) {   // (NaNs are there already, all along the row)
+                if (mine) open &= ~(((1ull << (4 * TN)) - 1) << (4 * TN * g));
+                continue;
+            }
+            float gate = 0.f, u = 0.f;
+            if (which & 1) gate = biased(f3_dot(x, W + (size_t)n * ldw, K), n);
+            if (which & 16) u = biased(f3_dot(x, W + (size_t)(N + n) * ldw, K), N + n);
+            if (mine) {
+                float* dst = C + (size_t)m * ldc + n;
+                if (which == 1) u = *dst;
+                if (which == 16) gate = *dst;
+                *dst = glu_act(gate, act) * u;
+                open &= ~(0x11ull << first);
+            }
+        }
+        return;
+    }
     // acc[t][g][e] of lane (r, q): output row m0 + 16 (wm's group + g) + r, column n0 + 16 (wn + t) + 4 q + e
 #pragma unroll
     for (int g = 0; g < TM; ++g) {
@@ -218,34 +285,46 @@ gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ X, const f
     }
 }
 
-// Cut tiles: the slices' sums in ascending order.  A thread takes the four outputs that a lane of the tile's workgroup held together.
-template <int BM, int BN, int WM, int WN>
+// Cut tiles: the slices' sums in ascending order.  A thread takes the four outputs that a lane of the tile's workgroup held together (GLU: those
+// of gate and of up).
+template <int BM, int BN, int WM, int WN, bool GLU>
 __global__ void __launch_bounds__(256)
 gemm_f32_sum_kernel(float* __restrict__ C, const float* __restrict__ ws, const float* __restrict__ X, const float* __restrict__ W,
                     const float* __restrict__ bias, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int m_tiles, int n_tiles,
-                    int vec_store, const FtCut cut) {
-    constexpr int TM = WM / 16, TN = WN / 16, EACH = BM * BN / 4;   // threads a tile
-    const int tile = cut.first + blockIdx.x / (EACH / 256);
-    const int i = blockIdx.x % (EACH / 256) * 256 + threadIdx.x, lane = i & 63, r = lane & 15, q = lane >> 4;
-    const int g = i / 64 % TM, t = i / (64 * TM) % TN, wave = i / (64 * TM * TN);
-    const f32x4* from = reinterpret_cast<const f32x4*>(ws) + (size_t)(tile - cut.first) * cut.slices * EACH + i;
-    f32x4 s[F3_SLICES];
+                    int vec_store, const FtCut cut, int act) {
+    constexpr int TM = WM / 16, TN = WN / 16, OF = GLU ? 2 : 1, EACH = BM * BN / 4, THREADS = EACH / OF;   // threads a tile
+    const int tile = cut.first + blockIdx.x / (THREADS / 256);
+    const int i = blockIdx.x % (THREADS / 256) * 256 + threadIdx.x, lane = i & 63, r = lane & 15, q = lane >> 4;
+    const int g = i / 64 % TM, t = i / (64 * TM) % (TN / OF), wave = i / (64 * TM * (TN / OF));
+    const f32x4* from = reinterpret_cast<const f32x4*>(ws) + (size_t)(tile - cut.first) * cut.slices * EACH + ((wave * TN + t * OF) * TM + g) * 64 + lane;
+    f32x4 s[OF][F3_SLICES], v[OF];
 #pragma unroll
-    for (int k = 0; k < F3_SLICES; ++k) s[k] = from[(size_t)(k < cut.slices ? k : 0) * EACH];
-    f32x4 v = s[0];
+    for (int h = 0; h < OF; ++h)
 #pragma unroll
-    for (int k = 1; k < F3_SLICES; ++k)
-        if (k < cut.slices) v += s[k];
+        for (int k = 0; k < F3_SLICES; ++k) s[h][k] = from[(size_t)(k < cut.slices ? k : 0) * EACH + h * TM * 64];
+#pragma unroll
+    for (int h = 0; h < OF; ++h) {
+        v[h] = s[h][0];
+#pragma unroll
+        for (int k = 1; k < F3_SLICES; ++k)
+            if (k < cut.slices) v[h] += s[h][k];
+    }
     int mt, nt;
     ft_place(tile, m_tiles, n_tiles, mt, nt);
-    const int m = mt * BM + (wave / (BN / WN) * TM + g) * 16 + r, n = nt * BN + (wave % (BN / WN) * TN + t) * 16 + 4 * q;
+    const int m = mt * BM + (wave / (BN / WN) * TM + g) * 16 + r, n = nt * (BN / OF) + (wave % (BN / WN) * (TN / OF) + t) * 16 + 4 * q;
     float o[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const bool live = m < M && n + e < N;
-        float x = f3_settle(v[e], live, X, W, m, n + e, K, lda, ldw);
+        float x = f3_settle(v[0][e], live, X, W, m, n + e, K, lda, ldw);
         if (bias != nullptr && live) x += bias[n + e];
-        o[e] = alpha * x;
+        if (GLU) {
+            float u = f3_settle(v[OF - 1][e], live, X, W, m, N + n + e, K, lda, ldw);
+            if (bias != nullptr && live) u += bias[N + n + e];
+            o[e] = glu_act(x, act) * u;
+        } else {
+            o[e] = alpha * x;
+        }
     }
     if (m >= M || n >= N) return;
     float* dst = C + (size_t)m * ldc + n;
@@ -299,11 +378,11 @@ static int ft_check(const char* name, const void* X, const void* W, int M, int N
     return 0;
 }
 #define FT_ARGS (float*)C, (const float*)X, (const float*)W, (const float*)bias, M, N, K, lda, ldw, ldc, alpha
-#define FT_RUN(BM_, BN_, WM_, WN_, CUT_, BLOCKS_)                                                                       \
+#define FT_RUN(BM_, BN_, WM_, WN_, CUT_, GLU_, BLOCKS_)                                                                       \
     {                                                                                                                   \
-        const int m_tiles = (M + BM_ - 1) / BM_, n_tiles = (N + BN_ - 1) / BN_;                                         \
-        gemm_f32_tile_kernel<BM_, BN_, WM_, WN_, CUT_><<<BLOCKS_, (BM_ / WM_) * (BN_ / WN_) * 64, 0, stream>>>(         \
-            FT_ARGS, m_tiles, n_tiles, vec_store, (float*)ws, cut);                                                     \
+        const int m_tiles = (M + BM_ - 1) / BM_, n_tiles = ((GLU_ ? 2 : 1) * N + BN_ - 1) / BN_;                         \
+        gemm_f32_tile_kernel<BM_, BN_, WM_, WN_, CUT_, GLU_><<<BLOCKS_, (BM_ / WM_) * (BN_ / WN_) * 64, 0, stream>>>(   \
+            FT_ARGS, m_tiles, n_tiles, vec_store, (float*)ws, cut, act);                                                \
         ILM_LAUNCH_CHECK("gemm_f32_tile");                                                                              \
     }
 
@@ -316,10 +395,11 @@ extern "C" int ilm_gemm_f32_tile(void* C, const void* X, const void* W, const vo
     int parts;
     void* ws = nullptr;
     const FtCut cut = {};
+    const int act = 0;
     if (tile == 0) tile = ft_form(M, N, K, 1, &parts);   // (of the whole forms)
-    if (tile == 1) FT_RUN(128, 256, 64, 64, false, m_tiles * n_tiles)
-    else if (tile == 2) FT_RUN(128, 128, 64, 32, false, m_tiles * n_tiles)
-    else FT_RUN(64, 64, 32, 32, false, m_tiles * n_tiles)
+    if (tile == 1) FT_RUN(128, 256, 64, 64, false, false, m_tiles * n_tiles)
+    else if (tile == 2) FT_RUN(128, 128, 64, 32, false, false, m_tiles * n_tiles)
+    else FT_RUN(64, 64, 32, 32, false, false, m_tiles * n_tiles)
     return 0;
 }
 
@@ -330,26 +410,54 @@ extern "C" long ilm_gemm_f32_cut_ws(int M, int N, int K) {
     return (long)ft_rest(M, N) * ft_slices(K) * 128 * 256;
 }
 
-// The same product with the tiles beyond whole rounds cut into their slices of K.  ws: ws_floats floats, at least as many as slices of such tiles hold.
-// `parts`: workgroups a tile, 0 the rule's.
-extern "C" int ilm_gemm_f32_cut(void* C, const void* X, const void* W, const void* bias, int M, int N, int K, int lda, int ldw, int ldc,
-                                float alpha, int parts, void* ws, long ws_floats, hipStream_t stream) {
-    if (ft_check("gemm_f32_cut", X, W, M, N, K, lda, ldw, ldc) != 0) return -1;
-    const int slices = ft_slices(K), rest = ft_rest(M, N), m_tiles = (M + 127) / 128, n_tiles = (N + 255) / 256;
+template <bool GLU>
+static int ft_cut(void* C, const void* X, const void* W, const void* bias, int M, int N, int K, int lda, int ldw, int ldc, float alpha, int act,
+                  int parts, void* ws, long ws_floats, hipStream_t stream) {
+    const int rows = GLU ? 2 * N : N, slices = ft_slices(K), rest = ft_rest(M, rows), m_tiles = (M + 127) / 128, n_tiles = (rows + 255) / 256;
     int rule = slices;
-    ft_form(M, N, K, slices, &rule);
+    ft_form(M, rows, K, slices, &rule);
     if (parts == 0) parts = rule;
     ILM_REQUIRE(parts >= 1 && parts <= slices, "gemm_f32_cut: %d workgroups for %d slices", parts, slices);
     ILM_REQUIRE(rest > 0 && ws != nullptr && ((uintptr_t)ws & 15) == 0 && ws_floats >= (long)rest * slices * 128 * 256,
                 "gemm_f32_cut: %d tiles of %d slices, a workspace of %ld floats", rest, slices, ws_floats);
     const int vec_store = (ldc % 4 == 0 && ((uintptr_t)C & 15) == 0) ? 1 : 0;
     const FtCut cut = {m_tiles * n_tiles - rest, slices, parts};
-    if (cut.first > 0) FT_RUN(128, 256, 64, 64, false, cut.first)
-    FT_RUN(128, 256, 64, 64, true, rest * parts)
-    gemm_f32_sum_kernel<128, 256, 64, 64><<<rest * (128 * 256 / 1024), 256, 0, stream>>>(
+    if (cut.first > 0) FT_RUN(128, 256, 64, 64, false, GLU, cut.first)
+    FT_RUN(128, 256, 64, 64, true, GLU, rest * parts)
+    gemm_f32_sum_kernel<128, 256, 64, 64, GLU><<<rest * (128 * 256 / 1024) / (GLU ? 2 : 1), 256, 0, stream>>>(
         (float*)C, (const float*)ws, (const float*)X, (const float*)W, (const float*)bias, M, N, K, lda, ldw, ldc, alpha, m_tiles, n_tiles, vec_store,
-        cut);
+        cut, act);
     ILM_LAUNCH_CHECK("gemm_f32_sum");
+    return 0;
+}
+
+// The same product with the tiles beyond whole rounds cut into their slices of K.  ws: ws_floats floats, at least as many as slices of such tiles hold.
+// `parts`: workgroups a tile, 0 the rule's.
+extern "C" int ilm_gemm_f32_cut(void* C, const void* X, const void* W, const void* bias, int M, int N, int K, int lda, int ldw, int ldc,
+                                float alpha, int parts, void* ws, long ws_floats, hipStream_t stream) {
+    if (ft_check("gemm_f32_cut", X, W, M, N, K, lda, ldw, ldc) != 0) return -1;
+    return ft_cut<false>(C, X, W, bias, M, N, K, lda, ldw, ldc, alpha, 0, parts, ws, ws_floats, stream);
+}
+
+// act(X Wg^T + bg) * (X Wu^T + bu), W = [Wg; Wu] with I rows each, in tiles of 128 rows and 128 outputs.  Whether these are the rule's for the product
+// alone (the smaller ones keep the activation apart), and that product's workspace
+extern "C" int ilm_gemm_f32_glu_tile_ok(int M, int I, int K) {
+    int parts;
+    if (M <= 0 || I <= 0 || K <= 0 || I >= 1 << 30) return 0;
+    const int form = ft_form(M, 2 * I, K, ft_slices(K), &parts);
+    return form == 1 || form == 4 ? 1 : 0;
+}
+// ws: null, or ilm_gemm_f32_cut_ws(M, 2 I, K) floats: with cut tiles
+extern "C" int ilm_gemm_f32_glu_tile(void* C, const void* X, const void* W, const void* bias, int M, int I, int K, int lda, int ldw, int ldc, int act,
+                                     void* ws, long ws_floats, hipStream_t stream) {
+    if (ft_check("gemm_f32_glu_tile", X, W, M, I, K, lda, ldw, ldc) != 0) return -1;
+    ILM_REQUIRE(I < 1 << 30, "gemm_f32_glu_tile: %d outputs", I);
+    const int N = I;
+    const float alpha = 1.f;
+    if (ws != nullptr) return ft_cut<true>(C, X, W, bias, M, N, K, lda, ldw, ldc, alpha, act, 0, ws, ws_floats, stream);
+    const int vec_store = (ldc % 4 == 0 && ((uintptr_t)C & 15) == 0) ? 1 : 0;
+    const FtCut cut = {};
+    FT_RUN(128, 256, 64, 64, false, true, m_tiles * n_tiles)
     return 0;
 }
 #undef FT_RUN

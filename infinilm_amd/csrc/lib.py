@@ -45,6 +45,7 @@ _SIGNATURES = {
     "ilm_gemm_f32_rope": [_P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "ilm_gemm_f32_tile": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "ilm_gemm_f32_cut": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _L, _P],
+    "ilm_gemm_f32_glu_tile": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _L, _P],
     "ilm_gemm_portion": [_P, _I, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _P],
     "ilm_gemm_portion_rope": [_P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "ilm_attn_f32": [_P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _F, _P],
@@ -154,6 +155,8 @@ def load(verbose: bool = True) -> ctypes.CDLL:
     lib.ilm_delta_chunk_ws.argtypes = [c_int, c_int]
     lib.ilm_gemm_f32_cut_ws.restype = c_long
     lib.ilm_gemm_f32_cut_ws.argtypes = [c_int, c_int, c_int]
+    lib.ilm_gemm_f32_glu_tile_ok.restype = c_int
+    lib.ilm_gemm_f32_glu_tile_ok.argtypes = [c_int, c_int, c_int]
     lib.ilm_sample_ws.restype = c_long
     lib.ilm_sample_ws.argtypes = [c_int, c_int]
     lib.ilm_moe_plan_few_ok.restype = c_int

@@ -479,8 +479,13 @@ def _few_span(M: int, N: int, K: int) -> int:
 
 def _f32_few_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the 32-bit products of few rows take these operands (`gemm` goes to the same kernels then)."""
+    return x.shape[0] <= F32_FEW_ROWS and _f32_pieces_ok(x, w)
+
+
+def _f32_pieces_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the 32-bit products in three pieces a float take these operands, few rows or many."""
     K = x.shape[1]
-    return (x.dtype == F32 and w.dtype == F32 and not FORCE_BASIC and x.shape[0] <= F32_FEW_ROWS and K % 4 == 0 and x.stride(1) == 1
+    return (x.dtype == F32 and w.dtype == F32 and not FORCE_BASIC and F32_FEW_ROWS > 0 and K % 4 == 0 and x.stride(1) == 1
             and w.stride(1) == 1 and x.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and max(x.stride(0), w.stride(0)) < 1 << 24)
 
@@ -826,14 +831,23 @@ def gateup_swiglu_gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Te
 
 
 def gateup_glu_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], act: str = "silu") -> Optional[torch.Tensor]:
-    """The same in float32, up to 64 rows: bit for bit the projection and the activation kernel one after the other."""
-    if not (USE_GATEUP_SWIGLU and _f32_few_rows(x, w) and w.shape[0] % 2 == 0 and w.shape[1] == x.shape[1]):
+    """The same in float32, up to 64 rows and where tiles of 128 rows and 128 outputs are the projection's best: bit for bit the projection and the
+    activation kernel one after the other."""
+    M, I, K = x.shape[0], w.shape[0] // 2, x.shape[1]
+    if not (USE_GATEUP_SWIGLU and _f32_pieces_ok(x, w) and w.shape[0] % 2 == 0 and w.shape[1] == K):
+        return None
+    if M > F32_FEW_ROWS and not (I > 0 and _lib().ilm_gemm_f32_glu_tile_ok(M, I, K)):
         return None
     _dev(x, w, bias)
-    M, I = x.shape[0], w.shape[0] // 2
     if bias is not None and (bias.shape != (2 * I,) or bias.dtype != F32 or not bias.is_contiguous()):
         raise KernelError("bias does not fit the fused gate/up projection")
     out = torch.empty((M, I), dtype=F32, device=x.device)
+    if M > F32_FEW_ROWS:
+        need = _lib().ilm_gemm_f32_cut_ws(M, 2 * I, K)
+        ws = torch.empty((need,), dtype=F32, device=x.device) if need else None
+        _run("ilm_gemm_f32_glu_tile", out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias), M, I, K, x.stride(0), w.stride(0), out.stride(0),
+             glu_code(act), _ptr(ws), need, _stream())
+        return out
     _run("ilm_gemm_f32_glu", out.data_ptr(), x.data_ptr(), w.data_ptr(), _ptr(bias), M, I, x.shape[1], x.stride(0), w.stride(0),
          out.stride(0), glu_code(act), _stream())
     return out

@@ -42,7 +42,7 @@ class SwiGLU(FeedForward):
                                              act=self.activation)
             return self.down.forward(act, allow_parts=not self.whole_output)
         frag = (lambda: self.gate_up.frag_weight("gate_up8")) if kernels.frag_weight_ok(self.gate_up.weight) else None
-        if x.dtype == torch.float32:   # few rows: activation in the epilogue
+        if x.dtype == torch.float32:   # the activation in the epilogue, where the rows and outputs suit
             act = kernels.gateup_glu_f32(x, self.gate_up.weight, self.gate_up.bias, act=self.activation)
         else:
             act = kernels.gateup_swiglu_gemm(x, self.gate_up.weight, self.gate_up.bias, frag_w=frag, act=self.activation)

@@ -1514,3 +1514,40 @@ def test_portion_gate_and_up_beyond_two_tiles_a_unit(K, M, N, K_):
     assert -(-M // 64) * -(-N // 64) > 2 * K._num_cus(torch.device(DEV)) or N == 2048
     got = K.portion_glu(x, w, None, "silu", 1)
     assert torch.equal(got, K.swiglu(K.portion_gemm(x, w, None, torch.empty((M, 2 * N), dtype=BF16, device=DEV), 1), "silu"))
+
+
+@pytest.mark.parametrize("M,I,K_,act", [(65, 31, 36, "silu"), (127, 128, 260, "gelu_tanh"), (129, 515, 132, "silu"), (300, 257, 1028, "silu"), (1100, 4101, 132, "gelu_tanh")])
+@pytest.mark.parametrize("odd", [False, True])
+def test_gemm_float32_tiles_with_the_activation_in_their_epilogue(K, M, I, K_, act, odd):
+    """Bit for bit the projection and the activation kernel one after the other, in whole tiles and in cut ones, with sums that the pieces cannot give in
+    the gate, in up and in both, and a bias; and where the rule takes them."""
+    from infinilm_amd.csrc import lib
+    L = lib.load()
+    g = torch.Generator().manual_seed(M + I + odd)
+    x, w, b = torch.randn((M, K_), generator=g), torch.randn((2 * I, K_), generator=g) * 0.2, torch.randn((2 * I,), generator=g)
+    if odd:
+        x[M // 3, 3], x[M // 2, K_ - 1], x[M - 1] = math.inf, math.nan, x[M - 1] * 2.0 ** -80
+        w[5, 7], w[I + 9, 8], w[I - 1, 9], w[2 * I - 1, 9] = math.inf, -math.inf, math.inf, -math.inf
+        w[I // 2, :2], w[I, :2], x[0, :2] = torch.tensor([3e38, -3e38]), torch.tensor([3e38, -3e38]), torch.tensor([3.0, 3.0])
+    x, w, b = x.to(DEV), w.to(DEV), b.to(DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    for bias in (None, b):
+        want = K.swiglu(K.gemm(x, w, bias), act)
+        assert not odd or not torch.isfinite(want).all()
+        ws = torch.empty(((-(-M // 128)) * (-(-I // 128)) * 8 * 128 * 256,), device=DEV)
+        for cut in (False, True):
+            got = torch.full((M, I), 7.0, device=DEV)
+            assert L.ilm_gemm_f32_glu_tile(got.data_ptr(), x.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(), M, I, K_, K_, K_, I,
+                                           K.glu_code(act), ws.data_ptr() if cut else None, ws.numel() if cut else 0, stream) == 0
+            _same(got, want)
+        ruled = K.gateup_glu_f32(x, w, bias, act)
+        assert (ruled is None) == (not L.ilm_gemm_f32_glu_tile_ok(M, I, K_))
+        if ruled is not None:
+            _same(ruled, want)
+
+
+def test_gemm_float32_tiles_with_the_activation_are_taken_for_large_projections(K):
+    """A whole number of rounds over the chip, and one that leaves tiles to be cut."""
+    for M, K_ in ((512, 256), (700, 4096)):
+        x, w = _rand((M, K_), 1).to(DEV), _rand((2 * 8192, K_), 2, scale=0.1).to(DEV)
+        _same(K.gateup_glu_f32(x, w, None), K.swiglu(K.gemm(x, w)))
