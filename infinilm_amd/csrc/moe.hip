@@ -33,6 +33,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 #define MOE_TN 64
 #define MOE_KS 64
 #define MOE_FEW_K 4096   // longest rows of the few-rows kernel: 16 k-steps of 32 for each of 8 waves
+#define MOE_FEW_RING 2   // pieces that a wave of it may be ahead of the next
 #define MOE_LD (MOE_KS + 8)   // bf16 elements a row of a tile in LDS (144 bytes)
 
 __device__ __forceinline__ float moe_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
@@ -504,23 +505,28 @@ moe_gemm_mfma_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict_
 }
 
 
-// bfloat16 on the matrix cores, few rows an expert (decoded tokens): bound by reading the experts' matrices once.  Block: 8 waves that split K; a
-// workgroup keeps a tile's rows (16 MG at a time) of its wave's K in registers and walks tiles of 16 rows of W (GLU: of gate and up), the
-// next one's loads in flight while the waves' sums meet in LDS, in wave order.  No barrier between loads, where the kernel above has two
-// every 64 k.  
-// us, with the kernel above and now, 2 of 14 experts a token: gate/up 2048 x 2048 1 token 23.8 / 9.6, 4 33.1 / 27.2, 16 49.8 / 44.4 (4.5 TB/s), 32 56.9 /
-// 51.5; down 19.7 / 6.0, 24.5 / 13.9, 31.3 / 23.2, 32.5 / 26.9; 16 of 2 of 16 experts 4096 x 4096 207 / 186 and 112 / 96.  Not below K 1024 (512: 26.6 /
-// 33.4), where the waves' sums meet more often than they multiply.  One workgroup a unit where a wave's part of K takes more than 128 registers.
+// bfloat16 on the matrix cores, few rows an expert (decoded tokens): bound by reading the experts' matrices once.  Block: 8 waves, of an eighth of K
+// each; a workgroup keeps a tile's rows (16 MG at a time) of its wave's K in registers and walks tiles of 16 rows of W (GLU: of gate and up).
+// An output's sum is one chain over K in steps of 32, the kernel above's, so a token has the same bits in a step of few tokens and in one of many:
+// a wave goes on with the sums of the wave before it, which hands them over in LDS (no barrier: a count of finished pieces a wave), and asks for its
+// part of the next piece meanwhile.
+// us, with the kernel above and with this one, 2 of 14 experts a token: gate/up 2048 x 2048 1 token 25.6 / 14.1, 4 34.3 / 30.5, 16 53.3 / 49.8, 32 53.4 / 52.0;
+// down 21.1 / 9.0, 22.5 / 14.7, 31.3 / 25.5, 31.4 / 26.9; 8 of 64 experts of 1408 x 2048 and 16 tokens 142 / 114 and 78 / 60.  The experts share the workgroups
+// out evenly, their tiles of W only in whole turns: 12 experts 21 workgroups each, 7 turns for 128 tiles where 6.1 would do.  Not below K 1024, where the waves
+// hand on more often than they multiply (at 1,024 32 tokens are there already: 16.9 / 17.9; 1 14.7 / 8.6).  One workgroup a unit where a wave's part of K takes more
+// than 128 registers.  Gate and up rows longer than 2,048 leave no registers for a second piece in flight: only up to two tokens (4096 x 4096, 2 of 16 experts, 2
+// tokens 61 / 50, 4 89 / 96, 16 207 / 206; 2304 x 2304 2 34.7 / 26.4, 8 49.9 / 54.6).
 template <bool GLU, int KSTEPS, int MG>
 __global__ void __launch_bounds__(512, KSTEPS * MG <= 4 ? 4 : 2)
 moe_gemm_few_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict__ X, int ldx, const int* __restrict__ perm, int top,
                     const float* __restrict__ pair_w, const bf16* __restrict__ W, size_t w_expert, int ldw, const int* __restrict__ tiles,
                     const int* __restrict__ n_tiles, int N, int K, float limit, float alpha, int act, int ks) {
     // D pieces of W (16 rows' part of a wave) in flight beside the one that is multiplied: gate and up rows where registers allow and both are
-    // long (45.2 -> 44.4 us; plain tiles in twos 23.2 -> 23.6).  EACH: pieces an output tile
-    constexpr int D = GLU && KSTEPS == 8 ? 2 : 1, EACH = GLU ? 2 : 1;
-    __shared__ float part[2][MG][8][64][4];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    // long.  EACH: pieces an output tile
+    constexpr int D = GLU && KSTEPS >= 6 && KSTEPS <= 8 ? 2 : 1, EACH = GLU ? 2 : 1;
+    __shared__ f32x4 pass[7][MOE_FEW_RING][MG][64];   // [wave that hands on][piece][rows][lane]
+    __shared__ int done[8];                           // pieces that a wave is through with
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
     const int nt_all = (N + 15) / 16, et_all = *n_tiles;
     if (et_all <= 0) return;
     const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
@@ -537,9 +543,15 @@ moe_gemm_few_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict__
     // the workgroups of an expert tile share its tiles of W (more expert tiles than workgroups: each takes several)
     const int sharers = (int)gridDim.x > et_all ? (int)gridDim.x / et_all : 1, share = blockIdx.x / et_all;
     if (share >= sharers || share >= nt_all) return;
-    const int et = threadIdx.x < 256 * MG ? threadIdx.x : 0, eg = et >> 8, e = et & 3, l = (et & 255) >> 2;
-    const int m = eg * 16 + (l & 15);
-    int buf = 0;
+    if (threadIdx.x < 8) done[threadIdx.x] = 0;
+    __syncthreads();
+    // until wave w is through with n pieces (a wave's LDS accesses stay in their order, so what it wrote before its count is there).  It always comes:
+    // a wave waits for the one before it to finish the piece that it wants, and for the one behind it to finish a piece that lies RING pieces back
+    auto wait_for = [&](int w, int n) {
+        while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(&done[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < n) __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");
+    };
+    int piece = 0;
 #pragma unroll 1
     for (int tile = blockIdx.x % et_all; tile < et_all; tile += gridDim.x) {
         const int place0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
@@ -579,18 +591,18 @@ moe_gemm_few_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict__
             if (D == 2) load(a[D - 1], share, 1);
 #pragma unroll 1
             for (int nt = share; nt < nt_all; nt += sharers) {
-                const int n = nt * 16 + (l >> 4) * 4 + e;
-                float gate = 0.f;
+                f32x4 gate[MG];
 #pragma unroll
                 for (int v = 0; v < EACH; ++v) {
                     f32x4 acc[MG];
-#pragma unroll
-                    for (int g = 0; g < MG; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
                     if (ragged) {
 #pragma unroll
                         for (int u = 0; u < KSTEPS; ++u)
                             if (!kok[u]) a[v % D][u] = zero;
                     }
+                    if (wave > 0) wait_for(wave - 1, piece + 1);
+#pragma unroll
+                    for (int g = 0; g < MG; ++g) acc[g] = wave > 0 ? pass[wave > 0 ? wave - 1 : 0][piece % MOE_FEW_RING][g][lane] : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int u = 0; u < KSTEPS; ++u)
 #pragma unroll
@@ -602,21 +614,31 @@ moe_gemm_few_kernel(bf16* __restrict__ out, int ld_out, const bf16* __restrict__
                     const int next = v + D < EACH ? nt : nt + sharers;
                     if (next < nt_all) load(a[v % D], next, (v + D) % EACH);
                     __builtin_amdgcn_sched_barrier(0);
+                    if (wave < 7) {
+                        wait_for(wave + 1, piece + 1 - MOE_FEW_RING);
 #pragma unroll
-                    for (int g = 0; g < MG; ++g) *reinterpret_cast<f32x4*>(&part[buf][g][wave][lane][0]) = acc[g];
-                    __syncthreads();
-                    float s = 0.f;
-#pragma unroll
-                    for (int w = 0; w < 8; ++w) s += part[buf][eg][w][l][e];
-                    buf ^= 1;   // (the other buffer's readers passed this barrier)
-                    if (GLU && v == 0) {
-                        gate = s;
-                        continue;
+                        for (int g = 0; g < MG; ++g) pass[wave < 7 ? wave : 0][piece % MOE_FEW_RING][g][lane] = acc[g];
                     }
-                    if (threadIdx.x < 256 * MG && n < N && row0 + m < rows) {
-                        if (GLU) s = moe_glu(gate, s, limit, alpha, act);
-                        else if (act == MOE_ACT_RELU2) { s = fmaxf(s, 0.f); s *= s; }
-                        out[(size_t)(place0 + row0 + m) * ld_out + n] = from_f32<bf16>(s);
+                    asm volatile("" ::: "memory");
+                    ++piece;
+                    if (lane == 0) __hip_atomic_store(&done[wave], piece, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (wave < 7) continue;
+                    // the last wave.  Lane (r, q): row m = 16 g + r, outputs 16 nt + 4 q + e
+#pragma unroll
+                    for (int g = 0; g < MG; ++g) {
+                        if (GLU && v == 0) gate[g] = acc[g];
+                        const int m = row0 + g * 16 + r;
+                        if (v < EACH - 1 || m >= rows) continue;
+                        bf16* orow = out + (size_t)(place0 + m) * ld_out;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int n = nt * 16 + 4 * q + e;
+                            if (n >= N) continue;
+                            float s = acc[g][e];
+                            if (GLU) s = moe_glu(gate[g][e], s, limit, alpha, act);
+                            else if (act == MOE_ACT_RELU2) { s = fmaxf(s, 0.f); s *= s; }
+                            orow[n] = from_f32<bf16>(s);
+                        }
                     }
                 }
             }
@@ -897,7 +919,8 @@ extern "C" int ilm_moe_gemm(void* out, int ld_out, const void* X, int ldx, const
         else if (glu) moe_gemm_mfma128_kernel<true, 2><<<big, 256, 0, stream>>>(MOE_ARGS(bf16), n_slices);
         else if (wide) moe_gemm_mfma128_kernel<false, 4><<<big, 512, 0, stream>>>(MOE_ARGS(bf16), n_slices);
         else moe_gemm_mfma128_kernel<false, 2><<<big, 256, 0, stream>>>(MOE_ARGS(bf16), n_slices);
-    } else if (dtype == ILM_DTYPE_BF16 && aligned && !force_plain && few_rows > 0 && few_rows <= 32 && K >= 1024 && K <= MOE_FEW_K) {
+    } else if (dtype == ILM_DTYPE_BF16 && aligned && !force_plain && few_rows > 0 && few_rows <= 32 && K >= 1024 && K <= MOE_FEW_K
+               && (!glu || K <= 2048 || few_rows <= 2)) {
         const long items = (long)max_tiles * ((N + 15) / 16);
         const int ks = ((K + 31) / 32 + 7) / 8, most = (ks <= 4 ? 2 : 1) * ilm_num_cus();
         const dim3 few((int)(items < most ? items : most));
@@ -906,11 +929,17 @@ extern "C" int ilm_moe_gemm(void* out, int ld_out, const void* X, int ldx, const
         if (glu) moe_gemm_few_kernel<true, KS_, MG_><<<few, 512, 0, stream>>>(MOE_ARGS(bf16), ks);           \
         else moe_gemm_few_kernel<false, KS_, MG_><<<few, 512, 0, stream>>>(MOE_ARGS(bf16), ks);              \
     }
-        if (few_rows <= 16) {
-            if (ks <= 4) MOE_FEW(4, 1) else if (ks <= 8) MOE_FEW(8, 1) else MOE_FEW(16, 1)
-        } else {
-            if (ks <= 4) MOE_FEW(4, 2) else if (ks <= 8) MOE_FEW(8, 2) else MOE_FEW(16, 2)
-        }
+        // (32 rows of more than 2,048 do not fit the registers: 16 at a time, for which W is read again where an expert has more)
+        if (few_rows > 16 && ks <= 8) {
+            if (ks <= 4) MOE_FEW(4, 2)
+            else if (ks <= 6) MOE_FEW(6, 2)
+            else MOE_FEW(8, 2)
+        } else if (ks <= 4) MOE_FEW(4, 1)
+        else if (ks <= 6) MOE_FEW(6, 1)
+        else if (ks <= 8) MOE_FEW(8, 1)
+        else if (ks <= 10) MOE_FEW(10, 1)
+        else if (ks <= 12) MOE_FEW(12, 1)
+        else MOE_FEW(16, 1)
 #undef MOE_FEW
     } else if (tile_rows != MOE_TM) {
         ILM_REQUIRE(false, "moe_gemm: tiles of %d rows are the bfloat16 matrix-core kernel's alone", tile_rows);

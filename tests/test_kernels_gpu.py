@@ -1462,6 +1462,32 @@ def test_experts_of_few_rows(K, T, E, top, K_, N):
         _close(torch.where(whole, got.to(F64), 0.0), torch.where(whole, want, 0.0), 2.0 ** -8)
 
 
+@pytest.mark.parametrize("T,E,top,K_,N", [(1, 3, 1, 1024, 40), (16, 14, 2, 1536, 33), (16, 5, 2, 2048, 200), (7, 600, 2, 1032, 17), (32, 3, 2, 2056, 48), (32, 14, 2, 1280, 100),
+                                          (32, 2, 2, 4096, 65), (12, 40, 4, 3848, 16)])
+def test_experts_of_few_rows_give_the_bits_of_many(K, monkeypatch, T, E, top, K_, N):
+    """A token's product by its expert in a step of few tokens and in one of more than the few-rows kernel takes, in every form: the same bits."""
+    g = torch.Generator().manual_seed(T + E + K_)
+    z, x = torch.randn((33, E), generator=g), torch.randn((33, K_), generator=g).to(BF16).to(DEV)
+    w = (torch.randn((E, 2 * N, K_), generator=g) / math.sqrt(K_)).to(BF16).to(DEV)
+    wp = w[:, :N].contiguous()
+    assert T <= K.MOE_FEW_TOKENS < 33
+
+    def pairs(tokens):
+        """[tokens, top, outputs] of every form"""
+        plan = K.moe_route(z[:tokens].to(DEV), E, top)
+        place = plan.inv.long()
+        rows = x[plan.perm.long() // top]
+        return [y[place].view(tokens, top, -1) for y in (K.moe_gemm(x[:tokens], w, plan, True, act="silu", weighted=False), K.moe_gemm(x[:tokens], w, plan, True, 0.8),
+                                                         K.moe_gemm(rows, wp, plan, False), K.moe_gemm(x[:tokens], wp, plan, False, gather=True, act="relu2"))]
+
+    few = pairs(T)
+    for a, b in zip(few, pairs(33)):
+        assert torch.equal(a, b[:T])
+    monkeypatch.setattr(K, "MOE_FEW_TOKENS", 0)
+    for a, b in zip(few, pairs(T)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("tile,M,N,K_", [(1, 1100, 1220, 64), (1, 1990, 700, 128), (2, 2041, 1000, 64), (2, 4000, 330, 192), (3, 4000, 1100, 64), (1, 130, 2000, 64)])
 def test_portion_product_walks_its_tiles_in_bands(K, tile, M, N, K_):
     """Products whose tiles are walked in bands of several rows of tiles, the last band lower than the others: every output once.  float sums of products of
