@@ -1044,12 +1044,14 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
             }
         }
     };
-    // Tiles [kb_a, kb_b) are seen whole by every token of the workgroup: from the window's edge of the
-    // last token (the start without a window) to the tile before the first token's own.  Three loops
-    // rather than one with a branch: each keeps its own registers.
-    const int lo_last = first_key(p_last, reach);
+    // Tiles [kb_a, kb_b) are seen whole by every token of the list's tile (PAIR: of the one that the wave's tokens belong to, so that they take the
+    // same path, and have the same bits, whether the tile is paired or not; every wave passes every barrier of the tiles in turn): from the window's
+    // edge of the last token (the start without a window) to the tile before the first token's own.  Three loops rather than one with a
+    // branch: each keeps its own registers.
+    const int own = PAIR ? (wave * NT * CT) & ~(ATT_TT - 1) : 0;
+    const int lo_last = first_key(PAIR ? pos_of(own + ATT_TT - 1) : p_last, reach);
     int kb_a = (lo_last + ATT_TK - 1) & ~(ATT_TK - 1);
-    int kb_b = ((p_first + 1) / ATT_TK) * ATT_TK;
+    int kb_b = (((PAIR ? pos_of(own) : p_first) + 1) / ATT_TK) * ATT_TK;
     if (D % 32 != 0 || kb_b < kb_a) kb_a = kb_b = kb0;
     int kb = kb0;
     for (; kb < kb_a && kb <= p_last; kb += ATT_TK) {

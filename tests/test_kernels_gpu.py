@@ -967,6 +967,28 @@ def test_attention_bfloat16_tiles_of_few_heads(K, monkeypatch, nh, nkv, d, page,
     _close(outs[0], outs[1], 1.2e-2)
 
 
+def _tiles_of(K, nh, nkv, d, page, lists, positions, n, window=0, v=None, seg=None, seed=5):
+    """bfloat16 attention of rows at `positions` of one request of `n` tokens, once for each list of tiles."""
+    k, q = _rand((n, nkv, d), seed, BF16), _rand((len(positions), nh, d), seed + 1, BF16, 2.0)
+    v = _rand((n, nkv, d), seed + 2, BF16) if v is None else v
+    kc, vc, bt = _paged([k], [v], page, -(-n // page) + 2, 4, BF16)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    return [K.paged_attention(q.reshape(-1, nh * d).to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), i32([0] * len(positions)), i32(positions), nh, nkv, d,
+                              d ** -0.5, window, max_total_len=n, tiles=i32(x)).cpu() for x in lists]
+
+
+@pytest.mark.parametrize("nh,nkv,d,page", [(32, 32, 64, 64), (64, 16, 128, 64), (48, 24, 96, 16), (48, 16, 128, 16)])
+@pytest.mark.parametrize("first", [41, 56, 59, 63, 120])
+@pytest.mark.parametrize("window", [0, 100])
+def test_attention_bfloat16_pairs_of_tiles_give_the_bits_of_each(K, nh, nkv, d, page, first, window):
+    """A token's result does not depend on whether its tile goes with the one beside it: where the two see different tiles of keys whole, too."""
+    T = 44
+    each = [[a, min(8, T - a)] for a in range(0, T, 8)]
+    apart = [x for t in each for x in (t, [0, 0])]
+    pairs, alone = _tiles_of(K, nh, nkv, d, page, (each, apart), list(range(first, first + T)), first + T, window)
+    assert torch.equal(pairs, alone)
+
+
 def test_attention_bfloat16_with_a_block_table_beyond_lds(K):
     """33,000 keys in pages of 16: more block-table entries than the tile kernel keeps in LDS, and
     the most chunks the single-token kernel cuts a context into."""
