@@ -541,7 +541,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
     } else {
         const int other = 2 * lead + 1 < n_tiles ? 2 * lead + 1 : 2 * lead;
         const int ta = tiles[4 * lead], na = tiles[4 * lead + 1], tb = tiles[2 * other], nb = other > 2 * lead ? tiles[2 * other + 1] : 0;
-        const bool run = na == ATT_TT && nb > 0 && tb == ta + ATT_TT && seg[tb] == seg[ta];
+        const bool run = na == ATT_TT && nb > 0 && tb == ta + ATT_TT && seg[tb] == seg[ta] && pos[tb] == pos[ta] + ATT_TT;
         t0 = second ? tb : ta;
         ntok = second ? (run ? 0 : nb) : (run ? na + nb : na);
     }

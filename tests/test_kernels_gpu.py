@@ -989,6 +989,13 @@ def test_attention_bfloat16_pairs_of_tiles_give_the_bits_of_each(K, nh, nkv, d, 
     assert torch.equal(pairs, alone)
 
 
+def test_attention_bfloat16_neighbouring_tiles_that_are_no_run(K):
+    """Two tiles of the same request in neighbouring rows whose positions do not follow one another."""
+    positions = list(range(0, 8)) + list(range(100, 108))
+    both, first, second = _tiles_of(K, 2, 1, 64, 64, ([[0, 8], [8, 8]], [[0, 8]], [[8, 8]]), positions, 120)
+    assert torch.equal(both, torch.cat([first[:8], second[8:]]))
+
+
 def test_attention_bfloat16_with_a_block_table_beyond_lds(K):
     """33,000 keys in pages of 16: more block-table entries than the tile kernel keeps in LDS, and
     the most chunks the single-token kernel cuts a context into."""
