@@ -7,6 +7,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 #define FA_CHUNK 128
 #define FA_TILES (FA_CHUNK / 16)
+#define FT_TOKENS 8   // most tokens a tile (attn_f32_tile.hip)
 #define FA_WS_PAD 4   // a partial result is d outputs, its maximum, its sum and two unused floats (16-byte rows)
 
 __device__ __forceinline__ f32x4 fa_mfma(float a, float b, f32x4 c) {
@@ -23,5 +24,7 @@ __device__ __forceinline__ void fa_fold_scales(float& M, float& L, float m, floa
     M = Mn;
 }
 
-// Folds the partial results of tokens 0 .. T - 1 (attn_f32.hip): ws[((t * nh + h) * nchunks + chunk) * (d + FA_WS_PAD)]
-int fa_fold(float* out, const float* ws, const int* pos, int T, int nh, int d, int nchunks, int out_stride, int reach, hipStream_t stream);
+// Folds partial results (attn_f32.hip): ws[((row * nh + h) * nchunks + chunk) * (d + FA_WS_PAD)], rows: eight of each of the n_tiles tiles (first token, count:
+// up to count of them hold something), then n_rows single tokens
+int fa_fold(float* out, const float* ws, const int* pos, const int* tiles, int n_tiles, const int* rows, int first, int n_rows, int nh, int d, int nchunks,
+            int out_stride, int reach, hipStream_t stream);

@@ -20,13 +20,13 @@
 #include "attn_f32.h"
 
 // DT: head size / 16.  !SPLIT: gridDim.z == 1 and the wave walks all chunks; SPLIT: blockIdx.z is the
-// chunk and the partial result goes to ws[((t * nh + h) * gridDim.z + chunk) * (d + FA_WS_PAD)].
-// `rows`: the launch's tokens, -1 for none; null: all.  P16: pages hold whole tiles of 16 keys.
+// chunk and the partial result goes to ws[((blockIdx.x * nh + h) * gridDim.z + chunk) * (d + FA_WS_PAD)].
+// `rows`: the launch's tokens, -1 for none; null: those from `first` on.  P16: pages hold whole tiles of 16 keys.
 template <int DT, bool SPLIT, bool P16>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(DT <= 8 ? 2 : 1)))
 attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __restrict__ qp, const float* __restrict__ kc,
                 const float* __restrict__ vc, const int* __restrict__ block_tables, const int* __restrict__ seg,
-                const int* __restrict__ pos, const int* __restrict__ rows, int nh, int nkv, int nsub, int page, int max_blocks, int q_stride,
+                const int* __restrict__ pos, const int* __restrict__ rows, int first, int nh, int nkv, int nsub, int page, int max_blocks, int q_stride,
                 int out_stride, float scale, int reach, float softcap) {
     constexpr int d = DT * 16;
     // tiles of keys (and of values) in flight: two, or one where the running result of the wave that walks all
@@ -37,7 +37,7 @@ attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __
     // 2 heads of 128 31.3 (36.6).  Four tiles in flight with the values started before the softmax spilled at four waves a
     // SIMD and was slower.
     constexpr int NB = (!SPLIT && DT > 6) ? 1 : 2;
-    const int t = rows != nullptr ? rows[blockIdx.x] : blockIdx.x;
+    const int t = rows != nullptr ? rows[blockIdx.x] : first + (int)blockIdx.x;
     if (t < 0) return;
     const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
     const int G = nh / nkv;
@@ -206,7 +206,7 @@ attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __
         // acc[i][e] of lane (r, q): head r, dim 16 i + 4 q + e
         if (SPLIT) {
             if (r < heads) {
-                float* dst = ws + (((size_t)t * nh + h) * gridDim.z + c) * (d + FA_WS_PAD);
+                float* dst = ws + (((size_t)blockIdx.x * nh + h) * gridDim.z + c) * (d + FA_WS_PAD);
 #pragma unroll
                 for (int i = 0; i < DT; ++i) *reinterpret_cast<f32x4*>(dst + 16 * i + 4 * q) = acc[i];
                 if (q == 0) {
@@ -241,11 +241,20 @@ attn_f32_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __
 // loads of FA_FOLD_AHEAD chunks are in flight together; the fold itself stays one chain in chunk order.
 // A token whose chunks do not all lie inside the workspace (the caller's bound was too small) gets a row of
 // NaNs instead of a silently wrong one.
+// The workspace's rows: eight of every tile, then `rows` or, null, the tokens from `first` on.
 #define FA_FOLD_AHEAD 8
 __global__ void __launch_bounds__(256)
-attn_f32_fold_kernel(float* __restrict__ out, const float* __restrict__ ws, const int* __restrict__ pos, int nh, int d,
-                     int nchunks, int out_stride, int reach) {
-    const int t = blockIdx.x, h = blockIdx.y, dim = threadIdx.x;
+attn_f32_fold_kernel(float* __restrict__ out, const float* __restrict__ ws, const int* __restrict__ pos, const int* __restrict__ tiles, int n_tiles,
+                     const int* __restrict__ rows, int first, int nh, int d, int nchunks, int out_stride, int reach) {
+    const int at = blockIdx.x, single = at - n_tiles * FT_TOKENS, h = blockIdx.y, dim = threadIdx.x;
+    int t;
+    if (single < 0) {
+        if (at % FT_TOKENS >= tiles[2 * (at / FT_TOKENS) + 1]) return;
+        t = tiles[2 * (at / FT_TOKENS)] + at % FT_TOKENS;
+    } else {
+        t = rows != nullptr ? rows[single] : first + single;
+        if (t < 0) return;
+    }
     const int p = pos[t];
     const int lo = first_key(p, reach);
     float* orow = out + (size_t)t * out_stride + (size_t)h * d;
@@ -255,7 +264,7 @@ attn_f32_fold_kernel(float* __restrict__ out, const float* __restrict__ ws, cons
     }
     const int dimc = dim < d ? dim : d - 1;
     const int c_last = p / FA_CHUNK;
-    const float* base = ws + ((size_t)t * nh + h) * nchunks * (d + FA_WS_PAD);
+    const float* base = ws + ((size_t)at * nh + h) * nchunks * (d + FA_WS_PAD);
     float M = -INFINITY, L = 0.f, ACC = 0.f;
     for (int c0 = lo / FA_CHUNK; c0 <= c_last; c0 += FA_FOLD_AHEAD) {
         float mm[FA_FOLD_AHEAD], ll[FA_FOLD_AHEAD], av[FA_FOLD_AHEAD];
@@ -279,8 +288,10 @@ attn_f32_fold_kernel(float* __restrict__ out, const float* __restrict__ ws, cons
     if (dim < d) orow[dim] = ACC * (1.0f / L);
 }
 
-int fa_fold(float* out, const float* ws, const int* pos, int T, int nh, int d, int nchunks, int out_stride, int reach, hipStream_t stream) {
-    attn_f32_fold_kernel<<<dim3(T, nh), 64 * ((d + 63) / 64), 0, stream>>>(out, ws, pos, nh, d, nchunks, out_stride, reach);
+int fa_fold(float* out, const float* ws, const int* pos, const int* tiles, int n_tiles, const int* rows, int first, int n_rows, int nh, int d, int nchunks,
+            int out_stride, int reach, hipStream_t stream) {
+    attn_f32_fold_kernel<<<dim3(n_tiles * FT_TOKENS + n_rows, nh), 64 * ((d + 63) / 64), 0, stream>>>(out, ws, pos, tiles, n_tiles, rows, first, nh, d, nchunks,
+                                                                                                     out_stride, reach);
     ILM_LAUNCH_CHECK("attn_f32_fold");
     return 0;
 }
@@ -288,12 +299,13 @@ int fa_fold(float* out, const float* ws, const int* pos, int T, int nh, int d, i
 extern "C" int ilm_attn_f32_chunk() { return FA_CHUNK; }
 extern "C" int ilm_attn_f32_ws_row(int d) { return d + FA_WS_PAD; }
 
-// rows: the T tokens this call serves (-1: none), null for tokens 0 .. T - 1.  fold: the step's tokens, T without `rows`.
-// ws: null (one wave walks all chunks of its token), or float [fold][nh][nchunks][d + 4] with
-// nchunks >= ceil((largest position + 1) / ilm_attn_f32_chunk()): one wave a chunk, then the fold.
+// rows: the T tokens this call serves (-1: none), null for tokens first .. first + T - 1.
+// ws: null (one wave walks all chunks of its token), or float [8 n_tiles + T][nh][nchunks][d + 4] with
+// nchunks >= ceil((largest position + 1) / ilm_attn_f32_chunk()): one wave a chunk, then the fold.  With it n_tiles > 0: the partial results of these
+// tiles (ilm_attn_f32_tile) lie there already, and the fold is theirs too.
 extern "C" int ilm_attn_f32(void* out, void* ws, int nchunks, const void* q, const void* kc, const void* vc,
-                            const void* block_tables, const void* seg, const void* pos, const void* rows, int T_, int fold, int nh, int nkv, int d,
-                            int page, int max_blocks, int q_stride, int out_stride, float scale, int reach, float softcap,
+                            const void* block_tables, const void* seg, const void* pos, const void* rows, int first, int T_, const void* tiles, int n_tiles,
+                            int nh, int nkv, int d, int page, int max_blocks, int q_stride, int out_stride, float scale, int reach, float softcap,
                             hipStream_t stream) {
     ILM_REQUIRE(T_ > 0 && nh > 0 && nkv > 0 && d > 0 && page > 0 && max_blocks > 0, "attn_f32: bad sizes");
     ILM_REQUIRE(nh % nkv == 0, "attn_f32: %d query heads do not divide into %d groups", nh, nkv);
@@ -303,13 +315,15 @@ extern "C" int ilm_attn_f32(void* out, void* ws, int nchunks, const void* q, con
                     && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 15) == 0 && (ws == nullptr || ((uintptr_t)ws & 15) == 0),
                 "attn_f32: rows must be 16-byte aligned");
     ILM_REQUIRE(ws == nullptr || (nchunks >= 1 && nchunks <= 65535), "attn_f32: %d chunks", nchunks);
-    ILM_REQUIRE(rows != nullptr || fold == T_, "attn_f32: %d tokens of %d", T_, fold);
+    ILM_REQUIRE(first >= 0 && n_tiles >= 0 && n_tiles <= 65535 && (n_tiles == 0 || (ws != nullptr && tiles != nullptr)), "attn_f32: first token %d, %d tiles",
+                first, n_tiles);
     const int G = nh / nkv, nsub = (G + 15) / 16;
     ILM_REQUIRE((long long)nkv * nsub <= 65535 && nh <= 65535, "attn_f32: too many heads");
     dim3 grid(T_, nkv * nsub, ws != nullptr ? nchunks : 1);
     const bool p16 = page % 16 == 0;
-#define FA_ARGS (float*)out, (float*)ws, (const float*)q, (const float*)kc, (const float*)vc, (const int*)block_tables, \
-                (const int*)seg, (const int*)pos, (const int*)rows, nh, nkv, nsub, page, max_blocks, q_stride, out_stride, scale, reach, softcap
+    float* own = (float*)ws + (size_t)n_tiles * FT_TOKENS * nh * nchunks * (d + FA_WS_PAD);
+#define FA_ARGS (float*)out, own, (const float*)q, (const float*)kc, (const float*)vc, (const int*)block_tables, \
+                (const int*)seg, (const int*)pos, (const int*)rows, first, nh, nkv, nsub, page, max_blocks, q_stride, out_stride, scale, reach, softcap
 #define FA_CASE(DT_)                                                                        \
     case DT_:                                                                               \
         if (ws != nullptr && p16) attn_f32_kernel<DT_, true, true><<<grid, 64, 0, stream>>>(FA_ARGS);  \
@@ -325,6 +339,8 @@ extern "C" int ilm_attn_f32(void* out, void* ws, int nchunks, const void* q, con
 #undef FA_CASE
 #undef FA_ARGS
     ILM_LAUNCH_CHECK("attn_f32");
-    if (ws != nullptr) return fa_fold((float*)out, (const float*)ws, (const int*)pos, fold, nh, d, nchunks, out_stride, reach, stream);
+    if (ws != nullptr)
+        return fa_fold((float*)out, (const float*)ws, (const int*)pos, (const int*)tiles, n_tiles, (const int*)rows, first, T_, nh, d, nchunks, out_stride, reach,
+                       stream);
     return 0;
 }

@@ -20,8 +20,6 @@
 typedef __attribute__((address_space(3))) void* lds_ptr;
 typedef const __attribute__((address_space(4))) int* const_ints;   // (read by the scalar unit whatever stands in between)
 
-#define FT_TOKENS 8
-
 // DT: head size / 16; NW: waves, of TPW tokens each
 template <int DT, int NW>
 struct FtShape {
@@ -31,7 +29,7 @@ struct FtShape {
     static_assert(DT % NW == 0 && FA_TILES % S == 0, "whole loads");
 };
 
-// SPLIT: blockIdx.z is the chunk, whose partial result goes to ws (attn_f32.h); else a workgroup walks all chunks of its tokens.
+// SPLIT: blockIdx.z is the chunk, whose partial result goes to ws (attn_f32.h: the rows of the tile's eight); else a workgroup walks all chunks of its tokens.
 template <int DT, int NW, int TPW, bool SPLIT>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
 attn_f32_tile_kernel(float* __restrict__ out, float* __restrict__ ws, const float* __restrict__ qp, const float* __restrict__ kc, const float* __restrict__ vc,
@@ -283,7 +281,7 @@ attn_f32_tile_kernel(float* __restrict__ out, float* __restrict__ ws, const floa
         }
         if (SPLIT) {
             if (live && sees) {
-                float* dst = ws + (((size_t)t * nh + h) * gridDim.z + c) * (d + FA_WS_PAD);
+                float* dst = ws + (((size_t)(tile * FT_TOKENS + part + wave * TPW + r / HW) * nh + h) * gridDim.z + c) * (d + FA_WS_PAD);
 #pragma unroll
                 for (int i = 0; i < DT; ++i) *reinterpret_cast<f32x4*>(dst + 16 * i + 4 * q) = acc[i];
                 if (q == 0) {
@@ -318,13 +316,17 @@ attn_f32_tile_kernel(float* __restrict__ out, float* __restrict__ ws, const floa
     }
 }
 
-// Whether the tile form takes such heads and pages
-extern "C" int ilm_attn_f32_tile_ok(int d, int page) { return (d == 64 || d == 128) && page > 0 && page % 16 == 0 ? 1 : 0; }
+// Whether the tile form takes such heads and pages.  Heads: the exchange of a row's pieces of 16 bytes wants a power of two of
+// at least 16 of them, which leaves out 32, 80, 96 and 192; 256, with twice the queries and sums in registers and twice the LDS a stage, was not built.
+extern "C" int ilm_attn_f32_tile_ok(int d, int page) {
+    return (d == 64 || d == 128) && page > 0 && page % 16 == 0 ? 1 : 0;
+}
 extern "C" int ilm_attn_f32_tile_tokens() { return FT_TOKENS; }
 
-// tiles: n_tiles pairs (first row, count <= 8; 0: nothing) of rows of consecutive tokens of one request; rows of `out` that no tile holds are left alone.
-// ws: null, or float [step's tokens][nh][nchunks][d + 4] (as ilm_attn_f32): a workgroup a chunk, and with `fold` (the step's tokens) the fold of all of them;
-// with fold 0 that is left to the call for the step's single tokens.
+// tiles: n_tiles pairs (first row, count <= 8; 0: nothing) of rows of consecutive tokens of one request;
+// rows of `out` that no tile holds are left alone.
+// ws: null, or float [8 n_tiles][nh][nchunks][d + 4] (as ilm_attn_f32): a workgroup a chunk, and with `fold` the fold of them; without, that is left to the
+// call for the step's single tokens.
 extern "C" int ilm_attn_f32_tile(void* out, void* ws, int nchunks, const void* q, const void* kc, const void* vc, const void* block_tables, const void* seg, const void* pos,
                                  const void* tiles, int n_tiles, int fold, int nh, int nkv, int d, int page, int max_blocks, int q_stride, int out_stride,
                                  float scale, int reach, float softcap, hipStream_t stream) {
@@ -362,6 +364,7 @@ extern "C" int ilm_attn_f32_tile(void* out, void* ws, int nchunks, const void* q
 #undef FT_ARGS
 #undef FT_RUN
     ILM_LAUNCH_CHECK("attn_f32_tile");
-    if (ws != nullptr && fold > 0) return fa_fold((float*)out, (const float*)ws, (const int*)pos, fold, nh, d, nchunks, out_stride, reach, stream);
+    if (ws != nullptr && fold)
+        return fa_fold((float*)out, (const float*)ws, (const int*)pos, (const int*)tiles, n_tiles, nullptr, 0, 0, nh, d, nchunks, out_stride, reach, stream);
     return 0;
 }

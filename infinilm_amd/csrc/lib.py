@@ -48,7 +48,7 @@ _SIGNATURES = {
     "ilm_gemm_f32_glu_tile": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _L, _P],
     "ilm_gemm_portion": [_P, _I, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _P],
     "ilm_gemm_portion_rope": [_P, _I, _P, _I, _P, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
-    "ilm_attn_f32": [_P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _F, _P],
+    "ilm_attn_f32": [_P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _F, _P],
     "ilm_attn_f32_tile": [_P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _F, _P],
     "ilm_gemm_basic": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P],
     "ilm_attn_basic": [_P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _F, _P],

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import functools
 import os
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -31,8 +31,8 @@ F32_ATTN_TILE_HEADS = (64, 128)   # head sizes of the kernel that takes portions
 # the portion need no launch of their own: 128 tokens of 32 heads of 128 over 2 19.7 us, in tiles 20.3; 300 38.4 / 34.1; 210 and three single ones of up
 # to 900 keys 31.4 / 40.1; 200 of 16 heads of 64 over 2 16.7 / 18.8, 300 23.0 / 19.6; 17 of 36 heads of 64 8.6 / 9.5, 40 11.7 / 11.4, 300 133 / 31.
 F32_ATTN_TILE_MIN = int(os.environ.get("INFINILM_AMD_F32_ATTN_TILE_MIN", "512"))
-# Waves up to which these kernels take one (a workgroup) a chunk.  In tiles, split / whole: 800 tokens of 32 heads of 128 over 2 (1,600 waves) 98 / 108 us,
-# 1,200 (2,400) 184 / 165; 300 of 36 heads of 64 (1,368) 31 / 34, 500 (2,268) 61 / 56; 300 at the end of 2,000 keys 140 / 222 and 168 / 214
+# Waves up to which these kernels take one (a workgroup) a chunk, tiles and single tokens each for themselves (`f32_attention`).  In tiles,
+# split / whole: 800 tokens of 32 heads of 128 over 2 (1,600 waves) 98 / 108 us, 1,200 (2,400) 184 / 165; 300 of 36 heads of 64 (1,368) 31 / 34, 500 (2,268) 61 / 56; 300 at the end of 2,000 keys 140 / 222 and 168 / 214
 F32_ATTN_SPLIT_WAVES = 2048
 # INFINILM_AMD_BASIC=1 runs the plain kernels everywhere (for telling a kernel's fault from the engine's)
 FORCE_BASIC = os.environ.get("INFINILM_AMD_BASIC", "0") == "1"
@@ -972,6 +972,28 @@ def attention_chunks(max_total_len: int, page: int, pairs: int, device, head_dim
     return span, -(-max_total_len // span)
 
 
+class F32Attention(NamedTuple):
+    """How the 32-bit path serves a step's tokens (`f32_attention`)."""
+    tiled: bool          # the list of tiles in the kernel for them, and then the single rows alone by the other one; else that one takes every row
+    chunks: int          # chunks of keys that the bound allows
+    split_tiles: bool    # a workgroup a chunk, and the fold
+    split_rows: bool     # a wave a chunk, and the fold
+
+
+def f32_attention(T: int, n_tiles: int, n_single: int, nh: int, nkv: int, d: int, page: int, bound: int) -> F32Attention:
+    """The rule by sizes: T tokens, a list of n_tiles tiles and one of n_single rows (0: none), contexts of up to `bound` keys.  A recorded step's lists are longer
+    than what they hold, so tiles count as what T tokens fill: the step recorded and eager go the same way."""
+    G = nh // nkv
+    groups = nkv * -(-G // 16)
+    full = min(n_tiles, -(-T // ATT_TILE_TOKENS))
+    tiled = (full > 0 and min(T, ATT_TILE_TOKENS * full) * groups > F32_ATTN_TILE_MIN and d in F32_ATTN_TILE_HEADS and page % 16 == 0)
+    rows = n_single if tiled else T
+    chunks = max(1, -(-bound // F32_ATTN_CHUNK))
+    split = F32_ATTN_SPLIT and chunks > 1
+    return F32Attention(tiled, chunks, tiled and split and full * groups * (8 if G > 8 else 4 if G > 4 else 2 if G > 2 else 1) <= F32_ATTN_SPLIT_WAVES,
+                        split and 0 < rows and rows * groups <= F32_ATTN_SPLIT_WAVES)
+
+
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor,
                     seg_of_token: torch.Tensor, positions: torch.Tensor, nh: int, nkv: int, d: int,
                     scale: float, window: int = 0, max_total_len: Optional[int] = None,
@@ -1039,29 +1061,25 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         # the 32-bit path: the group's heads side by side on the float matrix instruction.  Few tokens (decoding):
         # one wave a chunk of keys and a fold; many: one wave a token that walks its chunks; portions of prompts: tiles of
         # tokens that share their keys through LDS.  The same bits.
-        G = nh // nkv
-        groups = nkv * -(-G // 16)
-        rows, n_single, waves = None, T, T * groups
-        tiled = 0
-        if (tiles is not None and tiles.numel() > 0 and T * groups > F32_ATTN_TILE_MIN and d in F32_ATTN_TILE_HEADS and page % 16 == 0):
+        n_tiles, n_single = 0 if tiles is None else tiles.numel() // 2, 0 if single_rows is None else single_rows.numel()
+        how = f32_attention(T, n_tiles, n_single, nh, nkv, d, page, bound)
+        rows, n_rows = (single_rows, n_single) if how.tiled else (None, T)
+        if how.tiled:
             _i32(tiles, "tiles")
-            tiled = tiles.numel() // 2
-            waves = tiled * groups * (8 if G > 8 else 4 if G > 4 else 2 if G > 2 else 1)
-            rows, n_single = single_rows, 0 if single_rows is None else single_rows.numel()
             if n_single:
                 _i32(single_rows, "single_rows")
-        ws, nchunks = None, 1
-        if F32_ATTN_SPLIT and waves <= F32_ATTN_SPLIT_WAVES and bound > F32_ATTN_CHUNK:
-            nchunks = -(-bound // F32_ATTN_CHUNK)
-            ws = torch.empty((T * nh * nchunks * (d + 4),), dtype=F32, device=q.device)
-        if tiled:
-            _run("ilm_attn_f32_tile", out.data_ptr(), _ptr(ws), nchunks, q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-                 block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr(), tiles.data_ptr(), tiled, 0 if n_single else T, nh, nkv, d,
-                 page, block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
-        if n_single:
-            _run("ilm_attn_f32", out.data_ptr(), _ptr(ws), nchunks, q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-                 block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr(), _ptr(rows), n_single, T, nh, nkv, d, page,
-                 block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
+        in_tiles = ATT_TILE_TOKENS * n_tiles if how.split_tiles else 0
+        total = in_tiles + (n_rows if how.split_rows else 0)
+        ws = torch.empty((total * nh * how.chunks * (d + 4),), dtype=F32, device=q.device) if total else None
+        one_fold = how.split_tiles and how.split_rows
+        sizes = (nh, nkv, d, page, block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
+        operands = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr())
+        if how.tiled:
+            _run("ilm_attn_f32_tile", out.data_ptr(), _ptr(ws) if how.split_tiles else None, how.chunks, *operands, tiles.data_ptr(), n_tiles,
+                 int(not one_fold), *sizes)
+        if n_rows:
+            _run("ilm_attn_f32", out.data_ptr(), _ptr(ws) if how.split_rows else None, how.chunks, *operands, _ptr(rows), 0, n_rows,
+                 tiles.data_ptr() if one_fold else None, n_tiles if one_fold else 0, *sizes)
         return out
     # The plain kernel.  Few tokens over long contexts (decoding): one wave a chunk of keys and a fold of the
     # partial results, instead of one wave a head; the bits are the same (see attn_basic.hip).

@@ -85,3 +85,16 @@ def test_experts_are_chosen_and_ordered_in_one_kernel_for_few_tokens(monkeypatch
     monkeypatch.setattr(K, "_run", lambda name, *a, **k: called.append(name))
     K.moe_route(torch.zeros(T, 16), 16, 2, softmax=True, groups=4, keep=2, correction=torch.zeros(16), normalise=True)
     assert called == (["ilm_moe_plan_few"] if one else ["ilm_moe_route_groups", "ilm_moe_sort"])
+
+
+@pytest.mark.parametrize("T,tiles,singles,nh,nkv,d,bound,how", [
+    (768, 96 + 64, 64, 32, 2, 128, 16384, (True, True, True)), (740, 92, 5, 32, 2, 128, 16000, (True, True, True)),     # a recorded step's lists, an eager one's
+    (2048, 256 + 64, 64, 32, 2, 128, 16384, (True, False, True)), (2048, 256, 0, 32, 2, 128, 2048, (True, False, False)),
+    (1200, 13, 1100, 32, 2, 128, 4096, (False, False, False)),                                                          # a short portion beside many tokens
+    (2400, 163, 1100, 32, 2, 128, 4096, (True, False, False)), (300, 38, 3, 36, 36, 64, 2048, (True, True, True)), (300, 38, 60, 36, 36, 64, 2048, (True, True, False)),
+    (300, 38, 3, 36, 36, 64, 128, (True, False, False)), (300, 38, 3, 16, 2, 80, 2048, (False, False, True)), (64, 0, 0, 32, 2, 128, 4096, (False, False, True)),
+    (256, 32, 0, 32, 2, 128, 4096, (False, False, True)), (257, 33, 0, 32, 2, 128, 4096, (True, True, False))])
+def test_32_bit_attention_of_tiles_and_single_rows(T, tiles, singles, nh, nkv, d, bound, how):
+    """Each list is cut into chunks, or not, by its own length."""
+    got = K.f32_attention(T, tiles, singles, nh, nkv, d, 64, bound)
+    assert (got.tiled, got.split_tiles, got.split_rows) == how and got.chunks == -(-bound // K.F32_ATTN_CHUNK)
