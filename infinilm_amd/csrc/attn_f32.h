@@ -28,3 +28,4 @@ __device__ __forceinline__ void fa_fold_scales(float& M, float& L, float m, floa
 // up to count of them hold something), then n_rows single tokens
 int fa_fold(float* out, const float* ws, const int* pos, const int* tiles, int n_tiles, const int* rows, int first, int n_rows, int nh, int d, int nchunks,
             int out_stride, int reach, hipStream_t stream);
+extern "C" int ilm_attn_f32_tile_ok(int d, int page);   // attn_f32_tile.hip
