@@ -31,9 +31,19 @@ F32_ATTN_TILE_HEADS = (64, 128)   # head sizes of the kernel that takes portions
 # the portion need no launch of their own: 128 tokens of 32 heads of 128 over 2 19.7 us, in tiles 20.3; 300 38.4 / 34.1; 210 and three single ones of up
 # to 900 keys 31.4 / 40.1; 200 of 16 heads of 64 over 2 16.7 / 18.8, 300 23.0 / 19.6; 17 of 36 heads of 64 8.6 / 9.5, 40 11.7 / 11.4, 300 133 / 31.
 F32_ATTN_TILE_MIN = int(os.environ.get("INFINILM_AMD_F32_ATTN_TILE_MIN", "512"))
-# Waves up to which these kernels take one (a workgroup) a chunk, tiles and single tokens each for themselves (`f32_attention`).  In tiles,
-# split / whole: 800 tokens of 32 heads of 128 over 2 (1,600 waves) 98 / 108 us, 1,200 (2,400) 184 / 165; 300 of 36 heads of 64 (1,368) 31 / 34, 500 (2,268) 61 / 56; 300 at the end of 2,000 keys 140 / 222 and 168 / 214
+# Waves up to which these kernels take one (a workgroup) a chunk, tiles and single tokens each for themselves (`f32_attention`).
 F32_ATTN_SPLIT_WAVES = 2048
+# ... and tiles over contexts longer than F32_ATTN_LONG: their partial results then cost more than the chip's last gaps.  us, split / whole, tokens as many as make
+# the waves, over themselves and at the end of 2,300 and of 8,300 keys; 32 heads of 128 over 2: 1,280 waves 74 / 82, 278 / 327, 1,040 / 1,295;
+# 1,536 97 / 102, 321 / 328, 1,241 / 1,297; 1,792 119 / 120, 360 / 329, 1,424 / 1,301; 2,048 145 / 139, 397 / 331, 1,680 / 1,301; 3,072 282 / 215, 515 / 463,
+# 2,416 / 1,959.  16 of 128 over 2: 1,536 159 / 199, 276 / 315, 1,211 / 1,264; 2,048 258 / 276, 319 / 325, 1,612 / 1,266.  36 of 64: 1,536 40 / 39, 220 / 246,
+# 757 / 901; 2,048 52 / 49, 275 / 246, 991 / 908.
+F32_ATTN_SPLIT_WAVES_LONG, F32_ATTN_LONG = 1536, 2048
+# Bytes of partial results at once: beyond, tiles or tokens are taken in several launches over one workspace (a token of 32 heads of 128 over 32,768 keys has
+# 4.3 MB of them, and a step's other buffers share `loading.pages_that_fit`'s reserve of 4 GiB).  us in all at once / in 1,024 MB / in 256 MB, over 32,768
+# keys: 256 single tokens of 32 heads of 128 over 2 2,294 / 2,309 / 2,508; a portion of 512 tokens of them 3,417 / 3,467 / 3,680; of 300 of 36 heads of 64
+# 2,702 / 2,701 / 2,863.
+F32_ATTN_WS_BYTES = 1 << 30
 # INFINILM_AMD_BASIC=1 runs the plain kernels everywhere (for telling a kernel's fault from the engine's)
 FORCE_BASIC = os.environ.get("INFINILM_AMD_BASIC", "0") == "1"
 SKINNY_VARIANT = int(os.environ.get("INFINILM_AMD_SKINNY_VARIANT", "0"))  # 0: the kernel chooses
@@ -978,6 +988,7 @@ class F32Attention(NamedTuple):
     chunks: int          # chunks of keys that the bound allows
     split_tiles: bool    # a workgroup a chunk, and the fold
     split_rows: bool     # a wave a chunk, and the fold
+    most: int            # rows (eight a tile) whose partial results are held at once
 
 
 def f32_attention(T: int, n_tiles: int, n_single: int, nh: int, nkv: int, d: int, page: int, bound: int) -> F32Attention:
@@ -990,8 +1001,15 @@ def f32_attention(T: int, n_tiles: int, n_single: int, nh: int, nkv: int, d: int
     rows = n_single if tiled else T
     chunks = max(1, -(-bound // F32_ATTN_CHUNK))
     split = F32_ATTN_SPLIT and chunks > 1
-    return F32Attention(tiled, chunks, tiled and split and full * groups * (8 if G > 8 else 4 if G > 4 else 2 if G > 2 else 1) <= F32_ATTN_SPLIT_WAVES,
-                        split and 0 < rows and rows * groups <= F32_ATTN_SPLIT_WAVES)
+    waves = full * groups * (8 if G > 8 else 4 if G > 4 else 2 if G > 2 else 1)
+    return F32Attention(tiled, chunks, tiled and split and waves <= (F32_ATTN_SPLIT_WAVES if bound <= F32_ATTN_LONG else F32_ATTN_SPLIT_WAVES_LONG),
+                        split and 0 < rows and rows * groups <= F32_ATTN_SPLIT_WAVES, max(ATT_TILE_TOKENS, F32_ATTN_WS_BYTES // (4 * nh * chunks * (d + 4))))
+
+
+def _runs(n: int, most: int):
+    """(first, count) of as few runs of at most `most` as cover n, of about equal length."""
+    parts = -(-n // most)
+    return [(n * i // parts, n * (i + 1) // parts - n * i // parts) for i in range(parts)]
 
 
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor,
@@ -1070,16 +1088,16 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                 _i32(single_rows, "single_rows")
         in_tiles = ATT_TILE_TOKENS * n_tiles if how.split_tiles else 0
         total = in_tiles + (n_rows if how.split_rows else 0)
-        ws = torch.empty((total * nh * how.chunks * (d + 4),), dtype=F32, device=q.device) if total else None
-        one_fold = how.split_tiles and how.split_rows
+        ws = torch.empty((min(total, how.most) * nh * how.chunks * (d + 4),), dtype=F32, device=q.device) if total else None
+        one_fold = how.split_tiles and how.split_rows and total <= how.most
         sizes = (nh, nkv, d, page, block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
         operands = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr())
-        if how.tiled:
-            _run("ilm_attn_f32_tile", out.data_ptr(), _ptr(ws) if how.split_tiles else None, how.chunks, *operands, tiles.data_ptr(), n_tiles,
+        for first, n in _runs(n_tiles, how.most // ATT_TILE_TOKENS if how.split_tiles else n_tiles) if how.tiled else ():
+            _run("ilm_attn_f32_tile", out.data_ptr(), _ptr(ws) if how.split_tiles else None, how.chunks, *operands, tiles.data_ptr() + 8 * first, n,
                  int(not one_fold), *sizes)
-        if n_rows:
-            _run("ilm_attn_f32", out.data_ptr(), _ptr(ws) if how.split_rows else None, how.chunks, *operands, _ptr(rows), 0, n_rows,
-                 tiles.data_ptr() if one_fold else None, n_tiles if one_fold else 0, *sizes)
+        for first, n in _runs(n_rows, how.most if how.split_rows else n_rows) if n_rows else ():
+            _run("ilm_attn_f32", out.data_ptr(), _ptr(ws) if how.split_rows else None, how.chunks, *operands, None if rows is None else rows.data_ptr() + 4 * first,
+                 first, n, tiles.data_ptr() if one_fold else None, n_tiles if one_fold else 0, *sizes)
         return out
     # The plain kernel.  Few tokens over long contexts (decoding): one wave a chunk of keys and a fold of the
     # partial results, instead of one wave a head; the bits are the same (see attn_basic.hip).

@@ -817,7 +817,7 @@ def test_attention_float32_tiles_of_tokens_give_the_same_bits(K, monkeypatch, nh
 
 @pytest.mark.parametrize("nh,nkv,d", [(32, 2, 128), (10, 2, 64), (3, 3, 64)])
 def test_attention_float32_cuts_tiles_and_single_rows_each_for_itself(K, monkeypatch, nh, nkv, d):
-    """Either list in chunks with a fold of its own, both, neither: the bits of tokens one by one; what a list says of no token is skipped."""
+    """Either list in chunks with a fold of its own, both, neither, and in several launches that share a workspace: the bits of tokens one by one; what a list says of no token is skipped."""
     case = dict(lens=[1, 130, 300, 700, 523, 260], qlens=[1, 1, 21, 1, 12, 260], seed=14)
     monkeypatch.setattr(K, "F32_ATTN_TILE_MIN", 1 << 30)
     alone, want = _attention_case(K, torch.float32, nh, nkv, d, 64, **case)
@@ -826,10 +826,16 @@ def test_attention_float32_cuts_tiles_and_single_rows_each_for_itself(K, monkeyp
     i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
     monkeypatch.setattr(K, "paged_attention", lambda *a, tiles, single_rows, **k: attention(*a, tiles=pad(tiles, i32([[0, 0]])),
                                                                                            single_rows=pad(single_rows, i32([-1])), **k))
-    for tiles, rows in ((False, False), (True, False), (False, True), (True, True)):
-        monkeypatch.setattr(K, "f32_attention", lambda *a: rule(*a)._replace(split_tiles=tiles, split_rows=rows))
+    for tiles, rows, most in ((False, False, 8), (True, False, 1 << 20), (False, True, 1 << 20), (True, True, 1 << 20), (True, True, 8), (True, True, 24)):
+        monkeypatch.setattr(K, "f32_attention", lambda *a: rule(*a)._replace(split_tiles=tiles, split_rows=rows, most=most))
         out, _ = _attention_case(K, torch.float32, nh, nkv, d, 64, **case)
         assert torch.equal(out.cpu(), alone.cpu())
+    # rows one by one without a list, in several launches
+    monkeypatch.setattr(K, "paged_attention", attention)
+    monkeypatch.setattr(K, "F32_ATTN_TILE_MIN", 1 << 30)
+    monkeypatch.setattr(K, "f32_attention", lambda *a: rule(*a)._replace(split_rows=True, most=100))
+    out, _ = _attention_case(K, torch.float32, nh, nkv, d, 64, **case)
+    assert torch.equal(out.cpu(), alone.cpu())
     _close(alone, want, 3e-6)
 
 

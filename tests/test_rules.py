@@ -93,8 +93,23 @@ def test_experts_are_chosen_and_ordered_in_one_kernel_for_few_tokens(monkeypatch
     (1200, 13, 1100, 32, 2, 128, 4096, (False, False, False)),                                                          # a short portion beside many tokens
     (2400, 163, 1100, 32, 2, 128, 4096, (True, False, False)), (300, 38, 3, 36, 36, 64, 2048, (True, True, True)), (300, 38, 60, 36, 36, 64, 2048, (True, True, False)),
     (300, 38, 3, 36, 36, 64, 128, (True, False, False)), (300, 38, 3, 16, 2, 80, 2048, (False, False, True)), (64, 0, 0, 32, 2, 128, 4096, (False, False, True)),
+    (2048, 256, 0, 16, 2, 128, 2048, (True, True, False)), (2048, 256, 0, 16, 2, 128, 2049, (True, False, False)), (1536, 192, 0, 16, 2, 128, 32768, (True, True, False)),
+    (1537, 193, 0, 16, 2, 128, 32768, (True, False, False)), (1024, 0, 0, 32, 2, 128, 32768, (False, False, True)),
     (256, 32, 0, 32, 2, 128, 4096, (False, False, True)), (257, 33, 0, 32, 2, 128, 4096, (True, True, False))])
 def test_32_bit_attention_of_tiles_and_single_rows(T, tiles, singles, nh, nkv, d, bound, how):
     """Each list is cut into chunks, or not, by its own length."""
     got = K.f32_attention(T, tiles, singles, nh, nkv, d, 64, bound)
     assert (got.tiled, got.split_tiles, got.split_rows) == how and got.chunks == -(-bound // K.F32_ATTN_CHUNK)
+
+
+@pytest.mark.parametrize("T,tiles,singles,nh,nkv,d,bound", [(1536, 192, 0, 16, 2, 128, 32768), (768, 96, 0, 32, 2, 128, 32768), (300, 38, 40, 36, 36, 64, 32768),
+                                                            (1000, 0, 0, 32, 2, 128, 131072), (8, 1, 0, 128, 8, 256, 1 << 20), (512, 64 + 64, 64, 32, 2, 128, 65536)])
+def test_32_bit_attention_holds_a_bounded_workspace(T, tiles, singles, nh, nkv, d, bound):
+    """Long contexts whose tiles or tokens are cut into chunks: partial results of at most 1 GiB at once, or of eight tokens."""
+    how = K.f32_attention(T, tiles, singles, nh, nkv, d, 64, bound)
+    assert how.split_tiles or how.split_rows
+    row = 4 * nh * how.chunks * (d + 4)
+    assert how.most == 8 or how.most * row <= 1 << 30
+    for n, most in ((tiles, how.most // K.ATT_TILE_TOKENS), (singles or T, how.most)):
+        runs = K._runs(n, most) if n else []
+        assert all(0 < m <= most for _, m in runs) and [a for a, _ in runs] == [sum(m for _, m in runs[:i]) for i in range(len(runs))] and sum(m for _, m in runs) == n
