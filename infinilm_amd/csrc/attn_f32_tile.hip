@@ -316,10 +316,10 @@ attn_f32_tile_kernel(float* __restrict__ out, float* __restrict__ ws, const floa
     }
 }
 
-// Whether the tile form takes such heads and pages.  Heads: the exchange of a row's pieces of 16 bytes wants a power of two of
+// Whether the tile form takes such heads and pages (offsets inside a page take 32 bits).  Heads: the exchange of a row's pieces of 16 bytes wants a power of two of
 // at least 16 of them, which leaves out 32, 80, 96 and 192; 256, with twice the queries and sums in registers and twice the LDS a stage, was not built.
 extern "C" int ilm_attn_f32_tile_ok(int d, int page) {
-    return (d == 64 || d == 128) && page > 0 && page % 16 == 0 ? 1 : 0;
+    return (d == 64 || d == 128) && page > 0 && page % 16 == 0 && (long long)d * page < (1ll << 28) ? 1 : 0;
 }
 extern "C" int ilm_attn_f32_tile_tokens() { return FT_TOKENS; }
 
@@ -337,7 +337,6 @@ extern "C" int ilm_attn_f32_tile(void* out, void* ws, int nchunks, const void* q
                     && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 15) == 0 && (ws == nullptr || ((uintptr_t)ws & 15) == 0),
                 "attn_f32_tile: rows must be 16-byte aligned");
     ILM_REQUIRE(ws == nullptr || (nchunks >= 1 && nchunks <= 65535), "attn_f32_tile: %d chunks", nchunks);
-    ILM_REQUIRE((long long)d * page < (1ll << 28), "attn_f32_tile: pages of %d keys", page);   // (offsets inside a page take 32 bits)
     const int G = nh / nkv, nsub = (G + 15) / 16;
     ILM_REQUIRE(n_tiles <= 65535, "attn_f32_tile: %d tiles", n_tiles);
     const int shift = (page & (page - 1)) == 0 ? __builtin_ctz(page) : -1;

@@ -989,6 +989,7 @@ class F32Attention(NamedTuple):
     split_tiles: bool    # a workgroup a chunk, and the fold
     split_rows: bool     # a wave a chunk, and the fold
     most: int            # rows (eight a tile) whose partial results are held at once
+    most_tiles: int      # tiles a launch
 
 
 def f32_attention(T: int, n_tiles: int, n_single: int, nh: int, nkv: int, d: int, page: int, bound: int) -> F32Attention:
@@ -997,13 +998,16 @@ def f32_attention(T: int, n_tiles: int, n_single: int, nh: int, nkv: int, d: int
     G = nh // nkv
     groups = nkv * -(-G // 16)
     full = min(n_tiles, -(-T // ATT_TILE_TOKENS))
-    tiled = (full > 0 and min(T, ATT_TILE_TOKENS * full) * groups > F32_ATTN_TILE_MIN and d in F32_ATTN_TILE_HEADS and page % 16 == 0)
+    tiled = (full > 0 and min(T, ATT_TILE_TOKENS * full) * groups > F32_ATTN_TILE_MIN and d in F32_ATTN_TILE_HEADS and page % 16 == 0
+             and d * page < 1 << 28)   # (offsets inside a page take 32 bits)
     rows = n_single if tiled else T
     chunks = max(1, -(-bound // F32_ATTN_CHUNK))
     split = F32_ATTN_SPLIT and chunks > 1
     waves = full * groups * (8 if G > 8 else 4 if G > 4 else 2 if G > 2 else 1)
-    return F32Attention(tiled, chunks, tiled and split and waves <= (F32_ATTN_SPLIT_WAVES if bound <= F32_ATTN_LONG else F32_ATTN_SPLIT_WAVES_LONG),
-                        split and 0 < rows and rows * groups <= F32_ATTN_SPLIT_WAVES, max(ATT_TILE_TOKENS, F32_ATTN_WS_BYTES // (4 * nh * chunks * (d + 4))))
+    split_tiles = tiled and split and waves <= (F32_ATTN_SPLIT_WAVES if bound <= F32_ATTN_LONG else F32_ATTN_SPLIT_WAVES_LONG)
+    most = max(ATT_TILE_TOKENS, F32_ATTN_WS_BYTES // (4 * nh * chunks * (d + 4)))
+    return F32Attention(tiled, chunks, split_tiles, split and 0 < rows and rows * groups <= F32_ATTN_SPLIT_WAVES, most,
+                        min(65535, most // ATT_TILE_TOKENS if split_tiles else n_tiles))   # (what a grid's second dimension takes)
 
 
 def _runs(n: int, most: int):
@@ -1092,7 +1096,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         one_fold = how.split_tiles and how.split_rows and total <= how.most
         sizes = (nh, nkv, d, page, block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
         operands = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr())
-        for first, n in _runs(n_tiles, how.most // ATT_TILE_TOKENS if how.split_tiles else n_tiles) if how.tiled else ():
+        for first, n in _runs(n_tiles, how.most_tiles) if how.tiled else ():
             _run("ilm_attn_f32_tile", out.data_ptr(), _ptr(ws) if how.split_tiles else None, how.chunks, *operands, tiles.data_ptr() + 8 * first, n,
                  int(not one_fold), *sizes)
         for first, n in _runs(n_rows, how.most if how.split_rows else n_rows) if n_rows else ():

@@ -827,7 +827,7 @@ def test_attention_float32_cuts_tiles_and_single_rows_each_for_itself(K, monkeyp
     monkeypatch.setattr(K, "paged_attention", lambda *a, tiles, single_rows, **k: attention(*a, tiles=pad(tiles, i32([[0, 0]])),
                                                                                            single_rows=pad(single_rows, i32([-1])), **k))
     for tiles, rows, most in ((False, False, 8), (True, False, 1 << 20), (False, True, 1 << 20), (True, True, 1 << 20), (True, True, 8), (True, True, 24)):
-        monkeypatch.setattr(K, "f32_attention", lambda *a: rule(*a)._replace(split_tiles=tiles, split_rows=rows, most=most))
+        monkeypatch.setattr(K, "f32_attention", lambda *a: rule(*a)._replace(split_tiles=tiles, split_rows=rows, most=most, most_tiles=most // 8))
         out, _ = _attention_case(K, torch.float32, nh, nkv, d, 64, **case)
         assert torch.equal(out.cpu(), alone.cpu())
     # rows one by one without a list, in several launches

@@ -113,3 +113,10 @@ def test_32_bit_attention_holds_a_bounded_workspace(T, tiles, singles, nh, nkv, 
     for n, most in ((tiles, how.most // K.ATT_TILE_TOKENS), (singles or T, how.most)):
         runs = K._runs(n, most) if n else []
         assert all(0 < m <= most for _, m in runs) and [a for a, _ in runs] == [sum(m for _, m in runs[:i]) for i in range(len(runs))] and sum(m for _, m in runs) == n
+
+
+def test_32_bit_attention_takes_any_page_and_any_number_of_tiles():
+    """Pages beyond the tile kernel's 32-bit offsets go to the other one, tiles beyond a grid to several launches."""
+    assert K.f32_attention(2048, 256, 0, 32, 2, 128, (1 << 21) - 16, 2048).tiled and not K.f32_attention(2048, 256, 0, 32, 2, 128, 1 << 21, 2048).tiled
+    how = K.f32_attention(1 << 20, 1 << 17, 0, 4, 4, 64, 64, 2048)
+    assert how.tiled and how.most_tiles == 65535 and [n for _, n in K._runs(1 << 17, how.most_tiles)] == [43690, 43691, 43691]
