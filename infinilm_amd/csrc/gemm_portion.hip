@@ -60,7 +60,8 @@ __device__ __forceinline__ int gp_w_row(const GpArgs& A, int nt, int j) {
     return pc / half * A.d + pc % half + second * half;
 }
 
-template <int BM, int BN, int WM, int WN, int NS, int EPI>
+// BAND: the tiles are walked in bands of `group` m tiles (gp_group); else all m tiles of an n tile one after the other
+template <int BM, int BN, int WM, int WN, int NS, int EPI, bool BAND>
 __global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64, 2)
 gemm_portion_kernel(const GpArgs A) {
     constexpr int NW = (BM / WM) * (BN / WN), ROWS = BM + BN, GROUPS = ROWS / 8, PER = GROUPS / NW, TM = WM / 16, TN = WN / 16;
@@ -73,7 +74,11 @@ gemm_portion_kernel(const GpArgs A) {
     {
         const int total = A.m_tiles * A.n_tiles, per = total >> 3, rem = total & 7, xcd = blockIdx.x & 7;
         const int id = xcd * per + (xcd < rem ? xcd : rem) + ((int)blockIdx.x >> 3);
-        const int band = id / (A.group * A.n_tiles), first = band * A.group, rows = A.m_tiles - first < A.group ? A.m_tiles - first : A.group;
+        int first = 0, rows = A.m_tiles;
+        if (BAND) {
+            first = id / (A.group * A.n_tiles) * A.group;
+            rows = A.m_tiles - first < A.group ? A.m_tiles - first : A.group;
+        }
         const int at = id - first * A.n_tiles;
         mt = first + at % rows;
         nt = at / rows;
@@ -295,7 +300,8 @@ gemm_portion_kernel(const GpArgs A) {
 // its own L2: with all m tiles together all of X for each (2048 x 1024 x 4096 in tiles of 128 x 64: 134 MB in all, 67 MB where four m tiles are
 // walked with eight n tiles: 24.1 -> 22.4 us; 1000 x 1024 x 4096 15.2 -> 14.6).  But then a row of W is fetched by several: only where at most two
 // thirds of the rows are left (1000 x 2304 x 2304, four fifths, 18.0 -> 18.8), and not for q, k and v (2048 x 1280 x 1024, a round and a
-// quarter, in a model's step 16.1 -> 17.6).
+// quarter, in a model's step 16.1 -> 17.6).  Kernels of their own: with the band's two divisions and the arguments they wait for every workgroup starts
+// later, and what has no bands loses (985 x 4096 x 4096 36.8 us, 38.3 so; 600 x 4096 x 2048 18.1 and 19.0).
 static int gp_group(int m_tiles, int n_tiles, int bm, int bn) {
     const long long per = ((long long)m_tiles * n_tiles + 7) / 8;
     auto rows = [&](int g) { return (long long)g * bm + (per + g - 1) / g * bn; };
@@ -312,8 +318,13 @@ static int gp_group(int m_tiles, int n_tiles, int bm, int bn) {
         a.n_tiles = ((NCOLS_) + BN_ - 1) / BN_;                                                             \
         ILM_REQUIRE((long long)a.m_tiles * a.n_tiles < (1ll << 31), "gemm_portion: too many tiles");        \
         a.group = EPI_ == GP_PLAIN ? gp_group(a.m_tiles, a.n_tiles, BM_, BN_) : a.m_tiles;                  \
-        gemm_portion_kernel<BM_, BN_, WM_, WN_, NS_, EPI_>                                                  \
-            <<<a.m_tiles * a.n_tiles, (BM_ / WM_) * (BN_ / WN_) * 64, 0, stream>>>(a);                      \
+        const int threads = (BM_ / WM_) * (BN_ / WN_) * 64;                                                 \
+        if (EPI_ == GP_PLAIN && a.group < a.m_tiles)                                                        \
+            gemm_portion_kernel<BM_, BN_, WM_, WN_, NS_, EPI_, EPI_ == GP_PLAIN>                            \
+                <<<a.m_tiles * a.n_tiles, threads, 0, stream>>>(a);                                         \
+        else                                                                                                \
+            gemm_portion_kernel<BM_, BN_, WM_, WN_, NS_, EPI_, false>                                       \
+                <<<a.m_tiles * a.n_tiles, threads, 0, stream>>>(a);                                         \
     }
 
 static int gp_check(const char* what, int M, int rows, int K, const void* X, int lda, const void* W, int ldw) {
