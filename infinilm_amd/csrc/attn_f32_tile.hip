@@ -43,7 +43,13 @@ attn_f32_tile_kernel(float* __restrict__ out, float* __restrict__ ws, const floa
     const int tile = n_tiles - 1 - (int)blockIdx.y;
     // the tile's part of NW x TPW tokens (the later part of the same keys first)
     const int part = FT_TOKENS - NW * TPW - (int)(blockIdx.x / (nkv * nsub)) * (NW * TPW);
-    const int row0 = tiles[2 * tile] + part, count = min(tiles[2 * tile + 1] - part, NW * TPW);
+    const int row0 = tiles[2 * tile] + part, in_tile = tiles[2 * tile + 1], count = min(in_tile - part, NW * TPW);
+    if (in_tile < 0 && (!SPLIT || blockIdx.z == 0)) {   // rows of no request get zeros
+        const int G = nh / nkv, kvh = blockIdx.x / nsub % nkv, sub = blockIdx.x % nsub, of_row = min(16, G - sub * 16) * (d / 4);
+        const int n = min(-in_tile - part, NW * TPW) * of_row;
+        float* from = out + (size_t)row0 * out_stride + (size_t)(kvh * G + sub * 16) * d;
+        for (int i = threadIdx.x; i < n; i += NW * 64) reinterpret_cast<float4*>(from + (size_t)(i / of_row) * out_stride)[i % of_row] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
     if (count <= 0) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
     const int G = nh / nkv, kvh = blockIdx.x / nsub % nkv, sub = blockIdx.x % nsub;
@@ -323,7 +329,7 @@ extern "C" int ilm_attn_f32_tile_ok(int d, int page) {
 }
 extern "C" int ilm_attn_f32_tile_tokens() { return FT_TOKENS; }
 
-// tiles: n_tiles pairs (first row, count <= 8; 0: nothing) of rows of consecutive tokens of one request;
+// tiles: n_tiles pairs (first row, count <= 8; 0: nothing; below 0: that many rows of no request) of rows of consecutive tokens of one request;
 // rows of `out` that no tile holds are left alone.
 // ws: null, or float [8 n_tiles][nh][nchunks][d + 4] (as ilm_attn_f32): a workgroup a chunk, and with `fold` the fold of them; without, that is left to the
 // call for the step's single tokens.

@@ -48,7 +48,7 @@ class StepBatch:
         self.want_rows = None           # [num_wanted] rows of the flattened batch
         self.state_in = None            # [R] state row read at the start (0 = zeros)
         self.state_out = None           # [R] state row written at the end
-        self.att_tiles = None           # [n, 2] (first row, count): runs of <= 8 consecutive tokens of one request
+        self.att_tiles = None           # [n, 2] (first row, count): runs of <= 8 consecutive tokens of one request; count below 0: rows of none
         self.att_single_rows = None     # rows of requests that bring one token (None: no run of 2 or more exists)
         self.block_tables: List = []    # per group [R, max_blocks], -1 padded
         self.slots: List = []           # per group [T] slot of each new token
@@ -127,7 +127,7 @@ class StepRunner:
         `bounds` = (requests, wanted rows, attention tiles, single rows): every array of the metadata is laid out
         for that many entries (with `pad_rows` and `min_blocks` for the tokens and the block tables), so that a
         recorded step of mixed content finds every array at the same address at every replay: lists are
-        filled up with entries that do nothing (tiles of no tokens, a single row or a wanted row once more)."""
+        filled up with entries that do nothing (tiles of no tokens, single rows of -1, a wanted row once more)."""
         cache = self.cache
         V = self.model.spec.vocab_size
         if not entries and not pad_rows:
@@ -202,7 +202,9 @@ class StepRunner:
                     tiles += [a + k, min(TILE, n - k)]
         if not tiles and bounds is None:
             singles = []   # every token is single: the kernels take all rows
-        # (the rows of no request of a bounded layout are left out of the attention: nothing reads what they hold)
+        if bounds is not None:   # rows of no request: no attention, but zeros in 32-bit, as the products behind go by what a row holds
+            for k in range(int(offsets[R_real]), T, TILE):
+                tiles += [k, -min(TILE, T - k)]
         R_lay, want_lay, tiles_lay, singles_lay = R, n_want, len(tiles) // 2, len(singles)
         if bounds is not None:
             R_lay, want_lay, tiles_lay, singles_lay = bounds

@@ -1033,7 +1033,8 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     upper bound of position + 1 over the batch (the matrix-core kernel sizes its key chunks by it;
     without it the plain kernel runs).  `tiles` [n, 2] = (first row, count <= ATT_TILE_TOKENS) lists runs of
     consecutive tokens of one request and `single_rows` the remaining rows; without them every token
-    is served on its own.  Returns [T, nh*d]."""
+    is served on its own.  A tile of no tokens (0) or a single row of -1 fills a list up; a count below 0 stands for so many rows of no request, whose results
+    are finite in float32 and undefined in bfloat16, as those of rows in neither list are.  Returns [T, nh*d]."""
     _dev(q, k_cache, v_cache, block_tables, seg_of_token, positions)
     _i32(block_tables, "block_tables")
     _i32(seg_of_token, "seg_of_token")

@@ -982,3 +982,18 @@ def models_de(tmp_path_factory):
         d = str(tmp_path_factory.mktemp(f"mix_{name}_{dtype}"))
         out[(name, dtype)] = (cfg, d, make_model_dir(d, cfg, seed=60 + ord(name), store=dtype))
     return out
+
+
+def test_a_bounded_steps_lists_name_every_row_once(models_de):
+    """Tiles, single rows, and tiles of negative count for the rows that fill the shape up."""
+    from infinilm_amd.engine.loading import load_model, make_runner
+    from infinilm_amd.engine.step import StepEntry
+    cfg, d, _ = models_de[("B", "float32")]
+    r = make_runner(load_model(d, "float32", "cuda:0"), num_pages=8, page_size=64, max_requests=8)
+    for q in "abc":
+        r.cache.admit(q)
+    entries = [StepEntry("a", random_tokens(cfg, 17, 1), [16]), StepEntry("b", [1], [0]), StepEntry("c", random_tokens(cfg, 9, 2), [8])]
+    b = r.build_batch(entries, pad_rows=13, bounds=(9, 9, 5 + 9, 9))
+    tiles, singles = b.att_tiles.tolist(), b.att_single_rows.tolist()
+    assert [t for t in tiles if t[1]] == [[0, 8], [8, 8], [16, 1], [18, 8], [26, 1], [27, -8], [35, -5]]
+    assert singles == [17] + [-1] * 8 and len(tiles) == 14

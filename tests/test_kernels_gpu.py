@@ -839,6 +839,26 @@ def test_attention_float32_cuts_tiles_and_single_rows_each_for_itself(K, monkeyp
     _close(alone, want, 3e-6)
 
 
+@pytest.mark.parametrize("nh,nkv,d", [(32, 2, 128), (34, 2, 64), (10, 2, 64), (8, 2, 128), (3, 3, 64)])
+@pytest.mark.parametrize("split", [False, True])
+def test_attention_float32_gives_rows_of_no_request_zeros(K, monkeypatch, nh, nkv, d, split):
+    """A recorded step's lists: tiles of no tokens, tiles of rows of no request, single rows of none.  Served rows have their bits, and nothing of what the
+    results' and the workspace's memory held before is left in the others."""
+    n, page, none = 300, 64, 19
+    k, v, q = (_rand((m, h, d), s, torch.float32) for m, h, s in ((n, nkv, 1), (n, nkv, 2), (40 + 1 + none, nh, 3)))
+    kc, vc, bt = _paged([k, k[:1]], [v, v[:1]], page, 8, 4, torch.float32)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    args = (q.reshape(-1, nh * d).to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), i32([0] * 41 + [1] * none), i32(list(range(n - 40, n)) + [n - 1] + [0] * none), nh, nkv, d, 0.1)
+    alone = K.paged_attention(*args, max_total_len=n)
+    tiles = i32([[a, 8] for a in range(0, 40, 8)] + [[41, -8], [49, -8], [57, -3], [0, 0], [0, 0]])
+    monkeypatch.setattr(K, "F32_ATTN_TILE_MIN", 0)
+    monkeypatch.setattr(K, "F32_ATTN_SPLIT", split)
+    stale = [torch.full((m,), math.nan, device=DEV) for m in (alone.numel(), (8 * 10 + 4) * nh * 3 * (d + 4))]
+    del stale
+    out = K.paged_attention(*args, max_total_len=n, tiles=tiles, single_rows=i32([40, -1, -1, -1]))
+    assert torch.equal(out[:41].cpu(), alone[:41].cpu()) and not out[41:].any()
+
+
 @pytest.mark.parametrize("nh,nkv,d", [(9, 1, 64), (5, 1, 128), (3, 1, 64), (2, 2, 128)])
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_attention_float32_tiles_keep_later_values_from_earlier_tokens(K, monkeypatch, nh, nkv, d, bad):
