@@ -340,19 +340,20 @@ gemm_f32_sum_kernel(float* __restrict__ C, const float* __restrict__ ws, const f
 // Which of the three tiles, or 4: the first, with the tiles beyond whole rounds cut (`parts` workgroups a tile)
 static int ft_form(int M, int N, int K, int slices, int* parts) {
     // What ends soonest, by what a round of each takes (us at K 4096, measured on 256 units: the ratios count).  128 x
-    // 256 and 128 x 128 run one a unit, 325 and 197 a round; of 64 x 64 three share a unit: 95 alone, 142 two of them,
-    // 66 each when many follow one another.  2048 x 4096 outputs: 368, 405 and 529 us; 300 x 4608: 324, 197 and 142.
+    // 256 and 128 x 128 run one a unit, 325 and 197 a round; of 64 x 64 three share a unit: 95 alone, 142 two of them, 190 three
+    // (1024 x 2112 to 1024 x 3072: 184 to 197), 265 four, 66 each when many follow one another.  2048 x 4096 outputs: 368, 405 and 529 us; 300 x 4608: 324, 197 and 142.
     const long long cus = ilm_num_cus();
     auto count = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     const long long n1 = count(128, 256), t1 = 325 * ((n1 + cus - 1) / cus), t2 = 197 * ((count(128, 128) + cus - 1) / cus);
-    const long long n3 = count(64, 64), t3 = n3 <= cus ? 95 : n3 <= 2 * cus ? 142 : 66 * n3 / cus + 10;
+    const long long n3 = count(64, 64), t3 = n3 <= cus ? 95 : n3 <= 2 * cus ? 142 : n3 <= 3 * cus ? 190 : n3 <= 4 * cus ? 265 : 66 * n3 / cus + 10;
     const int form = t1 <= t2 && t1 <= t3 ? 1 : t2 <= t3 ? 2 : 3;
     const long long rest = n1 % cus;
     if (rest == 0 || slices < 2) return form;
     // Cut: rounds of workgroups of some slices each and 3 us for the start of a round, then the sum, 4 us and 0.03 a slice of a tile (128 KB, written and
-    // read).  By this rule / measured, and the best whole form: 2048 x 4608 x 4096 380 / 405 (578), 1024 x 4608 x 4096 257 / 248 (325), 300 x 4608
-    // x 4096 104 / 102 (144), 100 x 4608 x 4096 52 / 53 (102), 1024 x 4096 x 4096 209 / 210 (202), 2048 x 2304 x 2304 168 / 164 (182),
-    // 1024 x 2304 x 2304 99 / 96 (109), 2048 x 1024 x 1024 46 / 47 (42), 1024 x 6912 x 2304 237 / 245 (193), 1300 x 2048 x 12288 400 / 396 (568).
+    // read).  By this rule / measured, and the best whole form: 2048 x 4608 x 4096 380 / 382 (544), 1024 x 4608 x 4096 257 / 233 (305), 300 x 4608
+    // x 4096 101 / 93 (138), 100 x 4608 x 4096 52 / 51 (97), 1024 x 4096 x 4096 200 / 188 (197), 2048 x 2304 x 2304 168 / 152 (178),
+    // 1024 x 2304 x 2304 93 / 85 (106), 2048 x 1024 x 1024 43 / 44 (40), 2048 x 1280 x 1024 57 / 54 (52), 1024 x 6912 x 2304 237 / 228 (186), 1300 x 2048 x
+    // 12288 400 / 362 (532).
     const double unit = 325. / 4096 * K / slices;
     double best = 0.;
     for (int p = 2; p <= slices; ++p) {
@@ -403,7 +404,8 @@ extern "C" int ilm_gemm_f32_tile(void* C, const void* X, const void* W, const vo
     return 0;
 }
 
-// Floats of the workspace that the form with cut tiles takes, or 0 where one of the others ends sooner
+// Floats of the workspace that the form with cut tiles takes, or 0 where one of the others ends sooner.  At most the units less one times eight slices of
+// 128 KB, whatever the sizes: 267 MB on 256 units.
 extern "C" long ilm_gemm_f32_cut_ws(int M, int N, int K) {
     int parts;
     if (M <= 0 || N <= 0 || K <= 0 || ft_form(M, N, K, ft_slices(K), &parts) != 4) return 0;

@@ -1561,6 +1561,18 @@ def test_experts_of_few_rows_give_the_bits_of_many(K, monkeypatch, T, E, top, K_
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("M,N,K_,cut", [(1024, 2304, 2304, True), (1024, 2112, 2304, True), (2048, 1280, 1024, False), (2048, 1024, 1024, False), (1024, 6912, 2304, False),
+                                        (2048, 4608, 4096, True), (255 * 128, 256, 8192, False), (255 * 128, 200, 32768, False), (2048, 4096, 4096, False), (65, 60000, 4096, False),
+                                        (1, 1 << 20, 4, False), (65, 64, 1 << 20, True)])
+def test_float32_cut_tiles_by_size_and_their_workspace(K, M, N, K_, cut):
+    """Where two to three tiles of 64 x 64 a unit would run beyond one another the rule cuts, and no size asks for more than a slice's sums of every unit but one."""
+    from infinilm_amd.csrc import lib
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    need = lib.load().ilm_gemm_f32_cut_ws(M, N, K_)
+    assert 0 <= need <= (cus - 1) * 8 * 128 * 256
+    assert cus != 256 or (need > 0) == cut
+
+
 @pytest.mark.parametrize("tile,M,N,K_", [(1, 1100, 1220, 64), (1, 1990, 700, 128), (2, 2041, 1000, 64), (2, 4000, 330, 192), (3, 4000, 1100, 64), (1, 130, 2000, 64)])
 def test_portion_product_walks_its_tiles_in_bands(K, tile, M, N, K_):
     """Products whose tiles are walked in bands of several rows of tiles, the last band lower than the others: every output once.  float sums of products of
