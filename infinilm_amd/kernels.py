@@ -1094,7 +1094,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         in_tiles = ATT_TILE_TOKENS * n_tiles if how.split_tiles else 0
         total = in_tiles + (n_rows if how.split_rows else 0)
         ws = torch.empty((min(total, how.most) * nh * how.chunks * (d + 4),), dtype=F32, device=q.device) if total else None
-        one_fold = how.split_tiles and how.split_rows and total <= how.most
+        one_fold = how.split_tiles and how.split_rows and total <= how.most and n_tiles <= how.most_tiles   # (several launches of tiles share the workspace)
         sizes = (nh, nkv, d, page, block_tables.shape[1], q.stride(0), out.stride(0), float(scale), reach, float(softcap), _stream())
         operands = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), block_tables.data_ptr(), seg_of_token.data_ptr(), positions.data_ptr())
         for first, n in _runs(n_tiles, how.most_tiles) if how.tiled else ():

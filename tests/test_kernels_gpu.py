@@ -839,6 +839,24 @@ def test_attention_float32_cuts_tiles_and_single_rows_each_for_itself(K, monkeyp
     _close(alone, want, 3e-6)
 
 
+def test_attention_float32_lists_longer_than_a_launch_of_tiles(K, monkeypatch):
+    """Tiles beyond a grid's second dimension, nearly all of them of no tokens, beside single rows: both cut into chunks, and the launches of tiles, which share
+    the workspace, fold their own.  The bits of tokens one by one."""
+    n, T = 200, 150
+    k, v, q = (_rand((m, 1, 64), s, torch.float32) for m, s in ((n, 1), (n, 2), (T, 3)))
+    kc, vc, bt = _paged([k], [v], 64, 6, 4, torch.float32)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    args = (q.reshape(T, 64).to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), i32([0] * T), i32(list(range(n - T, n))), 1, 1, 64, 0.125)
+    alone = K.paged_attention(*args, max_total_len=n)
+    monkeypatch.setattr(K, "F32_ATTN_TILE_MIN", 0)
+    tiles = i32([[0, 0]] * 70000)
+    tiles[:9], tiles[-9:] = i32([[8 * a, 8] for a in range(9)]), i32([[72 + 8 * a, 8] for a in range(9)])
+    how = K.f32_attention(T, len(tiles), 6, 1, 1, 64, 64, n)
+    assert how.tiled and how.split_tiles and how.split_rows and how.most_tiles < len(tiles) and 8 * len(tiles) + 6 <= how.most
+    out = K.paged_attention(*args, max_total_len=n, tiles=tiles, single_rows=i32(list(range(144, T))))
+    assert torch.equal(out.cpu(), alone.cpu())
+
+
 @pytest.mark.parametrize("nh,nkv,d", [(32, 2, 128), (34, 2, 64), (10, 2, 64), (8, 2, 128), (3, 3, 64)])
 @pytest.mark.parametrize("split", [False, True])
 def test_attention_float32_gives_rows_of_no_request_zeros(K, monkeypatch, nh, nkv, d, split):
