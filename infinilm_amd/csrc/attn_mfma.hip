@@ -467,9 +467,9 @@ attn_merge_kernel(bf16* __restrict__ out, const float* __restrict__ ws_acc, cons
 
 // ------------------------------------------------------------------------------------------------
 // Tiles of up to ATT_TT consecutive tokens of one request (portions of prompts): the 4 waves of a
-// workgroup take 2 tokens (or groups of tokens) each and share every 64-key tile of K and V through LDS (the next tile is
-// already on its way: into registers, or, for heads of 128 and pages that hold whole tiles, straight
-// into a second pair of LDS buffers), so a tile is read from the cache once per 8 tokens x 16 heads.  No key chunks and no
+// workgroup take 2 tokens each (4 where a KV head has at most four heads, of two neighbouring tiles) and share every 64-key tile of K and V through LDS
+// (the next tile is already on its way: into registers, or, for heads of 128 and pages that hold whole tiles, straight
+// into a second pair of LDS buffers), so a tile is read from the cache once per 8 tokens x 16 heads, or 16 tokens x 4.  No key chunks and no
 // workspace: one workgroup walks all keys its tokens see, in ascending order of absolute key
 // index, 32 at a time.
 // ------------------------------------------------------------------------------------------------
@@ -483,9 +483,9 @@ __device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(
 // WF: see attn_mfma_kernel.  The 16 columns of the matrix instruction are CT tokens x 16 / CT heads, and a wave takes NT such groups.  9 to 16 heads: a token a
 // group, two groups a wave.  5 to 8: two tokens a group, one group a wave, so a tile of 8 tokens costs half the instructions that it costs with half of
 // the columns empty (2,048 tokens of 16 heads of 64 over 2 42.5 -> 33.1 us, of 128 55.6 -> 42.8, 37 tokens 7.2 -> 5.9; two groups a wave and 16 tokens a
-// workgroup 40.6, 52.3 and 7.8, better only for thousands of tokens over long contexts: 3,000 over 6,000 keys 144 against 175, 247 before).  Up to four:
-// four tokens a group, and a workgroup takes two neighbouring tiles, 16 tokens, where they are a run of a request (36 heads of 64, 2,048 tokens
-// 366 -> 121 us; 32 of 128 over 8 152 -> 59; 300 tokens 18.9 -> 9.2 and 13.9 -> 10.6).
+// workgroup 40.6, 52.3 and 7.8, better only for thousands of tokens over long contexts, for which there is no form: 3,000 over 6,000 keys 144 against 175,
+// 247 before).  Up to four: four tokens a group, and a workgroup takes two neighbouring tiles, 16 tokens, where they are a run of a request (36 heads of
+// 64, 2,048 tokens 366 -> 121 us; 32 of 128 over 8 152 -> 59; 300 tokens 18.9 -> 9.2 and 13.9 -> 10.6).
 template <int D16, bool PAGE64, bool WF, int CT>
 __global__ void __launch_bounds__(256, 2)
 attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16* __restrict__ kc,
@@ -730,7 +730,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
             __syncthreads();
         }
     };
-    // A tile that both tokens of the wave see whole (every tile but those on the diagonal and at a
+    // A tile that all tokens of the list's tile see whole (every tile but those on the diagonal and at a
     // window's edge) takes a path without masks, written so that matrix and vector instructions
     // alternate: a wave issues in order, so the vector work of one sub-tile has to stand between
     // the matrix instructions of another to run beside them.  While it issues matrix instructions a wave goes ahead of the unit's other ones
@@ -950,7 +950,7 @@ attn_tile_kernel(bf16* __restrict__ out, const bf16* __restrict__ q, const bf16*
 #pragma unroll
                 for (int j = 0; j < NT; ++j) s[sub][j][tau] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
-            // four independent accumulator chains (2 key tiles x 2 tokens), interleaved over d
+            // independent accumulator chains (2 key tiles x NT groups of tokens), interleaved over d
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks)
 #pragma unroll

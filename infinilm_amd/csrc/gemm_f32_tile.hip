@@ -13,8 +13,8 @@
 // the time), 4096 x 16384 1.42 against 2.67, 1024 x 1024 44 us against 106; 300 x 4608 x 4096 142 us against 416.
 // Tiles beyond whole rounds over the chip left most of it idle (288 tiles of 2048 x 4608 on 256 units: two rounds, the second an eighth full;
 // 300 x 4608 54 tiles): their eight slices of K go to as many workgroups, and a second kernel adds the slices' sums, 128 KB each, in their
-// order.  us, the best whole form before: 2048 x 4608 x 4096 578 -> 405, 300 x 4608 x 4096 144 -> 102, 100 x 4096 x 16384 391 -> 166, 2048 x 1024
-// x 4096 162 -> 106, 1024 x 2304 x 5760 262 -> 192.
+// order.  us, the best whole form and now: 2048 x 4608 x 4096 556 / 396, 300 x 4608 x 4096 142 / 98, 100 x 4096 x 16384 387 / 160, 2048 x 1024
+// x 4096 159 / 107, 1024 x 2304 x 5760 260 / 177.
 // K must be a multiple of 4 and rows 16-byte aligned.
 #include "f32_split.h"
 

@@ -17,7 +17,8 @@
 //                       plain form  x = rows in sorted order (or, with the list of pairs, the pairs' token rows), out = W_e x
 //                                   or the square of relu(W_e x)
 //                     bfloat16 on v_mfma_f32_16x16x32_bf16 (tiles of 64 rows x 64 outputs, operands through LDS in steps of
-//                     64 k, the next step's loads in flight), float32 and odd sizes by FMA in ascending k.
+//                     64 k, the next step's loads in flight; steps of up to 32 tokens: rows in registers, W streamed; from 96 pairs
+//                     an expert on: tiles of 128 rows), float32 and odd sizes by FMA in ascending k.
 //   ilm_moe_combine   (identity pairs take the token's row for out[place])
 //                     y[t] = sum over the token's slots of (weight of the pair *) out[place of (t, slot)] (+ shared[t] * sigmoid(sg[t])).
 //   ilm_glu_clamp     the experts' activation on fused [gate | up] rows of a dense product.

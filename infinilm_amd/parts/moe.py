@@ -9,8 +9,9 @@ The experts' matrices lie stacked in two tensors ([experts, 2 ff, hidden]: gate 
 checkpoint's tensors `e<j>.gate`, `e<j>.up`, `e<j>.down` are views into them.  The router's rows and the shared expert's
 weighing row are one float32-result product.  A step's (token, slot) pairs are ordered by expert on the device
 (`kernels.moe_route`) and the experts' products walk that order tile by tile (`kernels.moe_gemm`), so nothing depends on
-the host's view of the batch and a token's result does not depend on what else is in the step.  The shared expert is a
-dense feed-forward and takes the dense products.
+the host's view of the batch, and an expert's product of a row is one sum over k whatever else is in the step.  (In bfloat16 the
+number of a step's tokens chooses kernels: from 96 pairs an expert on average the score multiplies the float sums instead of the rounded
+input, which is the same but for rounding.)  The shared expert is a dense feed-forward and takes the dense products.
 """
 from __future__ import annotations
 
